@@ -83,7 +83,10 @@ LaunchPlan plan_launches(int T, int K, int E, int R, bool do_layout, bool do_mov
         MoveParams probe{};
         probe.T = T; probe.H = H; probe.row_bytes = row_bytes; probe.payload = payload; probe.do_expand = do_expand ? 1 : 0;
         probe.cast_pairs = tuning.cast_pairs; probe.copy_vecs = tuning.copy_vecs;
-        q.fused = dispatch_move_workgroups(probe) <= kMaxFusedMovers;
+        probe.K = K; probe.R = R; probe.fused = 1;
+        // BF16 rows from 300 MB on: 4096 x 7168 takes 78.7 us in one launch and 74.5 in two, 8192 x 7168 155 against 134, while
+        // 2048 x 7168 (154 MB) takes 40.2 against 44.3 and 16384 x 2048 top-6 (295 MB) 76.3 against 80.4.
+        q.fused = dispatch_move_workgroups(probe) <= kMaxFusedMovers && !copy_prefers_finished_layout(probe);
     }
     return q;
 }

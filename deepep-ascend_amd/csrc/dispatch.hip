@@ -20,6 +20,7 @@
 // before any mover can wait for them; every wait is bounded.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 
 #include "device_utils.h"
 #include "fp8_cast.h"
@@ -1268,18 +1269,68 @@ static int lds_bytes_per_cu() {
     return device_attribute(hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, cached, 160 * 1024);
 }
 
+// Destination rows of a token, on average, if the experts were chosen evenly: what decides how many stores follow a load.
+static double rows_per_token(const MoveParams& p) {
+    if (p.do_expand) return p.K;
+    return p.R * (1.0 - std::pow(1.0 - 1.0 / p.R, p.K));
+}
+
+// A call whose tokens go to nearly as many rows as they have selections (top-8 over 16 ranks: 6.4 rows): its stores are spread
+// over more buckets than those of eight ranks (5.3 rows).
+static bool many_rows_per_token(const MoveParams& p) { return rows_per_token(p) >= 5.8; }
+
+// The bytes of those rows.
+static double row_bytes_out(const MoveParams& p) {
+    const bool cast = p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8;
+    return double(p.T) * (cast ? p.H : p.row_bytes) * rows_per_token(p);
+}
+
+// Column tile of a move launch: 1024-channel segments per wavefront for the fused cast, KB of row per wavefront for
+// the pass-through payloads.
+static int move_tile(const MoveParams& p) {
+    const bool large_input = int64_t(p.T) * p.row_bytes >= (int64_t(64) << 20);
+    if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) {
+        // Two segments (2048 channels) measured best at hidden 7168 and 8 ranks: 92.8 us per dispatch against 93.7 (4
+        // segments) and 96.9 (7 segments, one wavefront per token).  With many rows per token one segment is ahead on a
+        // finished layout (16384 x 7168: 32 ranks 199 against 207 us, 16 ranks 185 against 189; 8192 x 7168 expanded 118
+        // against 124 us); in a single launch, whose workgroups each work out the row bases, only for the expanded layout
+        // of a large call.
+        if (p.cast_pairs != 0) return p.cast_pairs;
+        if (p.H <= 1024) return 1;
+        return (p.fused ? p.do_expand && large_input : many_rows_per_token(p)) ? 1 : 2;
+    }
+    if (p.copy_vecs != 0) return p.copy_vecs;
+    const int kb = (p.row_bytes + 1023) / 1024;
+    const int widest = kb <= 1 ? 1 : kb <= 2 ? 2 : 4;
+    // Small, latency-bound calls: up to 4 KB per wavefront, so that fewer wavefronts repeat the routing work (4096 rows
+    // of 4 KB: 19.5 us against 21.1 us with 1 KB tiles).  Calls that write a quarter of a gigabyte and more are bound by
+    // their stores: one KB per wavefront where a token goes to four rows and more (BF16, 8 ranks: 4096 x 7168 66.5
+    // against 73.4 us, 8192 x 7168 126 against 145, 16384 x 2048 top-6 69.5 against 74.1), two where it goes to fewer (8192 x 7168, 4 of
+    // 4 ranks: 75.6 us with four workgroups per CU against 79.4 with 1 KB and 84.9 with 4 KB; 4096 x 7168, 2 of 2 ranks,
+    // 88 MB of rows: 28.4 against 31.0 and 28.8).
+    if (p.fused) return large_input ? 1 : widest;
+    if (row_bytes_out(p) < 256e6) return widest;
+    return rows_per_token(p) >= 4.0 ? 1 : (kb >= 2 ? 2 : 1);
+}
+
 // How many workgroups of a move kernel launched on a finished layout a CU should hold at a time (0: as many as fit).
-// The fused cast streams fastest with fewer than the eight its registers allow - measured side by side at 8192 x 7168,
-// move phase in us with 8 / 7 / 6 / 5 / 4 per CU: compact layout 82.6 / 81.6 / 81.7 / 82.0 / 83.6 (16384 tokens: 162.5 with
-// eight, 156.5 with six), expanded layout 114.9 / 115.1 / 114.7 / 113.4 / 116.0 - while the BF16 copy does not care down
-// to six and loses 3 us at five.  Launches that would not fill two rounds of eight per CU are left alone.
+// Scattered stores stream fastest when not too many are under way.  Move phase in us, inputs read from memory, with
+// 8 / 6 / 5 / 4 / 3 workgroups per CU:
+//   fused cast, 8192 x 7168, 8 ranks           81.4 / 80.8 / 80.6 / 82.2;   expanded 119.9 / 120.0 / 118.4 / 119.0
+//   fused cast, 16384 x 7168, 32 ranks, 1 KB   212 / 201 / 199 / 203 / 228; 16384 x 4096, 64 ranks 150 / 133 / 130 / 134 / 153
+//   BF16, 16384 x 7168, 32 ranks, 1 KB         363 / 362 / 354 / 346 / 385; 16 ranks 312 / 312 / 304 / 314 / 357
+//   BF16, 16384 x 4096, 64 ranks, 1 KB         264 / 237 / 222 / 239 / 276
+//   BF16, 8192 x 7168, 8 ranks, 1 KB           126 / 126 / 128 / 137 / 151: left alone
+//   BF16, 8192 x 7168, 4 of 4 ranks, 2 KB       82 /  80 /  77 /  76;       16384 x 4096, 4 of 16 ranks 123 / 124 / 123 / 119 / 117
+// Launches that would not fill two rounds of eight per CU are left alone.
 static int move_workgroups_per_cu(const MoveParams& p) {
     if (p.fused) return 0;
     if (p.move_workgroups_per_cu != 0)       // two is the least an LDS share within a workgroup's 64 KB can enforce
         return p.move_workgroups_per_cu >= 8 ? 0 : (p.move_workgroups_per_cu < 2 ? 2 : p.move_workgroups_per_cu);
-    if (p.payload != DEEP_EP_HIP_PAYLOAD_CAST_FP8) return 0;
     if (int64_t(p.num_movers) < int64_t(compute_units()) * 16) return 0;
-    return p.do_expand ? 5 : 6;
+    if (many_rows_per_token(p)) return 5;
+    if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) return 6;
+    return move_tile(p) == 2 ? 4 : 0;
 }
 
 size_t move_lds_bytes(const MoveParams& p) {
@@ -1366,27 +1417,9 @@ int compute_units() {
     return device_attribute(hipDeviceAttributeMultiprocessorCount, cached, 256);
 }
 
-// Column tile of a move launch: 1024-channel segments per wavefront for the fused cast, KB of row per wavefront for
-// the pass-through payloads.
-static int move_tile(const MoveParams& p) {
-    if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) {
-        // Two segments (2048 channels, 8 wavefronts per SIMD) measured best at hidden 7168: 92.8 us per dispatch
-        // against 93.7 (4 segments) and 96.9 (7 segments, one wavefront per token).
-        // The expanded layout stores eight rows per token instead of five: in a large call (64 MB of input and more)
-        // one segment per wavefront is ahead there (8192 x 7168: move phase 119 us against 122 us, whole call 130
-        // against 131 us).
-        if (p.cast_pairs != 0) return p.cast_pairs;
-        const bool large = int64_t(p.T) * p.row_bytes >= (int64_t(64) << 20);
-        return (p.H <= 1024 || (p.do_expand && large)) ? 1 : 2;
-    }
-    // Large, bandwidth-bound calls: one 1 KB segment per wavefront measured best for this write-heavy stream (8192
-    // BF16 rows of 14 KB: 143 us per dispatch against 155-159 us with 2, 4, 7 or 8 segments).  Small, latency-bound
-    // calls: up to 4 KB per wavefront, so that fewer wavefronts repeat the routing work (4096 rows of 4 KB: 26 us
-    // against 32 us with 1 KB segments).
-    if (p.copy_vecs != 0) return p.copy_vecs;
-    const int kb = (p.row_bytes + 1023) / 1024;
-    const bool large = int64_t(p.T) * p.row_bytes >= (int64_t(64) << 20);
-    return large ? 1 : (kb <= 1 ? 1 : kb <= 2 ? 2 : 4);
+// More rows than this are copied in two launches: see plan_launches.
+bool copy_prefers_finished_layout(const MoveParams& p) {
+    return p.payload != DEEP_EP_HIP_PAYLOAD_CAST_FP8 && row_bytes_out(p) >= 300e6;
 }
 
 int64_t dispatch_move_workgroups(const MoveParams& p) {
