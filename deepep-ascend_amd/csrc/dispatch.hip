@@ -707,6 +707,11 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
         if (has_work && off < p.row_bytes) v[i] = load16_stream(src + off);
     }
 
+    // The caller's scale packs ride with tile 0: requested with the payload, once, not per destination row.
+    const bool packs = has_work && tile == 0 && p.recv_sf != nullptr;
+    uint32_t pack = 0;
+    if (packs && lane < p.num_sf_packs) pack = p.sf[int64_t(t) * p.sf_ts + int64_t(lane) * p.sf_hs];
+
     const RouteInputs route_in = load_route_inputs(p, t, lane);
     const int* flat_bases = nullptr;
     uint32_t word;
@@ -744,10 +749,11 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
             const int off = (tile * kVecs + i) * 1024 + lane * 16;
             if (off < p.row_bytes) store16_stream(dst + off, v[i]);
         }
-        if (tile == 0 && p.recv_sf != nullptr) {
-            for (int g = lane; g < p.num_sf_packs; g += kWaveSize)
-                p.recv_sf[int64_t(row) * p.rsf_ts + int64_t(g) * p.rsf_hs] =
-                    p.sf[int64_t(t) * p.sf_ts + int64_t(g) * p.sf_hs];
+        if (packs) {
+            uint32_t* to = p.recv_sf + int64_t(row) * p.rsf_ts;
+            if (lane < p.num_sf_packs) to[int64_t(lane) * p.rsf_hs] = pack;
+            for (int g = lane + kWaveSize; g < p.num_sf_packs; g += kWaveSize)        // rows beyond 8192 channels
+                to[int64_t(g) * p.rsf_hs] = p.sf[int64_t(t) * p.sf_ts + int64_t(g) * p.sf_hs];
         }
     }
 }
