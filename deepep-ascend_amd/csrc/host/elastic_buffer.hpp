@@ -222,7 +222,14 @@ public:
         args.tuning = process_tuning();
         void* stream_ptr = run.stream();
 
-        // Sizes of the outputs
+        // Sizes of the outputs.  With a CPU sync they are exact: known before the move is launched, or, for outputs small enough
+        // to be allocated at their bound, read from the mailbox once it is (allocation and launch run beside the layout).
+        const int64_t row_bound = int64_t(num_tokens) * std::min(num_topk, R);
+        const bool up_front = do_cpu_sync and not cached_mode and not do_expand and num_tokens > 0 and
+                              not previous_event_before_epilogue.has_value() and
+                              not (sf_dtype.has_value() and use_tma_aligned_col_major_sf) and      // its strides follow the row count
+                              row_bound * hidden * int64_t(c10::elementSize(out_dtype)) <= kUpFrontRowBytes;
+        int32_t* box = nullptr;
         int num_recv_tokens, num_expanded_tokens;
         std::vector<int> per_expert_list;
         if (cached_mode) {
@@ -230,23 +237,15 @@ public:
             num_expanded_tokens = *cached_num_expanded_tokens;
             per_expert_list = *cached_num_recv_tokens_per_expert_list;
         } else if (do_cpu_sync) {
-            // layout launch, then the host waits for the counts in its mailbox (no copy, no device synchronisation)
-            int32_t* box = fresh_mailbox(R + num_experts + 1);
+            // layout launch, which leaves the counts in the host's mailbox (no copy, no device synchronisation)
+            box = fresh_mailbox(R + num_experts + 1);
             args.phases = DEEP_EP_HIP_PHASE_LAYOUT;
             args.host_counts = box;
             check_abi(deep_ep_hip_launch_dispatch(&args, stream_ptr), "dispatch layout");
             args.host_counts = nullptr;
-            if (not await_mailbox(box, R + num_experts + 1, num_cpu_timeout_secs_))
-                throw EPException("DeepEP HIP backend: dispatch: timed out waiting for the layout counts");
-            if (box[R + num_experts] != 0) {
-                c10::hip::HIPStreamGuardMasqueradingAsCUDA on_run(run);
-                read_and_clear_status(workspace, "dispatch");          // raises, and leaves the workspace ready again
-            }
-            num_recv_tokens = 0;
-            for (int r = 0; r < R; ++r) num_recv_tokens += box[r];
+            num_recv_tokens = static_cast<int>(row_bound);
             num_expanded_tokens = 0;
-            per_expert_list.assign(box + R, box + R + num_experts);         // aligned counts
-            for (int e = 0; e < num_experts; ++e) num_expanded_tokens += per_expert_list[e];
+            if (not up_front) read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
         } else {
             num_recv_tokens = num_max_tokens_per_rank * R;
             num_expanded_tokens = num_max_tokens_per_rank * std::min(num_topk, num_experts) + (expert_alignment - 1) * num_experts;
@@ -257,14 +256,14 @@ public:
         torch::Tensor recv_x, recv_src_metadata;
         std::optional<torch::Tensor> recv_sf, recv_topk_idx, recv_topk_weights;
         int64_t rsf_ts = 0, rsf_hs = 0;
+        // what travels beside the payload (scales, indices, weights), in one allocation; the payload and the
+        // handle's metadata stay on their own, because callers keep them for different spans
+        TensorPack beside(device_);
+        int i_sf = -1, i_idx = -1, i_w = -1;
         {
             c10::hip::HIPStreamGuardMasqueradingAsCUDA on_run(run);
             recv_x = torch::empty({num_allocated, hidden}, torch::TensorOptions().dtype(out_dtype).device(device_));
             recv_src_metadata = cached_mode ? *cached_recv_src_metadata : torch::empty({num_recv_tokens, num_topk + 2}, i32);
-            // what travels beside the payload (scales, indices, weights), in one allocation; the payload and the
-            // handle's metadata stay on their own, because callers keep them for different spans
-            TensorPack beside(device_);
-            int i_sf = -1, i_idx = -1, i_w = -1;
             if (sf_dtype.has_value()) {
                 if (not use_tma_aligned_col_major_sf) {
                     rsf_ts = num_sf_packs; rsf_hs = 1;
@@ -294,6 +293,14 @@ public:
         args.recv_capacity = recv_src_metadata.size(0);
         args.expanded_capacity = do_expand ? num_expanded_tokens : 0;
         check_abi(deep_ep_hip_launch_dispatch(&args, stream_ptr), "dispatch");
+        if (up_front) {
+            read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
+            recv_x = first_rows(recv_x, num_recv_tokens);
+            recv_src_metadata = first_rows(recv_src_metadata, num_recv_tokens);
+            if (i_sf >= 0) recv_sf = beside.get(i_sf, num_recv_tokens);
+            if (i_idx >= 0) recv_topk_idx = beside.get(i_idx, num_recv_tokens);
+            if (i_w >= 0) recv_topk_weights = beside.get(i_w, num_recv_tokens);
+        }
         if (not cached_mode) slots_of_handle_.remember(recv_src_metadata, dst_slot);
 
         std::optional<EventHandle> event = scope.finish(
@@ -398,6 +405,23 @@ public:
     // V1 `get_dispatch_layout` on this buffer is inherited from HostRuntime.
 
 private:
+    // Waits for the counts of a layout in its mailbox; raises if a kernel flagged the routing.
+    void read_counts(int32_t* box, int num_experts, const Stream& run, const torch::Tensor& workspace, int& num_recv_tokens,
+                     int& num_expanded_tokens, std::vector<int>& per_expert_list) {
+        const int R = num_ranks_;
+        if (not await_mailbox(box, R + num_experts + 1, num_cpu_timeout_secs_))
+            throw EPException("DeepEP HIP backend: dispatch: timed out waiting for the layout counts");
+        if (box[R + num_experts] != 0) {
+            c10::hip::HIPStreamGuardMasqueradingAsCUDA on_run(run);
+            read_and_clear_status(workspace, "dispatch");          // raises, and leaves the workspace ready again
+        }
+        num_recv_tokens = 0;
+        for (int r = 0; r < R; ++r) num_recv_tokens += box[r];
+        num_expanded_tokens = 0;
+        per_expert_list.assign(box + R, box + R + num_experts);         // aligned counts
+        for (int e = 0; e < num_experts; ++e) num_expanded_tokens += per_expert_list[e];
+    }
+
     int64_t num_buffer_bytes_;
     bool allow_hybrid_mode_, allow_multiple_reduction_, prefer_overlap_with_compute_;
     int num_cpu_timeout_secs_;

@@ -204,8 +204,22 @@ public:
         args.workspace = workspace.data_ptr(); args.workspace_bytes = static_cast<uint64_t>(workspace.numel());
         void* stream_ptr = run.stream();
 
+        // With top-k tensors and outputs small enough to be allocated at their bound, the exact counts are read from the mailbox
+        // once the move is launched (see kUpFrontRowBytes).
+        const int64_t row_bound = int64_t(num_tokens) * std::min(num_topk, R);
+        const bool up_front = not cached_mode and num_worst_tokens == 0 and topk_idx.has_value() and num_tokens > 0 and
+                              row_bound * hidden * int64_t(x.element_size()) <= kUpFrontRowBytes;
+        int32_t* box = nullptr;
         int num_recv_tokens;
         std::vector<int> per_expert_list;
+        const auto read_counts = [&] {
+            if (not await_mailbox(box, R + num_experts + 1, 300))
+                throw EPException("DeepEP HIP backend: dispatch: timed out waiting for the layout counts");
+            if (box[R + num_experts] != 0) read_and_clear_status(workspace, "dispatch");      // raises
+            num_recv_tokens = 0;
+            for (int r = 0; r < R; ++r) num_recv_tokens += box[r];
+            per_expert_list.assign(box + R, box + R + num_experts);                           // aligned counts
+        };
         torch::Tensor rank_prefix_matrix, channel_prefix_matrix, recv_channel_prefix_matrix, send_head, recv_src_idx, counts;
         if (cached_mode) {
             num_recv_tokens = cached_num_recv_tokens;
@@ -244,19 +258,15 @@ public:
                 // (csrc/legacy/buffer.hpp:580-600).  With top-k tensors they arrive in the pinned mailbox; without,
                 // the per-expert counts are the caller's tensor and are copied back with the per-rank ones.
                 args.phases = DEEP_EP_HIP_PHASE_LAYOUT;
-                per_expert_list.resize(num_experts);
                 if (topk_idx.has_value()) {
-                    int32_t* box = fresh_mailbox(R + num_experts + 1);
+                    box = fresh_mailbox(R + num_experts + 1);
                     args.host_counts = box;
                     check_abi(deep_ep_hip_launch_intranode_dispatch(&args, stream_ptr), "intranode dispatch layout");
                     args.host_counts = nullptr;
-                    if (not await_mailbox(box, R + num_experts + 1, 300))
-                        throw EPException("DeepEP HIP backend: dispatch: timed out waiting for the layout counts");
-                    if (box[R + num_experts] != 0) read_and_clear_status(workspace, "dispatch");      // raises
-                    num_recv_tokens = 0;
-                    for (int r = 0; r < R; ++r) num_recv_tokens += box[r];
-                    std::copy(box + R, box + R + num_experts, per_expert_list.begin());               // aligned counts
+                    num_recv_tokens = static_cast<int>(row_bound);
+                    if (not up_front) read_counts();
                 } else {
+                    per_expert_list.resize(num_experts);
                     check_abi(deep_ep_hip_launch_intranode_dispatch(&args, stream_ptr), "intranode dispatch layout");
                     const torch::Tensor host = torch::cat({counts.slice(0, 0, R), *num_tokens_per_expert}).cpu();
                     const int32_t* h = host.data_ptr<int32_t>();
@@ -286,6 +296,14 @@ public:
         args.recv_topk_idx = ptr_of<int64_t>(recv_topk_idx); args.recv_topk_weights = ptr_of<float>(recv_topk_weights);
         args.recv_capacity = num_recv_tokens;
         check_abi(deep_ep_hip_launch_intranode_dispatch(&args, stream_ptr), "intranode dispatch");
+        if (up_front) {
+            read_counts();
+            recv_x = first_rows(recv_x, num_recv_tokens);
+            recv_src_idx = first_rows(recv_src_idx, num_recv_tokens);
+            recv_topk_idx = first_rows(*recv_topk_idx, num_recv_tokens);
+            recv_topk_weights = first_rows(*recv_topk_weights, num_recv_tokens);
+            if (recv_x_scales.has_value()) recv_x_scales = first_rows(*recv_x_scales, num_recv_tokens);
+        }
         if (not cached_mode) send_head_of_handle_.remember(rank_prefix_matrix, send_head);
 
         std::optional<EventHandle> event = scope.finish(

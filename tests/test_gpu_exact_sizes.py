@@ -1,0 +1,43 @@
+"""Exact-size dispatches on either side of the size up to which outputs are allocated at their bound (256 MiB of rows) before
+the counts are known: the tensors have the exact number of rows, are contiguous, and hold the tokens they should."""
+import pytest
+import torch
+
+import routing_cases as rc
+import routing_oracle as oracle
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {"at_the_limit": (2048, 8192, 8), "past_the_limit": (2049, 8192, 8), "one_token": (1, 1024, 8), "one_rank": (300, 1024, 1)}
+
+
+@pytest.mark.parametrize("surface", ["elastic", "legacy"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_exact_rows(shape, surface):
+    import deep_ep
+    T, H, R = SHAPES[shape]
+    E, K = 64, 8
+    small = rc.small(shape, T, 16, E, R, K, seed=60, masked_ratio=0.1)
+    ref = oracle.dispatch(small.x, small.topk_idx, small.topk_weights, E, R, 0, T)
+    x = torch.randn((T, H), generator=torch.Generator(device="cuda").manual_seed(61), device="cuda", dtype=torch.bfloat16)
+    idx, w = small.topk_idx.cuda(), small.topk_weights.cuda()
+    group = deep_ep.LogicalGroup(0, R)
+    for _ in range(2):
+        if surface == "elastic":
+            buf = deep_ep.ElasticBuffer(group, num_max_tokens_per_rank=T, hidden=H, num_topk=K)
+            recv_x, recv_idx, recv_w, handle, _ = buf.dispatch(x, idx, w, num_experts=E)
+            tokens, per_expert = handle.recv_src_metadata[:, 0].long(), handle.num_recv_tokens_per_expert_list
+            assert handle.num_recv_tokens == ref.num_recv_tokens
+            assert torch.equal(recv_w.cpu(), ref.recv_topk_weights)
+        else:
+            buf = deep_ep.Buffer(group)
+            per_rank, _, counts, in_rank, _ = buf.get_dispatch_layout(idx, E)
+            recv_x, recv_idx, recv_w, per_expert, handle, _ = buf.dispatch(
+                x, num_tokens_per_rank=per_rank, is_token_in_rank=in_rank, num_tokens_per_expert=counts, topk_idx=idx, topk_weights=w)
+            tokens = handle[3].long()
+        assert recv_x.shape == (ref.num_recv_tokens, H) and recv_x.is_contiguous()
+        assert recv_idx.shape == recv_w.shape == (ref.num_recv_tokens, K) and recv_idx.is_contiguous() and recv_w.is_contiguous()
+        assert torch.equal(recv_idx.cpu(), ref.recv_topk_idx)
+        assert list(per_expert) == ref.num_unaligned_recv_tokens_per_expert.tolist()
+        assert torch.equal(tokens.cpu().int(), ref.recv_src_metadata[:, 0])
+        assert torch.equal(recv_x, x[tokens])
