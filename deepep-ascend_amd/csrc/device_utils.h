@@ -131,14 +131,20 @@ __device__ __forceinline__ int row16_sum(int v) {
     return v;
 }
 
-// Inclusive prefix sum across the wave.
+// Inclusive prefix sum across the wave, as DPP operand modifiers: inside each row of 16 lanes by shifts of 1, 2, 4 and 8,
+// then the last lane of row 0 / 2 into row 1 / 3 and lane 31 into the upper half (bpermutes through LDS, as a shuffle
+// compiles to, took six dependent trips).  All lanes of the wavefront must be active.
+template <int kCtrl, int kRowMask, int kBankMask>
+__device__ __forceinline__ int dpp_or_zero(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, kBankMask, false);
+}
 __device__ __forceinline__ int wave_inclusive_sum(int v) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int off = 1; off < kWaveSize; off <<= 1) {
-        int o = __shfl_up(v, off, kWaveSize);
-        if (lane >= off) v += o;
-    }
+    v += dpp_or_zero<0x111, 0xf, 0xf>(v);      // row_shr:1
+    v += dpp_or_zero<0x112, 0xf, 0xf>(v);      // row_shr:2
+    v += dpp_or_zero<0x114, 0xf, 0xf>(v);      // row_shr:4
+    v += dpp_or_zero<0x118, 0xf, 0xf>(v);      // row_shr:8
+    v += dpp_or_zero<0x142, 0xa, 0xf>(v);      // row_bcast:15 into rows 1 and 3
+    v += dpp_or_zero<0x143, 0xc, 0xf>(v);      // row_bcast:31 into rows 2 and 3
     return v;
 }
 
@@ -171,6 +177,10 @@ __device__ __forceinline__ int load_agent(const int* p) {
 }
 __device__ __forceinline__ void store_agent(int* p, int v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A word the host polls in pinned memory: stored past every cache at once.
+__device__ __forceinline__ void store_system(int* p, int v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // kThrough: an agent-scope (write-through) store; otherwise an ordinary one.
 template <bool kThrough>

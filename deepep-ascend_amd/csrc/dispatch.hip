@@ -313,7 +313,7 @@ __device__ __forceinline__ unsigned movers_of_gate(const MoveParams& p, unsigned
 __device__ __forceinline__ void fused_count_block(const MoveParams& p) {
     extern __shared__ uint64_t count_lds[];
     const int c = int(blockIdx.x);
-    count_chunk<8, true>(p.lay, c, p.count_blocks, count_lds);
+    count_chunk<8, true>(p.lay, c, p.count_blocks, count_lds, nullptr, [] {});
     wait_for_own_stores();
     __syncthreads();
     if (threadIdx.x == 0) store_agent(p.chunk_done + c, 1);      // for the publisher
@@ -370,7 +370,7 @@ __device__ __forceinline__ void fused_publish_block(const MoveParams& p) {
     // with ordinary loads, the rank table (lines shared by the writers of 16 chunks) at agent scope.
     await_and_clear_flags(p, p.chunk_done, p.count_blocks);
     sum_expert_columns<kThreads>(tab, p.R, p.E, p.count_blocks, lds.totals);
-    publish_experts<kThreads>(p.pub, lds);
+    publish_experts<kThreads>(p.pub, lds, status_for_host(p.pub));
     if (p.do_expand && !bases_first) {
         __syncthreads();
         write_expert_bases<kThreads, true>(tab, tagged_bases, tag, p.E, p.count_blocks, lds);

@@ -21,15 +21,19 @@ namespace deep_ep_hip {
 static_assert(kLayoutChunk == 4 * kWaveSize, "the packed before-wave word holds three fields");
 
 // LDS the counting step needs: the bitmap words [(R + E)][4] and one packed word per bucket (see below).
-inline size_t count_lds_bytes(int R, int E) {
+__host__ __device__ inline size_t count_lds_bytes(int R, int E) {
     return size_t(R + E) * (kLayoutChunk / kWaveSize) * sizeof(uint64_t) + size_t(R + E) * sizeof(uint32_t);
 }
 
 // bitmap: LDS of count_lds_bytes(R, E) bytes.  Must be called by all 256 threads of the workgroup.
-// kThrough: positions and chunk totals are stored at agent scope (workgroups of the same launch read them); the
-// position words and the copy of the rank totals in p.tagged_rank carry the launch's tag.
-template <int KMAX, bool kThrough>
-__device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chunk, const int num_chunks, uint64_t* bitmap) {
+// kThrough: positions are stored at agent scope (workgroups of the same launch read them) and carry, like the copy of
+// the rank totals in p.tagged_rank, the launch's tag.  Chunk totals always go out at agent scope, to the count tables,
+// unless `lds_totals` is given: then the call's only chunk leaves them there ([R + E]).
+// hand_off() is called by all threads once the totals and the flags are on their way and before the positions are
+// stored: whoever waits for the totals does not wait for those.
+template <int KMAX, bool kThrough, typename HandOff>
+__device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chunk, const int num_chunks, uint64_t* bitmap,
+                                            int* lds_totals, HandOff hand_off) {
     constexpr int kThreads = kLayoutChunk;
     constexpr int kWaves = kThreads / kWaveSize;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -63,8 +67,17 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
             for (int k = 0; k < KMAX; ++k) raw[k] = -1;
         }
     } else {
+        // clamped columns instead of a branch around each load: all of a token's loads go out together
 #pragma unroll
-        for (int k = 0; k < KMAX; ++k) raw[k] = (active && k < p.K) ? p.topk_idx[int64_t(t) * p.K + k] : int64_t(-1);
+        for (int k = 0; k < KMAX; ++k) raw[k] = -1;
+        if (active) {
+            const int64_t* row = p.topk_idx + int64_t(t) * p.K;
+#pragma unroll
+            for (int k = 0; k < KMAX; ++k) raw[k] = row[min(k, p.K - 1)];
+#pragma unroll
+            for (int k = 0; k < KMAX; ++k)
+                if (k >= p.K) raw[k] = -1;
+        }
     }
 
     for (int i = tid; i < n * kWaves; i += kThreads) bitmap[i] = 0ull;
@@ -73,11 +86,13 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
     // Straight-line code from here on, no branch per routing lane: the LDS atomics of all lanes issue back to back, and
     // so do the LDS reads of the position step further down.  A lane without an expert ORs nothing into a word of its
     // own (not one word for all of them: atomics of one wavefront on one address take turns).
-    // With few ranks most lanes of a wavefront would meet on the same few rank words, so the rank bitmaps are taken by
-    // ballot instead: one per rank over "this token goes to rank r", no atomics.
-    constexpr int kBallotRanks = 16;
+    // Up to 64 ranks many lanes of a wavefront would meet on the same few rank words, so the rank bitmaps are taken by
+    // ballot instead: one per rank over "this token goes to rank r", no atomics (by atomics
+    // the bits took 3.5 us to set at 32 ranks, against 1.1 us by ballot at 8).
+    constexpr int kBallotRanks = 64;
     const bool ranks_by_ballot = p.R <= kBallotRanks;
     int e[KMAX], d[KMAX];
+    unsigned long long seen = 0;
     int flags = 0;
     const float rcp_experts_per_rank = 1.0f / float(p.E_l);
     const uint64_t my_bit = 1ull << lane;
@@ -85,12 +100,16 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
     uint64_t my_ranks = 0;                       // bit r: this token goes to rank r
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) {
-        const bool valid = raw[k] >= 0 && raw[k] < p.E;
-        if (raw[k] >= p.E) flags |= DEEP_EP_HIP_STATUS_EXPERT_OUT_OF_RANGE;
-        e[k] = valid ? int(raw[k]) : -1;
+        const uint32_t lo = uint32_t(raw[k]);
+        const int hi = int(raw[k] >> 32);
+        const bool valid = hi == 0 && lo < uint32_t(p.E);
+        if (hi >= 0 && !valid) flags |= DEEP_EP_HIP_STATUS_EXPERT_OUT_OF_RANGE;
+        e[k] = valid ? int(lo) : -1;
         d[k] = valid ? small_div(e[k], rcp_experts_per_rank) : -1;
         const uint64_t bit = valid ? my_bit : 0ull;
-        atomicOr(reinterpret_cast<unsigned long long*>(&bitmap[valid ? (p.R + e[k]) * kWaves + wave : idle_word]), bit);
+        unsigned long long* word = reinterpret_cast<unsigned long long*>(&bitmap[valid ? (p.R + e[k]) * kWaves + wave : idle_word]);
+        if constexpr (kThrough) atomicOr(word, bit);          // see the pairwise comparison below
+        else seen |= atomicOr(word, bit) & bit;              // a bit that is set already: the token names the expert twice
         if (valid) my_ranks |= 1ull << (d[k] & 63);            // used when num_ranks <= kBallotRanks
     }
     if (ranks_by_ballot) {
@@ -106,11 +125,15 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
             atomicOr(reinterpret_cast<unsigned long long*>(&bitmap[d[k] >= 0 ? d[k] * kWaves + wave : idle_word]),
                      d[k] >= 0 ? my_bit : 0ull);
     }
-    if (p.copied_topk_idx != nullptr && active) {
+    // The caller's copy of the indices: behind the hand-off, unless the registers they would occupy until then are scarce
+    // (the counting workgroups of a single launch are held to those of its movers).
+    auto copy_indices = [&] {
+        if (p.copied_topk_idx == nullptr || !active) return;
 #pragma unroll
         for (int k = 0; k < KMAX; ++k)
             if (k < p.K) p.copied_topk_idx[int64_t(t) * p.K + k] = raw[k];
-    }
+    };
+    if constexpr (kThrough) copy_indices();
     __syncthreads();
 
     // Per bucket: the chunk total goes out and the bits set by the wavefronts before each wavefront are packed into one LDS word (three 10-bit fields),
@@ -120,9 +143,13 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
         const int c0 = __popcll(bitmap[j * kWaves]), c1 = __popcll(bitmap[j * kWaves + 1]);
         const int c2 = __popcll(bitmap[j * kWaves + 2]), c3 = __popcll(bitmap[j * kWaves + 3]);
         before_wave[j] = uint32_t(c0) | (uint32_t(c0 + c1) << 10) | (uint32_t(c0 + c1 + c2) << 20);
+        if (!kThrough && lds_totals != nullptr) {
+            lds_totals[j] = c0 + c1 + c2 + c3;
+            continue;
+        }
         int32_t* at = j < p.R ? p.tab.rank_counts + int64_t(j) * p.tab.chunks_padded + chunk
                               : p.tab.expert_counts + int64_t(chunk) * p.tab.experts_padded + (j - p.R);
-        store_word<kThrough>(at, c0 + c1 + c2 + c3);
+        store_agent(at, c0 + c1 + c2 + c3);
         if constexpr (kThrough) {
             if (j < p.R && p.tagged_rank != nullptr)
                 store_agent(reinterpret_cast<int*>(p.tagged_rank) + j * p.tab.chunks_padded + chunk, int(uint32_t(c0 + c1 + c2 + c3) | tag));
@@ -132,10 +159,10 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
         }
     }
     const int pad = p.tab.chunks_padded - num_chunks;  // the padding columns of the rank table are cleared by the first workgroup
-    if (chunk == 0) {
+    if (chunk == 0 && lds_totals == nullptr) {
         for (int i = tid; i < p.R * pad; i += kThreads) {
             const int at = (i / pad) * p.tab.chunks_padded + num_chunks + i % pad;
-            store_word<kThrough>(p.tab.rank_counts + at, 0);
+            store_agent(p.tab.rank_counts + at, 0);
             if constexpr (kThrough)
                 if (p.tagged_rank != nullptr) store_agent(reinterpret_cast<int*>(p.tagged_rank) + at, int(tag));
         }
@@ -150,83 +177,90 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
         return uint32_t(__popcll(word & below)) + ((before >> wave_shift) & earlier_mask);
     };
 
-    if (active) {
-        if (p.pos != nullptr) {
-            // One word per (token, lane): the slot of the token inside its chunk for the lane's destination rank
-            // (master lanes only) and the position of the lane inside its chunk for its expert (kernels.h).
-            uint32_t packed[KMAX];
-            uint64_t word_r[KMAX];
-            uint32_t before_r[KMAX];
+    uint32_t packed[KMAX];
+    if (active && p.pos != nullptr) {
+        // One word per (token, lane): the slot of the token inside its chunk for the lane's destination rank
+        // (master lanes only) and the position of the lane inside its chunk for its expert (kernels.h).
+        uint64_t word_r[KMAX];
+        uint32_t before_r[KMAX];
+#pragma unroll
+        for (int k = 0; k < KMAX; ++k) {
+            const int bucket = d[k] >= 0 ? d[k] : 0;
+            word_r[k] = bitmap[bucket * kWaves + wave];
+            before_r[k] = before_wave[bucket];
+        }
+        // The master lane of a destination rank is the last lane that names it.
+        bool master[KMAX];
+        if (p.R <= 64) {
+            // walk the lanes backwards with the set of ranks seen so far
+            uint64_t later_ranks = 0;
+#pragma unroll
+            for (int k = KMAX - 1; k >= 0; --k) {
+                const uint64_t rank_bit = d[k] >= 0 ? 1ull << (d[k] & 63) : 0ull;
+                master[k] = (rank_bit & ~later_ranks) != 0;
+                later_ranks |= rank_bit;
+            }
+        } else {
 #pragma unroll
             for (int k = 0; k < KMAX; ++k) {
-                const int bucket = d[k] >= 0 ? d[k] : 0;
-                word_r[k] = bitmap[bucket * kWaves + wave];
-                before_r[k] = before_wave[bucket];
+                master[k] = d[k] >= 0;
+#pragma unroll
+                for (int j = k + 1; j < KMAX; ++j)
+                    if (d[j] == d[k]) master[k] = false;
             }
-            // The master lane of a destination rank is the last lane that names it.
-            bool master[KMAX];
-            if (p.R <= 64) {
-                // walk the lanes backwards with the set of ranks seen so far
-                uint64_t later_ranks = 0;
+        }
 #pragma unroll
-                for (int k = KMAX - 1; k >= 0; --k) {
-                    const uint64_t rank_bit = d[k] >= 0 ? 1ull << (d[k] & 63) : 0ull;
-                    master[k] = (rank_bit & ~later_ranks) != 0;
-                    later_ranks |= rank_bit;
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < KMAX; ++k) {
-                    master[k] = d[k] >= 0;
-#pragma unroll
-                    for (int j = k + 1; j < KMAX; ++j)
-                        if (d[j] == d[k]) master[k] = false;
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < KMAX; ++k) {
+        for (int k = 0; k < KMAX; ++k) {
+            if constexpr (kThrough) {      // a mover's register budget does not hold eight answers of the LDS: compared pairwise
 #pragma unroll
                 for (int j = k + 1; j < KMAX; ++j)
                     if (e[k] >= 0 && e[j] == e[k]) flags |= DEEP_EP_HIP_STATUS_DUPLICATE_EXPERT;
-                packed[k] = (master[k] ? position(word_r[k], before_r[k]) : kNoPosition) | tag;
             }
-            if (p.expert_bases) {                         // only the expanded layout places rows by expert
-#pragma unroll
-                for (int k = 0; k < KMAX; ++k) {
-                    const int bucket = e[k] >= 0 ? p.R + e[k] : 0;
-                    word_r[k] = bitmap[bucket * kWaves + wave];
-                    before_r[k] = before_wave[bucket];
-                }
-#pragma unroll
-                for (int k = 0; k < KMAX; ++k)
-                    packed[k] |= (e[k] >= 0 ? position(word_r[k], before_r[k]) : kNoPosition) << kExpertPositionShift;
-            } else {
-#pragma unroll
-                for (int k = 0; k < KMAX; ++k) packed[k] |= kNoPosition << kExpertPositionShift;
-            }
-            if (KMAX == 8 && p.K == 8) {
-                vec16* dst = reinterpret_cast<vec16*>(p.pos + int64_t(t) * 8);
-                const vec16 lo{packed[0], packed[1], packed[2], packed[3]}, hi{packed[4], packed[5], packed[6], packed[7]};
-                if constexpr (kThrough) {
-                    store16_agent(dst, lo);
-                    store16_agent(dst + 1, hi);
-                } else {
-                    dst[0] = lo;
-                    dst[1] = hi;
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < KMAX; ++k)
-                    if (k < p.K) store_word<kThrough>(reinterpret_cast<int*>(p.pos) + int64_t(t) * p.K + k, int(packed[k]));
-            }
+            packed[k] = (master[k] ? position(word_r[k], before_r[k]) : kNoPosition) | tag;
         }
-        if (p.is_token_in_rank != nullptr) {
-            for (int r = 0; r < p.R; ++r)
-                p.is_token_in_rank[int64_t(t) * p.R + r] = uint8_t((bitmap[r * kWaves + wave] >> lane) & 1ull);
+        if (p.expert_bases) {                         // only the expanded layout places rows by expert
+#pragma unroll
+            for (int k = 0; k < KMAX; ++k) {
+                const int bucket = e[k] >= 0 ? p.R + e[k] : 0;
+                word_r[k] = bitmap[bucket * kWaves + wave];
+                before_r[k] = before_wave[bucket];
+            }
+#pragma unroll
+            for (int k = 0; k < KMAX; ++k)
+                packed[k] |= (e[k] >= 0 ? position(word_r[k], before_r[k]) : kNoPosition) << kExpertPositionShift;
+        } else {
+#pragma unroll
+            for (int k = 0; k < KMAX; ++k) packed[k] |= kNoPosition << kExpertPositionShift;
         }
     }
+    if (p.pos != nullptr && seen != 0) flags |= DEEP_EP_HIP_STATUS_DUPLICATE_EXPERT;
     if (flags != 0) atomicOr(p.status, flags);
 
+    hand_off();
+
+    if (!active) return;
+    if (p.pos != nullptr) {
+        if (KMAX == 8 && p.K == 8) {
+            vec16* dst = reinterpret_cast<vec16*>(p.pos + int64_t(t) * 8);
+            const vec16 lo{packed[0], packed[1], packed[2], packed[3]}, hi{packed[4], packed[5], packed[6], packed[7]};
+            if constexpr (kThrough) {
+                store16_agent(dst, lo);
+                store16_agent(dst + 1, hi);
+            } else {
+                dst[0] = lo;
+                dst[1] = hi;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < KMAX; ++k)
+                if (k < p.K) store_word<kThrough>(reinterpret_cast<int*>(p.pos) + int64_t(t) * p.K + k, int(packed[k]));
+        }
+    }
+    if constexpr (!kThrough) copy_indices();
+    if (p.is_token_in_rank != nullptr) {
+        for (int r = 0; r < p.R; ++r)
+            p.is_token_in_rank[int64_t(t) * p.R + r] = uint8_t((bitmap[r * kWaves + wave] >> lane) & 1ull);
+    }
 }
 
 }  // namespace deep_ep_hip

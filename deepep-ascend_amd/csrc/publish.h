@@ -71,7 +71,7 @@ template <int kThreads>
 __device__ void publish_ranks(const PublishParams& q, const PublishLds& s) {
     for (int r = threadIdx.x; r < q.R; r += kThreads) {
         if (q.num_tokens_per_rank != nullptr) q.num_tokens_per_rank[r] = s.totals[r];
-        if (q.host_counts != nullptr) q.host_counts[r] = -s.totals[r] - 1;
+        if (q.host_counts != nullptr) store_system(q.host_counts + r, -s.totals[r] - 1);
     }
     __syncthreads();
     block_inclusive_scan<kThreads>(s.totals, q.R, s.scan_tmp);
@@ -136,7 +136,7 @@ __device__ void scan_rank_counts(const PublishParams& q, const LayoutTables& t, 
     for (int r = tid; r < R; r += kThreads) {
         const int total = s.totals[r] - (r > 0 ? s.totals[r - 1] : 0);
         if (q.num_tokens_per_rank != nullptr) q.num_tokens_per_rank[r] = total;
-        if (q.host_counts != nullptr) q.host_counts[r] = -total - 1;
+        if (q.host_counts != nullptr) store_system(q.host_counts + r, -total - 1);
         if (q.psum_rank != nullptr) q.psum_rank[r] = s.totals[r];
     }
     if (tid == 0 && q.totals_out != nullptr) q.totals_out[0] = s.totals[R - 1];
@@ -162,9 +162,19 @@ __device__ void sum_expert_columns(const LayoutTables& t, int R, int E, int num_
     __syncthreads();
 }
 
+// First thread: the status word as the counting workgroups left it (they are all done when a workgroup publishes), for
+// the host's mailbox.  Asked for early: the trip to memory passes beside the prefix sums.
+__device__ __forceinline__ int status_for_host(const PublishParams& q) {
+    return threadIdx.x == 0 && q.host_counts != nullptr && q.status != nullptr ? load_agent(q.status) : 0;
+}
+
 // Per-expert outputs; afterwards the region of expert j starts at s.aligned_incl[j] - s.aligned[j].
+//
+// The words of the mailbox are stored at system scope, each valid by itself (v as -v-1): the host sees a word as soon as
+// it has crossed the bus, and no fence follows.  With a system-scope fence, which writes the whole L2 back and waits for
+// it, a layout launch took 1 to 2 us longer.
 template <int kThreads>
-__device__ void publish_experts(const PublishParams& q, const PublishLds& s) {
+__device__ void publish_experts(const PublishParams& q, const PublishLds& s, const int status) {
     for (int j = threadIdx.x; j < q.E; j += kThreads) {
         const int cnt = s.totals[q.R + j];
         const int al = (cnt + q.A - 1) / q.A * q.A;
@@ -173,7 +183,7 @@ __device__ void publish_experts(const PublishParams& q, const PublishLds& s) {
         if (q.num_tokens_per_expert != nullptr) q.num_tokens_per_expert[j] = cnt;
         if (q.num_unaligned != nullptr) q.num_unaligned[j] = cnt;
         if (q.cumulative_stats != nullptr) q.cumulative_stats[j] += cnt;
-        if (q.host_counts != nullptr) q.host_counts[q.R + j] = -al - 1;
+        if (q.host_counts != nullptr) store_system(q.host_counts + q.R + j, -al - 1);
     }
     __syncthreads();
     block_inclusive_scan<kThreads>(s.aligned_incl, q.E, s.scan_tmp);
@@ -183,12 +193,9 @@ __device__ void publish_experts(const PublishParams& q, const PublishLds& s) {
         if (q.psum_expert != nullptr) q.psum_expert[j] = q.do_expand ? start + s.totals[q.R + j] : s.aligned_incl[j];
     }
     if (threadIdx.x == 0 && q.totals_out != nullptr) q.totals_out[1] = q.E > 0 ? s.aligned_incl[q.E - 1] : 0;
-    if (q.host_counts != nullptr) {
-        // The status word as the counting workgroups left it (they are all done when a workgroup publishes): a host that
-        // sizes its outputs from this mailbox learns about bad routing input without a second trip to the device.
-        if (threadIdx.x == 0) q.host_counts[q.R + q.E] = -(q.status != nullptr ? load_agent(q.status) : 0) - 1;
-        __threadfence_system();
-    }
+    // The status word: a host that sizes its outputs from this mailbox learns about bad routing input without a second
+    // trip to the device.
+    if (threadIdx.x == 0 && q.host_counts != nullptr) store_system(q.host_counts + q.R + q.E, -status - 1);
 }
 
 // table[c][e] = start of expert e's region + sum of expert_counts[0..c)[e], each word ORed with `tag`.
@@ -275,65 +282,131 @@ __device__ bool write_expert_bases_from_registers(const LayoutTables& t, const u
     return all_complete != 0;
 }
 
-// publish_layout for the common sizes (at most 32 chunks, num_experts <= kThreads, R * chunks_padded <= 4 * kThreads) in one
-// trip to memory instead of four: every thread first loads all it will ever need - four entries of the flattened rank
-// table and its expert's column of chunk totals, kept in registers - and totals, prefix sums, public outputs and both
-// base tables are worked out from those.
-template <int kThreads>
-__device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutTables& t, int num_chunks, bool expert_bases, int* lds) {
-    const PublishLds s = carve_publish_lds(lds, q.R, q.E);
+// publish_layout for the common sizes: num_experts <= kThreads, R * chunks_padded <= 16 * kThreads.  A workgroup of its
+// own on the critical path of every call: what it costs is the chain of barriers, LDS trips and instruction fetches, so
+// there is one trip to memory (every thread first loads all it needs: up to 16 consecutive entries of the flattened rank
+// table and its expert's column of chunk totals, of which 32 stay in registers), one pair of prefix sums, taken
+// together, and two barriers; outputs go out from registers.  kOneChunk: `totals` ([R + E], LDS) holds the only
+// chunk's totals and nothing is loaded.  scratch: LDS of publish_scratch_ints.
+// From the ticket to the end it took 3.4 us at 16 chunks, 9 us at 64 chunks over 32 ranks, with LDS scans of five
+// barriers and 32 chunks at most; the whole launch went from 10.0 to 8.3 and from 14.8 to 11.5 us.
+inline __host__ __device__ int publish_scratch_ints(int R, int threads) { return R + 2 * (threads / kWaveSize); }
+
+template <int kThreads, bool kOneChunk>
+__device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutTables& t, int num_chunks, bool expert_bases,
+                                           const int* totals, int* scratch) {
+    constexpr int kWavesHere = kThreads / kWaveSize;
+    constexpr int kMaxVecs = kOneChunk ? 1 : 4, kColumn = kOneChunk ? 1 : 32;
+    int* rank_end = scratch;                             // [R] inclusive prefix sum over the ranks
+    int* wave_sums = scratch + q.R;                      // [2][kWavesHere]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int flat = q.R * t.chunks_padded;              // a multiple of 4: a thread's entries share a row
-    const int begin = tid * 4;
-    vec16 rv{0, 0, 0, 0};
-    if (begin < flat) rv = load16(t.rank_counts + begin);
-    int v[32];
-    if (tid < q.E) {
+    const bool has_expert = tid < q.E;
+    const int status = status_for_host(q);
+    const int flat = q.R * t.chunks_padded;              // a multiple of 4: four entries share a row
+    const int vecs = kOneChunk ? 1 : (flat + 4 * kThreads - 1) / (4 * kThreads);
+    vec16 rv[kMaxVecs];
+    int v[kColumn];
+    int rows = 0, count = 0;
+    if constexpr (kOneChunk) {
+        rv[0] = vec16{tid < q.R ? uint32_t(totals[tid]) : 0u, 0, 0, 0};          // rows of four, three of them padding
+        v[0] = has_expert ? totals[q.R + tid] : 0;
+        rows = int(rv[0].x);
+        count = v[0];
+    } else {
 #pragma unroll
-        for (int u = 0; u < 32; ++u) {
-            const int row_start = __builtin_amdgcn_readfirstlane(min(u, num_chunks - 1) * t.experts_padded);
-            v[u] = t.expert_counts[row_start + tid];
+        for (int i = 0; i < kMaxVecs; ++i) {
+            rv[i] = vec16{0, 0, 0, 0};
+            const int begin = (tid * vecs + i) * 4;
+            if (i < vecs && begin < flat) rv[i] = load16(t.rank_counts + begin);
         }
+        const int column = has_expert ? tid : 0;
+        auto load_sixteen = [&](int first, int* to) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                // a row start common to the workgroup plus the thread's column: one address register serves all loads
+                const int row_start = __builtin_amdgcn_readfirstlane(min(first + u, num_chunks - 1) * t.experts_padded);
+                to[u] = t.expert_counts[row_start + column];
+            }
+        };
+        auto sum_sixteen = [&](int first, const int* of) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) count += first + u < num_chunks ? of[u] : 0;
+        };
+        load_sixteen(0, v);
+        if (num_chunks > 16) load_sixteen(16, v + 16);
+        for (int c0 = 32; c0 < num_chunks; c0 += 16) {
+            int w[16];
+            load_sixteen(c0, w);
+            sum_sixteen(c0, w);
+        }
+        sum_sixteen(0, v);
+        if (num_chunks > 16) sum_sixteen(16, v + 16);
+#pragma unroll
+        for (int i = 0; i < kMaxVecs; ++i) rows += int(rv[i].x) + int(rv[i].y) + int(rv[i].z) + int(rv[i].w);
+    }
+    int aligned = 0;
+    if (has_expert) aligned = q.A == 1 ? count : int((unsigned(count) + unsigned(q.A) - 1u) / unsigned(q.A)) * q.A;
+
+    const int rows_incl = wave_inclusive_sum(rows), aligned_incl = wave_inclusive_sum(aligned);
+    if (lane == kWaveSize - 1) {
+        wave_sums[wave] = rows_incl;
+        wave_sums[kWavesHere + wave] = aligned_incl;
+    }
+    __syncthreads();
+    int run = rows_incl - rows, start = aligned_incl - aligned;
+#pragma unroll
+    for (int w = 0; w < kWavesHere - 1; ++w) {
+        run += w < wave ? wave_sums[w] : 0;
+        start += w < wave ? wave_sums[kWavesHere + w] : 0;
     }
 
-    // rank part: exclusive prefix over the flattened table = first compact row of every (rank, chunk)
-    const int sum = int(rv.x) + int(rv.y) + int(rv.z) + int(rv.w);
-    const int inc = wave_inclusive_sum(sum);
-    if (lane == kWaveSize - 1) s.scan_tmp[wave] = inc;
-    __syncthreads();
-    int run = inc - sum;
-    for (int w = 0; w < wave; ++w) run += s.scan_tmp[w];
-    if (begin < flat) {
-        if (t.rank_bases != nullptr) {
-            const uint32_t b0 = uint32_t(run), b1 = b0 + rv.x, b2 = b1 + rv.y, b3 = b2 + rv.z;
-            store16(t.rank_bases + begin, vec16{b0, b1, b2, b3});
-        }
-        if ((begin + 4) % t.chunks_padded == 0) s.totals[begin / t.chunks_padded] = run + sum;   // inclusive prefix of the rank
+    // experts: the region of an expert starts at the aligned rows of those before it
+    if (has_expert) {
+        if (q.host_counts != nullptr) store_system(q.host_counts + q.R + tid, -aligned - 1);
+        if (q.num_tokens_per_expert != nullptr) q.num_tokens_per_expert[tid] = count;
+        if (q.num_unaligned != nullptr) q.num_unaligned[tid] = count;
+        if (q.cumulative_stats != nullptr) q.cumulative_stats[tid] += count;
+        if (q.expert_start != nullptr) q.expert_start[tid] = start;
+        if (q.psum_expert != nullptr) q.psum_expert[tid] = q.do_expand ? start + count : start + aligned;
+        if (tid == q.E - 1 && q.totals_out != nullptr) q.totals_out[1] = start + aligned;
     }
-    if (tid < q.E) {
-        int total = 0;
+    // ranks: the exclusive prefix over the flattened table is the first compact row of every (rank, chunk)
+    const float rcp_row = 1.0f / float(t.chunks_padded);
 #pragma unroll
-        for (int u = 0; u < 32; ++u) total += u < num_chunks ? v[u] : 0;
-        s.totals[q.R + tid] = total;
+    for (int i = 0; i < kMaxVecs; ++i) {
+        const int begin = (tid * vecs + i) * 4;
+        if (i >= vecs || begin >= flat) break;
+        const uint32_t b0 = uint32_t(run), b1 = b0 + rv[i].x, b2 = b1 + rv[i].y, b3 = b2 + rv[i].z;
+        run = int(b3 + rv[i].w);
+        if (t.rank_bases != nullptr) store16(t.rank_bases + begin, vec16{b0, b1, b2, b3});
+        const int r = small_div(begin, rcp_row);
+        if (begin + 4 == (r + 1) * t.chunks_padded) rank_end[r] = run;
     }
     __syncthreads();
     for (int r = tid; r < q.R; r += kThreads) {
-        const int total = s.totals[r] - (r > 0 ? s.totals[r - 1] : 0);
+        const int end = rank_end[r], total = end - (r > 0 ? rank_end[r - 1] : 0);
+        if (q.host_counts != nullptr) store_system(q.host_counts + r, -total - 1);
         if (q.num_tokens_per_rank != nullptr) q.num_tokens_per_rank[r] = total;
-        if (q.host_counts != nullptr) q.host_counts[r] = -total - 1;
-        if (q.psum_rank != nullptr) q.psum_rank[r] = s.totals[r];
+        if (q.psum_rank != nullptr) q.psum_rank[r] = end;
+        if (r == q.R - 1 && q.totals_out != nullptr) q.totals_out[0] = end;
     }
-    if (tid == 0 && q.totals_out != nullptr) q.totals_out[0] = s.totals[q.R - 1];
+    if (tid == 0 && q.host_counts != nullptr) store_system(q.host_counts + q.R + q.E, -status - 1);
 
-    publish_experts<kThreads>(q, s);
-    if (t.expert_bases != nullptr && expert_bases && tid < q.E) {
-        int at = s.aligned_incl[tid] - s.aligned[tid];
+    if (t.expert_bases != nullptr && expert_bases && has_expert) {
+        int at = start;
 #pragma unroll
-        for (int u = 0; u < 32; ++u) {
+        for (int u = 0; u < kColumn; ++u) {
             if (u < num_chunks) {
-                const int row_start = __builtin_amdgcn_readfirstlane(u * t.experts_padded);
-                t.expert_bases[row_start + tid] = at;
+                t.expert_bases[__builtin_amdgcn_readfirstlane(u * t.experts_padded) + tid] = at;
                 at += v[u];
+            }
+        }
+        if constexpr (!kOneChunk) {
+            for (int c = kColumn; c < num_chunks; ++c) {
+                const int row_start = c * t.experts_padded;
+                const int here = t.expert_counts[row_start + tid];
+                t.expert_bases[row_start + tid] = at;
+                at += here;
             }
         }
     }
@@ -343,17 +416,18 @@ __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutT
 // totals, public outputs, and - when the caller has room for them - the base tables.
 template <int kThreads>
 __device__ void publish_layout(const PublishParams& q, const LayoutTables& t, int num_chunks, bool expert_bases, int* lds) {
-    if (num_chunks <= 32 && q.E <= kThreads && q.R * t.chunks_padded <= 4 * kThreads) {
-        publish_layout_in_one_trip<kThreads>(q, t, num_chunks, expert_bases, lds);
+    if (q.E <= kThreads && q.R * t.chunks_padded <= 16 * kThreads) {
+        publish_layout_in_one_trip<kThreads, false>(q, t, num_chunks, expert_bases, nullptr, lds);
         return;
     }
     const PublishLds s = carve_publish_lds(lds, q.R, q.E);
+    const int status = status_for_host(q);
     sum_rank_rows<kThreads>(t, q.R, s.totals);
     sum_expert_columns<kThreads>(t, q.R, q.E, num_chunks, s.totals);
     publish_ranks<kThreads>(q, s);
     __syncthreads();
     if (t.rank_bases != nullptr) write_rank_bases<kThreads>(t, q.R, s);
-    publish_experts<kThreads>(q, s);
+    publish_experts<kThreads>(q, s, status);
     if (t.expert_bases != nullptr && expert_bases) {
         __syncthreads();
         write_expert_bases<kThreads, false>(t, t.expert_bases, 0u, q.E, num_chunks, s);
