@@ -308,7 +308,7 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
     lay.pos = reinterpret_cast<uint32_t*>(ws + w.pos);
 
     if (do_layout && !plan.fused) {
-        hipError_t err = launch_layout_kernel(lay, stream);
+        hipError_t err = launch_layout_kernel(lay, IntranodePrefixParams{}, stream);
         if (err != hipSuccess) return hip_fail(err, "dispatch layout launch");
     }
 
@@ -440,7 +440,7 @@ int deep_ep_hip_launch_layout(const deep_ep_hip_layout_args* a, void* stream) {
     p.tab = carve_tables(ws, w, p.T, p.E);
     p.tab.rank_bases = nullptr;       // a layout-only call publishes counts, not row bases
     p.tab.expert_bases = nullptr;
-    hipError_t err = launch_layout_kernel(p, static_cast<hipStream_t>(stream));
+    hipError_t err = launch_layout_kernel(p, IntranodePrefixParams{}, static_cast<hipStream_t>(stream));
     if (err != hipSuccess) return hip_fail(err, "layout launch");
     return DEEP_EP_HIP_OK;
 }
@@ -624,24 +624,18 @@ int deep_ep_hip_launch_intranode_dispatch(const deep_ep_hip_intranode_dispatch_a
     lay.pos = reinterpret_cast<uint32_t*>(ws + w.pos);
 
     if (do_layout) {
-        hipError_t err = hipSuccess;
-        if (!plan.fused) {
-            err = launch_layout_kernel(lay, stream);
-            if (err != hipSuccess) return hip_fail(err, "intranode dispatch layout launch");
-        }
-
+        IntranodePrefixParams prefix{};
         if (a->rank_prefix_matrix != nullptr || a->channel_prefix_matrix != nullptr ||
             a->recv_channel_prefix_matrix != nullptr) {
             REQUIRE(a->is_token_in_rank != nullptr || T == 0, "the prefix matrices are computed from is_token_in_rank");
-            IntranodePrefixParams q{};
-            q.mask = a->is_token_in_rank;
-            q.T = T; q.R = R; q.C = a->num_channels; q.rank_idx = a->rank_idx;
-            q.rank_prefix_matrix = a->rank_prefix_matrix;
-            q.channel_prefix_matrix = a->channel_prefix_matrix;
-            q.recv_channel_prefix_matrix = a->recv_channel_prefix_matrix;
-            err = launch_intranode_prefix(q, stream);
-            if (err != hipSuccess) return hip_fail(err, "intranode prefix launch");
+            prefix.mask = a->is_token_in_rank;
+            prefix.T = T; prefix.R = R; prefix.C = a->num_channels; prefix.rank_idx = a->rank_idx;
+            prefix.rank_prefix_matrix = a->rank_prefix_matrix;
+            prefix.channel_prefix_matrix = a->channel_prefix_matrix;
+            prefix.recv_channel_prefix_matrix = a->recv_channel_prefix_matrix;
         }
+        const hipError_t err = plan.fused ? launch_intranode_prefix(prefix, stream) : launch_layout_kernel(lay, prefix, stream);
+        if (err != hipSuccess) return hip_fail(err, "intranode dispatch layout launch");
     }
 
     if (do_move) {

@@ -1218,37 +1218,6 @@ __global__ __launch_bounds__(kThreads) void cast_kernel(const CastParams p) {
     if ((lane & 7) == 0 && group < groups && elem < p.H) p.scales[int64_t(t) * groups + group] = scale_inv;
 }
 
-// ---- V1 handle bookkeeping (csrc/kernels/legacy/intranode.cu:94-125): one workgroup per destination rank
-// counts the tokens of each channel (contiguous token range) that go there, then prefix-sums over channels ----
-__global__ __launch_bounds__(kThreads) void intranode_prefix_kernel(const IntranodePrefixParams p) {
-    extern __shared__ int channel_counts[];     // [C]
-    const int d = blockIdx.x;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int per_channel = (p.T + p.C - 1) / p.C;
-    for (int c = wave; c < p.C; c += kWavesPerBlock) {
-        const int begin = min(per_channel * c, p.T), end = min(begin + per_channel, p.T);
-        int count = 0;
-        for (int t = begin + lane; t < end; t += kWaveSize) count += p.mask[int64_t(t) * p.R + d] != 0 ? 1 : 0;
-        count = wave_inclusive_sum(count);
-        if (lane == kWaveSize - 1) channel_counts[c] = count;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int run = 0;
-        for (int c = 0; c < p.C; ++c) {
-            if (p.recv_channel_prefix_matrix != nullptr) p.recv_channel_prefix_matrix[d * p.C + c] = run;
-            run += channel_counts[c];
-            if (p.channel_prefix_matrix != nullptr) p.channel_prefix_matrix[d * p.C + c] = run;
-            channel_counts[c] = run;
-        }
-    }
-    __syncthreads();
-    // Only this source rank sends in a one-GPU call: the prefix over source ranks steps once, at rank_idx.
-    const int total = p.C > 0 ? channel_counts[p.C - 1] : 0;
-    if (p.rank_prefix_matrix != nullptr)
-        for (int i = threadIdx.x; i < p.R; i += kThreads) p.rank_prefix_matrix[i * p.R + d] = i >= p.rank_idx ? total : 0;
-}
-
 // ---- rows of recv_topk_idx beyond the received ones read -1 (csrc/kernels/legacy/intranode.cu:535-545) ----
 __global__ __launch_bounds__(kThreads) void fill_tail_kernel(const FillTailParams p) {
     const int64_t first = int64_t(*p.total_rows) * p.K;
@@ -1463,12 +1432,6 @@ hipError_t launch_zero_padding(const PadParams& p, hipStream_t stream) {
     const int64_t waves = int64_t(p.E) * (p.A - 1);
     const unsigned blocks = unsigned((waves + kWavesPerBlock - 1) / kWavesPerBlock);
     hipLaunchKernelGGL(zero_padding_kernel, dim3(blocks), dim3(kThreads), 0, stream, p);
-    return hipGetLastError();
-}
-
-hipError_t launch_intranode_prefix(const IntranodePrefixParams& p, hipStream_t stream) {
-    if (p.R == 0 || p.C == 0) return hipSuccess;
-    hipLaunchKernelGGL(intranode_prefix_kernel, dim3(p.R), dim3(kThreads), size_t(p.C) * sizeof(int), stream, p);
     return hipGetLastError();
 }
 

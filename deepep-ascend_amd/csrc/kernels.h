@@ -115,7 +115,18 @@ struct LayoutParams {
     const uint32_t* generation;
 };
 
-hipError_t launch_layout_kernel(const LayoutParams& p, hipStream_t stream);
+// The channel matrices of a V1 handle; R = 0: not wanted.
+struct IntranodePrefixParams {
+    const uint8_t* mask;             // [T, R]
+    int T, R, C, rank_idx;
+    int32_t* rank_prefix_matrix;         // [R, R]
+    int32_t* channel_prefix_matrix;      // [R, C] inclusive over channels
+    int32_t* recv_channel_prefix_matrix; // [R, C] exclusive starts
+};
+
+// `prefix`, if wanted, rides in the same launch.
+hipError_t launch_layout_kernel(const LayoutParams& p, const IntranodePrefixParams& prefix, hipStream_t stream);
+hipError_t launch_intranode_prefix(const IntranodePrefixParams& p, hipStream_t stream);
 
 struct MoveParams {
     const uint8_t* x;
@@ -202,16 +213,6 @@ struct PadParams {
 hipError_t launch_zero_padding(const PadParams& p, hipStream_t stream);
 
 // V1 (intranode) handle bookkeeping computed from is_token_in_rank, and the -1 fill of unused recv_topk_idx rows.
-struct IntranodePrefixParams {
-    const uint8_t* mask;             // [T, R]
-    int T, R, C, rank_idx;
-    int32_t* rank_prefix_matrix;         // [R, R]
-    int32_t* channel_prefix_matrix;      // [R, C] inclusive over channels
-    int32_t* recv_channel_prefix_matrix; // [R, C] exclusive starts
-};
-
-hipError_t launch_intranode_prefix(const IntranodePrefixParams& p, hipStream_t stream);
-
 struct FillTailParams {
     int64_t* recv_topk_idx;          // [capacity, K]
     const int32_t* total_rows;       // device: rows in use
