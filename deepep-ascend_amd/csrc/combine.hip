@@ -12,8 +12,14 @@
 // lane order rounded to BF16.  Expanded layout without multiple reduction: every valid lane is its
 // own term, in lane order.
 //
-// One wavefront owns one (token, column tile of kVecs * 512 channels).
+// One wavefront owns one (token, column tile of kVecs * 512 channels).  Large calls are bound by memory, small ones by the chain
+// of trips to it: routing loads, rows of the first batch, rows of the second.  With a start that waited for the index, biases and
+// weights waited for in front of the rows and a branch around every load it took (combine kernel and its launch, us before ->
+// now): 1237 x 2888 top-9 over 6 ranks 11.5 -> 9.8, 4096 x 2048 top-6 19.1 -> 17.3, 8192 x 7168 4 of 4 ranks 73.9 -> 67.6,
+// 8192 x 7168 top-8 over 8 ranks 118.4 -> 117.0 and 16384 over 32 ranks 333 -> 321 (1.9 GB, 5.8 TB/s -> 6.0).  Eight rows
+// a batch instead of four measured the same.
 #include <algorithm>
+#include <cmath>
 
 #include "device_utils.h"
 #include "kernels.h"
@@ -41,15 +47,14 @@ __device__ __forceinline__ void add_row(float (&acc)[kVecs][8], const vec16 (&v)
     }
 }
 
+// The row is the same for the whole wavefront, so it is read through a buffer descriptor of its own (base: the row; range:
+// its bytes, none for row < 0): channels past the row's end and missing rows read as zero in the load itself.  With a branch
+// around each load instead, the compiler put waits and address arithmetic between the loads of a batch.
 template <int kVecs>
-__device__ __forceinline__ void load_row(vec16 (&v)[kVecs], const uint8_t* base, int64_t row, int row_bytes,
-                                         int tile, int lane) {
+__device__ __forceinline__ void load_row(vec16 (&v)[kVecs], const uint8_t* base, int row, int row_bytes, int tile, int lane) {
+    const auto of_row = buffer_of(base + int64_t(max(row, 0)) * row_bytes, row >= 0 ? row_bytes : 0);
 #pragma unroll
-    for (int i = 0; i < kVecs; ++i) {
-        const int off = (tile * kVecs + i) * 1024 + lane * 16;
-        v[i] = vec16{0, 0, 0, 0};
-        if (row >= 0 && off < row_bytes) v[i] = load16_stream(base + row * row_bytes + off);
-    }
+    for (int i = 0; i < kVecs; ++i) v[i] = buffer_load16_stream(of_row, (tile * kVecs + i) * 1024 + lane * 16);
 }
 
 // acc += sum of rows named by the lanes in `mask` (ascending lane order); row_of_lane < 0 adds nothing.
@@ -78,11 +83,12 @@ __device__ __forceinline__ void accumulate_rows(float (&acc)[kVecs][8], uint64_t
 
 // kLayout: what the rows of x are.  Each gets a kernel of its own, so that the sequencing registers of the expanded
 // layout do not cost the compact layout occupancy.
-enum : int { kCompactRows = 0, kExpandedRows = 1, kExpandedRowsReducedPerRank = 2 };
+// kRankRows: V1 conventions (CombineParams::rank_mode).
+enum : int { kCompactRows = 0, kExpandedRows = 1, kExpandedRowsReducedPerRank = 2, kRankRows = 3 };
 
 template <int kVecs, int kLayout>
 __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p) {
-    constexpr bool kExpanded = kLayout != kCompactRows;
+    constexpr bool kExpanded = kLayout == kExpandedRows || kLayout == kExpandedRowsReducedPerRank;
     const int lane = threadIdx.x & 63;
     const unsigned work = wave_work_index(blockIdx.x, kWavesPerBlock);
     if (work >= unsigned(p.T) * unsigned(p.tiles)) return;
@@ -90,7 +96,18 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p
     const int tile = int(work - unsigned(t) * unsigned(p.tiles));
     const int row_bytes = p.H * 2;
 
-    // Biases first: their loads do not depend on the routing metadata.
+    // Routing of this token: lanes [0, K).  Indices, slots and the ends of the ranks' regions (lane r: rank r) are asked for
+    // together, on clamped columns instead of behind branches, and the biases with them: where a rank's region starts then
+    // comes from another lane, not from a load that waits for the index.
+    const int64_t at = int64_t(t) * p.K + min(lane, p.K - 1);
+    const int slot = p.slot[at];
+    int64_t raw = -1;
+    int rank_end = 0;
+    if constexpr (kLayout != kRankRows) {
+        raw = p.topk_idx[at];
+        rank_end = p.psum_rank[min(lane, p.R - 1)];
+    }
+
     float acc[kVecs][8];
 #pragma unroll
     for (int i = 0; i < kVecs; ++i)
@@ -107,17 +124,13 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p
         add_row<kVecs>(acc, v);
     }
 
-    // Routing of this token: lanes [0, K).
     int e = -1, d = -1, row_c = -1, my_row = -1, erow = -1;
-    if (p.rank_mode) {
+    if constexpr (kLayout == kRankRows) {
         // V1 handle: lane q < R reads the receive row of this token on rank q; rows are added in ascending
         // rank order and the weights of all rows are summed (csrc/kernels/legacy/intranode.cu:940-1033).
-        if (lane < p.K) {
-            const int v = p.slot[int64_t(t) * p.K + lane];
-            if (v >= 0) {
-                if (v < p.num_x_rows) row_c = v;
-                else atomicOr(p.status, DEEP_EP_HIP_STATUS_ROW_OVERFLOW);
-            }
+        if (lane < p.K && slot >= 0) {
+            if (slot < p.num_x_rows) row_c = slot;
+            else atomicOr(p.status, DEEP_EP_HIP_STATUS_ROW_OVERFLOW);
         }
         const uint64_t rows_of_token = __ballot(row_c >= 0);      // taken with every lane active
         if (tile == 0 && p.out_w != nullptr && lane < p.Kw) {
@@ -131,25 +144,28 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p
             }
             p.out_w[int64_t(t) * p.Kw + lane] = w;
         }
-    } else if (lane < p.K) {
-        const int64_t raw = p.topk_idx[int64_t(t) * p.K + lane];
-        if (raw >= 0 && raw < p.E) e = int(raw);
-        const int v = p.slot[int64_t(t) * p.K + lane];
-        if (e >= 0) {
+    } else {
+        if (lane < p.K && raw >= 0 && raw < p.E) {
+            e = int(raw);
             d = small_div(e, 1.0f / float(p.E_l));
-            if (v >= 0) {
-                row_c = (d > 0 ? p.psum_rank[d - 1] : 0) + (v - p.rank_idx * p.M);
-                if (!kExpanded && row_c >= p.num_x_rows) {
-                    atomicOr(p.status, DEEP_EP_HIP_STATUS_ROW_OVERFLOW);
-                    row_c = -1;
-                }
+        }
+        int start = __shfl(rank_end, max(d - 1, 0) & 63, kWaveSize);
+        if (p.R > kWaveSize && d > 0) start = p.psum_rank[d - 1];
+        if (e >= 0 && slot >= 0) {
+            row_c = (d > 0 ? start : 0) + (slot - p.rank_idx * p.M);
+            if (!kExpanded && row_c >= p.num_x_rows) {
+                atomicOr(p.status, DEEP_EP_HIP_STATUS_ROW_OVERFLOW);
+                row_c = -1;
             }
         }
     }
-    for (int j = 0; j < p.K && !p.rank_mode; ++j) {
-        const int dj = read_lane(d, j);
-        const int rj = read_lane(row_c, j);
-        if (d >= 0 && dj == d && rj >= 0) my_row = rj;
+    const bool returns_weights = kLayout != kRankRows && tile == 0 && p.out_w != nullptr;
+    if (kExpanded || returns_weights) {
+        for (int j = 0; j < p.K; ++j) {
+            const int dj = read_lane(d, j);
+            const int rj = read_lane(row_c, j);
+            if (d >= 0 && dj == d && rj >= 0) my_row = rj;
+        }
     }
     if (kExpanded && my_row >= 0 && my_row < p.num_meta_rows) {
         erow = p.meta[int64_t(my_row) * (p.K + 2) + 2 + lane];
@@ -159,20 +175,18 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p
         }
     }
 
-    // Weights travel back to the lane that owns them.
-    if (tile == 0 && p.out_w != nullptr && lane < p.K && !p.rank_mode) {
-        float w = 0.f;
-        if (p.topk_weights != nullptr) {
-            if (kExpanded) {
-                if (erow >= 0) w = p.topk_weights[erow];
-            } else if (my_row >= 0) {
-                w = p.topk_weights[int64_t(my_row) * p.K + lane];
-            }
+    // Weights travel back to the lane that owns them: asked for in front of the rows, stored behind them, so that the rows
+    // are not held up by the wait.
+    float w = 0.f;
+    if (returns_weights && p.topk_weights != nullptr && lane < p.K) {
+        if (kExpanded) {
+            if (erow >= 0) w = p.topk_weights[erow];
+        } else if (my_row >= 0) {
+            w = p.topk_weights[int64_t(my_row) * p.K + lane];
         }
-        p.out_w[int64_t(t) * p.K + lane] = w;
     }
 
-    if constexpr (kLayout == kCompactRows) {
+    if constexpr (kLayout == kCompactRows || kLayout == kRankRows) {
         accumulate_rows<kVecs>(acc, __ballot(row_c >= 0), row_c, p.x, row_bytes, tile, lane);
     } else if constexpr (kLayout == kExpandedRows) {
         accumulate_rows<kVecs>(acc, __ballot(erow >= 0), erow, p.x, row_bytes, tile, lane);
@@ -250,11 +264,36 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p
             store16_stream(dst + off, o);
         }
     }
+    if (returns_weights && lane < p.K) p.out_w[int64_t(t) * p.K + lane] = w;
+}
+
+// Rows a token has, on average: as if its experts were chosen evenly, and no more than there are.
+double rows_per_token(const CombineParams& p) {
+    const double returned = double(p.num_x_rows) / p.T;
+    const int selections = p.rank_mode ? p.Kw : p.K;
+    if (selections == 0) return returned;
+    const int ranks = p.rank_mode ? p.K : p.R;
+    return std::min(returned, p.do_expand && !p.rank_mode ? double(selections) : ranks * (1.0 - std::pow(1.0 - 1.0 / ranks, selections)));
+}
+
+// How many workgroups a CU should hold at a time (0: the eight its registers allow).  Scattered rows stream fastest when not
+// too many are under way.  us with 8 / 6 / 5 / 4 per CU, 1 KB tiles, top-8, hidden 7168 unless said:
+//   8 ranks (5.3 rows a token)   4096 tokens  60.0 / 59.5 / 60.3 / 63.2;   8192  119.6 / 117.0 / 117.5 / 123.7;  16384  247 / 237 / 233 / 247
+//   16 ranks (6.4)               8192 tokens 149.1 / 145.4 / 141.7 / 143.8;  16384  303 / 297 / 287 / 286
+//   32 ranks (7.2)               4096 tokens  81.3 / 80.1 / 78.5 / 78.6;   16384  336 / 330 / 321 / 312
+//   4 of 4 ranks (2.7)           8192 tokens  67.6 / 71.3 / 76.0;   16384 x 2048 top-6 (4.4) 60.9 / 62.2 / 64.1
+//   expanded (8 rows)            4096 tokens  91.4 / 92.6 / 96.7;   8192  180.3 / 179.4 / 189.1;   16384  373 / 363 / 376
+// Smaller calls lose by any limit (4096 x 2048 top-6: 17.3 / 18.3).
+int workgroups_per_cu(const CombineParams& p) {
+    const double rows = rows_per_token(p), bytes = rows * p.T * p.H * 2;
+    if (p.do_expand && !p.rank_mode) return bytes >= 600e6 ? 6 : 0;
+    if (bytes < 300e6 || rows < 5.0) return 0;
+    return rows >= 5.8 ? 5 : 6;
 }
 
 template <int kVecs, int kLayout>
 hipError_t launch_layout(const CombineParams& p, unsigned blocks, hipStream_t stream) {
-    hipLaunchKernelGGL((combine_kernel<kVecs, kLayout>), dim3(blocks), dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((combine_kernel<kVecs, kLayout>), dim3(blocks), dim3(kThreads), lds_for_residency(workgroups_per_cu(p)), stream, p);
     return hipGetLastError();
 }
 
@@ -264,7 +303,8 @@ hipError_t launch(CombineParams p, hipStream_t stream) {
     p.tiles = (row_bytes + kVecs * 1024 - 1) / (kVecs * 1024);
     const int64_t waves = int64_t(p.T) * p.tiles;
     const unsigned blocks = unsigned((waves + kWavesPerBlock - 1) / kWavesPerBlock);
-    if (!p.do_expand || p.rank_mode) return launch_layout<kVecs, kCompactRows>(p, blocks, stream);
+    if (p.rank_mode) return launch_layout<kVecs, kRankRows>(p, blocks, stream);
+    if (!p.do_expand) return launch_layout<kVecs, kCompactRows>(p, blocks, stream);
     if (!p.multi_red) return launch_layout<kVecs, kExpandedRows>(p, blocks, stream);
     return launch_layout<kVecs, kExpandedRowsReducedPerRank>(p, blocks, stream);
 }
@@ -313,11 +353,15 @@ hipError_t launch_rebuild_slot_map(const SlotMapParams& p, hipStream_t stream) {
 
 hipError_t launch_combine_kernel(CombineParams p, hipStream_t stream) {
     if (p.T == 0) return hipSuccess;
-    // Column tile per wavefront, in KB of a BF16 row.  Compact rows: 1 KB (512 channels, 41 registers, eight wavefronts
-    // per SIMD) measured best - 8192 tokens x 7168: 117.9 us against 122.7 (2 KB) and 119.6 (4 KB); after a cache flush
-    // 123.6 / 126.6 / 124.4; 4096 x 2048: 18.2 / 18.2 / 19.7.  Expanded rows are insensitive (181.7 / 181.7 / 180.5 us).
+    // Column tile per wavefront, in KB of a BF16 row: 1 KB (512 channels, 41 registers, eight wavefronts per SIMD) measured
+    // best, at the residency above - 8192 tokens x 7168: 117.0 us against 117.9 (2 KB), expanded 179.4 against 179.8.  Calls
+    // of rows up to 6 KB that are over in one round of workgroups are ahead with 2 KB, which repeats the routing work half as
+    // often: 1237 x 2888 top-9 9.8 against 10.7, 512 x 1024 6.8 against 7.2 (512 x 7168: 9.9 against 9.6).
     int vecs = p.vecs;
-    if (vecs == 0) vecs = (p.do_expand && !p.rank_mode && p.H * 2 > 1024) ? 2 : 1;
+    if (vecs == 0) {
+        const int kb = (p.H * 2 + 1023) / 1024;
+        vecs = kb >= 2 && kb <= 6 && int64_t(p.T) * kb <= int64_t(compute_units()) * 8 * kWavesPerBlock ? 2 : 1;
+    }
     switch (vecs) {
         case 1: return launch<1>(p, stream);
         case 4: return launch<4>(p, stream);

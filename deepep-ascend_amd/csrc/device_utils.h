@@ -131,6 +131,16 @@ __device__ __forceinline__ int row16_sum(int v) {
     return v;
 }
 
+// A range of memory that is the same for the whole wavefront, as a buffer descriptor; loads past its end return zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const uint8_t* base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, bytes, 0x00027000);
+}
+__device__ __forceinline__ vec16 buffer_load16_stream(__amdgpu_buffer_rsrc_t from, int offset) {
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(from, offset, 0, 2 /* nt */);
+    return vec16{v.x, v.y, v.z, v.w};
+}
+
 // Inclusive prefix sum across the wave, as DPP operand modifiers: inside each row of 16 lanes by shifts of 1, 2, 4 and 8,
 // then the last lane of row 0 / 2 into row 1 / 3 and lane 31 into the upper half (bpermutes through LDS, as a shuffle
 // compiles to, took six dependent trips).  All lanes of the wavefront must be active.

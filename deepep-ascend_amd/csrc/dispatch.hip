@@ -1308,14 +1308,18 @@ static int move_workgroups_per_cu(const MoveParams& p) {
     return move_tile(p) == 2 ? 4 : 0;
 }
 
+}  // namespace
+
+// The limit is set with LDS the kernel never touches: a share that is just too large for one workgroup more, whatever
+// granule the LDS is handed out in.
+size_t lds_for_residency(int per_cu) {
+    return per_cu == 0 ? 0 : (size_t(lds_bytes_per_cu() / (per_cu + 1)) + 256) & ~size_t(255);
+}
+
+namespace {
+
 size_t move_lds_bytes(const MoveParams& p) {
-    if (!p.fused) {
-        // The limit is set with LDS the kernel never touches: a share that is just too large for one workgroup more,
-        // whatever granule the LDS is handed out in.
-        const int per_cu = move_workgroups_per_cu(p);
-        if (per_cu == 0) return 0;
-        return (size_t(lds_bytes_per_cu() / (per_cu + 1)) + 256) & ~size_t(255);
-    }
+    if (!p.fused) return lds_for_residency(move_workgroups_per_cu(p));
     const size_t publish = publish_lds_bytes(p.R, p.E, kThreads);
     const size_t bitmap = count_lds_bytes(p.R, p.E);
     const size_t bases = (size_t(p.R) * p.tab.chunks_padded + kWavesPerBlock) * sizeof(int);

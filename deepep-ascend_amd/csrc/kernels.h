@@ -296,6 +296,9 @@ struct LLDispatchParams {
 // Compute units of the current device (asked once per device).
 int compute_units();
 
+// LDS a workgroup asks for so that a CU holds at most `per_cu` of them (0: no limit).
+size_t lds_for_residency(int per_cu);
+
 hipError_t launch_ll_dispatch(const LLDispatchParams& p, hipStream_t stream);
 
 struct LLCombineParams {
