@@ -238,7 +238,7 @@ public:
             per_expert_list = *cached_num_recv_tokens_per_expert_list;
         } else if (do_cpu_sync) {
             // layout launch, which leaves the counts in the host's mailbox (no copy, no device synchronisation)
-            box = fresh_mailbox(R + num_experts + 1);
+            box = fresh_mailbox(R + num_experts + 1, run, num_cpu_timeout_secs_);
             args.phases = DEEP_EP_HIP_PHASE_LAYOUT;
             args.host_counts = box;
             check_abi(deep_ep_hip_launch_dispatch(&args, stream_ptr), "dispatch layout");

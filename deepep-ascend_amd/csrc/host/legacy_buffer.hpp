@@ -259,7 +259,7 @@ public:
                 // the per-expert counts are the caller's tensor and are copied back with the per-rank ones.
                 args.phases = DEEP_EP_HIP_PHASE_LAYOUT;
                 if (topk_idx.has_value()) {
-                    box = fresh_mailbox(R + num_experts + 1);
+                    box = fresh_mailbox(R + num_experts + 1, run, 300);
                     args.host_counts = box;
                     check_abi(deep_ep_hip_launch_intranode_dispatch(&args, stream_ptr), "intranode dispatch layout");
                     args.host_counts = nullptr;

@@ -313,10 +313,19 @@ protected:
         device_ = torch::Device(torch::kCUDA, comm_stream_.device_index());
     }
 
+    // The mailbox goes back to a pool that other pinned tensors come from: not while a launch may still write to it.
+    ~HostRuntime() {
+        try {
+            drain_mailbox(0);
+        } catch (...) {
+        }
+    }
+
     void release() {
         EP_HIP_HOST_ASSERT(explicitly_destroy_);
         EP_HIP_HOST_ASSERT(not destroyed_);
         c10::hip::device_synchronize();
+        mail_stream_.reset();
         workspace_.reset();
         status_read_.reset();
         destroyed_ = true;
@@ -414,20 +423,38 @@ protected:
     // The mailbox through which a layout launch tells the host its counts (deep_ep_hip_dispatch_args::host_counts): pinned
     // host memory the kernel writes directly, zeroed here, so that sizing the outputs takes no device-to-host copy and no
     // device synchronisation (the reference's host-mapped counters, csrc/elastic/buffer.hpp:1019-1066).
-    int32_t* fresh_mailbox(int entries) {
+    // A call that has thrown since its layout launch, before its wait, has left a launch behind that will still write here: the
+    // mailbox is handed out again only when `mail_stream_`, where that launch was queued, has run dry (waited for `timeout_secs`).
+    int32_t* fresh_mailbox(int entries, const Stream& stream, int timeout_secs) {
         if (not mailbox_.has_value())
             mailbox_ = torch::zeros({DEEP_EP_HIP_MAX_RANKS + DEEP_EP_HIP_MAX_EXPERTS + 1},
                                     torch::TensorOptions().dtype(torch::kInt32).pinned_memory(true));
         EP_HIP_HOST_ASSERT(entries <= mailbox_->numel());
+        if (not drain_mailbox(timeout_secs))
+            throw EPException("DeepEP HIP backend: dispatch: timed out waiting for the layout launch of an earlier call");
         int32_t* box = mailbox_->data_ptr<int32_t>();
         std::fill(box, box + entries, 0);
+        mail_stream_ = stream;
         return box;
+    }
+
+    // Waits until no launch can write to the mailbox any more; false on a timeout.
+    bool drain_mailbox(int timeout_secs) {
+        const auto deadline = deadline_after(timeout_secs);
+        while (mail_stream_.has_value() and not mail_stream_->query())
+            if (std::chrono::steady_clock::now() > deadline) return false;
+        mail_stream_.reset();
+        return true;
+    }
+
+    static std::chrono::steady_clock::time_point deadline_after(int timeout_secs) {
+        return std::chrono::steady_clock::now() + std::chrono::seconds(timeout_secs > 0 ? timeout_secs : 300);
     }
 
     // Waits (bounded by the buffer's CPU timeout) until the kernel has published all `entries` values; decodes them in
     // place.  Returns false on a timeout.
-    static bool await_mailbox(int32_t* box, int entries, int timeout_secs) {
-        const auto deadline = std::chrono::steady_clock::now() + std::chrono::seconds(timeout_secs > 0 ? timeout_secs : 300);
+    bool await_mailbox(int32_t* box, int entries, int timeout_secs) {
+        const auto deadline = deadline_after(timeout_secs);
         volatile int32_t* watched = box;
         uint32_t spins = 0;
         for (int i = 0; i < entries; ++i) {
@@ -437,6 +464,7 @@ protected:
             }
             box[i] = -watched[i] - 1;
         }
+        mail_stream_.reset();
         return true;
     }
 
@@ -468,6 +496,7 @@ protected:
     torch::Device device_ = torch::Device(torch::kCUDA, 0);
     std::optional<torch::Tensor> workspace_;
     std::optional<torch::Tensor> mailbox_;            // pinned: counts of a layout launch for a call that waits for them
+    std::optional<Stream> mail_stream_;               // stream of a layout launch whose counts have not been read yet
     std::optional<torch::Tensor> status_host_;        // one pinned int32: where poll_device_status has the status copied
     std::optional<EventHandle> status_read_;          // recorded after the read in flight
 };
