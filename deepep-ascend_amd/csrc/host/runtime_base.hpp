@@ -345,7 +345,7 @@ protected:
     struct StreamScope {
         HostRuntime& buffer;
         Stream compute_stream, run_stream;
-        bool allocate_on_comm_stream, async_with_compute_stream, switched = false;
+        bool allocate_on_comm_stream, async_with_compute_stream, switched = false, finished = false;
 
         StreamScope(HostRuntime& b, const std::optional<EventHandle>& previous_event, bool allocate_on_comm, bool async,
                     bool v1_rules = false)
@@ -367,12 +367,19 @@ protected:
             else if (run_stream != compute_stream) stream_wait(run_stream, compute_stream);
         }
 
+        // A call that threw may have queued launches that read the caller's tensors: what follows on the caller's stream, which
+        // may reuse their memory, is ordered behind them.
         ~StreamScope() {
             if (switched) c10::hip::setCurrentHIPStreamMasqueradingAsCUDA(compute_stream);
+            if (finished or run_stream == compute_stream) return;
+            try {
+                stream_wait(compute_stream, run_stream);
+            } catch (...) {
+            }
         }
 
         std::optional<EventHandle> finish(std::initializer_list<std::optional<torch::Tensor>> tensors) {
-            buffer.last_stream_ = run_stream;
+            finished = true;
             std::optional<EventHandle> event;
             if (run_stream != compute_stream) {
                 if (async_with_compute_stream) {
@@ -410,6 +417,7 @@ protected:
             c10::hip::HIPStreamGuardMasqueradingAsCUDA on_run(run);
             workspace_ = torch::zeros({size}, torch::TensorOptions().dtype(torch::kUInt8).device(device_));
         }
+        last_stream_ = run;                      // already now: a call that throws further down may have queued launches
         return *workspace_;
     }
 

@@ -67,3 +67,49 @@ def test_counts_of_a_thrown_call_are_not_taken_for_the_next_ones(surface):
     assert torch.equal(recv_x.cpu().view(torch.int16), ref.recv_x.view(torch.int16))
     assert torch.equal(recv_idx.cpu(), ref.recv_topk_idx)
     del keep
+
+
+@pytest.mark.parametrize("surface", ["elastic", "legacy"])
+def test_work_after_a_thrown_call_is_ordered_behind_it(surface):
+    """The thrown call's launches read its inputs and use the buffer's workspace: neither what follows on the caller's stream nor the
+    next call on the buffer, on whatever stream, may run before them."""
+    buf = _buffer(surface)
+    end, keep = _throw_behind_a_busy_stream(buf, surface)
+    after = torch.cuda.Event()
+    after.record()
+    after.synchronize()
+    assert end.query(), "the caller's stream did not wait for the launches of the call that threw"
+
+    end, keep = _throw_behind_a_busy_stream(buf, surface)
+    other = torch.cuda.Stream()
+    with torch.cuda.stream(other):
+        buf.get_dispatch_layout(keep[0], E)
+        after.record()
+    after.synchronize()
+    assert end.query(), "the next call on the buffer did not wait for the launches of the call that threw"
+
+
+def test_a_low_latency_call_does_not_stand_for_the_dispatches_before_it():
+    """It uses a workspace of its own: a later call on its stream still waits for dispatches queued on another."""
+    import deep_ep
+    buf = deep_ep.Buffer(deep_ep.LogicalGroup(0, R), low_latency_mode=True)
+    case = rc.small("behind", 64, 512, E, R, K, seed=72)
+    x, idx, w = case.x.cuda(), case.topk_idx.cuda(), case.topk_weights.cuda()
+    a, b = torch.randn((8192, 8192), device="cuda"), torch.empty((8192, 8192), device="cuda")
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    for products in (1, 12):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(first):
+            for _ in range(products):
+                torch.mm(a, a, out=b)
+            buf.get_dispatch_layout(idx, E)
+            end = torch.cuda.Event()
+            end.record()
+        with torch.cuda.stream(second):
+            buf.low_latency_dispatch(x, idx, 64, E, use_fp8=False)
+            assert products == 1 or not end.query(), "the products were over too early for this test to say anything"
+            buf.get_dispatch_layout(idx, E)
+            after = torch.cuda.Event()
+            after.record()
+        after.synchronize()
+        assert end.query()
