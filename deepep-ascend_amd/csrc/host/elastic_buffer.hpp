@@ -225,10 +225,12 @@ public:
         // Sizes of the outputs.  With a CPU sync they are exact: known before the move is launched, or, for outputs small enough
         // to be allocated at their bound, read from the mailbox once it is (allocation and launch run beside the layout).
         const int64_t row_bound = int64_t(num_tokens) * std::min(num_topk, R);
+        const int64_t bytes_by_row = hidden * int64_t(c10::elementSize(out_dtype)) + num_sf_packs * 4 + (num_topk + 2) * 4 + num_topk * 8 +
+                                     (topk_weights.has_value() ? num_topk * 4 : 0);
         const bool up_front = do_cpu_sync and not cached_mode and not do_expand and num_tokens > 0 and
                               not previous_event_before_epilogue.has_value() and
                               not (sf_dtype.has_value() and use_tma_aligned_col_major_sf) and      // its strides follow the row count
-                              row_bound * hidden * int64_t(c10::elementSize(out_dtype)) <= kUpFrontRowBytes;
+                              row_bound * bytes_by_row <= kUpFrontBytes;
         int32_t* box = nullptr;
         int num_recv_tokens, num_expanded_tokens;
         std::vector<int> per_expert_list;

@@ -205,10 +205,11 @@ public:
         void* stream_ptr = run.stream();
 
         // With top-k tensors and outputs small enough to be allocated at their bound, the exact counts are read from the mailbox
-        // once the move is launched (see kUpFrontRowBytes).
+        // once the move is launched (see kUpFrontBytes).
         const int64_t row_bound = int64_t(num_tokens) * std::min(num_topk, R);
+        const int64_t bytes_by_row = hidden * int64_t(x.element_size()) + num_scales * 4 + 4 + num_topk * 12;
         const bool up_front = not cached_mode and num_worst_tokens == 0 and topk_idx.has_value() and num_tokens > 0 and
-                              row_bound * hidden * int64_t(x.element_size()) <= kUpFrontRowBytes;
+                              row_bound * bytes_by_row <= kUpFrontBytes;
         int32_t* box = nullptr;
         int num_recv_tokens;
         std::vector<int> per_expert_list;

@@ -172,14 +172,16 @@ inline torch::Tensor first_rows(const torch::Tensor& t, int64_t rows) {
     return torch::Tensor(std::move(impl));
 }
 
-// Outputs of up to this many bytes are allocated for as many rows as the call could receive, so that a call that returns exact
-// sizes allocates them and launches its move while its layout launch runs, and waits for the counts last.  With the wait in
-// between the GPU idled while the host allocated and launched: 1237 x 2888 BF16 over 6 ranks, dispatch + combine, takes
-// 38.0 us instead of 43.0, 128 x 1024 over 2 ranks 28.0 instead of 31.8.
-// Rows then hold about half as much again as needed (uniform top-8 routing over 8 ranks); beyond this size that is worth more
-// than the few microseconds.  (A single launch in place of the two is no gain here: its publisher hands the counts to the
-// host later than a layout launch does.)
-constexpr int64_t kUpFrontRowBytes = int64_t(256) << 20;
+// A call that returns exact sizes allocates its outputs for as many rows as it could receive, and launches its move, while its
+// layout launch runs, and waits for the counts last, if all it would allocate by the row - payload, scales, indices, weights, the
+// handle's row records - comes to no more than this.  With the wait in between the GPU idled while the host allocated and
+// launched: 1237 x 2888 BF16 top-9 over 6 ranks (44 MB), dispatch + combine, takes 38.0 us instead of 43.0, 128 x 1024 over 2
+// ranks 28.0 instead of 31.8.  (A single launch in place of the two is no gain here: its publisher hands the counts to the host
+// later than a layout launch does.)
+// The tensors keep that memory: half as much again as they need with uniform top-8 routing over 8 ranks, min(top-k, ranks) times
+// as much where every token goes to one rank, without limit where selections are masked.  The bound is on what a call can hold
+// in vain; a call that could receive more allocates what it does receive.
+constexpr int64_t kUpFrontBytes = int64_t(64) << 20;
 
 // A few (key tensor -> companion tensor) pairs a buffer remembers about handles it has produced.  The key is held
 // weakly and compared by identity, so an entry can only be found through the very tensor object the buffer returned:

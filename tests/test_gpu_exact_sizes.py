@@ -1,5 +1,6 @@
-"""Exact-size dispatches on either side of the size up to which outputs are allocated at their bound (256 MiB of rows) before
-the counts are known: the tensors have the exact number of rows, are contiguous, and hold the tokens they should."""
+"""Exact-size dispatches on either side of the size up to which outputs are allocated at their bound (64 MiB in all) before the
+counts are known: the tensors have the exact number of rows, are contiguous, hold the tokens they should, and past that size no
+memory beyond them."""
 import pytest
 import torch
 
@@ -8,7 +9,7 @@ import routing_oracle as oracle
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = {"at_the_limit": (2048, 8192, 8), "past_the_limit": (2049, 8192, 8), "one_token": (1, 1024, 8), "one_rank": (300, 1024, 1)}
+SHAPES = {"at_the_limit": (507, 8192, 8), "past_the_limit": (509, 8192, 8), "far_past_the_limit": (2049, 8192, 8), "one_token": (1, 1024, 8), "one_rank": (300, 1024, 1)}
 
 
 @pytest.mark.parametrize("surface", ["elastic", "legacy"])
@@ -41,3 +42,37 @@ def test_exact_rows(shape, surface):
         assert list(per_expert) == ref.num_unaligned_recv_tokens_per_expert.tolist()
         assert torch.equal(tokens.cpu().int(), ref.recv_src_metadata[:, 0])
         assert torch.equal(recv_x, x[tokens])
+
+
+# T, H, R, K, FP8: rows of 776 bytes of which the payload is 256, so that 4096 x 32 of them pass the limit by what travels beside
+# it; and whole rows, FP8 with scales and BF16
+MASKED = {"narrow_rows": (4096, 128, 32, 32, False), "fp8_rows": (4096, 7168, 8, 8, True), "bf16_rows": (2049, 7168, 8, 8, False),
+          "small": (300, 7168, 8, 8, True)}
+
+
+@pytest.mark.parametrize("surface", ["elastic", "legacy"])
+@pytest.mark.parametrize("shape", MASKED)
+def test_memory_kept_with_mostly_masked_routing(shape, surface):
+    import deep_ep
+    from deep_ep.utils.math import per_token_cast_to_fp8
+    T, H, R, K, fp8 = MASKED[shape]
+    E = 64
+    case = rc.small(shape, T, H, E, R, K, seed=62, masked_ratio=0.97)
+    x, idx, w = case.x.cuda(), case.topk_idx.cuda(), case.topk_weights.cuda()
+    payload = per_token_cast_to_fp8(x) if fp8 else x
+    if surface == "elastic":
+        buf = deep_ep.ElasticBuffer(deep_ep.LogicalGroup(0, R), num_max_tokens_per_rank=T, hidden=H, num_topk=K)
+        recv, recv_idx, recv_w, handle, _ = buf.dispatch(payload, idx, w, num_experts=E)
+        records = handle.recv_src_metadata
+    else:
+        buf = deep_ep.Buffer(deep_ep.LogicalGroup(0, R))
+        per_rank, _, counts, in_rank, _ = buf.get_dispatch_layout(idx, E)
+        recv, recv_idx, recv_w, _, handle, _ = buf.dispatch(payload, num_tokens_per_rank=per_rank, is_token_in_rank=in_rank,
+                                                            num_tokens_per_expert=counts, topk_idx=idx, topk_weights=w)
+        records = handle[3]
+    tensors = [*(recv if fp8 else (recv,)), recv_idx, recv_w, records]
+    kept = sum({t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() for t in tensors}.values())
+    needed = sum(t.numel() * t.element_size() for t in tensors)
+    assert kept <= (64 << 20)
+    if shape != "small":
+        assert kept <= needed + 256 * len(tensors)
