@@ -290,6 +290,8 @@ __device__ bool write_expert_bases_from_registers(const LayoutTables& t, const u
 // chunk's totals and nothing is loaded.  scratch: LDS of publish_scratch_ints.
 // From the ticket to the end it took 3.4 us at 16 chunks, 9 us at 64 chunks over 32 ranks, with LDS scans of five
 // barriers and 32 chunks at most; the whole launch went from 10.0 to 8.3 and from 14.8 to 11.5 us.
+// Chunks past the 32 in registers are read again for the expert bases, sixteen a trip: one at a time, each load behind the store
+// before it, an expanded layout took 41.7 us at 65536 tokens over 8 ranks, 13.8 at 16384 over 32, and takes 29.1 and 12.2.
 inline __host__ __device__ int publish_scratch_ints(int R, int threads) { return R + 2 * (threads / kWaveSize); }
 
 template <int kThreads, bool kOneChunk>
@@ -307,6 +309,15 @@ __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutT
     vec16 rv[kMaxVecs];
     int v[kColumn];
     int rows = 0, count = 0;
+    const int column = has_expert ? tid : 0;
+    auto load_sixteen = [&](int first, int* to) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            // a row start common to the workgroup plus the thread's column: one address register serves all loads
+            const int row_start = __builtin_amdgcn_readfirstlane(min(first + u, num_chunks - 1) * t.experts_padded);
+            to[u] = t.expert_counts[row_start + column];
+        }
+    };
     if constexpr (kOneChunk) {
         rv[0] = vec16{tid < q.R ? uint32_t(totals[tid]) : 0u, 0, 0, 0};          // rows of four, three of them padding
         v[0] = has_expert ? totals[q.R + tid] : 0;
@@ -319,15 +330,6 @@ __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutT
             const int begin = (tid * vecs + i) * 4;
             if (i < vecs && begin < flat) rv[i] = load16(t.rank_counts + begin);
         }
-        const int column = has_expert ? tid : 0;
-        auto load_sixteen = [&](int first, int* to) {
-#pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                // a row start common to the workgroup plus the thread's column: one address register serves all loads
-                const int row_start = __builtin_amdgcn_readfirstlane(min(first + u, num_chunks - 1) * t.experts_padded);
-                to[u] = t.expert_counts[row_start + column];
-            }
-        };
         auto sum_sixteen = [&](int first, const int* of) {
 #pragma unroll
             for (int u = 0; u < 16; ++u) count += first + u < num_chunks ? of[u] : 0;
@@ -402,11 +404,16 @@ __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutT
             }
         }
         if constexpr (!kOneChunk) {
-            for (int c = kColumn; c < num_chunks; ++c) {
-                const int row_start = c * t.experts_padded;
-                const int here = t.expert_counts[row_start + tid];
-                t.expert_bases[row_start + tid] = at;
-                at += here;
+            for (int c0 = kColumn; c0 < num_chunks; c0 += 16) {
+                int w[16];
+                load_sixteen(c0, w);
+#pragma unroll
+                for (int u = 0; u < 16; ++u) {
+                    if (c0 + u < num_chunks) {
+                        t.expert_bases[__builtin_amdgcn_readfirstlane((c0 + u) * t.experts_padded) + tid] = at;
+                        at += w[u];
+                    }
+                }
             }
         }
     }

@@ -1,6 +1,7 @@
 """The layout pass at the sizes where it changes its way of working: one chunk of 256 tokens (handed over in LDS) and more, 16 and
-32 chunks (columns held in registers), 64 ranks (membership by ballot), 8 and 12 routing lanes (kernel variants), more experts
-than threads (the general publishing step).  Counts, prefix sums and placements are integers: exactly the oracle's."""
+32 chunks (columns held in registers), 48 and one more (sixteen a trip beyond), 64 ranks (membership by ballot), 8 and 12 routing
+lanes (kernel variants), more experts than threads (the general publishing step).  Counts, prefix sums and placements are
+integers: exactly the oracle's."""
 import pytest
 import torch
 
@@ -12,7 +13,7 @@ pytestmark = pytest.mark.gpu
 SHAPES = [  # T, K, E, R
     (1, 8, 256, 8), (256, 8, 256, 8), (257, 8, 256, 8), (255, 12, 256, 64), (256, 3, 65, 65), (256, 8, 320, 8), (100, 1, 1, 1),
     (4096, 8, 256, 16), (4097, 9, 256, 17), (1237, 13, 72, 6), (8193, 8, 256, 32), (8192, 8, 320, 64), (16385, 8, 128, 64),
-    (2048, 2, 130, 65),
+    (2048, 2, 130, 65), (12288, 4, 64, 8), (12289, 4, 64, 8),
 ]
 
 
