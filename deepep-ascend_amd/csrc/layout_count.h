@@ -86,10 +86,11 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
     // Straight-line code from here on, no branch per routing lane: the LDS atomics of all lanes issue back to back, and
     // so do the LDS reads of the position step further down.  A lane without an expert ORs nothing into a word of its
     // own (not one word for all of them: atomics of one wavefront on one address take turns).
-    // Up to 64 ranks many lanes of a wavefront would meet on the same few rank words, so the rank bitmaps are taken by
-    // ballot instead: one per rank over "this token goes to rank r", no atomics (by atomics
-    // the bits took 3.5 us to set at 32 ranks, against 1.1 us by ballot at 8).
-    constexpr int kBallotRanks = 64;
+    // With few ranks most lanes of a wavefront would meet on the same few rank words, so the rank bitmaps are taken by
+    // ballot instead: one per rank over "this token goes to rank r", no atomics.  Past 16 ranks the ballots cost more than the
+    // atomics (layout launch of 4096 tokens, top-8: 24 ranks 8.2 us by ballot and 7.7 by atomics, 32 ranks 8.7 and 7.8, 64 ranks
+    // 9.9 and 7.8; 4096 x 2048 fused cast in one launch over 64 ranks 28.5 and 24.2).
+    constexpr int kBallotRanks = 16;
     const bool ranks_by_ballot = p.R <= kBallotRanks;
     int e[KMAX], d[KMAX];
     unsigned long long seen = 0;
