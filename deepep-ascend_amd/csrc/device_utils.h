@@ -158,6 +158,18 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
     return v;
 }
 
+// The same by shuffles, for workgroups of which several share a CU with others that hold loads under way: single-launch
+// movers with the DPP form took about 0.7 us longer (1024 x 7168 fused cast, 8 ranks: 19.9 against 19.0 us).
+__device__ __forceinline__ int wave_inclusive_sum_by_shuffles(int v) {
+    const int lane = lane_id();
+#pragma unroll
+    for (int off = 1; off < kWaveSize; off <<= 1) {
+        const int o = __shfl_up(v, off, kWaveSize);
+        if (lane >= off) v += o;
+    }
+    return v;
+}
+
 // Workgroups are handed to the 8 XCDs (each with its own L2) round-robin: workgroup i runs on XCD i % 8.
 // This renumbering gives every XCD one contiguous range of logical workgroups, so that neighbouring
 // work items (which write neighbouring output rows) share an L2 and their partial-line writes merge.

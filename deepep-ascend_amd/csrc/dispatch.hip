@@ -440,7 +440,7 @@ __device__ __forceinline__ bool build_rank_bases(const MoveParams& p, uint64_t l
     const int v0 = int(uint32_t(lo) & kTagValueMask), v1 = int(uint32_t(lo >> 32) & kTagValueMask);
     const int v2 = int(uint32_t(hi) & kTagValueMask), v3 = int(uint32_t(hi >> 32) & kTagValueMask);
     const int sum = v0 + v1 + v2 + v3;
-    const int inc = wave_inclusive_sum(sum);
+    const int inc = wave_inclusive_sum_by_shuffles(sum);
     if (lane == kWaveSize - 1) scan_tmp[wave] = inc;
     const int all_complete = __syncthreads_and(complete ? 1 : 0);
     int run = inc - sum;

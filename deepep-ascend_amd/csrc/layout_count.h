@@ -67,10 +67,11 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
             for (int k = 0; k < KMAX; ++k) raw[k] = -1;
         }
     } else {
-        // clamped columns instead of a branch around each load: all of a token's loads go out together
+        // Clamped columns instead of a branch around each load: all of a token's loads go out together.  Not beside movers,
+        // whose payload the loads of absent lanes would wait with.
 #pragma unroll
-        for (int k = 0; k < KMAX; ++k) raw[k] = -1;
-        if (active) {
+        for (int k = 0; k < KMAX; ++k) raw[k] = kThrough && active && k < p.K ? p.topk_idx[int64_t(t) * p.K + k] : int64_t(-1);
+        if (!kThrough && active) {
             const int64_t* row = p.topk_idx + int64_t(t) * p.K;
 #pragma unroll
             for (int k = 0; k < KMAX; ++k) raw[k] = row[min(k, p.K - 1)];
@@ -101,11 +102,9 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
     uint64_t my_ranks = 0;                       // bit r: this token goes to rank r
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) {
-        const uint32_t lo = uint32_t(raw[k]);
-        const int hi = int(raw[k] >> 32);
-        const bool valid = hi == 0 && lo < uint32_t(p.E);
-        if (hi >= 0 && !valid) flags |= DEEP_EP_HIP_STATUS_EXPERT_OUT_OF_RANGE;
-        e[k] = valid ? int(lo) : -1;
+        const bool valid = raw[k] >= 0 && raw[k] < p.E;
+        if (raw[k] >= p.E) flags |= DEEP_EP_HIP_STATUS_EXPERT_OUT_OF_RANGE;
+        e[k] = valid ? int(raw[k]) : -1;
         d[k] = valid ? small_div(e[k], rcp_experts_per_rank) : -1;
         const uint64_t bit = valid ? my_bit : 0ull;
         unsigned long long* word = reinterpret_cast<unsigned long long*>(&bitmap[valid ? (p.R + e[k]) * kWaves + wave : idle_word]);
@@ -235,12 +234,9 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
         }
     }
     if (p.pos != nullptr && seen != 0) flags |= DEEP_EP_HIP_STATUS_DUPLICATE_EXPERT;
-    if (flags != 0) atomicOr(p.status, flags);
 
-    hand_off();
-
-    if (!active) return;
-    if (p.pos != nullptr) {
+    auto store_positions = [&] {
+        if (!active || p.pos == nullptr) return;
         if (KMAX == 8 && p.K == 8) {
             vec16* dst = reinterpret_cast<vec16*>(p.pos + int64_t(t) * 8);
             const vec16 lo{packed[0], packed[1], packed[2], packed[3]}, hi{packed[4], packed[5], packed[6], packed[7]};
@@ -256,9 +252,17 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
             for (int k = 0; k < KMAX; ++k)
                 if (k < p.K) store_word<kThrough>(reinterpret_cast<int*>(p.pos) + int64_t(t) * p.K + k, int(packed[k]));
         }
+    };
+    if constexpr (kThrough) store_positions();           // movers of this launch are waiting for them
+    if (flags != 0) atomicOr(p.status, flags);
+
+    hand_off();
+
+    if constexpr (!kThrough) {
+        store_positions();
+        copy_indices();
     }
-    if constexpr (!kThrough) copy_indices();
-    if (p.is_token_in_rank != nullptr) {
+    if (active && p.is_token_in_rank != nullptr) {
         for (int r = 0; r < p.R; ++r)
             p.is_token_in_rank[int64_t(t) * p.R + r] = uint8_t((bitmap[r * kWaves + wave] >> lane) & 1ull);
     }
