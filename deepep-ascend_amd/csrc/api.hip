@@ -58,7 +58,7 @@ struct LaunchPlan {
 constexpr int64_t kMaxFusedMovers = 16384;
 
 LaunchPlan plan_launches(int T, int K, int E, int R, bool do_layout, bool do_move, bool do_expand, int alignment, int payload, int H,
-                         int row_bytes, const deep_ep_hip_tuning& tuning) {
+                         int row_bytes, const deep_ep_hip_tuning& tuning, int64_t rows_of_rank_lanes = -1 /* no top-k: rows received */) {
     LaunchPlan q{};
     q.chunks = T > 0 ? (T + kLayoutChunk - 1) / kLayoutChunk : 1;
     q.chunks_padded = (q.chunks + 3) / 4 * 4;
@@ -84,6 +84,7 @@ LaunchPlan plan_launches(int T, int K, int E, int R, bool do_layout, bool do_mov
         probe.T = T; probe.H = H; probe.row_bytes = row_bytes; probe.payload = payload; probe.do_expand = do_expand ? 1 : 0;
         probe.cast_pairs = tuning.cast_pairs; probe.copy_vecs = tuning.copy_vecs;
         probe.K = K; probe.R = R; probe.fused = 1;
+        probe.rank_lanes = rows_of_rank_lanes >= 0 ? 1 : 0; probe.recv_capacity = rows_of_rank_lanes;
         // BF16 rows from 300 MB on: 4096 x 7168 takes 78.7 us in one launch and 74.5 in two, 8192 x 7168 155 against 134, while
         // 2048 x 7168 (154 MB) takes 40.2 against 44.3 and 16384 x 2048 top-6 (295 MB) 76.3 against 80.4.
         q.fused = dispatch_move_workgroups(probe) <= kMaxFusedMovers && !copy_prefers_finished_layout(probe);
@@ -612,7 +613,8 @@ int deep_ep_hip_launch_intranode_dispatch(const deep_ep_hip_intranode_dispatch_a
     pub.expert_start = reinterpret_cast<int32_t*>(ws + w.expert_start);
     pub.totals_out = reinterpret_cast<int32_t*>(ws + w.totals);
 
-    const LaunchPlan plan = plan_launches(T, K, E, R, do_layout, do_move, false, 1, a->payload, H, H * elem_in, a->tuning);
+    const LaunchPlan plan = plan_launches(T, K, E, R, do_layout, do_move, false, 1, a->payload, H, H * elem_in, a->tuning,
+                                          with_topk ? -1 : a->recv_capacity);
     LayoutParams lay{};
     lay.topk_idx = a->topk_idx;
     lay.route_mask = with_topk ? nullptr : a->is_token_in_rank;
