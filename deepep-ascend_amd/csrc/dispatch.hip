@@ -754,6 +754,7 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
             if (lane < p.num_sf_packs) to[int64_t(lane) * p.rsf_hs] = pack;
             for (int g = lane + kWaveSize; g < p.num_sf_packs; g += kWaveSize)        // rows beyond 8192 channels
                 to[int64_t(g) * p.rsf_hs] = p.sf[int64_t(t) * p.sf_ts + int64_t(g) * p.sf_hs];
+            if (!kFused && p.row_by_row) wait_for_own_stores();
         }
     }
 }
@@ -1264,6 +1265,13 @@ static double row_bytes_out(const MoveParams& p) {
     return double(p.T) * (cast ? p.H : p.row_bytes) * rows_per_token(p);
 }
 
+// A launch of so many workgroups of this tile that they fill `rounds` rounds of eight per CU.
+static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
+    const int bytes = p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? p.H : p.row_bytes;
+    const int64_t wavefronts = int64_t(p.T) * ((bytes + tile * 1024 - 1) / (tile * 1024));
+    return wavefronts >= int64_t(compute_units()) * rounds * 8 * kWavesPerBlock;
+}
+
 // Column tile of a move launch: 1024-channel segments per wavefront for the fused cast, KB of row per wavefront for
 // the pass-through payloads.
 static int move_tile(const MoveParams& p) {
@@ -1292,6 +1300,16 @@ static int move_tile(const MoveParams& p) {
     return rows_per_token(p) >= 4.0 ? 1 : (kb >= 2 ? 2 : 1);
 }
 
+// Rows of one KB tile with scale packs: their payload and packs, 32 bytes to a row, are partial lines of as many buckets as there
+// are ranks, which the caches merge the better the fewer of them are under way.  A wavefront that waits for the stores of a
+// row before it starts the next takes, against none that does (65536 x 1024 top-8): 8 ranks 98.7 us for 102.6, 32 ranks 123
+// for 141, 64 ranks 134 for 164; 16384 tokens over 8 ranks 30.5 for 30.9.  Wider rows gain by it over 64 ranks and lose over 8
+// (32768 x 4096: 231 us for 246, 162 for 157).
+static bool stores_row_by_row(const MoveParams& p) {
+    return !p.fused && p.payload != DEEP_EP_HIP_PAYLOAD_CAST_FP8 && p.recv_sf != nullptr && p.row_bytes <= 1024 &&
+           rows_per_token(p) >= 3.5 && fills_rounds(p, 1, 2);
+}
+
 // How many workgroups of a move kernel launched on a finished layout a CU should hold at a time (0: as many as fit).
 // Scattered stores stream fastest when not too many are under way.  Move phase in us, inputs read from memory, with
 // 8 / 6 / 5 / 4 / 3 workgroups per CU:
@@ -1307,7 +1325,7 @@ static int move_workgroups_per_cu(const MoveParams& p) {
     if (p.move_workgroups_per_cu != 0)       // two is the least an LDS share within a workgroup's 64 KB can enforce
         return p.move_workgroups_per_cu >= 8 ? 0 : (p.move_workgroups_per_cu < 2 ? 2 : p.move_workgroups_per_cu);
     if (int64_t(p.num_movers) < int64_t(compute_units()) * 16) return 0;
-    if (many_rows_per_token(p)) return 5;
+    if (many_rows_per_token(p)) return stores_row_by_row(p) ? 0 : 5;
     if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) return 6;
     return move_tile(p) == 2 ? 4 : 0;
 }
@@ -1417,6 +1435,7 @@ hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream) {
     p.rcp_E_l = 1.0f / float(p.E_l);
     p.num_cus = p.fused ? compute_units() : 0;
     const int tile = move_tile(p);
+    p.row_by_row = stores_row_by_row(p) ? 1 : 0;
     if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) {
         switch (tile) {
             case 1: return launch_cast<1>(p, stream);

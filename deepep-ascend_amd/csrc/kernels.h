@@ -154,6 +154,7 @@ struct MoveParams {
     int payload;         // DEEP_EP_HIP_PAYLOAD_*
     int row_bytes;       // input row bytes
     int tiles;           // column tiles per token
+    int row_by_row;      // a wavefront waits for the stores of a row before it starts the next (set by the launcher)
     unsigned warm_lds_offset;   // single-launch cast: byte offset (in the dynamic LDS) of the 4 KB landing area of the
                                 // cache-warming loads, 0 = none
     unsigned warm_ahead;        // ... and how many work items ahead of its own a wavefront warms
