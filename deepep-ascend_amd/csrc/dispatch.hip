@@ -670,7 +670,8 @@ __device__ __forceinline__ bool warm_next_rounds_of_rows(const MoveParams& p, un
 }
 
 // ---- pass-through payload (BF16, or FP8 with caller-provided scale packs) ----
-template <int kVecs, bool kFused>
+// kScales: rows may come with scale packs (p.recv_sf).
+template <int kVecs, bool kFused, bool kScales>
 __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
     if constexpr (kFused) {
         if (blockIdx.x <= unsigned(p.count_blocks)) {
@@ -708,7 +709,7 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
     }
 
     // The caller's scale packs ride with tile 0: requested with the payload, once, not per destination row.
-    const bool packs = has_work && tile == 0 && p.recv_sf != nullptr;
+    const bool packs = kScales && has_work && tile == 0 && p.recv_sf != nullptr;
     uint32_t pack = 0;
     if (packs && lane < p.num_sf_packs) pack = p.sf[int64_t(t) * p.sf_ts + int64_t(lane) * p.sf_hs];
 
@@ -1110,13 +1111,13 @@ __global__ __launch_bounds__(kQueueThreads) void dispatch_cast_queue_kernel(cons
 // The kernels.  The single-launch forms also hold the counting and publishing code, whose register needs must not cost
 // the movers their occupancy: they are held to six wavefronts per SIMD (80 registers) - six workgroups per CU, which
 // is also where the move streams fastest (more were slower when tried with a leaner counting step, fewer are slower too).
-template <int kVecs>
+template <int kVecs, bool kScales>
 __global__ __launch_bounds__(kThreads) void dispatch_copy_kernel(const MoveParams p) {
-    dispatch_copy<kVecs, false>(p);
+    dispatch_copy<kVecs, false, kScales>(p);
 }
-template <int kVecs>
+template <int kVecs, bool kScales>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void dispatch_copy_single_launch_kernel(const MoveParams p) {
-    dispatch_copy<kVecs, true>(p);
+    dispatch_copy<kVecs, true, kScales>(p);
 }
 template <int kPairs>
 __global__ __launch_bounds__(kThreads) void dispatch_cast_kernel(const MoveParams p) {
@@ -1378,8 +1379,14 @@ hipError_t launch_copy(MoveParams p, hipStream_t stream) {
     p.tiles = (p.row_bytes + kVecs * 1024 - 1) / (kVecs * 1024);
     const unsigned blocks = move_grid(p, int64_t(p.T) * p.tiles);
     plan_cache_warming(p);
-    if (p.fused) hipLaunchKernelGGL((dispatch_copy_single_launch_kernel<kVecs>), dim3(blocks), dim3(kThreads), move_lds_bytes(p), stream, p);
-    else hipLaunchKernelGGL((dispatch_copy_kernel<kVecs>), dim3(blocks), dim3(kThreads), move_lds_bytes(p), stream, p);
+    // Rows without scale packs, in tiles of one and two KB: a kernel without the branch on the packs, with which they took 3 to 8 %
+    // longer (16384 x 7168 top-2, 1 KB tiles: 126 against 119 us; 65536 x 256 top-8 84.4 against 77.1).  Tiles of four KB and many wide
+    // rows to a token are the other way round (8192 x 2048 top-2 21.9 us without the branch, 20.5 with it; 16384 x 7168 top-8 254, 249).
+    constexpr bool kSmallTile = kVecs <= 2;
+    const bool plain = kSmallTile && p.recv_sf == nullptr && (rows_per_token(p) < 5.0 || p.row_bytes < 4096);
+    const auto kernel = p.fused ? (plain ? dispatch_copy_single_launch_kernel<kVecs, !kSmallTile> : dispatch_copy_single_launch_kernel<kVecs, true>)
+                                : (plain ? dispatch_copy_kernel<kVecs, !kSmallTile> : dispatch_copy_kernel<kVecs, true>);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), move_lds_bytes(p), stream, p);
     return hipGetLastError();
 }
 
