@@ -1256,10 +1256,6 @@ static double rows_per_token(const MoveParams& p) {
     return p.R * (1.0 - std::pow(1.0 - 1.0 / p.R, p.K));
 }
 
-// A call whose tokens go to nearly as many rows as they have selections (top-8 over 16 ranks: 6.4 rows): its stores are spread
-// over more buckets than those of eight ranks (5.3 rows).
-static bool many_rows_per_token(const MoveParams& p) { return rows_per_token(p) >= 5.8; }
-
 // The bytes of those rows.
 static double row_bytes_out(const MoveParams& p) {
     const bool cast = p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8;
@@ -1274,31 +1270,40 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 }
 
 // Column tile of a move launch: 1024-channel segments per wavefront for the fused cast, KB of row per wavefront for
-// the pass-through payloads.
+// the pass-through payloads.  A tile of one whose last wavefront of a row would be half idle loses to one of two: 65536
+// tokens x 768 BF16 over 16 ranks 152 against 175 us, fused cast of 32768 x 1152 over 32 ranks 82 against 104 us.
 static int move_tile(const MoveParams& p) {
     const bool large_input = int64_t(p.T) * p.row_bytes >= (int64_t(64) << 20);
+    const double rows = rows_per_token(p);
     if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) {
         // Two segments (2048 channels) measured best at hidden 7168 and 8 ranks: 92.8 us per dispatch against 93.7 (4
         // segments) and 96.9 (7 segments, one wavefront per token).  With many rows per token one segment is ahead on a
-        // finished layout (16384 x 7168: 32 ranks 199 against 207 us, 16 ranks 185 against 189; 8192 x 7168 expanded 118
-        // against 124 us); in a single launch, whose workgroups each work out the row bases, only for the expanded layout
-        // of a large call.
+        // finished layout, in calls of four rounds and more (16384 x 7168: 32 ranks 199 against 207 us, 16 ranks 185
+        // against 189; but 4096 x 4096 over 32 ranks 4 % behind), and in the expanded layout from two rounds on (8192 x
+        // 7168 118 against 124 us, 16384 x 4096 top-8 134 against 139); in a single launch, whose workgroups each work out
+        // the row bases, only for the expanded layout of a large call.
         if (p.cast_pairs != 0) return p.cast_pairs;
         if (p.H <= 1024) return 1;
-        return (p.fused ? p.do_expand && large_input : many_rows_per_token(p)) ? 1 : 2;
+        if (p.fused) return p.do_expand && large_input ? 1 : 2;
+        if (p.H * 8 <= (p.H + 1023) / 1024 * 7 * 1024) return 2;
+        return (p.do_expand ? fills_rounds(p, 1, 2) : rows >= 5.8 && fills_rounds(p, 1, 4)) ? 1 : 2;
     }
     if (p.copy_vecs != 0) return p.copy_vecs;
     const int kb = (p.row_bytes + 1023) / 1024;
     const int widest = kb <= 1 ? 1 : kb <= 2 ? 2 : 4;
     // Small, latency-bound calls: up to 4 KB per wavefront, so that fewer wavefronts repeat the routing work (4096 rows
-    // of 4 KB: 19.5 us against 21.1 us with 1 KB tiles).  Calls that write a quarter of a gigabyte and more are bound by
-    // their stores: one KB per wavefront where a token goes to four rows and more (BF16, 8 ranks: 4096 x 7168 66.5
-    // against 73.4 us, 8192 x 7168 126 against 145, 16384 x 2048 top-6 69.5 against 74.1), two where it goes to fewer (8192 x 7168, 4 of
-    // 4 ranks: 75.6 us with four workgroups per CU against 79.4 with 1 KB and 84.9 with 4 KB; 4096 x 7168, 2 of 2 ranks,
-    // 88 MB of rows: 28.4 against 31.0 and 28.8).
+    // of 4 KB: 19.5 us against 21.1 us with 1 KB tiles).  Calls that write 200 MB and more are bound by their stores.
+    // Rows of up to 3 KB then take 2 KB (32768 x 1536 top-8: 8 ranks 97 against 104 us, 64 ranks 133 against 146), wider
+    // (whole KB in the expanded layout and in V1 calls without top-k tensors, which write little or nothing beside the rows, 1 KB:
+// 32768 x 1024 top-8 over 8 ranks 119 against 127 us, cached V1 77 against 84) ones 1 KB where a token goes to 3.5 rows and more (BF16, 8 ranks: 4096 x 7168 66.5 against 73.4 us, 8192 x 7168 126
+    // against 145; 16384 x 7168 top-4 of 16 ranks, 3.6 rows, 194 against 206), 2 KB where it goes to fewer (8192 x 7168, 4 of
+    // 4 ranks: 75.6 us with four workgroups per CU against 79.4 with 1 KB and 84.9 with 4 KB) and, below five, over 64 ranks
+    // (32768 x 2048 top-4: 126 us against 147).  At 183 MB (16384 x 2048, 4 of 4 ranks) 2 and 4 KB measured the same.
     if (p.fused) return large_input ? 1 : widest;
-    if (row_bytes_out(p) < 256e6) return widest;
-    return rows_per_token(p) >= 4.0 ? 1 : (kb >= 2 ? 2 : 1);
+    if (row_bytes_out(p) < 200e6) return widest;
+    const bool whole = p.row_bytes * 8 > kb * 7 * 1024;           // no wavefront of 1 KB would be half idle
+    if (kb <= 3) return kb == 1 || (p.rank_lanes && rows >= 5.0) || ((p.rank_lanes || p.do_expand) && whole) ? 1 : 2;
+    return rows >= (p.rank_lanes ? 2.5 : 3.5) && !(p.R >= 64 && rows < 5.0) ? 1 : 2;
 }
 
 // Rows of one KB tile with scale packs: their payload and packs, 32 bytes to a row, are partial lines of as many buckets as there
@@ -1312,23 +1317,38 @@ static bool stores_row_by_row(const MoveParams& p) {
 }
 
 // How many workgroups of a move kernel launched on a finished layout a CU should hold at a time (0: as many as fit).
-// Scattered stores stream fastest when not too many are under way.  Move phase in us, inputs read from memory, with
-// 8 / 6 / 5 / 4 / 3 workgroups per CU:
-//   fused cast, 8192 x 7168, 8 ranks           81.4 / 80.8 / 80.6 / 82.2;   expanded 119.9 / 120.0 / 118.4 / 119.0
-//   fused cast, 16384 x 7168, 32 ranks, 1 KB   212 / 201 / 199 / 203 / 228; 16384 x 4096, 64 ranks 150 / 133 / 130 / 134 / 153
-//   BF16, 16384 x 7168, 32 ranks, 1 KB         363 / 362 / 354 / 346 / 385; 16 ranks 312 / 312 / 304 / 314 / 357
-//   BF16, 16384 x 4096, 64 ranks, 1 KB         264 / 237 / 222 / 239 / 276
-//   BF16, 8192 x 7168, 8 ranks, 1 KB           126 / 126 / 128 / 137 / 151: left alone
-//   BF16, 8192 x 7168, 4 of 4 ranks, 2 KB       82 /  80 /  77 /  76;       16384 x 4096, 4 of 16 ranks 123 / 124 / 123 / 119 / 117
-// Launches that would not fill two rounds of eight per CU are left alone.
+// Scattered stores stream fastest when not too many are under way: the more rows a token has, the more ranks they are spread
+// over and the wider they are, the fewer.  Move phase in us, inputs read from memory, with 8 / 6 / 5 / 4 workgroups per CU:
+//   fused cast, 8192 x 7168, 8 ranks           81.4 / 80.8 / 80.6 / 82.2;   16384 x 7168, 64 ranks 1 KB 272 / 241 / 228
+//   fused cast, expanded, 16384 x 4096 top-4    84 /  89 /  92;              8192 x 7168 top-8 1 KB 122 / 123 / 121: left alone
+//   BF16, 16384 x 7168, 32 ranks, 1 KB         363 / 362 / 354 / 346;       16 ranks 312 / 312 / 304 / 314
+//   BF16, 16384 x 7168, 8 ranks, 1 KB          255 / 249 / 254 / 271;       16384 x 2048 80.8 / 82.2 / 86.8: left alone
+//   BF16, 16384 x 2048, 64 ranks top-6, 1 KB   116 /  95 /  97 / 105;       16 ranks top-8 99.7 / 99.7 / 101 / 109
+//   BF16, 65536 x 768, 2 KB, top-8: 8 ranks    122 / 117 / 116 / 122;       64 ranks top-6 203 / 168 / 143 / 140
+//   BF16, 65536 x 768, 2 KB, top-2 of 2 ranks 50.9 / 52.1 / 55.0 / 62.0: left alone
+//   BF16, 65536 x 512, 64 ranks top-6, 1 KB    140 / 122 / 118 / 123;       65536 x 256 77 / 83 / 88 / 98 (8 ranks): left alone
+//   BF16, 8192 x 7168, 4 of 4 ranks, 2 KB       82 /  80 /  77 /  76;       32768 x 2048, 2 of 2 ranks 60.4 / 62.5 / 63 / 64.3
+//   BF16, 16384 x 7168 top-2 of 8 ranks, 2 KB 123 / 121 / 119 / 118;       the same in FP8 63.5 / 67.1 / 66 / 68.4: left alone
+//   BF16, cached V1, 32768 x 2048, 32 ranks    201 / 211, 65536 x 768, 16 ranks 137 / 137 / 153: left alone
+// Launches that would not fill two rounds of eight per CU, and copies of less than 200 MB (but for rows of 2 KB over 64 ranks:
+// 32768 x 768 top-4, 198 MB, 70 us without, 58 with four), are left alone.
 static int move_workgroups_per_cu(const MoveParams& p) {
     if (p.fused) return 0;
     if (p.move_workgroups_per_cu != 0)       // two is the least an LDS share within a workgroup's 64 KB can enforce
         return p.move_workgroups_per_cu >= 8 ? 0 : (p.move_workgroups_per_cu < 2 ? 2 : p.move_workgroups_per_cu);
-    if (int64_t(p.num_movers) < int64_t(compute_units()) * 16) return 0;
-    if (many_rows_per_token(p)) return stores_row_by_row(p) ? 0 : 5;
-    if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) return 6;
-    return move_tile(p) == 2 ? 4 : 0;
+    const int tile = move_tile(p);
+    if (!fills_rounds(p, tile, 2)) return 0;
+    const double rows = rows_per_token(p);
+    if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) return p.do_expand ? 0 : tile == 1 && p.R >= 64 ? 5 : 6;
+    const int kb = (p.row_bytes + 1023) / 1024;
+    const bool spread = rows >= 5.5 || p.R >= 64;
+    if (kb == 2 && p.R >= 64 && !p.rank_lanes) return 4;
+    if (row_bytes_out(p) < 200e6 || (p.rank_lanes && kb < 8)) return 0;
+    if (kb == 1) return spread && p.row_bytes > 512 && !stores_row_by_row(p) ? 5 : 0;
+    if (tile == 2 && kb <= 3) return spread ? 4 : rows >= 3.0 ? 5 : 0;
+    if (tile == 2) return rows < (p.payload == DEEP_EP_HIP_PAYLOAD_FP8 && p.R < 64 ? 2.5 : 1.7) ? 0 : 4;
+    if (spread) return rows >= 5.8 && kb >= 8 ? 5 : 6;
+    return kb * rows >= 40.0 ? 6 : 0;
 }
 
 }  // namespace

@@ -13,7 +13,13 @@ CASES = {
     "bf16_few_rows_2kb": (7003, 7160, 64, 4, 4, False, False),          # 2 KB tiles, 4 workgroups per CU
     "cast_many_rows": (3001, 7040, 256, 32, 8, True, False),            # one 1024-channel segment
     "cast_many_rows_small": (37, 2176, 64, 32, 8, True, False),         # ... without a residency limit
+    "cast_many_rows_large": (6011, 7040, 256, 32, 8, True, False),      # one segment, four rounds
+    "cast_half_empty_segment": (9001, 1152, 256, 32, 8, True, False),   # rows whose second segment would be an eighth full
     "cast_expanded": (2503, 7040, 128, 16, 8, True, True),
+    "bf16_two_kb": (25009, 760, 64, 8, 8, False, False),                # whole rows, 5 workgroups per CU
+    "bf16_two_kb_many_ranks": (16411, 760, 64, 64, 4, False, False),    # ... and 4, below the size of the other limits
+    "bf16_one_kb_many_ranks": (36007, 504, 64, 64, 6, False, False),
+    "bf16_two_kb_expanded": (16411, 1024, 64, 8, 8, False, True),       # 1 KB tiles
 }
 
 
