@@ -1447,7 +1447,7 @@ int compute_units() {
 
 // More rows than this are copied in two launches: see plan_launches.
 bool copy_prefers_finished_layout(const MoveParams& p) {
-    return p.payload != DEEP_EP_HIP_PAYLOAD_CAST_FP8 && row_bytes_out(p) >= 300e6;
+    return p.payload != DEEP_EP_HIP_PAYLOAD_CAST_FP8 && row_bytes_out(p) >= (p.row_bytes > 4096 ? 300e6 : 345e6);
 }
 
 int64_t dispatch_move_workgroups(const MoveParams& p) {
