@@ -1320,7 +1320,8 @@ static bool stores_row_by_row(const MoveParams& p) {
 // Scattered stores stream fastest when not too many are under way: the more rows a token has, the more ranks they are spread
 // over and the wider they are, the fewer.  Move phase in us, inputs read from memory, with 8 / 6 / 5 / 4 workgroups per CU:
 //   fused cast, 8192 x 7168, 8 ranks           81.4 / 80.8 / 80.6 / 82.2;   16384 x 7168, 64 ranks 1 KB 272 / 241 / 228
-//   fused cast, expanded, 16384 x 4096 top-4    84 /  89 /  92;              8192 x 7168 top-8 1 KB 122 / 123 / 121: left alone
+//   fused cast, expanded, 16384 x 4096 top-8   134 / 139 / 141: left alone;           8192 x 7168 top-8 1 KB 122 / 123 / 121,
+//                                              and 2 % of the whole pass with inputs that change
 //   BF16, 16384 x 7168, 32 ranks, 1 KB         363 / 362 / 354 / 346;       16 ranks 312 / 312 / 304 / 314
 //   BF16, 16384 x 7168, 8 ranks, 1 KB          255 / 249 / 254 / 271;       16384 x 2048 80.8 / 82.2 / 86.8: left alone
 //   BF16, 16384 x 2048, 64 ranks top-6, 1 KB   116 /  95 /  97 / 105;       16 ranks top-8 99.7 / 99.7 / 101 / 109
@@ -1339,7 +1340,10 @@ static int move_workgroups_per_cu(const MoveParams& p) {
     const int tile = move_tile(p);
     if (!fills_rounds(p, tile, 2)) return 0;
     const double rows = rows_per_token(p);
-    if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) return p.do_expand ? 0 : tile == 1 && p.R >= 64 ? 5 : 6;
+    if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) {
+        if (p.do_expand) return rows * p.H >= 40 * 1024 ? 5 : 0;
+        return tile == 1 && p.R >= 64 ? 5 : 6;
+    }
     const int kb = (p.row_bytes + 1023) / 1024;
     const bool spread = rows >= 5.5 || p.R >= 64;
     if (kb == 2 && p.R >= 64 && !p.rank_lanes) return 4;
