@@ -76,3 +76,82 @@ def test_memory_kept_with_mostly_masked_routing(shape, surface):
     assert kept <= (64 << 20)
     if shape != "small":
         assert kept <= needed + 256 * len(tensors)
+
+
+# T, H, R, K: both sides of the limit
+SIZES = {"up_front": (300, 1024, 8, 6), "afterwards": (1500, 7168, 8, 6)}
+
+
+def _call(buf, payload, idx, w, E, on_stream=False, **kw):
+    """One exact-size dispatch on either surface: rows, scales, indices, weights, source tokens."""
+    import deep_ep
+    legacy = isinstance(buf, deep_ep.Buffer)
+    if on_stream:
+        kw.update(previous_event=buf.capture(), allocate_on_comm_stream=True, **{"async_finish" if legacy else "async_with_compute_stream": True})
+    if legacy:
+        per_rank, _, counts, in_rank, _ = buf.get_dispatch_layout(idx, E)
+        if on_stream:
+            kw["previous_event"] = buf.capture()
+        recv, recv_idx, recv_w, _, handle, event = buf.dispatch(payload, num_tokens_per_rank=per_rank, is_token_in_rank=in_rank,
+                                                                num_tokens_per_expert=counts, topk_idx=idx, topk_weights=w, **kw)
+    else:
+        recv, recv_idx, recv_w, handle, event = buf.dispatch(payload, idx, w, num_experts=E, **kw)
+    if on_stream:
+        event.current_stream_wait()
+    tokens = handle[3] if legacy else handle.recv_src_metadata[:, 0]
+    return (*(recv if isinstance(recv, tuple) else (recv, None)), recv_idx, recv_w, tokens.long())
+
+
+@pytest.mark.parametrize("on_stream", [False, True])
+@pytest.mark.parametrize("form", ["elastic_pair", "elastic_cast", "elastic_column_major", "legacy_pair"])
+@pytest.mark.parametrize("size", SIZES)
+def test_exact_scales(size, form, on_stream):
+    import deep_ep
+    from deep_ep.utils.math import per_token_cast_to_fp8
+    T, H, R, K = SIZES[size]
+    E = 64
+    small = rc.small(size, T, 16, E, R, K, seed=63, masked_ratio=0.2)
+    ref = oracle.dispatch(small.x, small.topk_idx, small.topk_weights, E, R, 0, T)
+    x = torch.randn((T, H), generator=torch.Generator(device="cuda").manual_seed(64), device="cuda", dtype=torch.bfloat16)
+    q, sf = per_token_cast_to_fp8(x)
+    idx, w = small.topk_idx.cuda(), small.topk_weights.cuda()
+    group = deep_ep.LogicalGroup(0, R)
+    buf = deep_ep.Buffer(group) if form == "legacy_pair" else deep_ep.ElasticBuffer(group, num_max_tokens_per_rank=T, hidden=H, num_topk=K)
+    kw = {"elastic_cast": dict(cast_to_fp8=True), "elastic_column_major": dict(cast_to_fp8=True, use_tma_aligned_col_major_sf=True)}.get(form, {})
+    for _ in range(2):
+        recv, recv_sf, recv_idx, _, tokens = _call(buf, (q, sf) if form.endswith("pair") else x, idx, w, E, on_stream, **kw)
+        assert recv.shape == (ref.num_recv_tokens, H) and recv_sf.shape == (ref.num_recv_tokens, H // 128)
+        assert recv_sf.is_contiguous() == (form != "elastic_column_major")
+        assert torch.equal(tokens.cpu().int(), ref.recv_src_metadata[:, 0]) and torch.equal(recv_idx.cpu(), ref.recv_topk_idx)
+        assert torch.equal(recv.view(torch.uint8), q[tokens].view(torch.uint8)) and torch.equal(recv_sf, sf[tokens])
+
+
+@pytest.mark.parametrize("fault", ["out_of_range", "twice"])
+@pytest.mark.parametrize("surface", ["elastic", "legacy"])
+@pytest.mark.parametrize("size", SIZES)
+def test_bad_routing_raises_and_the_next_call_is_clean(size, surface, fault):
+    """Up front the move of the bad routing is queued before its layout's verdict is read."""
+    import deep_ep
+    T, H, R, K = SIZES[size]
+    E = 64
+    small = rc.small(size, T, 16, E, R, K, seed=65, masked_ratio=0.2)
+    ref = oracle.dispatch(small.x, small.topk_idx, small.topk_weights, E, R, 0, T)
+    x = torch.randn((T, H), generator=torch.Generator(device="cuda").manual_seed(66), device="cuda", dtype=torch.bfloat16)
+    idx, w = small.topk_idx.cuda(), small.topk_weights.cuda()
+    group = deep_ep.LogicalGroup(0, R)
+    buf = deep_ep.Buffer(group) if surface == "legacy" else deep_ep.ElasticBuffer(group, num_max_tokens_per_rank=T, hidden=H, num_topk=K)
+    if surface == "legacy":
+        layout = buf.get_dispatch_layout(idx, E)                   # of the good routing: only the dispatch sees the bad one
+        call = lambda i: buf.dispatch(x, num_tokens_per_rank=layout[0], is_token_in_rank=layout[3], num_tokens_per_expert=layout[2],
+                                      topk_idx=i, topk_weights=w)
+    else:
+        call = lambda i: buf.dispatch(x, i, w, num_experts=E)
+    bad = idx.clone()
+    bad[T // 2, 0] = E + 5 if fault == "out_of_range" else 7
+    if fault == "twice":
+        bad[T // 2, 1] = 7
+    with pytest.raises(RuntimeError, match="expert"):
+        call(bad)
+    recv, recv_idx, recv_w, *_ = call(idx)
+    tokens = ref.recv_src_metadata[:, 0].long().cuda()
+    assert torch.equal(recv, x[tokens]) and torch.equal(recv_idx.cpu(), ref.recv_topk_idx)
