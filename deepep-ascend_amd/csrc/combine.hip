@@ -282,18 +282,21 @@ double rows_per_token(const CombineParams& p) {
 //   16 ranks (6.4)               8192 tokens 149.1 / 145.4 / 141.7 / 143.8;  16384  303 / 297 / 287 / 286
 //   32 ranks (7.2)               4096 tokens  81.3 / 80.1 / 78.5 / 78.6;   16384  336 / 330 / 321 / 312
 //   4 of 4 ranks (2.7)           8192 tokens  67.6 / 71.3 / 76.0;   16384 x 2048 top-6 (4.4) 60.9 / 62.2 / 64.1
-//   2048 channels (32768 tokens) 8 ranks 142 / 139 / 139;                64 ranks 205 / 199 / 195;   4096 channels (16384) 207 / 206 / 206
-// Smaller calls lose by any limit (4096 x 2048 top-6: 17.3 / 18.3; 8192 x 4096 top-6 over 64 ranks, 388 MB, 79.5 / 83.2), and so do
-// narrower rows (65536 x 768 over 16 ranks 125 / 137 / 146).
+//   top-6 of 8 ranks (4.4)       4096 tokens  53.5 / 52.6 / 54.0;   8192  103.4 / 100.6 / 102.8;   16384  210 / 199 / 202
+//   top-4 of 16 ranks (3.6)      8192 tokens  88.1 / 87.3 / 88.7;   16384  176 / 172 / 175;   of 8 ranks (3.3)   158 / 157 / 162
+//   2048 channels (32768 tokens) 8 ranks 142 / 139 / 139;                64 ranks 205 / 199 / 195
+//   8192 channels (16384 tokens) top-6 of 8 ranks 238 / 247 / 252;   4096 channels (8192) of 64 ranks 79.5 / 83.2 / 83.2: rows a
+//   power of two apart are left alone
+// Smaller calls lose by any limit (4096 x 2048 top-6: 17.3 / 18.3), and so do narrower rows (65536 x 768 over 16 ranks 125 / 137 /
+// 146).
 // The limit is kept with LDS, which a product on another stream then lacks: beside products of 4096^3 BF16 that share the GPU,
 // twenty combines and 24 products together take 4.44 ms without it and 4.58 with six at 8192 tokens over 8 ranks (alone 122 and
 // 119 us a combine), 8.24 and 8.45 with five at 16384 over 32 (337 and 322).  Expanded rows are left alone: there it gave 1 %
 // alone (187.7 and 185.6) and took 4 % beside products (5.68 and 5.93).
 int workgroups_per_cu(const CombineParams& p) {
     const double rows = rows_per_token(p), bytes = rows * p.T * p.H * 2;
-    if (p.H < 2048 || (p.H < 6144 && bytes < 600e6)) return 0;
-    if (p.do_expand && !p.rank_mode) return 0;
-    if (bytes < 300e6 || rows < 5.0) return 0;
+    if ((p.do_expand && !p.rank_mode) || p.H < 2048 || p.H % 4096 == 0) return 0;
+    if (p.H < 6144 ? rows < 5.0 || bytes < 600e6 : rows >= 5.0 ? bytes < 300e6 : rows < 3.5 || bytes < 450e6) return 0;
     return rows >= 5.8 ? 5 : 6;
 }
 
