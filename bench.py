@@ -36,17 +36,17 @@ HBM_PEAK_GBS = 8000.0
 # the whole call (one kernel where the single launch applies, layout kernel + move kernel otherwise).
 MEASURED_TRAFFIC_BYTES = {
     # profiles/bench_C3_hbm_counters.md
-    ("C3", "compact", "fp8", "dispatch"): 459281822,
-    ("C3", "compact", "fp8", "combine"): 751991366,
-    ("C3", "expanded", "fp8", "dispatch"): 1862368 + 613156339,
-    ("C3", "expanded", "fp8", "combine"): 1074426190,
-    ("C3", "compact", "bf16", "dispatch"): 1844575 + 755717968,
-    ("C3", "compact", "bf16", "combine"): 751994813,
+    ("C3", "compact", "fp8", "dispatch"): 459294014,
+    ("C3", "compact", "fp8", "combine"): 752000765,
+    ("C3", "expanded", "fp8", "dispatch"): 1087375 + 613255416,
+    ("C3", "expanded", "fp8", "combine"): 1078618617,
+    ("C3", "compact", "bf16", "dispatch"): 1056154 + 755775749,
+    ("C3", "compact", "bf16", "combine"): 752000758,
     # profiles/bench_C4_C2_hbm_counters.md
-    ("C4", "compact", "fp8", "dispatch"): 425752286,
-    ("C4", "compact", "fp8", "combine"): 690500110,
-    ("C2", "compact", "bf16", "dispatch"): 97414801,
-    ("C2", "compact", "bf16", "combine"): 96362205,
+    ("C4", "compact", "fp8", "dispatch"): 425760944,
+    ("C4", "compact", "fp8", "combine"): 690503978,
+    ("C2", "compact", "bf16", "dispatch"): 97441507,
+    ("C2", "compact", "bf16", "combine"): 96352156,
     # profiles/bench_C5_low_latency_hbm_counters.md
     ("C5", "packed", "fp8", "ll_dispatch"): 23993245,
     ("C5", "packed", "fp8", "ll_combine"): 30425179,

@@ -91,8 +91,8 @@ typedef struct {
                                   launch give up at once: for tests of that path - every kernel still runs to its end and
                                   the workspace stays consistent) */
     int32_t move_workgroups_per_cu;  /* dispatch move kernel launched on a finished layout: workgroups a CU holds at a
-                                        time (2..7; 8 and more = as many as fit; 0 = six / five for the compact / expanded
-                                        layout of a large fused-cast call, no limit otherwise) */
+                                        time (2..7; 8 and more = as many as fit; 0 = four to six in large calls, by payload,
+                                        rows per token and row width, no limit otherwise) */
     int32_t warm_rounds;       /* single-launch dispatch: the movers that are resident at launch also
                                   load, into the caches only, the tiles of the work items this many rounds of resident
                                   workgroups ahead of their own (0 = 2, or 1 in launches of one and a half to two rounds;
