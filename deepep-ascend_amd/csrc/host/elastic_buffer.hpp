@@ -231,6 +231,9 @@ public:
                               not previous_event_before_epilogue.has_value() and
                               not (sf_dtype.has_value() and use_tma_aligned_col_major_sf) and      // its strides follow the row count
                               row_bound * bytes_by_row <= kUpFrontBytes;
+        // Larger calls allocate for evenly chosen experts while the layout runs, and again if the counts say otherwise.
+        const bool by_guess = do_cpu_sync and not cached_mode and not do_expand and num_tokens > 0 and not up_front and
+                              not (sf_dtype.has_value() and use_tma_aligned_col_major_sf);
         int32_t* box = nullptr;
         int num_recv_tokens, num_expanded_tokens;
         std::vector<int> per_expert_list;
@@ -245,25 +248,26 @@ public:
             args.host_counts = box;
             check_abi(deep_ep_hip_launch_dispatch(&args, stream_ptr), "dispatch layout");
             args.host_counts = nullptr;
-            num_recv_tokens = static_cast<int>(row_bound);
+            num_recv_tokens = static_cast<int>(by_guess ? guessed_rows(num_tokens, num_topk, num_experts, R) : row_bound);
             num_expanded_tokens = 0;
-            if (not up_front) read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
+            if (not up_front and not by_guess) read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
         } else {
             num_recv_tokens = num_max_tokens_per_rank * R;
             num_expanded_tokens = num_max_tokens_per_rank * std::min(num_topk, num_experts) + (expert_alignment - 1) * num_experts;
             num_expanded_tokens = static_cast<int>(align_up(num_expanded_tokens, expert_alignment));
         }
 
-        const int64_t num_allocated = do_expand ? num_expanded_tokens : num_recv_tokens;
         torch::Tensor recv_x, recv_src_metadata;
         std::optional<torch::Tensor> recv_sf, recv_topk_idx, recv_topk_weights;
         int64_t rsf_ts = 0, rsf_hs = 0;
         // what travels beside the payload (scales, indices, weights), in one allocation; the payload and the
         // handle's metadata stay on their own, because callers keep them for different spans
-        TensorPack beside(device_);
+        std::optional<TensorPack> pack;
         int i_sf = -1, i_idx = -1, i_w = -1;
-        {
+        const auto allocate_outputs = [&] {
             c10::hip::HIPStreamGuardMasqueradingAsCUDA on_run(run);
+            const int64_t num_allocated = do_expand ? num_expanded_tokens : num_recv_tokens;
+            TensorPack& beside = pack.emplace(device_);
             recv_x = torch::empty({num_allocated, hidden}, torch::TensorOptions().dtype(out_dtype).device(device_));
             recv_src_metadata = cached_mode ? *cached_recv_src_metadata : torch::empty({num_recv_tokens, num_topk + 2}, i32);
             if (sf_dtype.has_value()) {
@@ -281,6 +285,26 @@ public:
             if (i_sf >= 0) recv_sf = beside.get(i_sf);
             if (i_idx >= 0) recv_topk_idx = beside.get(i_idx);
             if (i_w >= 0) recv_topk_weights = beside.get(i_w);
+        };
+        const auto narrow_outputs = [&] {
+            recv_x = first_rows(recv_x, num_recv_tokens);
+            recv_src_metadata = first_rows(recv_src_metadata, num_recv_tokens);
+            if (i_sf >= 0) recv_sf = pack->get(i_sf, num_recv_tokens);
+            if (i_idx >= 0) recv_topk_idx = pack->get(i_idx, num_recv_tokens);
+            if (i_w >= 0) recv_topk_weights = pack->get(i_w, num_recv_tokens);
+        };
+        allocate_outputs();
+        bool narrow_last = up_front;                 // behind the launch, which does not wait for it
+        if (by_guess) {
+            const int64_t guess = num_recv_tokens;
+            read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
+            narrow_last = guess_serves(guess, num_recv_tokens);
+            if (not narrow_last) {
+                pack.reset();
+                recv_x = recv_src_metadata = torch::Tensor();
+                recv_sf = recv_topk_idx = recv_topk_weights = std::nullopt;
+                allocate_outputs();
+            }
         }
 
         if (previous_event_before_epilogue.has_value()) stream_wait(run, *previous_event_before_epilogue);
@@ -295,14 +319,8 @@ public:
         args.recv_capacity = recv_src_metadata.size(0);
         args.expanded_capacity = do_expand ? num_expanded_tokens : 0;
         check_abi(deep_ep_hip_launch_dispatch(&args, stream_ptr), "dispatch");
-        if (up_front) {
-            read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
-            recv_x = first_rows(recv_x, num_recv_tokens);
-            recv_src_metadata = first_rows(recv_src_metadata, num_recv_tokens);
-            if (i_sf >= 0) recv_sf = beside.get(i_sf, num_recv_tokens);
-            if (i_idx >= 0) recv_topk_idx = beside.get(i_idx, num_recv_tokens);
-            if (i_w >= 0) recv_topk_weights = beside.get(i_w, num_recv_tokens);
-        }
+        if (up_front) read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
+        if (narrow_last) narrow_outputs();
         if (not cached_mode) slots_of_handle_.remember(recv_src_metadata, dst_slot);
 
         std::optional<EventHandle> event = scope.finish(

@@ -210,6 +210,8 @@ public:
         const int64_t bytes_by_row = hidden * int64_t(x.element_size()) + num_scales * 4 + 4 + num_topk * 12;
         const bool up_front = not cached_mode and num_worst_tokens == 0 and topk_idx.has_value() and num_tokens > 0 and
                               row_bound * bytes_by_row <= kUpFrontBytes;
+        // Larger ones allocate for evenly chosen experts while the layout runs, and again if the counts say otherwise.
+        const bool by_guess = not cached_mode and num_worst_tokens == 0 and topk_idx.has_value() and num_tokens > 0 and not up_front;
         int32_t* box = nullptr;
         int num_recv_tokens;
         std::vector<int> per_expert_list;
@@ -264,8 +266,8 @@ public:
                     args.host_counts = box;
                     check_abi(deep_ep_hip_launch_intranode_dispatch(&args, stream_ptr), "intranode dispatch layout");
                     args.host_counts = nullptr;
-                    num_recv_tokens = static_cast<int>(row_bound);
-                    if (not up_front) read_counts();
+                    num_recv_tokens = static_cast<int>(by_guess ? guessed_rows(num_tokens, num_topk, num_experts, R) : row_bound);
+                    if (not up_front and not by_guess) read_counts();
                 } else {
                     per_expert_list.resize(num_experts);
                     check_abi(deep_ep_hip_launch_intranode_dispatch(&args, stream_ptr), "intranode dispatch layout");
@@ -278,33 +280,48 @@ public:
                 args.phases = DEEP_EP_HIP_PHASE_MOVE;
             }
         }
-        recv_src_idx = torch::empty({num_recv_tokens}, i32);
-
-        torch::Tensor recv_x = torch::empty({num_recv_tokens, hidden}, x.options());
+        torch::Tensor recv_x;
         std::optional<torch::Tensor> recv_x_scales, recv_topk_idx, recv_topk_weights;
-        if (topk_idx.has_value()) {
-            recv_topk_idx = torch::empty({num_recv_tokens, num_topk}, topk_idx->options());
-            recv_topk_weights = torch::empty({num_recv_tokens, num_topk}, topk_weights->options());
-        }
-        if (x_scales.has_value()) {
-            recv_x_scales = torch::empty({num_recv_tokens, num_scales}, x_scales->options().memory_format(torch::MemoryFormat::Contiguous));
-            args.recv_scale_token_stride = num_scales; args.recv_scale_hidden_stride = 1;
+        const auto allocate_outputs = [&] {
+            recv_src_idx = torch::empty({num_recv_tokens}, i32);
+            recv_x = torch::empty({num_recv_tokens, hidden}, x.options());
+            if (topk_idx.has_value()) {
+                recv_topk_idx = torch::empty({num_recv_tokens, num_topk}, topk_idx->options());
+                recv_topk_weights = torch::empty({num_recv_tokens, num_topk}, topk_weights->options());
+            }
+            if (x_scales.has_value()) {
+                recv_x_scales = torch::empty({num_recv_tokens, num_scales}, x_scales->options().memory_format(torch::MemoryFormat::Contiguous));
+                args.recv_scale_token_stride = num_scales; args.recv_scale_hidden_stride = 1;
+            }
+        };
+        const auto narrow_outputs = [&] {
+            recv_x = first_rows(recv_x, num_recv_tokens);
+            recv_src_idx = first_rows(recv_src_idx, num_recv_tokens);
+            recv_topk_idx = first_rows(*recv_topk_idx, num_recv_tokens);
+            recv_topk_weights = first_rows(*recv_topk_weights, num_recv_tokens);
+            if (recv_x_scales.has_value()) recv_x_scales = first_rows(*recv_x_scales, num_recv_tokens);
+        };
+        allocate_outputs();
+        bool narrow_last = up_front;                 // behind the launch, which does not wait for it
+        if (by_guess) {
+            const int64_t guess = num_recv_tokens;
+            read_counts();
+            narrow_last = guess_serves(guess, num_recv_tokens);
+            if (not narrow_last) {
+                recv_x = recv_src_idx = torch::Tensor();
+                recv_x_scales = recv_topk_idx = recv_topk_weights = std::nullopt;
+                allocate_outputs();
+            }
         }
         args.send_head = static_cast<int32_t*>(send_head.data_ptr());
         args.recv_src_idx = (cached_mode and cached_send_head.has_value()) ? nullptr : static_cast<int32_t*>(recv_src_idx.data_ptr());
         args.recv_x = recv_x.data_ptr();
         args.recv_x_scales = recv_x_scales.has_value() ? recv_x_scales->data_ptr() : nullptr;
         args.recv_topk_idx = ptr_of<int64_t>(recv_topk_idx); args.recv_topk_weights = ptr_of<float>(recv_topk_weights);
-        args.recv_capacity = num_recv_tokens;
+        args.recv_capacity = recv_x.size(0);
         check_abi(deep_ep_hip_launch_intranode_dispatch(&args, stream_ptr), "intranode dispatch");
-        if (up_front) {
-            read_counts();
-            recv_x = first_rows(recv_x, num_recv_tokens);
-            recv_src_idx = first_rows(recv_src_idx, num_recv_tokens);
-            recv_topk_idx = first_rows(*recv_topk_idx, num_recv_tokens);
-            recv_topk_weights = first_rows(*recv_topk_weights, num_recv_tokens);
-            if (recv_x_scales.has_value()) recv_x_scales = first_rows(*recv_x_scales, num_recv_tokens);
-        }
+        if (up_front) read_counts();
+        if (narrow_last) narrow_outputs();
         if (not cached_mode) send_head_of_handle_.remember(rank_prefix_matrix, send_head);
 
         std::optional<EventHandle> event = scope.finish(

@@ -1,6 +1,6 @@
 """Exact-size dispatches on either side of the size up to which outputs are allocated at their bound (64 MiB in all) before the
 counts are known: the tensors have the exact number of rows, are contiguous, hold the tokens they should, and past that size no
-memory beyond them."""
+memory beyond a fifteenth more."""
 import pytest
 import torch
 
@@ -155,3 +155,32 @@ def test_bad_routing_raises_and_the_next_call_is_clean(size, surface, fault):
     recv, recv_idx, recv_w, *_ = call(idx)
     tokens = ref.recv_src_metadata[:, 0].long().cuda()
     assert torch.equal(recv, x[tokens]) and torch.equal(recv_idx.cpu(), ref.recv_topk_idx)
+
+
+@pytest.mark.parametrize("surface", ["elastic", "legacy"])
+@pytest.mark.parametrize("routing", ["even", "spread", "one_rank", "nowhere"])
+def test_outputs_allocated_for_even_routing(routing, surface):
+    """Past the limit outputs are allocated for evenly chosen experts before the counts are known: kept where those fit (and hold
+    at most 16 / 15 of what they need), too few where every token goes to every rank, far too many where all go to one or none."""
+    import deep_ep
+    T, H, R, E, K = 2049, 4096, 8, 64, 8
+    gen = torch.Generator().manual_seed(67)
+    idx = torch.stack([torch.randperm(E, generator=gen)[:K] for _ in range(T)])
+    if routing == "spread":
+        idx = torch.arange(K).mul(E // R).add(torch.randint(0, E // R, (T, K), generator=gen))
+    elif routing == "one_rank":
+        idx = torch.stack([torch.randperm(E // R, generator=gen)[:K] for _ in range(T)]) + 3 * (E // R)
+    elif routing == "nowhere":
+        idx = torch.full((T, K), -1)
+        idx[5, 2] = 9
+    w = torch.rand((T, K), generator=gen)
+    ref = oracle.dispatch(torch.zeros((T, 16), dtype=torch.bfloat16), idx, w, E, R, 0, T)
+    x = torch.randn((T, H), generator=torch.Generator(device="cuda").manual_seed(68), device="cuda", dtype=torch.bfloat16)
+    group = deep_ep.LogicalGroup(0, R)
+    buf = deep_ep.Buffer(group) if surface == "legacy" else deep_ep.ElasticBuffer(group, num_max_tokens_per_rank=T, hidden=H, num_topk=K)
+    for _ in range(2):
+        recv, _, recv_idx, recv_w, tokens = _call(buf, x, idx.cuda(), w.cuda(), E)
+        assert recv.shape == (ref.num_recv_tokens, H) and recv.is_contiguous()
+        assert torch.equal(tokens.cpu().int(), ref.recv_src_metadata[:, 0]) and torch.equal(recv_idx.cpu(), ref.recv_topk_idx)
+        assert torch.equal(recv, x[tokens])
+        assert recv.untyped_storage().nbytes() * 15 <= recv.numel() * 2 * 16
