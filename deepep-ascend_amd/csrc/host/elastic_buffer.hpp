@@ -293,12 +293,17 @@ public:
             if (i_idx >= 0) recv_topk_idx = pack->get(i_idx, num_recv_tokens);
             if (i_w >= 0) recv_topk_weights = pack->get(i_w, num_recv_tokens);
         };
-        allocate_outputs();
-        bool narrow_last = up_front;                 // behind the launch, which does not wait for it
-        if (by_guess) {
-            const int64_t guess = num_recv_tokens;
-            read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
-            narrow_last = guess_serves(guess, num_recv_tokens);
+        bool counts_read = not up_front and not by_guess, narrow_last = false;       // narrowed behind the launch, which does not wait for it
+        if (counts_read) {
+            allocate_outputs();
+        } else {
+            const int64_t rows = num_recv_tokens;
+            narrow_last = allocates(allocate_outputs);
+            if (by_guess or not narrow_last) {
+                read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
+                counts_read = true;
+            }
+            if (by_guess and not guess_serves(rows, num_recv_tokens)) narrow_last = false;
             if (not narrow_last) {
                 pack.reset();
                 recv_x = recv_src_metadata = torch::Tensor();
@@ -319,7 +324,7 @@ public:
         args.recv_capacity = recv_src_metadata.size(0);
         args.expanded_capacity = do_expand ? num_expanded_tokens : 0;
         check_abi(deep_ep_hip_launch_dispatch(&args, stream_ptr), "dispatch");
-        if (up_front) read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
+        if (not counts_read) read_counts(box, num_experts, run, workspace, num_recv_tokens, num_expanded_tokens, per_expert_list);
         if (narrow_last) narrow_outputs();
         if (not cached_mode) slots_of_handle_.remember(recv_src_metadata, dst_slot);
 

@@ -301,12 +301,17 @@ public:
             recv_topk_weights = first_rows(*recv_topk_weights, num_recv_tokens);
             if (recv_x_scales.has_value()) recv_x_scales = first_rows(*recv_x_scales, num_recv_tokens);
         };
-        allocate_outputs();
-        bool narrow_last = up_front;                 // behind the launch, which does not wait for it
-        if (by_guess) {
-            const int64_t guess = num_recv_tokens;
-            read_counts();
-            narrow_last = guess_serves(guess, num_recv_tokens);
+        bool counts_read = not up_front and not by_guess, narrow_last = false;       // narrowed behind the launch, which does not wait for it
+        if (counts_read) {
+            allocate_outputs();
+        } else {
+            const int64_t rows = num_recv_tokens;
+            narrow_last = allocates(allocate_outputs);
+            if (by_guess or not narrow_last) {
+                read_counts();
+                counts_read = true;
+            }
+            if (by_guess and not guess_serves(rows, num_recv_tokens)) narrow_last = false;
             if (not narrow_last) {
                 recv_x = recv_src_idx = torch::Tensor();
                 recv_x_scales = recv_topk_idx = recv_topk_weights = std::nullopt;
@@ -320,7 +325,7 @@ public:
         args.recv_topk_idx = ptr_of<int64_t>(recv_topk_idx); args.recv_topk_weights = ptr_of<float>(recv_topk_weights);
         args.recv_capacity = recv_x.size(0);
         check_abi(deep_ep_hip_launch_intranode_dispatch(&args, stream_ptr), "intranode dispatch");
-        if (up_front) read_counts();
+        if (not counts_read) read_counts();
         if (narrow_last) narrow_outputs();
         if (not cached_mode) send_head_of_handle_.remember(rank_prefix_matrix, send_head);
 

@@ -197,6 +197,17 @@ inline int64_t guessed_rows(int64_t num_tokens, int num_topk, int num_experts, i
 }
 inline bool guess_serves(int64_t guess, int64_t rows) { return rows <= guess and (guess - rows) * 16 <= guess; }
 
+// Outputs for more rows than a call may turn out to receive: false if there is no memory for so many, which is no error yet.
+template <typename Allocate>
+bool allocates(const Allocate& allocate_outputs) {
+    try {
+        allocate_outputs();
+        return true;
+    } catch (const c10::OutOfMemoryError&) {
+        return false;
+    }
+}
+
 // A few (key tensor -> companion tensor) pairs a buffer remembers about handles it has produced.  The key is held
 // weakly and compared by identity, so an entry can only be found through the very tensor object the buffer returned:
 // a clone, a view or another tensor that happens to reuse the freed memory misses, and the caller falls back to

@@ -184,3 +184,31 @@ def test_outputs_allocated_for_even_routing(routing, surface):
         assert torch.equal(tokens.cpu().int(), ref.recv_src_metadata[:, 0]) and torch.equal(recv_idx.cpu(), ref.recv_topk_idx)
         assert torch.equal(recv, x[tokens])
         assert recv.untyped_storage().nbytes() * 15 <= recv.numel() * 2 * 16
+
+
+@pytest.mark.parametrize("surface", ["elastic", "legacy"])
+@pytest.mark.parametrize("T", [500, 2049])
+def test_memory_for_what_is_received_is_enough(T, surface):
+    """Where there is memory for the rows a call receives but not for those it could, it still runs."""
+    import deep_ep
+    H, R, E, K = 4096, 8, 64, 8
+    idx = torch.full((T, K), -1, device="cuda")
+    idx[7, 3], idx[T - 1, 0] = 9, 60
+    w = torch.ones((T, K), device="cuda")
+    x = torch.randn((T, H), device="cuda").to(torch.bfloat16)
+    group = deep_ep.LogicalGroup(0, R)
+    buf = deep_ep.Buffer(group) if surface == "legacy" else deep_ep.ElasticBuffer(group, num_max_tokens_per_rank=T, hidden=H, num_topk=K)
+    for _ in range(2):                                            # what a call keeps exists
+        _call(buf, x, idx, w, E)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (12 << 20)) / total)
+    try:
+        recv, _, recv_idx, recv_w, tokens = _call(buf, x, idx, w, E)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert tokens.tolist() == [7, T - 1] and torch.equal(recv, x[tokens]) and recv_idx.shape == recv_w.shape == (2, K)
+    buf_status = getattr(buf, "check_device_status", None)
+    if buf_status is not None:
+        buf_status()
