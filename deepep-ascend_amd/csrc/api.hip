@@ -133,7 +133,6 @@ void fill_fused(MoveParams& m, const LayoutParams& lay, const LaunchPlan& plan, 
 
 WorkspaceLayout make_workspace_layout(int num_max_tokens, int num_topk, int num_experts, int num_ranks) {
     WorkspaceLayout w{};
-    const size_t n = size_t(num_ranks) + num_experts;
     const size_t chunks = num_max_tokens > 0 ? (size_t(num_max_tokens) + kLayoutChunk - 1) / kLayoutChunk : 1;
     const size_t chunks_padded = (chunks + 3) / 4 * 4;
     const size_t lanes = size_t(num_max_tokens > 0 ? num_max_tokens : 1) * num_topk;
@@ -740,7 +739,6 @@ size_t deep_ep_hip_ll_workspace_bytes(int num_src_ranks, int src_token_stride, i
     if (num_src_ranks < 1 || src_token_stride < 1 || num_topk < 1 || num_local_experts < 1) return 0;
     const size_t chunks = size_t(num_src_ranks) * ((size_t(src_token_stride) + kLayoutChunk - 1) / kLayoutChunk);
     size_t off = 256;
-    off = align_up(off + chunks * num_local_experts * 4, 256) ;
     off = align_up(off + chunks * num_local_experts * 4, 256);
     off = align_up(off + size_t(num_src_ranks) * src_token_stride * num_topk * 4, 256);
     return off;
@@ -793,9 +791,7 @@ int deep_ep_hip_launch_ll_dispatch(const deep_ep_hip_ll_dispatch_args* a, void* 
     p.lane_slot = a->lane_rows;
     size_t off = 256;
     p.status = reinterpret_cast<int32_t*>(ws);
-    p.done_counter = reinterpret_cast<uint32_t*>(ws + 4);
     p.chunk_counts = reinterpret_cast<int32_t*>(ws + off); off = align_up(off + chunks * p.E_l * 4, 256);
-    p.chunk_base = reinterpret_cast<int32_t*>(ws + off);   off = align_up(off + chunks * p.E_l * 4, 256);
     p.pos_expert = reinterpret_cast<int32_t*>(ws + off);
     p.pairs = a->tuning.ll_pairs; p.threads = a->tuning.ll_threads; p.two_kernels = a->tuning.ll_two_kernels;
     hipError_t err = launch_ll_dispatch(p, static_cast<hipStream_t>(stream));

@@ -286,10 +286,8 @@ struct LLDispatchParams {
     int32_t* lane_slot;      // optional [S*stride, K]: packed row (le * rows + slot) of every (token, lane), -1 none
     // workspace
     int32_t* status;
-    uint32_t* done_counter;
-    int32_t* chunk_counts;   // [C][E_l]
-    int32_t* chunk_base;     // [C][E_l]
-    int32_t* pos_expert;     // [S*stride*K]
+    int32_t* chunk_counts;   // [E_l][C]: rows chunk c (256 tokens of one source) brings to a local expert
+    int32_t* pos_expert;     // [S*stride*K]: position of a local selection inside its chunk
     // launch-shape overrides, 0 = choose
     int pairs, threads, two_kernels;
 };
