@@ -354,6 +354,7 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
         m.gates = reinterpret_cast<uint32_t*>(ws + w.gates);               // a persistent move kernel keeps its item counter there
         m.gates_finished = reinterpret_cast<uint32_t*>(ws + w.gates_finished);
         if (plan.fused) fill_fused(m, lay, plan, ws, w);
+        m.sf_blocked = a->do_zero_padding && scales_in_blocks(m, a->expert_alignment) ? 1 : 0;
 
         hipError_t err = launch_dispatch_move(m, stream);
         if (err != hipSuccess) return hip_fail(err, "dispatch move launch");
@@ -370,6 +371,7 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
             z.expanded_capacity = a->expanded_capacity;
             z.E = E; z.A = a->expert_alignment;
             z.out_row_bytes = H * elem_out;
+            z.sf_blocked = m.sf_blocked;
             err = launch_zero_padding(z, stream);
             if (err != hipSuccess) return hip_fail(err, "zero padding launch");
         }

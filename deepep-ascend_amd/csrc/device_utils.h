@@ -192,6 +192,13 @@ __device__ __forceinline__ int small_div(int x, float rcp_d) {
     return int((float(x) + 0.5f) * rcp_d);
 }
 
+// Where the scales of a column-major tensor (columns `stride` apart) stand while they are in blocks of `block` rows (kernels.h):
+// place `index` of the block that starts at row r0 and has `rows` rows.
+__device__ __forceinline__ int64_t place_in_block(int index, int block, int rows, int64_t r0, int64_t stride) {
+    const int column = rows == block ? index / block : int(unsigned(index) / unsigned(rows));
+    return column * stride + r0 + (index - column * rows);
+}
+
 // Agent-scope relaxed load / store (no caching that another XCD's workgroups could not see through), for words
 // workgroups of one launch hand to each other.
 __device__ __forceinline__ int load_agent(const int* p) {

@@ -264,6 +264,15 @@ __device__ __forceinline__ uint64_t destination_lanes(const MoveParams& p, const
     return __ballot(row_of_lane >= 0);
 }
 
+// Where scale `group` of a (wave-uniform) row goes.  kBlocked: scales_in_blocks.
+template <bool kBlocked>
+__device__ __forceinline__ uint32_t* scale_place(const MoveParams& p, int row, int group) {
+    if constexpr (!kBlocked) return p.recv_sf + (int64_t(row) * p.rsf_ts + int64_t(group) * p.rsf_hs);
+    const int r0 = row & ~(kScaleBlockRows - 1);
+    const int rows = int(min(p.expanded_capacity - r0, int64_t(kScaleBlockRows)));
+    return p.recv_sf + place_in_block((row - r0) * p.num_sf_packs + group, kScaleBlockRows, rows, r0, p.rsf_hs);
+}
+
 // ---- single-launch dispatch ----
 //
 // Grid: C counting workgroups (one 256-token chunk each), one publishing workgroup, then the movers.  A mover cannot
@@ -671,7 +680,9 @@ __device__ __forceinline__ bool warm_next_rounds_of_rows(const MoveParams& p, un
 
 // ---- pass-through payload (BF16, or FP8 with caller-provided scale packs) ----
 // kScales: rows may come with scale packs (p.recv_sf).
-template <int kVecs, bool kFused, bool kScales>
+enum : int { kNoScales = 0, kScalesInPlace = 1, kScalesInBlocks = 2 };
+
+template <int kVecs, bool kFused, int kScales>
 __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
     if constexpr (kFused) {
         if (blockIdx.x <= unsigned(p.count_blocks)) {
@@ -709,7 +720,7 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
     }
 
     // The caller's scale packs ride with tile 0: requested with the payload, once, not per destination row.
-    const bool packs = kScales && has_work && tile == 0 && p.recv_sf != nullptr;
+    const bool packs = kScales != kNoScales && has_work && tile == 0 && p.recv_sf != nullptr;
     uint32_t pack = 0;
     if (packs && lane < p.num_sf_packs) pack = p.sf[int64_t(t) * p.sf_ts + int64_t(lane) * p.sf_hs];
 
@@ -751,10 +762,9 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
             if (off < p.row_bytes) store16_stream(dst + off, v[i]);
         }
         if (packs) {
-            uint32_t* to = p.recv_sf + int64_t(row) * p.rsf_ts;
-            if (lane < p.num_sf_packs) to[int64_t(lane) * p.rsf_hs] = pack;
+            if (lane < p.num_sf_packs) *scale_place<kScales == kScalesInBlocks>(p, row, lane) = pack;
             for (int g = lane + kWaveSize; g < p.num_sf_packs; g += kWaveSize)        // rows beyond 8192 channels
-                to[int64_t(g) * p.rsf_hs] = p.sf[int64_t(t) * p.sf_ts + int64_t(g) * p.sf_hs];
+                *scale_place<kScales == kScalesInBlocks>(p, row, g) = p.sf[int64_t(t) * p.sf_ts + int64_t(g) * p.sf_hs];
             if (!kFused && p.row_by_row) wait_for_own_stores();
         }
     }
@@ -770,7 +780,7 @@ __device__ long long wave_stamps[3 * kMaxStampedWaves];
 #endif
 
 // ---- fused BF16 -> e4m3 cast: lane owns 16 consecutive channels, 8 lanes own one 128-group ----
-template <int kPairs, bool kFused>
+template <int kPairs, bool kFused, bool kBlocked>
 __device__ __forceinline__ void dispatch_cast(const MoveParams& p) {
     if constexpr (kFused) {
         if (blockIdx.x <= unsigned(p.count_blocks)) {
@@ -882,8 +892,7 @@ __device__ __forceinline__ void dispatch_cast(const MoveParams& p) {
             const int elem = (tile * kPairs + q) * 1024 + lane * 16;
             if (elem < p.H) store16_stream(dst + elem, out[q]);
         }
-        if (owns_scale)
-            p.recv_sf[int64_t(row) * p.rsf_ts + int64_t(group) * p.rsf_hs] = __float_as_uint(my_scale);
+        if (owns_scale) *scale_place<kBlocked>(p, row, group) = __float_as_uint(my_scale);
     }
 #ifdef DEEP_EP_HIP_WAVE_STAMPS
     if (lane == 0 && work < unsigned(kMaxStampedWaves)) {
@@ -1111,27 +1120,59 @@ __global__ __launch_bounds__(kQueueThreads) void dispatch_cast_queue_kernel(cons
 // The kernels.  The single-launch forms also hold the counting and publishing code, whose register needs must not cost
 // the movers their occupancy: they are held to six wavefronts per SIMD (80 registers) - six workgroups per CU, which
 // is also where the move streams fastest (more were slower when tried with a leaner counting step, fewer are slower too).
-template <int kVecs, bool kScales>
+template <int kVecs, int kScales>
 __global__ __launch_bounds__(kThreads) void dispatch_copy_kernel(const MoveParams p) {
     dispatch_copy<kVecs, false, kScales>(p);
 }
-template <int kVecs, bool kScales>
+template <int kVecs, int kScales>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void dispatch_copy_single_launch_kernel(const MoveParams p) {
     dispatch_copy<kVecs, true, kScales>(p);
 }
-template <int kPairs>
+template <int kPairs, bool kBlocked>
 __global__ __launch_bounds__(kThreads) void dispatch_cast_kernel(const MoveParams p) {
-    dispatch_cast<kPairs, false>(p);
+    dispatch_cast<kPairs, false, kBlocked>(p);
 }
-template <int kPairs>
+template <int kPairs, bool kBlocked>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void dispatch_cast_single_launch_kernel(const MoveParams p) {
-    dispatch_cast<kPairs, true>(p);
+    dispatch_cast<kPairs, true, kBlocked>(p);
 }
 
-// ---- zero the alignment padding rows of the expanded layout ----
-__global__ __launch_bounds__(kThreads) void zero_padding_kernel(const PadParams p) {
+// ---- zero the alignment padding rows of the expanded layout, and put scales that came in blocks into their columns ----
+// Workgroups [0, scale_blocks) turn a block each, those behind them zero rows.
+__global__ __launch_bounds__(kThreads) void zero_padding_kernel(const PadParams p, const int scale_blocks) {
+    extern __shared__ uint32_t scales[];              // [kScaleBlockRows][G + 1]
+    if (int(blockIdx.x) < scale_blocks) {
+        __shared__ unsigned long long padding;        // rows of the block that are padding
+        const int G = p.num_sf_packs, tid = threadIdx.x;
+        const int64_t r0 = int64_t(blockIdx.x) * kScaleBlockRows;
+        const int last = p.num_unaligned[p.E - 1];
+        const int64_t total = int64_t(p.psum_expert[p.E - 1]) - last + (int64_t(last) + p.A - 1) / p.A * p.A;
+        if (r0 >= total) return;
+        const int rows = int(min(p.expanded_capacity - r0, int64_t(kScaleBlockRows)));
+        const float rcp_G = 1.0f / float(G);
+        if (tid == 0) padding = 0ull;
+        for (int i = tid; i < rows * G; i += kThreads) {
+            const int r = small_div(i, rcp_G);
+            scales[r * (G + 1) + (i - r * G)] = p.recv_sf[place_in_block(i, kScaleBlockRows, rows, r0, p.rsf_hs)];
+        }
+        __syncthreads();
+        for (int e = tid; e < p.E; e += kThreads) {
+            const int cnt = p.num_unaligned[e];
+            const int64_t from = max(int64_t(p.psum_expert[e]) - r0, int64_t(0));
+            const int64_t to = min(int64_t(p.psum_expert[e]) + ((cnt + p.A - 1) / p.A * p.A - cnt) - r0, int64_t(kScaleBlockRows));
+            if (from < to) atomicOr(&padding, (to == 64 ? ~0ull : (1ull << to) - 1ull) & ~((1ull << from) - 1ull));
+        }
+        __syncthreads();
+        const unsigned long long none = padding | (total - r0 < kScaleBlockRows ? ~((1ull << (total - r0)) - 1ull) : 0ull);
+        for (int i = tid; i < rows * G; i += kThreads) {
+            const int g = rows == kScaleBlockRows ? i / kScaleBlockRows : int(unsigned(i) / unsigned(rows));
+            const int r = i - g * rows;
+            p.recv_sf[r0 + r + g * p.rsf_hs] = (none >> r) & 1ull ? 0u : scales[r * (G + 1) + g];
+        }
+        return;
+    }
     const int lane = threadIdx.x & 63;
-    const int64_t work = int64_t(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
+    const int64_t work = int64_t(int(blockIdx.x) - scale_blocks) * kWavesPerBlock + (threadIdx.x >> 6);
     const int pad_slots = p.A - 1;
     if (work >= int64_t(p.E) * pad_slots) return;
     const int e = int(work / pad_slots);
@@ -1144,7 +1185,7 @@ __global__ __launch_bounds__(kThreads) void zero_padding_kernel(const PadParams 
     uint8_t* dst = p.recv_x + row * p.out_row_bytes;
     const vec16 zero{0, 0, 0, 0};
     for (int off = lane * 16; off < p.out_row_bytes; off += kWaveSize * 16) store16(dst + off, zero);
-    if (p.recv_sf != nullptr)
+    if (p.recv_sf != nullptr && !p.sf_blocked)
         for (int g = lane; g < p.num_sf_packs; g += kWaveSize) p.recv_sf[row * p.rsf_ts + int64_t(g) * p.rsf_hs] = 0u;
     if (p.recv_topk_weights != nullptr && lane == 0) p.recv_topk_weights[row] = 0.f;
 }
@@ -1406,10 +1447,12 @@ hipError_t launch_copy(MoveParams p, hipStream_t stream) {
     // Rows without scale packs, in tiles of one and two KB: a kernel without the branch on the packs, with which they took 3 to 8 %
     // longer (16384 x 7168 top-2, 1 KB tiles: 126 against 119 us; 65536 x 256 top-8 84.4 against 77.1).  Tiles of four KB and many wide
     // rows to a token are the other way round (8192 x 2048 top-2 21.9 us without the branch, 20.5 with it; 16384 x 7168 top-8 254, 249).
-    constexpr bool kSmallTile = kVecs <= 2;
-    const bool plain = kSmallTile && p.recv_sf == nullptr && (rows_per_token(p) < 5.0 || p.row_bytes < 4096);
-    const auto kernel = p.fused ? (plain ? dispatch_copy_single_launch_kernel<kVecs, !kSmallTile> : dispatch_copy_single_launch_kernel<kVecs, true>)
-                                : (plain ? dispatch_copy_kernel<kVecs, !kSmallTile> : dispatch_copy_kernel<kVecs, true>);
+    constexpr int kPlain = kVecs <= 2 ? kNoScales : kScalesInPlace;
+    const bool plain = kPlain == kNoScales && p.recv_sf == nullptr && (rows_per_token(p) < 5.0 || p.row_bytes < 4096);
+    auto kernel = p.fused ? (plain ? dispatch_copy_single_launch_kernel<kVecs, kPlain> : dispatch_copy_single_launch_kernel<kVecs, kScalesInPlace>)
+                          : (plain ? dispatch_copy_kernel<kVecs, kPlain> : dispatch_copy_kernel<kVecs, kScalesInPlace>);
+    if constexpr (kVecs <= 4)
+        if (p.sf_blocked) kernel = p.fused ? dispatch_copy_single_launch_kernel<kVecs, kScalesInBlocks> : dispatch_copy_kernel<kVecs, kScalesInBlocks>;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), move_lds_bytes(p), stream, p);
     return hipGetLastError();
 }
@@ -1421,7 +1464,8 @@ hipError_t launch_cast(MoveParams p, hipStream_t stream) {
     plan_cache_warming(p);
     if constexpr (kPairs <= 2) {
         if (p.fused) {
-            hipLaunchKernelGGL((dispatch_cast_single_launch_kernel<kPairs>), dim3(blocks), dim3(kThreads), move_lds_bytes(p), stream, p);
+            const auto kernel = p.sf_blocked ? dispatch_cast_single_launch_kernel<kPairs, true> : dispatch_cast_single_launch_kernel<kPairs, false>;
+            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), move_lds_bytes(p), stream, p);
             return hipGetLastError();
         }
     }
@@ -1438,7 +1482,10 @@ hipError_t launch_cast(MoveParams p, hipStream_t stream) {
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((dispatch_cast_kernel<kPairs>), dim3(blocks), dim3(kThreads), move_lds_bytes(p), stream, p);
+    auto kernel = dispatch_cast_kernel<kPairs, false>;
+    if constexpr (kPairs <= 2)
+        if (p.sf_blocked) kernel = dispatch_cast_kernel<kPairs, true>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), move_lds_bytes(p), stream, p);
     return hipGetLastError();
 }
 
@@ -1485,11 +1532,27 @@ hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream) {
     }
 }
 
+// From 128 K scales on.  Move + pad kernel in us, scales stored into their columns / in blocks, fused cast and pass-through of the
+// same rows, top-8 of 256 experts, alignment 128: 8192 x 7168 134.2 + 19.7 / 117.4 + 22.1 and 106.8 + 19.5 / 100.0 + 21.3; 2048 x
+// 7168 37.1 + 20.0 / 35.5 + 18.4; 512 x 7168 11.9 + 31.9 / 11.4 + 28.4 (a padding row's zeroes are single dwords too); top-6 of 64
+// experts, 8192 x 1024 21.8 + 5.0 / 19.7 + 4.5, 1024 x 2048 in one launch (98 K scales) 15.7 + 4.4 / 15.6 + 4.9; 64 x 2048 6.7 + 6.0 /
+// 7.2 + 6.1.
+bool scales_in_blocks(const MoveParams& m, int alignment) {
+    constexpr int64_t kFromScales = int64_t(1) << 17;
+    const bool tile_known = m.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? m.cast_pairs >= 0 && m.cast_pairs <= 2
+                                                                      : m.copy_vecs >= 0 && m.copy_vecs <= 4 && m.copy_vecs != 3;
+    return m.do_expand && alignment > 1 && m.payload != DEEP_EP_HIP_PAYLOAD_BF16 && m.recv_sf != nullptr && m.rsf_ts == 1 &&
+           m.rsf_hs >= m.expanded_capacity && m.num_sf_packs >= 2 && m.num_sf_packs <= kMaxBlockedScales && tile_known &&
+           int64_t(m.T) * m.K * m.num_sf_packs >= kFromScales;
+}
+
 hipError_t launch_zero_padding(const PadParams& p, hipStream_t stream) {
     if (p.A <= 1 || p.E == 0) return hipSuccess;
     const int64_t waves = int64_t(p.E) * (p.A - 1);
     const unsigned blocks = unsigned((waves + kWavesPerBlock - 1) / kWavesPerBlock);
-    hipLaunchKernelGGL(zero_padding_kernel, dim3(blocks), dim3(kThreads), 0, stream, p);
+    const int scale_blocks = p.sf_blocked ? int((p.expanded_capacity + kScaleBlockRows - 1) / kScaleBlockRows) : 0;
+    const size_t lds = p.sf_blocked ? size_t(kScaleBlockRows) * (p.num_sf_packs + 1) * sizeof(uint32_t) : 0;
+    hipLaunchKernelGGL(zero_padding_kernel, dim3(blocks + unsigned(scale_blocks)), dim3(kThreads), lds, stream, p, scale_blocks);
     return hipGetLastError();
 }
 

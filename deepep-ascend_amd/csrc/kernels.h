@@ -154,6 +154,7 @@ struct MoveParams {
     int payload;         // DEEP_EP_HIP_PAYLOAD_*
     int row_bytes;       // input row bytes
     int tiles;           // column tiles per token
+    int sf_blocked;      // recv_sf is column-major and the pad kernel follows: scales go out in blocks (below)
     int row_by_row;      // a wavefront waits for the stores of a row before it starts the next (set by the launcher)
     unsigned warm_lds_offset;   // single-launch cast: byte offset (in the dynamic LDS) of the 4 KB landing area of the
                                 // cache-warming loads, 0 = none
@@ -209,7 +210,18 @@ struct PadParams {
     const int32_t* num_unaligned;
     int64_t expanded_capacity;
     int E, A, out_row_bytes;
+    int sf_blocked;                  // recv_sf is in blocks: turned here
 };
+
+// Column-major scales of an expanded dispatch on their way.  A row's scales belong into as many columns as it has scales, a
+// dword each, 128 bytes of a column being the work of 32 rows that are moved far apart in time and by different XCDs: every
+// such store is a partial line of its own.  So where the pad kernel follows, the move kernel stores a row's scales side by side
+// and the pad kernel puts them into their columns.  Both in the same memory: the scales of 64 rows r0 .. r0 + 63 (the last
+// block: what is left) occupy 64 dwords of every column, and in between these places hold the same block row by row.
+constexpr int kScaleBlockRows = 64;
+constexpr int kMaxBlockedScales = 128;     // scales of a row: the pad kernel turns a block in LDS
+
+bool scales_in_blocks(const MoveParams& m, int alignment);
 
 hipError_t launch_zero_padding(const PadParams& p, hipStream_t stream);
 
