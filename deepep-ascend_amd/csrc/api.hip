@@ -52,11 +52,6 @@ struct LaunchPlan {
     bool fused;       // one launch: counting workgroups at the front of the move kernel
 };
 
-// Past this many mover workgroups the per-workgroup cost of the single-launch protocol (a look at the layout, one
-// atomic, two workgroup barriers) outweighs the launch it saves: 28 672 workgroups of 8192 BF16 rows of 14 KB take
-// 155 us in one launch against 134 us in two; 8 192 workgroups of the same rows cast to FP8 take 86 us against 92 us.
-constexpr int64_t kMaxFusedMovers = 16384;
-
 LaunchPlan plan_launches(int T, int K, int E, int R, bool do_layout, bool do_move, bool do_expand, int alignment, int payload, int H,
                          int row_bytes, const deep_ep_hip_tuning& tuning, int64_t rows_of_rank_lanes = -1 /* no top-k: rows received */) {
     LaunchPlan q{};
@@ -85,12 +80,7 @@ LaunchPlan plan_launches(int T, int K, int E, int R, bool do_layout, bool do_mov
         probe.cast_pairs = tuning.cast_pairs; probe.copy_vecs = tuning.copy_vecs;
         probe.K = K; probe.R = R; probe.fused = 1;
         probe.rank_lanes = rows_of_rank_lanes >= 0 ? 1 : 0; probe.recv_capacity = rows_of_rank_lanes;
-        // Rows copied as they are, from 300 MB of them on (345 MB of rows of up to 4 KB).  One launch / two, us, BF16 unless said:
-        //   3072 x 7168: 8 ranks 231 MB 59 / 63, 16 ranks 284 MB 71.8 / 71.4, 32 ranks 316 MB 77.0 / 79.0
-        //   4096 x 7168: 4 of 4 ranks 160 MB 48 / 51, 8 ranks 308 MB 80.5 / 77.7, 16 ranks 378 MB 97 / 90;   6144 x 7168, 8 ranks 462 MB 117 / 109
-        //   12288 x 2048: 8 ranks 264 MB 68 / 73, 16 ranks 324 MB 81.3 / 84.7, 32 ranks 361 MB 94 / 94;      8192 x 4096, 8 ranks 352 MB 100 / 93
-        //   FP8 with scales, 12288 x 4096: 8 ranks 264 MB 69 / 74, 16 ranks 324 MB 82.7 / 87.4, 32 ranks 361 MB 98 / 98
-        q.fused = dispatch_move_workgroups(probe) <= kMaxFusedMovers && !copy_prefers_finished_layout(probe);
+        q.fused = !move_prefers_finished_layout(probe, q.chunks);
     }
     return q;
 }

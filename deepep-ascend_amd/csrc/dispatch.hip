@@ -1303,6 +1303,8 @@ static double row_bytes_out(const MoveParams& p) {
     return double(p.T) * (cast ? p.H : p.row_bytes) * rows_per_token(p);
 }
 
+static bool is_large_input(const MoveParams& p) { return int64_t(p.T) * p.row_bytes >= (int64_t(64) << 20); }
+
 // A launch of so many workgroups of this tile that they fill `rounds` rounds of eight per CU.
 static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
     const int bytes = p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? p.H : p.row_bytes;
@@ -1314,7 +1316,6 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 // the pass-through payloads.  A tile of one whose last wavefront of a row would be half idle loses to one of two: 65536
 // tokens x 768 BF16 over 16 ranks 152 against 175 us, fused cast of 32768 x 1152 over 32 ranks 82 against 104 us.
 static int move_tile(const MoveParams& p) {
-    const bool large_input = int64_t(p.T) * p.row_bytes >= (int64_t(64) << 20);
     const double rows = rows_per_token(p);
     if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) {
         // Two segments (2048 channels) measured best at hidden 7168 and 8 ranks: 92.8 us per dispatch against 93.7 (4
@@ -1325,7 +1326,7 @@ static int move_tile(const MoveParams& p) {
         // the row bases, only for the expanded layout of a large call.
         if (p.cast_pairs != 0) return p.cast_pairs;
         if (p.H <= 1024) return 1;
-        if (p.fused) return p.do_expand && large_input ? 1 : 2;
+        if (p.fused) return p.do_expand && is_large_input(p) ? 1 : 2;
         if (p.H * 8 <= (p.H + 1023) / 1024 * 7 * 1024) return 2;
         return (p.do_expand ? fills_rounds(p, 1, 2) : rows >= 5.8 && fills_rounds(p, 1, 4)) ? 1 : 2;
     }
@@ -1340,8 +1341,7 @@ static int move_tile(const MoveParams& p) {
     // against 145; 16384 x 7168 top-4 of 16 ranks, 3.6 rows, 194 against 206), 2 KB where it goes to fewer (8192 x 7168, 4 of
     // 4 ranks: 75.6 us with four workgroups per CU against 79.4 with 1 KB and 84.9 with 4 KB) and, below five, over 64 ranks
     // (32768 x 2048 top-4: 126 us against 147).  At 183 MB (16384 x 2048, 4 of 4 ranks) 2 and 4 KB measured the same.
-    if (p.fused) return large_input ? 1 : widest;
-    if (row_bytes_out(p) < 200e6) return widest;
+    if (p.fused || row_bytes_out(p) < 200e6) return widest;
     const bool whole = p.row_bytes * 8 > kb * 7 * 1024;           // no wavefront of 1 KB would be half idle
     if (kb <= 3) return kb == 1 || (p.rank_lanes && rows >= 5.0) || ((p.rank_lanes || p.do_expand) && whole) ? 1 : 2;
     return rows >= (p.rank_lanes ? 2.5 : 3.5) && !(p.R >= 64 && rows < 5.0) ? 1 : 2;
@@ -1496,16 +1496,36 @@ int compute_units() {
     return device_attribute(hipDeviceAttributeMultiprocessorCount, cached, 256);
 }
 
-// More rows than this are copied in two launches: see plan_launches.
-bool copy_prefers_finished_layout(const MoveParams& p) {
-    return p.payload != DEEP_EP_HIP_PAYLOAD_CAST_FP8 && row_bytes_out(p) >= (p.row_bytes > 4096 ? 300e6 : 345e6);
-}
-
-int64_t dispatch_move_workgroups(const MoveParams& p) {
+// Mover workgroups launch_dispatch_move would start for p.
+static int64_t move_workgroups(const MoveParams& p) {
     const int tile = move_tile(p);
     const int64_t tiles = p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? (p.H + tile * 1024 - 1) / (tile * 1024)
                                                                     : (p.row_bytes + tile * 1024 - 1) / (tile * 1024);
     return (int64_t(p.T) * tiles + kWavesPerBlock - 1) / kWavesPerBlock;
+}
+
+// Where the per-workgroup cost of the single-launch protocol (a look at the layout, one atomic, two workgroup barriers) outweighs
+// the launch it saves:
+// - rows copied as they are, from 64 MB of input on (one launch / two, us; 1 KB tiles, as wide ones do not help there): BF16 16384 x
+//   2048 top-2 of 2 ranks 68.5 / 41.9, 4 of 4 ranks 82.5 / 57.8, top-6 of 16 ranks 108 / 91.6; 8192 x 4096 top-2 of 8 ranks 70.8 / 47.8;
+//   FP8 16384 x 4096 4 of 4 ranks 86.0 / 57.6 (6144 x 4096 BF16, 50 MB: 43.8 / 46.9);
+// - rows copied as they are, from 300 MB of them on (345 MB of rows of up to 4 KB), BF16 unless said:
+//   3072 x 7168: 8 ranks 231 MB 59 / 63, 16 ranks 284 MB 71.8 / 71.4, 32 ranks 316 MB 77.0 / 79.0
+//   4096 x 7168: 4 of 4 ranks 160 MB 48 / 51, 8 ranks 308 MB 80.5 / 77.7, 16 ranks 378 MB 97 / 90;   12288 x 2048, 8 ranks 264 MB
+//   68 / 73, 16 ranks 324 MB 81.3 / 84.7, 32 ranks 361 MB 94 / 94;   FP8 with scales, 12288 x 4096: 8 ranks 264 MB 69 / 74, 16
+//   ranks 324 MB 82.7 / 87.4, 32 ranks 361 MB 98 / 98
+// - a fused cast whose movers fill a little more than the first round of residents, all of whom wait for the layout: the rest
+//   then runs as a round of its own, while seven per CU of a plain move are under way at once.  Top-8, 1600 movers, one / two:
+//   2048 channels 8 ranks 33.8 / 30.7, 32 ranks 39.9 / 37.0; 1024 channels 8 ranks 27.6 / 24.3, 32 ranks 31.8 / 27.3; 7168 channels
+//   29.3 / 29.7 and 34.7 / 33.6.  1500 movers (2048 channels) 27.1 / 29.6, 1900 36.4 / 37.5; 4 of 4 ranks (2.7 rows) 23.9 / 23.5
+//   and with 7168 channels 23.4 / 23.9: left alone;
+// - more than 16384 movers of narrow rows, and of a fused cast.
+bool move_prefers_finished_layout(const MoveParams& p, int count_blocks) {
+    const int64_t movers = move_workgroups(p), round = int64_t(compute_units()) * kResidentWorkgroupsPerCu;
+    if (movers > 16384) return true;
+    if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8)
+        return !p.do_expand && rows_per_token(p) >= 4.0 && movers + count_blocks >= round && movers <= round + compute_units();
+    return is_large_input(p) || row_bytes_out(p) >= (p.row_bytes > 4096 ? 300e6 : 345e6);
 }
 
 hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream) {

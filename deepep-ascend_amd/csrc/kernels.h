@@ -195,10 +195,9 @@ struct MoveParams {
 };
 
 hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream);
-// Mover workgroups launch_dispatch_move would start for p (p.T, p.H, p.row_bytes, p.payload and the tile overrides set).
-int64_t dispatch_move_workgroups(const MoveParams& p);
-// A pass-through call with so many bytes of rows that the layout kernel and a move of its own are faster than one launch.
-bool copy_prefers_finished_layout(const MoveParams& p);
+// A call for which the layout kernel and a move of its own are faster than one launch (p.T, p.H, p.row_bytes, p.payload, the
+// routing shape and the tile overrides set, p.fused = 1).
+bool move_prefers_finished_layout(const MoveParams& p, int count_blocks);
 
 struct PadParams {
     uint8_t* recv_x;
