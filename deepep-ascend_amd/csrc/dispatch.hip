@@ -1315,8 +1315,19 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 // Column tile of a move launch: 1024-channel segments per wavefront for the fused cast, KB of row per wavefront for
 // the pass-through payloads.  A tile of one whose last wavefront of a row would be half idle loses to one of two: 65536
 // tokens x 768 BF16 over 16 ranks 152 against 175 us, fused cast of 32768 x 1152 over 32 ranks 82 against 104 us.
+//
+// Calls that leave the chip half empty take the narrowest tile that still gives a CU no more than eight wavefronts (ten with 2 KB
+// tiles): what a wavefront does is a chain, and a shorter one is over sooner.  Layout and move of compact calls with 1 / 2 / 4 KB tiles, us:
+// BF16 top-8 of 8 ranks 128 x 4096 14.0 / 14.2 / 14.9, 512 x 2048 16.7 / 16.9 / 17.5, 1237 x 2048 18.6 / 18.4 / 19.3 (2474 wavefronts of
+// 2 KB), 512 x 7168 23.0 / 20.6 / 19.7 (3584): left alone; fused cast, 1 / 2 segments, 300 x 7168 18.0 / 18.3, 512 x 2048 16.8 / 17.4,
+// 512 x 7168 (3584) 19.2 / 18.9.  Not in a single launch, where neighbours of the counting workgroups wait: 512 x 2048 BF16 16.7 / 16.5
+// / 15.6, though 300 x 7168 takes 16.7 / 16.3 / 17.5.
 static int move_tile(const MoveParams& p) {
     const double rows = rows_per_token(p);
+    const auto wavefronts_per_cu_at_most = [&](int tile, int most) {
+        const int bytes = p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? p.H : p.row_bytes;
+        return !p.fused && !p.do_expand && int64_t(p.T) * ((bytes + tile * 1024 - 1) / (tile * 1024)) <= int64_t(compute_units()) * most;
+    };
     if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) {
         // Two segments (2048 channels) measured best at hidden 7168 and 8 ranks: 92.8 us per dispatch against 93.7 (4
         // segments) and 96.9 (7 segments, one wavefront per token).  With many rows per token one segment is ahead on a
@@ -1325,13 +1336,15 @@ static int move_tile(const MoveParams& p) {
         // 7168 118 against 124 us, 16384 x 4096 top-8 134 against 139); in a single launch, whose workgroups each work out
         // the row bases, only for the expanded layout of a large call.
         if (p.cast_pairs != 0) return p.cast_pairs;
-        if (p.H <= 1024) return 1;
+        if (p.H <= 1024 || wavefronts_per_cu_at_most(1, 8)) return 1;
         if (p.fused) return p.do_expand && is_large_input(p) ? 1 : 2;
         if (p.H * 8 <= (p.H + 1023) / 1024 * 7 * 1024) return 2;
         return (p.do_expand ? fills_rounds(p, 1, 2) : rows >= 5.8 && fills_rounds(p, 1, 4)) ? 1 : 2;
     }
     if (p.copy_vecs != 0) return p.copy_vecs;
     const int kb = (p.row_bytes + 1023) / 1024;
+    if (wavefronts_per_cu_at_most(1, 8)) return 1;
+    if (kb > 2 && wavefronts_per_cu_at_most(2, 10)) return 2;
     const int widest = kb <= 1 ? 1 : kb <= 2 ? 2 : 4;
     // Small, latency-bound calls: up to 4 KB per wavefront, so that fewer wavefronts repeat the routing work (4096 rows
     // of 4 KB: 19.5 us against 21.1 us with 1 KB tiles).  Calls that write 200 MB and more are bound by their stores.

@@ -48,3 +48,26 @@ def test_both_ways_place_the_same_rows(payload, T, H, R, K, E):
                        [ri[:n], rw[:n], h.recv_src_metadata[:n], h.dst_buffer_slot_idx, h.psum_num_recv_tokens_per_expert])
     assert all(torch.equal(a, b) for a, b in zip(*results))
     buf.check_device_status()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("payload,T,H", [("bf16", 512, 2048), ("bf16", 513, 2048),       # 2048 tiles of 1 KB, and past them
+                                         ("bf16", 1280, 2056), ("bf16", 853, 2056),      # 2 KB tiles, the last 16 bytes wide: 2559 and past 2560
+                                         ("cast", 292, 7168), ("cast", 293, 7168), ("cast", 3, 16256)])
+def test_tiles_of_small_calls_place_the_same_rows(payload, T, H):
+    """Exact-size calls that leave the chip half empty take narrow tiles: both sides of the lines against the widest tile."""
+    import deep_ep
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.randn((T, H), generator=gen, device="cuda", dtype=torch.bfloat16)
+    w, idx = torch.topk(torch.rand((T, 32), generator=gen, device="cuda"), 6, dim=1)
+    buf = deep_ep.ElasticBuffer(deep_ep.LogicalGroup(0, 4), num_max_tokens_per_rank=T, hidden=H, num_topk=6)
+    knob, results = "cast_pairs" if payload == "cast" else "copy_vecs", []
+    for tile in (0, 4):
+        setattr(deep_ep.tuning, knob, tile)
+        try:
+            recv, ri, rw, h, _ = buf.dispatch(x, idx, w, num_experts=32, cast_to_fp8=payload == "cast")
+        finally:
+            setattr(deep_ep.tuning, knob, 0)
+        parts = recv if isinstance(recv, tuple) else (recv,)
+        results.append([p.view(torch.uint8) if p.dtype != torch.float32 else p for p in parts] + [ri, rw, h.recv_src_metadata, h.dst_buffer_slot_idx])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
