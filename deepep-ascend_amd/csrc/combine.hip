@@ -300,6 +300,30 @@ int workgroups_per_cu(const CombineParams& p) {
     return rows >= 5.8 ? 5 : 6;
 }
 
+// Column tile per wavefront: 1 KB of a BF16 row (512 channels, 41 registers, eight wavefronts per SIMD), or 2 KB.  us with 1 / 2 KB:
+// - many rows a token: 1 KB, at the residency above.  8 ranks top-8, compact: 8192 x 7168 120.7 / 125.3, 2048 x 4096 22.0 / 22.6, 1365 x
+//   2048 11.0 / 11.7, 512 x 1024 7.4 / 8.0; expanded 512 x 7168 16.8 / 18.2, 128 x 2048 8.4 / 9.5.
+// - few rows a token (top-2, or two ranks): 2 KB from one and a half wavefronts per place on (two and a half for rows past 8 KB).
+//   Compact, 2 ranks: 16384 x 7168 107.3 / 98.5, 2048 x 4096 13.2 / 12.5 (8 ranks 13.7 / 13.3), 2048 x 2888 11.6 / 11.1, 2048 x 2048
+//   9.0 / 9.5; 8 ranks 1365 x 7168 15.1 / 15.5.  4 of 4 ranks (2.7 rows) 16384 x 7168 137 / 145.  Expanded rows, whose routing is one trip longer, from half a wavefront per place on: top-2 16384 x 7168
+//   146.5 / 128.5, 1237 x 2048 9.2 / 8.5, 512 x 7168 10.3 / 9.9, 512 x 2048 7.3 / 7.5.
+// - expanded rows of up to 6 KB that fill half of the places to all of them: 2 KB.  Top-4: 1237 x 2048 11.0 / 10.5, 2048 x 2048 13.6 / 12.9,
+//   4096 x 1024 13.5 / 13.0; top-8 the same within 0.2.
+// - compact rows of up to 6 KB and four rows a token and more that fill seven eighths of the places: 2 KB.  1237 x 2888, top-9 of 6 ranks
+//   13.4 / 12.9, top-8 of 8 13.7 / 13.2; 2048 x 2048 13.6 / 13.4 and 13.9 / 13.9; 4 of 4 ranks 1237 x 3072 9.6 / 10.2.
+// - V1 rows of 2 KB that fill half of the places: 2 KB.  2048 x 1024, top-9 of 6 ranks 10.5 / 10.1, top-8 of 8 10.7 / 10.4; 2048 x 2048
+//   14.5 / 15.1 and 14.9 / 15.6.
+bool takes_two_kb_tiles(const CombineParams& p) {
+    const int kb = (p.H * 2 + 1023) / 1024;
+    if (kb < 2) return false;
+    const int64_t places = int64_t(compute_units()) * 8 * kWavesPerBlock, waves = int64_t(p.T) * kb;
+    const bool expanded = p.do_expand && !p.rank_mode, fits = kb <= 6 && waves <= places;
+    const double rows = rows_per_token(p);
+    if (rows < 2.3 && 2 * waves >= (expanded ? 1 : kb <= 8 ? 3 : 5) * places) return true;
+    if (p.rank_mode) return kb == 2 && fits && 2 * waves >= places;
+    return fits && (expanded ? 2 * waves > places : rows >= 4.0 && 8 * waves > 7 * places);
+}
+
 template <int kVecs, int kLayout>
 hipError_t launch_layout(const CombineParams& p, unsigned blocks, hipStream_t stream) {
     hipLaunchKernelGGL((combine_kernel<kVecs, kLayout>), dim3(blocks), dim3(kThreads), lds_for_residency(workgroups_per_cu(p)), stream, p);
@@ -362,15 +386,7 @@ hipError_t launch_rebuild_slot_map(const SlotMapParams& p, hipStream_t stream) {
 
 hipError_t launch_combine_kernel(CombineParams p, hipStream_t stream) {
     if (p.T == 0) return hipSuccess;
-    // Column tile per wavefront, in KB of a BF16 row: 1 KB (512 channels, 41 registers, eight wavefronts per SIMD) measured
-    // best, at the residency above - 8192 tokens x 7168: 117.0 us against 117.9 (2 KB), expanded 179.4 against 179.8.  Calls
-    // of rows up to 6 KB that are over in one round of workgroups are ahead with 2 KB, which repeats the routing work half as
-    // often: 1237 x 2888 top-9 9.8 against 10.7, 512 x 1024 6.8 against 7.2 (512 x 7168: 9.9 against 9.6).
-    int vecs = p.vecs;
-    if (vecs == 0) {
-        const int kb = (p.H * 2 + 1023) / 1024;
-        vecs = kb >= 2 && kb <= 6 && int64_t(p.T) * kb <= int64_t(compute_units()) * 8 * kWavesPerBlock ? 2 : 1;
-    }
+    const int vecs = p.vecs != 0 ? p.vecs : takes_two_kb_tiles(p) ? 2 : 1;
     switch (vecs) {
         case 1: return launch<1>(p, stream);
         case 4: return launch<4>(p, stream);

@@ -771,11 +771,10 @@ hipError_t launch_ll_combine(const LLCombineParams& p, hipStream_t stream) {
     if (p.S <= 0 || p.src_token_stride <= 0) return hipSuccess;
     int vecs = p.vecs;
     if (vecs != 1 && vecs != 2 && vecs != 4 && vecs != 7) {
-        // Decode-sized calls are over before a second round of workgroups could start: 2 KB per wavefront is the widest
-        // tile whose whole grid is resident at once (measured at 1024 tokens x 7168: 1 KB 8.4 us, 2 KB 7.9, 4 KB 9.2,
-        // 7 KB 9.3).  Large batches stream with 4 KB tiles.
-        const int64_t tokens = int64_t(p.S) * p.src_token_stride;
-        vecs = p.H * 2 <= 1024 ? 1 : tokens <= 4096 ? 2 : 4;
+        // 2 KB is the widest tile whose whole grid is resident at once at decode sizes (1024 tokens x 7168: 1 KB 8.4 us, 2 KB 7.9, 4 KB
+        // 9.2, 7 KB 9.3), and the best one in large batches (8192 tokens x 7168 over 8 ranks 48.0 / 43.7 / 45.4 / 47.7, over 16 ranks
+        // 43.6 / 34.2 / 35.6 / 38.3, 8192 x 2048 17.8 / 16.4 / 16.7 / 21.5).
+        vecs = p.H * 2 <= 1024 ? 1 : 2;
     }
     if (p.use_logfmt) vecs = p.H % 1024 == 0 ? 2 : 1;                                     // one codec chunk per wavefront
     const int tiles = (p.H * 2 + vecs * 1024 - 1) / (vecs * 1024);
@@ -786,17 +785,14 @@ hipError_t launch_ll_combine(const LLCombineParams& p, hipStream_t stream) {
         else hipLaunchKernelGGL((ll_combine_kernel<1, true>), dim3(blocks), dim3(kMoveThreads), 0, stream, p, tiles);
         return hipGetLastError();
     }
-    // Decode-sized calls: one wavefront per workgroup.  The wavefronts share nothing, and single-wavefront workgroups are
-    // placed and retired one by one instead of in fours (1024 tokens x 7168: 7.55 against 8.1 us; large batches and the
-    // routing kernels of the high-throughput path measured no difference).
-    if (int64_t(p.S) * p.src_token_stride <= 4096 && (vecs == 1 || vecs == 2)) {
+    // One wavefront per workgroup: the wavefronts share nothing, and single-wavefront workgroups are placed and retired one by one
+    // instead of in fours (1024 tokens x 7168: 7.55 against 8.1 us).
+    if (vecs == 1 || vecs == 2) {
         if (vecs == 1) hipLaunchKernelGGL((ll_combine_kernel<1, false, kWaveSize>), dim3(unsigned(waves)), dim3(kWaveSize), 0, stream, p, tiles);
         else hipLaunchKernelGGL((ll_combine_kernel<2, false, kWaveSize>), dim3(unsigned(waves)), dim3(kWaveSize), 0, stream, p, tiles);
         return hipGetLastError();
     }
-    if (vecs == 1) hipLaunchKernelGGL(ll_combine_kernel<1>, dim3(blocks), dim3(kMoveThreads), 0, stream, p, tiles);
-    else if (vecs == 2) hipLaunchKernelGGL(ll_combine_kernel<2>, dim3(blocks), dim3(kMoveThreads), 0, stream, p, tiles);
-    else if (vecs == 4) hipLaunchKernelGGL(ll_combine_kernel<4>, dim3(blocks), dim3(kMoveThreads), 0, stream, p, tiles);
+    if (vecs == 4) hipLaunchKernelGGL(ll_combine_kernel<4>, dim3(blocks), dim3(kMoveThreads), 0, stream, p, tiles);
     else hipLaunchKernelGGL(ll_combine_kernel<7>, dim3(blocks), dim3(kMoveThreads), 0, stream, p, tiles);
     return hipGetLastError();
 }
