@@ -50,15 +50,15 @@ __device__ __forceinline__ void add_row(float (&acc)[kVecs][8], const vec16 (&v)
 // The row is the same for the whole wavefront, so it is read through a buffer descriptor of its own (base: the row; range:
 // its bytes, none for row < 0): channels past the row's end and missing rows read as zero in the load itself.  With a branch
 // around each load instead, the compiler put waits and address arithmetic between the loads of a batch.
-template <int kVecs>
+template <int kVecs, bool kStream>
 __device__ __forceinline__ void load_row(vec16 (&v)[kVecs], const uint8_t* base, int row, int row_bytes, int tile, int lane) {
     const auto of_row = buffer_of(base + int64_t(max(row, 0)) * row_bytes, row >= 0 ? row_bytes : 0);
 #pragma unroll
-    for (int i = 0; i < kVecs; ++i) v[i] = buffer_load16_stream(of_row, (tile * kVecs + i) * 1024 + lane * 16);
+    for (int i = 0; i < kVecs; ++i) v[i] = buffer_load16_as<kStream>(of_row, (tile * kVecs + i) * 1024 + lane * 16);
 }
 
 // acc += sum of rows named by the lanes in `mask` (ascending lane order); row_of_lane < 0 adds nothing.
-template <int kVecs>
+template <int kVecs, bool kStream>
 __device__ __forceinline__ void accumulate_rows(float (&acc)[kVecs][8], uint64_t mask, int row_of_lane,
                                                 const uint8_t* x, int row_bytes, int tile, int lane) {
     while (mask) {
@@ -74,7 +74,7 @@ __device__ __forceinline__ void accumulate_rows(float (&acc)[kVecs][8], uint64_t
         }
         vec16 v[kBatch][kVecs];
 #pragma unroll
-        for (int b = 0; b < kBatch; ++b) load_row<kVecs>(v[b], x, rows[b], row_bytes, tile, lane);
+        for (int b = 0; b < kBatch; ++b) load_row<kVecs, kStream>(v[b], x, rows[b], row_bytes, tile, lane);
 #pragma unroll
         for (int b = 0; b < kBatch; ++b)
             if (rows[b] >= 0) add_row<kVecs>(acc, v[b]);
@@ -86,7 +86,8 @@ __device__ __forceinline__ void accumulate_rows(float (&acc)[kVecs][8], uint64_t
 // kRankRows: V1 conventions (CombineParams::rank_mode).
 enum : int { kCompactRows = 0, kExpandedRows = 1, kExpandedRowsReducedPerRank = 2, kRankRows = 3 };
 
-template <int kVecs, int kLayout>
+// kStream: rows are read past the memory-side cache (reads_past_the_cache).
+template <int kVecs, int kLayout, bool kStream>
 __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p) {
     constexpr bool kExpanded = kLayout == kExpandedRows || kLayout == kExpandedRowsReducedPerRank;
     const int lane = threadIdx.x & 63;
@@ -115,12 +116,12 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p
         for (int c = 0; c < 8; ++c) acc[i][c] = 0.f;
     if (p.bias0 != nullptr) {
         vec16 v[kVecs];
-        load_row<kVecs>(v, p.bias0, t, row_bytes, tile, lane);
+        load_row<kVecs, true>(v, p.bias0, t, row_bytes, tile, lane);
         add_row<kVecs>(acc, v);
     }
     if (p.bias1 != nullptr) {
         vec16 v[kVecs];
-        load_row<kVecs>(v, p.bias1, t, row_bytes, tile, lane);
+        load_row<kVecs, true>(v, p.bias1, t, row_bytes, tile, lane);
         add_row<kVecs>(acc, v);
     }
 
@@ -187,9 +188,9 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p
     }
 
     if constexpr (kLayout == kCompactRows || kLayout == kRankRows) {
-        accumulate_rows<kVecs>(acc, __ballot(row_c >= 0), row_c, p.x, row_bytes, tile, lane);
+        accumulate_rows<kVecs, kStream>(acc, __ballot(row_c >= 0), row_c, p.x, row_bytes, tile, lane);
     } else if constexpr (kLayout == kExpandedRows) {
-        accumulate_rows<kVecs>(acc, __ballot(erow >= 0), erow, p.x, row_bytes, tile, lane);
+        accumulate_rows<kVecs, kStream>(acc, __ballot(erow >= 0), erow, p.x, row_bytes, tile, lane);
     } else {
         // One term per destination rank, in ascending order of the rank's master lane; a rank's rows are summed in
         // lane order and the sum is rounded to BF16 before it is added.  The rows are put into that order first (each
@@ -229,7 +230,7 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p
             }
             vec16 v[kBatch][kVecs];
 #pragma unroll
-            for (int b = 0; b < kBatch; ++b) load_row<kVecs>(v[b], p.x, rows[b], row_bytes, tile, lane);
+            for (int b = 0; b < kBatch; ++b) load_row<kVecs, kStream>(v[b], p.x, rows[b], row_bytes, tile, lane);
 #pragma unroll
             for (int b = 0; b < kBatch; ++b) {
                 if (rows[b] < 0) continue;
@@ -324,9 +325,18 @@ bool takes_two_kb_tiles(const CombineParams& p) {
     return fits && (expanded ? 2 * waves > places : rows >= 4.0 && 8 * waves > 7 * places);
 }
 
+// The rows a combine adds up have just been written, by the experts or by the dispatch itself: up to 110 MB of them are read with plain
+// loads, which find them in the memory-side cache.  Dispatch and combine of BF16 rows, us, streaming / plain rows (the dispatch stores
+// accordingly, keeps_rows): 4096 x 2048 top-6 of 8 ranks, forward and backward (74 MB) 91.2 / 84.9, 16384 x 2048 of 2 ranks (100 MB) 77.5
+// / 76.0; combine of rows an expert has just written, with an FP8 dispatch in front, 1024 x 7168 (78 MB) 42.3 / 36.7, 700 x 4096 (30 MB) 27.4 /
+// 26.6; rows that are in HBM while the cache is full of what others have written are the other way round (41.0 / 53.5).  More rows than
+// the cache holds beside other traffic are read past it: 2100 x 7168 (160 MB) 67.5 / 74.0, 4096 x 7168 (311 MB) 134 / 170.
+bool reads_past_the_cache(const CombineParams& p) { return rows_per_token(p) * p.T * p.H * 2 > 110e6; }
+
 template <int kVecs, int kLayout>
 hipError_t launch_layout(const CombineParams& p, unsigned blocks, hipStream_t stream) {
-    hipLaunchKernelGGL((combine_kernel<kVecs, kLayout>), dim3(blocks), dim3(kThreads), lds_for_residency(workgroups_per_cu(p)), stream, p);
+    const auto kernel = reads_past_the_cache(p) ? combine_kernel<kVecs, kLayout, true> : combine_kernel<kVecs, kLayout, false>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), lds_for_residency(workgroups_per_cu(p)), stream, p);
     return hipGetLastError();
 }
 

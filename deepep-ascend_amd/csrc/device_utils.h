@@ -36,7 +36,8 @@ __device__ __forceinline__ vec16 load16(const void* p) {
 __device__ __forceinline__ void store16(void* p, const vec16& v) {
     *reinterpret_cast<vec16*>(p) = v;
 }
-// Streaming (non-temporal) forms for payload that is touched exactly once.
+// Streaming (non-temporal) forms: past the 256 MB memory-side cache, which a plain load or store fills.  A line that is there,
+// written and not yet in HBM, costs a streaming load more than a plain one.
 __device__ __forceinline__ vec16 load16_stream(const void* p) {
     const uint32_t* q = reinterpret_cast<const uint32_t*>(p);
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -47,6 +48,17 @@ __device__ __forceinline__ void store16_stream(void* p, const vec16& v) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     u32x4 t = {v.x, v.y, v.z, v.w};
     __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
+}
+
+template <bool kStream>
+__device__ __forceinline__ vec16 load16_as(const void* p) {
+    if constexpr (kStream) return load16_stream(p);
+    else return load16(p);
+}
+template <bool kStream>
+__device__ __forceinline__ void store16_as(void* p, const vec16& v) {
+    if constexpr (kStream) store16_stream(p, v);
+    else store16(p, v);
 }
 
 // bf16 <-> fp32 on raw bits.
@@ -135,9 +147,10 @@ __device__ __forceinline__ int row16_sum(int v) {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const uint8_t* base, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, bytes, 0x00027000);
 }
-__device__ __forceinline__ vec16 buffer_load16_stream(__amdgpu_buffer_rsrc_t from, int offset) {
+template <bool kStream>
+__device__ __forceinline__ vec16 buffer_load16_as(__amdgpu_buffer_rsrc_t from, int offset) {
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(from, offset, 0, 2 /* nt */);
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(from, offset, 0, kStream ? 2 /* nt */ : 0);
     return vec16{v.x, v.y, v.z, v.w};
 }
 

@@ -682,7 +682,10 @@ __device__ __forceinline__ bool warm_next_rounds_of_rows(const MoveParams& p, un
 // kScales: rows may come with scale packs (p.recv_sf).
 enum : int { kNoScales = 0, kScalesInPlace = 1, kScalesInBlocks = 2 };
 
-template <int kVecs, bool kFused, int kScales>
+// kCached: what goes through the memory-side cache (cached_side).
+enum : int { kNeither = 0, kInput = 1, kRows = 2 };
+
+template <int kVecs, bool kFused, int kScales, int kCached>
 __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
     if constexpr (kFused) {
         if (blockIdx.x <= unsigned(p.count_blocks)) {
@@ -716,7 +719,7 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
     for (int i = 0; i < kVecs; ++i) {
         const int off = (tile * kVecs + i) * 1024 + lane * 16;
         v[i] = vec16{0, 0, 0, 0};
-        if (has_work && off < p.row_bytes) v[i] = load16_stream(src + off);
+        if (has_work && off < p.row_bytes) v[i] = load16_as<kCached != kInput>(src + off);
     }
 
     // The caller's scale packs ride with tile 0: requested with the payload, once, not per destination row.
@@ -759,7 +762,7 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
 #pragma unroll
         for (int i = 0; i < kVecs; ++i) {
             const int off = (tile * kVecs + i) * 1024 + lane * 16;
-            if (off < p.row_bytes) store16_stream(dst + off, v[i]);
+            if (off < p.row_bytes) store16_as<kCached != kRows>(dst + off, v[i]);
         }
         if (packs) {
             if (lane < p.num_sf_packs) *scale_place<kScales == kScalesInBlocks>(p, row, lane) = pack;
@@ -1120,13 +1123,13 @@ __global__ __launch_bounds__(kQueueThreads) void dispatch_cast_queue_kernel(cons
 // The kernels.  The single-launch forms also hold the counting and publishing code, whose register needs must not cost
 // the movers their occupancy: they are held to six wavefronts per SIMD (80 registers) - six workgroups per CU, which
 // is also where the move streams fastest (more were slower when tried with a leaner counting step, fewer are slower too).
-template <int kVecs, int kScales>
+template <int kVecs, int kScales, int kCached>
 __global__ __launch_bounds__(kThreads) void dispatch_copy_kernel(const MoveParams p) {
-    dispatch_copy<kVecs, false, kScales>(p);
+    dispatch_copy<kVecs, false, kScales, kCached>(p);
 }
-template <int kVecs, int kScales>
+template <int kVecs, int kScales, int kCached>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void dispatch_copy_single_launch_kernel(const MoveParams p) {
-    dispatch_copy<kVecs, true, kScales>(p);
+    dispatch_copy<kVecs, true, kScales, kCached>(p);
 }
 template <int kPairs, bool kBlocked>
 __global__ __launch_bounds__(kThreads) void dispatch_cast_kernel(const MoveParams p) {
@@ -1452,22 +1455,47 @@ void plan_cache_warming(MoveParams& p) {
     p.warm_ahead = rounds * first_round * unsigned(kWavesPerBlock);
 }
 
-template <int kVecs>
-hipError_t launch_copy(MoveParams p, hipStream_t stream) {
-    p.tiles = (p.row_bytes + kVecs * 1024 - 1) / (kVecs * 1024);
-    const unsigned blocks = move_grid(p, int64_t(p.T) * p.tiles);
-    plan_cache_warming(p);
+// Which side of a copy goes through the memory-side cache (256 MB).
+// - BF16, up to 110 MB of rows: the rows, which whoever is next then finds there; the combine reads as many with plain loads.
+// - BF16, more: the input, which the layer in front has just written; so many rows would drive it and each other out.  Dispatch and
+//   combine, us, neither / input: 2600 x 7168 over 8 ranks (198 MB) 103.4 / 96.5, 3400 x 7168 (258 MB) 123.7 / 116.5, 8192 x 7168 (622 MB) 261.7 /
+//   261.5, V1 4096 x 7168 150.2 / 141.8, expanded 4096 x 4096 top-8 143.3 / 134.8; with the input just written behind 400 MB of other writes 103.7 /
+//   99.4, 125.8 / 118.2, 274.8 / 247.4, 151.5 / 141.5, 143.9 / 137.5; with an input that has left the cache by then 103.3 / 110.1, 125.7 /
+//   131.3, 265.4 / 275.7, 153.2 / 159.4, 146.1 / 150.6.
+// - FP8: neither.  Cast, dispatch and combine, neither / input / rows: 1024 x 7168 (39 MB) 43.2 / 44.3 / 43.4, 2100 x 7168 (80 MB) 71.0 / 71.4 /
+//   69.1, 4096 x 7168 (156 MB) 130.1 / 127.4 / 125.4 with three inputs in turn, 126.9 / - / 129.4 with more.
+static int cached_side(const MoveParams& p) {
+    if (p.payload != DEEP_EP_HIP_PAYLOAD_BF16) return kNeither;
+    return row_bytes_out(p) <= 110e6 ? kRows : kInput;
+}
+
+template <int kVecs, int kCached>
+hipError_t launch_copy_cached(const MoveParams& p, unsigned blocks, hipStream_t stream) {
     // Rows without scale packs, in tiles of one and two KB: a kernel without the branch on the packs, with which they took 3 to 8 %
     // longer (16384 x 7168 top-2, 1 KB tiles: 126 against 119 us; 65536 x 256 top-8 84.4 against 77.1).  Tiles of four KB and many wide
     // rows to a token are the other way round (8192 x 2048 top-2 21.9 us without the branch, 20.5 with it; 16384 x 7168 top-8 254, 249).
     constexpr int kPlain = kVecs <= 2 ? kNoScales : kScalesInPlace;
     const bool plain = kPlain == kNoScales && p.recv_sf == nullptr && (rows_per_token(p) < 5.0 || p.row_bytes < 4096);
-    auto kernel = p.fused ? (plain ? dispatch_copy_single_launch_kernel<kVecs, kPlain> : dispatch_copy_single_launch_kernel<kVecs, kScalesInPlace>)
-                          : (plain ? dispatch_copy_kernel<kVecs, kPlain> : dispatch_copy_kernel<kVecs, kScalesInPlace>);
+    auto kernel = p.fused ? (plain ? dispatch_copy_single_launch_kernel<kVecs, kPlain, kCached> : dispatch_copy_single_launch_kernel<kVecs, kScalesInPlace, kCached>)
+                          : (plain ? dispatch_copy_kernel<kVecs, kPlain, kCached> : dispatch_copy_kernel<kVecs, kScalesInPlace, kCached>);
     if constexpr (kVecs <= 4)
-        if (p.sf_blocked) kernel = p.fused ? dispatch_copy_single_launch_kernel<kVecs, kScalesInBlocks> : dispatch_copy_kernel<kVecs, kScalesInBlocks>;
+        if (p.sf_blocked) kernel = p.fused ? dispatch_copy_single_launch_kernel<kVecs, kScalesInBlocks, kCached> : dispatch_copy_kernel<kVecs, kScalesInBlocks, kCached>;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), move_lds_bytes(p), stream, p);
     return hipGetLastError();
+}
+
+template <int kVecs>
+hipError_t launch_copy(MoveParams p, hipStream_t stream) {
+    p.tiles = (p.row_bytes + kVecs * 1024 - 1) / (kVecs * 1024);
+    const unsigned blocks = move_grid(p, int64_t(p.T) * p.tiles);
+    plan_cache_warming(p);
+    if constexpr (kVecs <= 4) {
+        switch (cached_side(p)) {
+            case kInput: return launch_copy_cached<kVecs, kInput>(p, blocks, stream);
+            case kRows: return launch_copy_cached<kVecs, kRows>(p, blocks, stream);
+        }
+    }
+    return launch_copy_cached<kVecs, kNeither>(p, blocks, stream);
 }
 
 template <int kPairs>

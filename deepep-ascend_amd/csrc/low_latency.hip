@@ -119,28 +119,21 @@ constexpr int kMoveThreads = 256;
 constexpr int kMoveWaves = kMoveThreads / kWaveSize;
 constexpr int kFusedTokens = 3072;      // the single-kernel path: a lane per 64 tokens of the routing table, within its LDS
 
-// Loads one column tile (kPairs * 1024 channels) of token g: lane owns 16 consecutive channels per pair.  kClamped:
-// a pair past the end of the row loads the row's last 32 bytes instead of being skipped (no branch around the load;
-// what it brings is never stored).
-template <int kPairs, bool kClamped = false>
+// Loads one column tile (kPairs * 1024 channels) of token g: lane owns 16 consecutive channels per pair.  A pair past the end of
+// the row loads the row's last 32 bytes instead of being skipped (no branch around the load; what it brings is never stored).
+// Plain loads: a decode step has just written the tokens, and a streaming load of a line the memory-side cache holds unwritten
+// takes longer.  Dispatch and combine, streaming / plain, tokens just written by a copy behind 400 MB of other writes, us: 1024
+// tokens x 7168 FP8 20.8 / 20.1, 4096 tokens 50.3 / 48.1, 8192 x 2048 of 16 ranks 30.3 / 28.9; called over and over 21.8 / 18.9, 46.9 /
+// 43.8, 28.8 / 26.3; tokens left in HBM by then 21.1 / 23.8, 48.8 / 52.9, 30.3 / 31.3.
+template <int kPairs>
 __device__ __forceinline__ void ll_load_tile(const uint8_t* x, int hidden, int64_t g, int tile, int lane,
                                              vec16 (&in)[kPairs][2]) {
     const uint8_t* src = x + g * (int64_t(hidden) * 2);
 #pragma unroll
     for (int q = 0; q < kPairs; ++q) {
-        const int elem = (tile * kPairs + q) * 1024 + lane * 16;
-        if constexpr (kClamped) {
-            const int at = min(elem, hidden - 16);
-            in[q][0] = load16_stream(src + int64_t(at) * 2);
-            in[q][1] = load16_stream(src + int64_t(at) * 2 + 16);
-        } else {
-            in[q][0] = vec16{0, 0, 0, 0};
-            in[q][1] = vec16{0, 0, 0, 0};
-            if (elem < hidden) {
-                in[q][0] = load16_stream(src + int64_t(elem) * 2);
-                in[q][1] = load16_stream(src + int64_t(elem) * 2 + 16);
-            }
-        }
+        const int at = min((tile * kPairs + q) * 1024 + lane * 16, hidden - 16);
+        in[q][0] = load16(src + int64_t(at) * 2);
+        in[q][1] = load16(src + int64_t(at) * 2 + 16);
     }
 }
 
@@ -271,7 +264,7 @@ __global__ __launch_bounds__(kBlockThreads) void ll_move_kernel(const LLDispatch
                 for (int i = lane + kWaveSize; i < chunk; i += kWaveSize) v[b] += totals[i];
             }
         }
-        if (!loaded) ll_load_tile<kPairs, true>(p.x, p.H, g, tile, lane, in);
+        if (!loaded) ll_load_tile<kPairs>(p.x, p.H, g, tile, lane, in);
         loaded = true;
 #pragma unroll
         for (int b = 0; b < kBatch; ++b) {
@@ -338,7 +331,7 @@ __global__ __launch_bounds__(kFusedThreads) void ll_fused_kernel(const LLDispatc
     const int64_t own_loaded = p.topk_idx[g * p.K + min(lane, p.K - 1)];
     // the payload tile: queued behind the index loads, in flight while the routing pass runs
     vec16 in[kPairs][2];
-    ll_load_tile<kPairs, true>(p.x, p.H, g, tile, lane, in);
+    ll_load_tile<kPairs>(p.x, p.H, g, tile, lane, in);
     __builtin_amdgcn_sched_barrier(0);
 
     // An entry sets a bit iff it names a local expert: a negative or oversized id has a non-zero upper half or a lower

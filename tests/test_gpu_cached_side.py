@@ -1,0 +1,36 @@
+"""BF16 dispatches and combines on both sides of the line up to which rows go through the memory-side cache, in one launch and in two, with
+the last column tile of a row partly filled: every received row is the row of its source token, and a combine of the rows as they are is
+the token times the number of its rows (exact: at most eight equal terms of seven-bit values)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,H,E,R,K,sync", [
+    (17700, 2056, 32, 2, 2, True), (18100, 2056, 32, 2, 2, True),         # two launches: 109 and 112 MB of rows
+    (5050, 2056, 256, 8, 8, False), (5200, 2056, 256, 8, 8, False),       # one launch
+])
+@pytest.mark.parametrize("expand", [False, True])
+def test_rows_and_sums(T, H, E, R, K, sync, expand):
+    import deep_ep
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randint(-127, 128, (T, H), generator=gen, device="cuda").to(torch.bfloat16) / 16
+    w, idx = torch.topk(torch.rand((T, E), generator=gen, device="cuda"), K, dim=1)
+    idx = idx.masked_fill(torch.rand((T, K), generator=gen, device="cuda") < 0.05, -1)
+    buf = deep_ep.ElasticBuffer(deep_ep.LogicalGroup(0, R), num_max_tokens_per_rank=T, hidden=H, num_topk=K, allow_multiple_reduction=False)
+    recv, _, _, handle, _ = buf.dispatch(x, idx, w, num_experts=E, do_cpu_sync=sync, do_expand=expand)
+    rank = torch.where(idx >= 0, idx // (E // R), -1)
+    per_rank = torch.stack([(rank == r).any(dim=1) for r in range(R)], dim=1)
+    n = int(per_rank.sum())
+    meta = handle.recv_src_metadata[:n].long()
+    if expand:
+        lanes = meta[:, 2:]
+        rows, tokens = lanes[lanes >= 0], meta[:, :1].expand(-1, K)[lanes >= 0]
+        copies = (idx >= 0).sum(dim=1, keepdim=True)
+    else:
+        rows, tokens, copies = torch.arange(n, device="cuda"), meta[:, 0], per_rank.sum(dim=1, keepdim=True)
+    assert rows.numel() == int(copies.sum()) and torch.equal(recv[rows], x[tokens])
+    out, _, _ = buf.combine(recv, handle)
+    assert torch.equal(out.float(), (x.float() * copies).to(torch.bfloat16).float())
+    buf.check_device_status()
