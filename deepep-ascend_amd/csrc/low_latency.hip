@@ -725,21 +725,35 @@ hipError_t launch_fused_by_width(const LLDispatchParams& p, hipStream_t stream, 
     }
 }
 
+// Decode-sized calls: one kernel, every workgroup of which derives the slots itself.  How many threads a workgroup has, or 0 for the
+// two kernels.  Every workgroup passes over all selections, so the more there are the fewer workgroups a CU may have and the more
+// wavefronts share a pass.  Dispatch, us, 256 / 512 / 1024 threads / two kernels, FP8, top-1 over 16 ranks, top-4 over 4, the rest 8:
+//   up to 4096 selections       2048 x 2048 top-1 8.7 / 9.2 / 10.1 / 10.2;   1024 x 4096 top-4 8.6 / 10.1 / 12.1 / 11.7;
+//                               3072 x 7168 top-1 (6144 wavefronts) 13.6 / 13.9 / 15.8 / 13.9;   2048 x 7168 top-2 12.4 / 12.9 / 13.3 / 13.5
+//   up to 8192, 16 a CU         2240 x 2048 top-2 9.6 / 9.2 / 9.9 / 10.8;   1024 x 7168 top-8 12.0 / 11.0 / 14.2 / 13.1;   2048 x 7168 top-4
+//                               (4096 wavefronts) 15.7 / 14.6 / 15.4 / 15.9;   2560 x 7168 top-2 (5120) 15.5 / 14.6 / 17.0 / 14.6
+//   more, 8 wavefronts a CU     2048 x 2048 top-8 12.8 / 10.8 / 10.9 / 11.8;   2048 x 4096 top-8 15.1 / 13.3 / 13.3 / 14.1
+//   up to 16384, 16 a CU, 2048 tokens   1280 x 7168 top-8 15.0 / 15.1 / 13.2 / 14.1;   2048 x 7168 19.8 / 17.6 / 15.9 / 16.4
+//                               (over 16 ranks 18.3 / 15.4 / 14.7 / 14.5: the one point of the line where the two kernels are ahead)
+//   beyond                      2240 x 4096 top-8 17.7 / 16.9 / 14.5 / 14.1;   3072 x 7168 top-8 29.0 / 23.9 / 24.0 / 18.6
+static int fused_threads(const LLDispatchParams& p) {
+    const int64_t tokens = int64_t(p.S) * p.src_token_stride, selections = tokens * p.K;
+    const int64_t waves = tokens * ((p.H + fused_pairs(p) * 1024 - 1) / (fused_pairs(p) * 1024)), per_cu_8 = int64_t(compute_units()) * 8;
+    if (p.threads == 256 || p.threads == 512 || p.threads == 1024) return p.threads;
+    if (selections <= 4096) return 256;
+    if (waves <= per_cu_8) return 512;
+    if (waves > 2 * per_cu_8) return 0;
+    return selections <= 8192 ? 512 : selections <= 16384 && tokens <= 2048 ? 1024 : 0;
+}
+
 hipError_t launch_ll_dispatch(const LLDispatchParams& p, hipStream_t stream) {
     if (p.S <= 0 || p.src_token_stride <= 0) return hipSuccess;
-    // Decode-sized calls: one kernel, every workgroup derives the slots itself, as long as every wavefront has one item with one
-    // workgroup per compute unit - with a second item each it loses to the two kernels (their dispatch against it, us: FP8 top-8 over
-    // 8 ranks 7168 channels 1280 tokens 15.2 / 17.4, 2048 18.0 / 21.8, 3072 21.7 / 25.6; 4096 channels 2560 tokens 16.1 / 19.1;
-    // 2048 channels 3072 tokens 13.0 / 14.4; BF16 7168 channels 3072 tokens 25.5 / 28.1; up to that line it is 1 to 3 us ahead:
-    // 1024 tokens of 7168 channels 14.0 / 11.9, 2048 of 2048 12.6 / 11.5).
     const int64_t total_tokens = int64_t(p.S) * p.src_token_stride;
     // the routing table of the single-kernel path, plus one spare 32-bit word per lane
     const size_t fused_lds = size_t(p.E_l) * ((total_tokens + 63) / 64) * sizeof(uint64_t) + kWaveSize * sizeof(uint32_t);
     const bool table_fits = (reinterpret_cast<uintptr_t>(p.topk_idx) & 15) == 0 && total_tokens * p.K >= 2 && p.H >= 16;
-    const int threads = p.threads == 256 || p.threads == 1024 ? p.threads : 512;
-    const int64_t items = total_tokens * ((p.H + fused_pairs(p) * 1024 - 1) / (fused_pairs(p) * 1024));
-    const bool one_item_each = items <= int64_t(compute_units()) * (threads / kWaveSize);
-    if (one_item_each && total_tokens <= kFusedTokens && fused_lds <= 33 * 1024 && table_fits && !p.two_kernels) {
+    const int threads = fused_threads(p);
+    if (threads != 0 && total_tokens <= kFusedTokens && fused_lds <= 33 * 1024 && table_fits && !p.two_kernels) {
         if (threads == 256) return launch_fused_by_width<256>(p, stream, fused_lds);
         if (threads == 1024) return launch_fused_by_width<1024>(p, stream, fused_lds);
         return launch_fused_by_width<512>(p, stream, fused_lds);

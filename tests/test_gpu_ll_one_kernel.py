@@ -1,0 +1,44 @@
+"""Low-latency dispatch as a single kernel, at the lines between its workgroup sizes and the two kernels: 4096, 8192 and 16384 selections,
+eight and sixteen wavefronts a compute unit (256 of them), 2048 and 3072 tokens.  Every line from both sides against the oracle."""
+import pytest
+import torch
+
+import routing_cases as rc
+import routing_oracle as oracle
+from test_gpu_parity import assert_equal
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("R,T,H,E,K,payload", [
+    (8, 384, 4112, 16, 1, "bf16"),         # 3072 tokens, 6144 wavefronts (two tiles a token)
+    (8, 385, 4112, 16, 1, "bf16"),         # 3080: two kernels
+    (4, 512, 1152, 16, 2, "fp8"),          # 4096 selections
+    (4, 513, 1152, 16, 2, "fp8"),          # 4104: 512 threads
+    (8, 256, 4112, 16, 4, "bf16"),         # 8192 selections, 4096 wavefronts: 512 threads
+    (8, 257, 4112, 16, 4, "bf16"),         # 8224, 4112: two kernels
+    (8, 256, 4608, 16, 5, "ue8m0"),        # 10240 selections, 4096 wavefronts: 1024 threads
+    (8, 256, 4224, 16, 8, "fp8"),          # 16384
+    (8, 256, 4224, 16, 9, "fp8"),          # 18432: two kernels
+    (8, 257, 512, 16, 7, "bf16"),          # 14392 selections of 2056 tokens: two kernels
+    (8, 256, 512, 16, 10, "bf16"),         # 2048 wavefronts: 512 threads at any number of selections
+], ids=lambda v: str(v))
+def test_single_kernel_lines(R, T, H, E, K, payload):
+    import deep_ep
+    x, idx, w = rc.c5_sources(seed=23, R=R, T=T, H=H, E=E, K=K)
+    idx = idx.masked_fill(torch.rand(idx.shape, generator=torch.Generator().manual_seed(5)) < 0.1, -1)
+    fp8, ue8m0 = payload != "bf16", payload == "ue8m0"
+    M = -(-T // 4) * 4
+    dst = R - 1
+    buf = deep_ep.Buffer(deep_ep.LogicalGroup(dst, R), low_latency_mode=True)
+    recv, count, handle, _, _ = buf.low_latency_dispatch(x.cuda(), idx.cuda(), M, E, use_fp8=fp8, round_scale=ue8m0, use_ue8m0=ue8m0)
+    px, ps, cnt, info, rng = oracle.ll_dispatch(list(x), list(idx), M, E, R, dst, fp8, round_scale=ue8m0)
+    assert_equal(count, cnt, "packed_recv_count")
+    assert_equal(handle[1], rng, "packed_recv_layout_range")
+    got = recv[0] if fp8 else recv
+    for e in range(E // R):
+        n = int(cnt[e])
+        assert_equal(handle[0][e, :n], info[e, :n], f"src_info[{e}]")
+        assert_equal(got[e, :n], px[e, :n], f"packed_recv_x[{e}]")
+        if fp8:
+            assert_equal(recv[1][e, :n], oracle.pack_ue8m0(ps[e, :n]) if ue8m0 else ps[e, :n], f"scales[{e}]")
