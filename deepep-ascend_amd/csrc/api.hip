@@ -2,6 +2,7 @@
 // The declarations (and the reference interfaces they stand in for) are in include/deep_ep_hip.h.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -345,6 +346,8 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
         m.gates_finished = reinterpret_cast<uint32_t*>(ws + w.gates_finished);
         if (plan.fused) fill_fused(m, lay, plan, ws, w);
         m.sf_blocked = a->do_zero_padding && scales_in_blocks(m, a->expert_alignment) ? 1 : 0;
+
+        m.zeroed_rows = a->do_zero_padding ? int(std::min<int64_t>(int64_t(E) * (a->expert_alignment - 1) / 2, INT32_MAX)) : 0;
 
         hipError_t err = launch_dispatch_move(m, stream);
         if (err != hipSuccess) return hip_fail(err, "dispatch move launch");

@@ -1464,9 +1464,14 @@ void plan_cache_warming(MoveParams& p) {
 //   131.3, 265.4 / 275.7, 153.2 / 159.4, 146.1 / 150.6.
 // - FP8: neither.  Cast, dispatch and combine, neither / input / rows: 1024 x 7168 (39 MB) 43.2 / 44.3 / 43.4, 2100 x 7168 (80 MB) 71.0 / 71.4 /
 //   69.1, 4096 x 7168 (156 MB) 130.1 / 127.4 / 125.4 with three inputs in turn, 126.9 / - / 129.4 with more.
+// - BF16, the input larger than that cache or followed by 150 MB and more of zeroed rows (half an alignment for each expert): neither.
+//   Input called over and over, 20000 x 7168 (287 MB) 597.7 / 603.0; expanded over 256 experts aligned to 128 rows 4883 x 6728 (220 MB of zeros)
+//   309.7 / 313.2, 10714 x 6896 (225 MB) 601.2 / 611.5; over 128 (113 MB) it is 567.3 / 565.9 and, input just written, 580.1 / 552.4.
 static int cached_side(const MoveParams& p) {
     if (p.payload != DEEP_EP_HIP_PAYLOAD_BF16) return kNeither;
-    return row_bytes_out(p) <= 110e6 ? kRows : kInput;
+    if (row_bytes_out(p) <= 110e6) return kRows;
+    const double zeroed = p.zeroed_rows * double(p.row_bytes);
+    return double(p.T) * p.row_bytes <= 256e6 && zeroed < 150e6 ? kInput : kNeither;
 }
 
 template <int kVecs, int kCached>

@@ -34,3 +34,20 @@ def test_rows_and_sums(T, H, E, R, K, sync, expand):
     out, _, _ = buf.combine(recv, handle)
     assert torch.equal(out.float(), (x.float() * copies).to(torch.bfloat16).float())
     buf.check_device_status()
+
+
+@pytest.mark.parametrize("alignment", [280, 288])          # 147 and 151 MB of zeroed rows expected
+def test_rows_in_front_of_many_zeroed_ones(alignment):
+    import deep_ep
+    T, H, E, R, K = 5200, 2056, 256, 8, 8
+    gen = torch.Generator(device="cuda").manual_seed(alignment)
+    x = torch.randint(-127, 128, (T, H), generator=gen, device="cuda").to(torch.bfloat16) / 16
+    w, idx = torch.topk(torch.rand((T, E), generator=gen, device="cuda"), K, dim=1)
+    buf = deep_ep.ElasticBuffer(deep_ep.LogicalGroup(0, R), num_max_tokens_per_rank=T, hidden=H, num_topk=K, allow_multiple_reduction=False)
+    recv, _, _, handle, _ = buf.dispatch(x, idx, w, num_experts=E, do_expand=True, do_zero_padding=True, expert_alignment=alignment)
+    lanes = handle.recv_src_metadata[:, 2:].long()
+    rows = lanes[lanes >= 0]
+    assert torch.equal(recv[rows], x[handle.recv_src_metadata[:, :1].long().expand(-1, K)[lanes >= 0]])
+    recv[rows] = 0
+    assert rows.unique().numel() == T * K and not recv.any()
+    buf.check_device_status()
