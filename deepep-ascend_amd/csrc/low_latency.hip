@@ -735,6 +735,9 @@ hipError_t launch_fused_by_width(const LLDispatchParams& p, hipStream_t stream, 
 //   more, 8 wavefronts a CU     2048 x 2048 top-8 12.8 / 10.8 / 10.9 / 11.8;   2048 x 4096 top-8 15.1 / 13.3 / 13.3 / 14.1
 //   up to 16384, 16 a CU, 2048 tokens   1280 x 7168 top-8 15.0 / 15.1 / 13.2 / 14.1;   2048 x 7168 19.8 / 17.6 / 15.9 / 16.4
 //                               (over 16 ranks 18.3 / 15.4 / 14.7 / 14.5: the one point of the line where the two kernels are ahead)
+//   up to 24576, 16 a CU, 2048 channels   2288 x 1024 top-8 13.3 / 12.2 / 11.5 / 11.8;   2560 x 2048 top-6 13.4 / 12.0 / 10.8 / 11.6;   3072 x 2048
+//                               top-8 17.3 / 14.4 / 12.9 / 12.5, where a launch less is worth more than that: dispatch and combine of the
+//                               first 18.8 in three launches, 15.1 in two
 //   beyond                      2240 x 4096 top-8 17.7 / 16.9 / 14.5 / 14.1;   3072 x 7168 top-8 29.0 / 23.9 / 24.0 / 18.6
 static int fused_threads(const LLDispatchParams& p) {
     const int64_t tokens = int64_t(p.S) * p.src_token_stride, selections = tokens * p.K;
@@ -743,7 +746,8 @@ static int fused_threads(const LLDispatchParams& p) {
     if (selections <= 4096) return 256;
     if (waves <= per_cu_8) return 512;
     if (waves > 2 * per_cu_8) return 0;
-    return selections <= 8192 ? 512 : selections <= 16384 && tokens <= 2048 ? 1024 : 0;
+    if (selections <= 8192) return 512;
+    return selections <= 24576 && (p.H <= 2048 || (selections <= 16384 && tokens <= 2048)) ? 1024 : 0;
 }
 
 hipError_t launch_ll_dispatch(const LLDispatchParams& p, hipStream_t stream) {

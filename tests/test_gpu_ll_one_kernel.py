@@ -1,5 +1,5 @@
-"""Low-latency dispatch as a single kernel, at the lines between its workgroup sizes and the two kernels: 4096, 8192 and 16384 selections,
-eight and sixteen wavefronts a compute unit (256 of them), 2048 and 3072 tokens.  Every line from both sides against the oracle."""
+"""Low-latency dispatch as a single kernel, at the lines between its workgroup sizes and the two kernels: 4096, 8192, 16384 and 24576
+selections, eight and sixteen wavefronts a compute unit (256 of them), 2048 and 3072 tokens.  Every line from both sides against the oracle."""
 import pytest
 import torch
 
@@ -20,7 +20,10 @@ pytestmark = pytest.mark.gpu
     (8, 256, 4608, 16, 5, "ue8m0"),        # 10240 selections, 4096 wavefronts: 1024 threads
     (8, 256, 4224, 16, 8, "fp8"),          # 16384
     (8, 256, 4224, 16, 9, "fp8"),          # 18432: two kernels
-    (8, 257, 512, 16, 7, "bf16"),          # 14392 selections of 2056 tokens: two kernels
+    (8, 257, 2064, 16, 7, "bf16"),         # 14392 selections of 2056 tokens: two kernels
+    (8, 257, 2048, 16, 7, "bf16"),         # ... of at most 2048 channels: 1024 threads
+    (8, 384, 512, 16, 8, "fp8"),           # 24576 selections: 1024 threads
+    (8, 384, 512, 16, 9, "fp8"),           # 27648: two kernels
     (8, 256, 512, 16, 10, "bf16"),         # 2048 wavefronts: 512 threads at any number of selections
 ], ids=lambda v: str(v))
 def test_single_kernel_lines(R, T, H, E, K, payload):
