@@ -75,7 +75,8 @@ __global__ __launch_bounds__(kThreads) void intranode_prefix_kernel(const Intran
 // call of one chunk hands its totals over in LDS instead.  Launch time, mailbox included, with everything
 // waited for before the ticket and everything read back -> now: 128 tokens top-2 9.6 -> 6.1 us, 1237 top-9 13.0 -> 9.8,
 // 4096 top-8 10.0 -> 8.3, 16384 top-8 over 32 ranks 14.8 -> 11.5.
-template <int KMAX, bool kOneChunk>
+// kExpertsPerThread: of the publishing step in one trip, 0 = publish_layout.
+template <int KMAX, bool kOneChunk, int kExpertsPerThread>
 __global__ __launch_bounds__(kThreads) void layout_kernel(const LayoutParams p, const IntranodePrefixParams prefix) {
     extern __shared__ uint64_t bitmap[];   // [(R + E)][kWaves]
     __shared__ int is_last;
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(kThreads) void layout_kernel(const LayoutParams p, 
         count_chunk<KMAX, false>(p, 0, 1, bitmap, totals, [&] {
             wait_for_own_stores();                         // flags ORed into the status word, if any
             __syncthreads();
-            publish_layout_in_one_trip<kThreads, true>(p.pub, p.tab, 1, p.expert_bases != 0, totals, totals + p.R + p.E);
+            publish_layout_in_one_trip<kThreads, true, kExpertsPerThread>(p.pub, p.tab, 1, p.expert_bases != 0, totals, totals + p.R + p.E);
         });
     } else {
         // Hand the chunk totals to whichever workgroup finishes last: they were stored at agent scope (written through),
@@ -107,15 +108,21 @@ __global__ __launch_bounds__(kThreads) void layout_kernel(const LayoutParams p, 
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 
         // ---- last workgroup: per-bucket totals, the public prefix sums and the row bases (LDS is re-carved) ----
-        publish_layout<kThreads>(p.pub, p.tab, num_chunks, p.expert_bases != 0, reinterpret_cast<int*>(bitmap));
+        int* lds = reinterpret_cast<int*>(bitmap);
+        if constexpr (kExpertsPerThread == 0) publish_layout<kThreads>(p.pub, p.tab, num_chunks, p.expert_bases != 0, lds);
+        else publish_layout_in_one_trip<kThreads, false, kExpertsPerThread>(p.pub, p.tab, num_chunks, p.expert_bases != 0, nullptr, lds);
         if (tid == 0) *p.done_counter = 0u;                // ready for the next launch
     }
 }
 
 template <int KMAX>
 void launch_layout(const LayoutParams& q, const IntranodePrefixParams& prefix, dim3 grid, size_t lds, bool one_chunk, hipStream_t stream) {
-    if (one_chunk) hipLaunchKernelGGL((layout_kernel<KMAX, true>), grid, dim3(kThreads), lds, stream, q, prefix);
-    else hipLaunchKernelGGL((layout_kernel<KMAX, false>), grid, dim3(kThreads), lds, stream, q, prefix);
+    const bool by_one = fits_one_trip(1, q.R, q.E, q.tab.chunks_padded, kThreads), by_two = fits_one_trip(2, q.R, q.E, q.tab.chunks_padded, kThreads);
+    auto kernel = one_chunk ? (by_one ? layout_kernel<KMAX, true, 1> : layout_kernel<KMAX, true, 2>)
+                : by_one    ? layout_kernel<KMAX, false, 1>
+                : by_two    ? layout_kernel<KMAX, false, 2>
+                            : layout_kernel<KMAX, false, 0>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), lds, stream, q, prefix);
 }
 
 }  // namespace
@@ -135,7 +142,7 @@ hipError_t launch_layout_kernel(const LayoutParams& p, const IntranodePrefixPara
     const size_t bitmap_bytes = count_lds_bytes(p.R, p.E);
     const size_t publish_bytes = publish_lds_bytes(p.R, p.E, kThreads);
     const size_t behind = (size_t(p.R + p.E) + publish_scratch_ints(p.R, kThreads)) * sizeof(int);
-    const bool one_chunk = num_chunks == 1 && p.R <= kThreads && p.E <= kThreads;
+    const bool one_chunk = num_chunks == 1 && p.R <= kThreads && fits_one_trip(2, p.R, p.E, p.tab.chunks_padded, kThreads);
     size_t lds = one_chunk ? bitmap_bytes + behind : bitmap_bytes > publish_bytes ? bitmap_bytes : publish_bytes;
     if (prefix.R != 0 && lds < size_t(prefix.C) * sizeof(int)) lds = size_t(prefix.C) * sizeof(int);
     LayoutParams q = p;

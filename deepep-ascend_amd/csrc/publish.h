@@ -282,47 +282,59 @@ __device__ bool write_expert_bases_from_registers(const LayoutTables& t, const u
     return all_complete != 0;
 }
 
-// publish_layout for the common sizes: num_experts <= kThreads, R * chunks_padded <= 16 * kThreads.  A workgroup of its
+// publish_layout for the common sizes: num_experts <= kPerThread * kThreads, R * chunks_padded <= 16 * kThreads (fits_one_trip).  A workgroup of its
 // own on the critical path of every call: what it costs is the chain of barriers, LDS trips and instruction fetches, so
 // there is one trip to memory (every thread first loads all it needs: up to 16 consecutive entries of the flattened rank
-// table and its expert's column of chunk totals, of which 32 stay in registers), one pair of prefix sums, taken
+// table and its experts' columns of chunk totals, of which 32 stay in registers), one pair of prefix sums, taken
 // together, and two barriers; outputs go out from registers.  kOneChunk: `totals` ([R + E], LDS) holds the only
 // chunk's totals and nothing is loaded.  scratch: LDS of publish_scratch_ints.
 // From the ticket to the end it took 3.4 us at 16 chunks, 9 us at 64 chunks over 32 ranks, with LDS scans of five
 // barriers and 32 chunks at most; the whole launch went from 10.0 to 8.3 and from 14.8 to 11.5 us.
 // Chunks past the 32 in registers are read again for the expert bases, sixteen a trip: one at a time, each load behind the store
 // before it, an expanded layout took 41.7 us at 65536 tokens over 8 ranks, 13.8 at 16384 over 32, and takes 29.1 and 12.2.
+// Two experts a thread: the layout launch over 512 experts of 16 ranks took 11.8 us at 57 tokens, 13.3 at 8192 (expanded 16.6) and 18.0 at
+// 20000 (26.0) in the steps of publish_layout, and takes 7.0, 9.3 (10.8) and 11.5 (16.2).  A launch's kernel holds only its own way of
+// publishing: with the two-expert one beside it the launch took 0.2 to 0.4 us longer over 256 experts.
+inline bool fits_one_trip(int per_thread, int R, int E, int chunks_padded, int threads) {
+    return E <= per_thread * threads && R * chunks_padded <= 16 * threads;
+}
+
 inline __host__ __device__ int publish_scratch_ints(int R, int threads) { return R + 2 * (threads / kWaveSize); }
 
-template <int kThreads, bool kOneChunk>
+template <int kThreads, bool kOneChunk, int kPerThread>
 __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutTables& t, int num_chunks, bool expert_bases,
-                                           const int* totals, int* scratch) {
+                                           int* totals, int* scratch) {
     constexpr int kWavesHere = kThreads / kWaveSize;
-    constexpr int kMaxVecs = kOneChunk ? 1 : 4, kColumn = kOneChunk ? 1 : 32;
+    constexpr int kMaxVecs = kOneChunk ? 1 : 4, kColumn = kOneChunk ? 1 : 32 / kPerThread;
     int* rank_end = scratch;                             // [R] inclusive prefix sum over the ranks
     int* wave_sums = scratch + q.R;                      // [2][kWavesHere]
+    // kPerThread > 1: [E] what the mailbox gets, of which a thread writes the entries it has read the totals from
+    int* for_host = kOneChunk ? totals + q.R : scratch + publish_scratch_ints(q.R, kThreads);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const bool has_expert = tid < q.E;
+    const int first_expert = tid * kPerThread;
+    const bool has_expert = first_expert < q.E;
     const int status = status_for_host(q);
     const int flat = q.R * t.chunks_padded;              // a multiple of 4: four entries share a row
     const int vecs = kOneChunk ? 1 : (flat + 4 * kThreads - 1) / (4 * kThreads);
+    // The thread's experts of a chunk: columns the table pads with (experts_padded is a multiple of 32) come along and count nothing.
+    struct alignas(4 * kPerThread) Columns { int of[kPerThread]; };
     vec16 rv[kMaxVecs];
-    int v[kColumn];
-    int rows = 0, count = 0;
-    const int column = has_expert ? tid : 0;
-    auto load_sixteen = [&](int first, int* to) {
+    Columns v[kColumn];
+    int rows = 0, count[kPerThread] = {};
+    const int column = has_expert ? first_expert : 0;
+    auto load_sixteen = [&](int first, Columns* to) {
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
             // a row start common to the workgroup plus the thread's column: one address register serves all loads
             const int row_start = __builtin_amdgcn_readfirstlane(min(first + u, num_chunks - 1) * t.experts_padded);
-            to[u] = t.expert_counts[row_start + column];
+            to[u] = *reinterpret_cast<const Columns*>(t.expert_counts + row_start + column);
         }
     };
     if constexpr (kOneChunk) {
         rv[0] = vec16{tid < q.R ? uint32_t(totals[tid]) : 0u, 0, 0, 0};          // rows of four, three of them padding
-        v[0] = has_expert ? totals[q.R + tid] : 0;
+#pragma unroll
+        for (int j = 0; j < kPerThread; ++j) v[0].of[j] = count[j] = first_expert + j < q.E ? totals[q.R + first_expert + j] : 0;
         rows = int(rv[0].x);
-        count = v[0];
     } else {
 #pragma unroll
         for (int i = 0; i < kMaxVecs; ++i) {
@@ -330,47 +342,60 @@ __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutT
             const int begin = (tid * vecs + i) * 4;
             if (i < vecs && begin < flat) rv[i] = load16(t.rank_counts + begin);
         }
-        auto sum_sixteen = [&](int first, const int* of) {
+        auto sum_sixteen = [&](int first, const Columns* of) {
 #pragma unroll
-            for (int u = 0; u < 16; ++u) count += first + u < num_chunks ? of[u] : 0;
+            for (int u = 0; u < 16; ++u)
+#pragma unroll
+                for (int j = 0; j < kPerThread; ++j) count[j] += first + u < num_chunks ? of[u].of[j] : 0;
         };
         load_sixteen(0, v);
-        if (num_chunks > 16) load_sixteen(16, v + 16);
-        for (int c0 = 32; c0 < num_chunks; c0 += 16) {
-            int w[16];
+        if (kColumn > 16 && num_chunks > 16) load_sixteen(16, v + (kColumn - 16));
+        for (int c0 = kColumn; c0 < num_chunks; c0 += 16) {
+            Columns w[16];
             load_sixteen(c0, w);
             sum_sixteen(c0, w);
         }
         sum_sixteen(0, v);
-        if (num_chunks > 16) sum_sixteen(16, v + 16);
+        if (kColumn > 16 && num_chunks > 16) sum_sixteen(16, v + (kColumn - 16));
 #pragma unroll
         for (int i = 0; i < kMaxVecs; ++i) rows += int(rv[i].x) + int(rv[i].y) + int(rv[i].z) + int(rv[i].w);
     }
-    int aligned = 0;
-    if (has_expert) aligned = q.A == 1 ? count : int((unsigned(count) + unsigned(q.A) - 1u) / unsigned(q.A)) * q.A;
+    int aligned[kPerThread], all_aligned = 0;
+#pragma unroll
+    for (int j = 0; j < kPerThread; ++j) {
+        aligned[j] = 0;
+        if (first_expert + j < q.E) aligned[j] = q.A == 1 ? count[j] : int((unsigned(count[j]) + unsigned(q.A) - 1u) / unsigned(q.A)) * q.A;
+        all_aligned += aligned[j];
+    }
 
-    const int rows_incl = wave_inclusive_sum(rows), aligned_incl = wave_inclusive_sum(aligned);
+    const int rows_incl = wave_inclusive_sum(rows), aligned_incl = wave_inclusive_sum(all_aligned);
     if (lane == kWaveSize - 1) {
         wave_sums[wave] = rows_incl;
         wave_sums[kWavesHere + wave] = aligned_incl;
     }
     __syncthreads();
-    int run = rows_incl - rows, start = aligned_incl - aligned;
+    int run = rows_incl - rows, start = aligned_incl - all_aligned;
 #pragma unroll
     for (int w = 0; w < kWavesHere - 1; ++w) {
         run += w < wave ? wave_sums[w] : 0;
         start += w < wave ? wave_sums[kWavesHere + w] : 0;
     }
+    Columns base;                                        // the region of an expert starts at the aligned rows of those before it
+#pragma unroll
+    for (int j = 0, at = start; j < kPerThread; at += aligned[j], ++j) base.of[j] = at;
 
-    // experts: the region of an expert starts at the aligned rows of those before it
-    if (has_expert) {
-        if (q.host_counts != nullptr) store_system(q.host_counts + q.R + tid, -aligned - 1);
-        if (q.num_tokens_per_expert != nullptr) q.num_tokens_per_expert[tid] = count;
-        if (q.num_unaligned != nullptr) q.num_unaligned[tid] = count;
-        if (q.cumulative_stats != nullptr) q.cumulative_stats[tid] += count;
-        if (q.expert_start != nullptr) q.expert_start[tid] = start;
-        if (q.psum_expert != nullptr) q.psum_expert[tid] = q.do_expand ? start + count : start + aligned;
-        if (tid == q.E - 1 && q.totals_out != nullptr) q.totals_out[1] = start + aligned;
+#pragma unroll
+    for (int j = 0; j < kPerThread; ++j) {
+        const int e = first_expert + j;
+        if (e >= q.E) break;
+        if constexpr (kPerThread > 1) for_host[e] = aligned[j];
+        else if (q.host_counts != nullptr) store_system(q.host_counts + q.R + e, -aligned[j] - 1);
+        if (q.num_tokens_per_expert != nullptr) q.num_tokens_per_expert[e] = count[j];
+        if (q.num_unaligned != nullptr) q.num_unaligned[e] = count[j];
+        if (q.cumulative_stats != nullptr) q.cumulative_stats[e] += count[j];
+        if (q.expert_start != nullptr) q.expert_start[e] = base.of[j];
+        if (q.psum_expert != nullptr) q.psum_expert[e] = q.do_expand ? base.of[j] + count[j] : base.of[j] + aligned[j];
+        if (e == q.E - 1 && q.totals_out != nullptr) q.totals_out[1] = base.of[j] + aligned[j];
     }
     // ranks: the exclusive prefix over the flattened table is the first compact row of every (rank, chunk)
     const float rcp_row = 1.0f / float(t.chunks_padded);
@@ -385,6 +410,11 @@ __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutT
         if (begin + 4 == (r + 1) * t.chunks_padded) rank_end[r] = run;
     }
     __syncthreads();
+    // Neighbouring lanes store neighbouring words: every second word at a time the bus takes them one by one, which kept the host
+    // waiting 45 us longer over 512 experts.
+    if constexpr (kPerThread > 1)
+        if (q.host_counts != nullptr)
+            for (int e = tid; e < q.E; e += kThreads) store_system(q.host_counts + q.R + e, -for_host[e] - 1);
     for (int r = tid; r < q.R; r += kThreads) {
         const int end = rank_end[r], total = end - (r > 0 ? rank_end[r - 1] : 0);
         if (q.host_counts != nullptr) store_system(q.host_counts + r, -total - 1);
@@ -395,38 +425,30 @@ __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutT
     if (tid == 0 && q.host_counts != nullptr) store_system(q.host_counts + q.R + q.E, -status - 1);
 
     if (t.expert_bases != nullptr && expert_bases && has_expert) {
-        int at = start;
+        auto store_base = [&](int chunk, const Columns& counts) {
+            *reinterpret_cast<Columns*>(t.expert_bases + __builtin_amdgcn_readfirstlane(chunk * t.experts_padded) + first_expert) = base;
 #pragma unroll
-        for (int u = 0; u < kColumn; ++u) {
-            if (u < num_chunks) {
-                t.expert_bases[__builtin_amdgcn_readfirstlane(u * t.experts_padded) + tid] = at;
-                at += v[u];
-            }
-        }
+            for (int j = 0; j < kPerThread; ++j) base.of[j] += counts.of[j];
+        };
+#pragma unroll
+        for (int u = 0; u < kColumn; ++u)
+            if (u < num_chunks) store_base(u, v[u]);
         if constexpr (!kOneChunk) {
             for (int c0 = kColumn; c0 < num_chunks; c0 += 16) {
-                int w[16];
+                Columns w[16];
                 load_sixteen(c0, w);
 #pragma unroll
-                for (int u = 0; u < 16; ++u) {
-                    if (c0 + u < num_chunks) {
-                        t.expert_bases[__builtin_amdgcn_readfirstlane((c0 + u) * t.experts_padded) + tid] = at;
-                        at += w[u];
-                    }
-                }
+                for (int u = 0; u < 16; ++u)
+                    if (c0 + u < num_chunks) store_base(c0 + u, w[u]);
             }
         }
     }
 }
 
 // Everything at once, for a workgroup that publishes after all counting is over (the stand-alone layout kernel):
-// totals, public outputs, and - when the caller has room for them - the base tables.
+// totals, public outputs, and - when the caller has room for them - the base tables.  Any sizes.
 template <int kThreads>
 __device__ void publish_layout(const PublishParams& q, const LayoutTables& t, int num_chunks, bool expert_bases, int* lds) {
-    if (q.E <= kThreads && q.R * t.chunks_padded <= 16 * kThreads) {
-        publish_layout_in_one_trip<kThreads, false>(q, t, num_chunks, expert_bases, nullptr, lds);
-        return;
-    }
     const PublishLds s = carve_publish_lds(lds, q.R, q.E);
     const int status = status_for_host(q);
     sum_rank_rows<kThreads>(t, q.R, s.totals);
