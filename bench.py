@@ -710,8 +710,8 @@ def bench_low_latency(args, torch, rc, _abi, dev):
     d_bytes, c_bytes = ll.dispatch_bytes, ll.combine_bytes
     sweep = None
     if args.ll_batch_sweep:
-        # other batch sizes of the same shape: the single-kernel dispatch (one item per wavefront up to 128 tokens per
-        # rank here, several beyond) against the counting + move kernels, and the combine
+        # other batch sizes of the same shape: the dispatch as its size has it (the single kernel up to 2048 tokens here)
+        # against the counting + move kernels, and the combine
         sweep = {}
         for t in (64, 128, 192, 256, 384, 512):
             one, two = LowLatencyCalls(torch, rc, _abi, dev, t), LowLatencyCalls(torch, rc, _abi, dev, t, two_kernels=True)
