@@ -121,10 +121,14 @@ constexpr int kFusedTokens = 3072;      // the single-kernel path: a lane per 64
 
 // Loads one column tile (kPairs * 1024 channels) of token g: lane owns 16 consecutive channels per pair.  A pair past the end of
 // the row loads the row's last 32 bytes instead of being skipped (no branch around the load; what it brings is never stored).
-// Plain loads: a decode step has just written the tokens, and a streaming load of a line the memory-side cache holds unwritten
-// takes longer.  Dispatch and combine, streaming / plain, tokens just written by a copy behind 400 MB of other writes, us: 1024
-// tokens x 7168 FP8 20.8 / 20.1, 4096 tokens 50.3 / 48.1, 8192 x 2048 of 16 ranks 30.3 / 28.9; called over and over 21.8 / 18.9, 46.9 /
-// 43.8, 28.8 / 26.3; tokens left in HBM by then 21.1 / 23.8, 48.8 / 52.9, 30.3 / 31.3.
+// Plain loads, of tokens that stay on this rank only: a decode step has just written its tokens, and a streaming load of a line the
+// memory-side cache holds unwritten takes longer.  A line that is not there pushes another out, which has to be written to HBM first
+// where the cache is full of what others have written, so nothing is loaded that is not stored.  Dispatch, us, tokens in the cache
+// (called over and over) / just written behind 400 MB of other writes / in HBM / in HBM behind 1 GB of other writes:
+//   plain          1024 x 7168 FP8 9.8 / 11.2 / 10.9 / 12.3;   2048 x 7168 BF16 17.9 / 19.9 / 20.8 / 22.3;   4096 x 7168 (two kernels) 21.4 / 25.3 /
+//                  24.6 / 30.1
+//   streaming      10.4 / 12.1 / 11.2 / 11.9;   20.1 / 22.1 / 21.0 / 21.6;   26.1 / 28.3 / 25.7 / 26.3
+//   plain, also the tokens that stay nowhere here   10.6 / 11.9 / 11.4 / 14.4;   20.2 / 22.0 / 23.6 / 27.8
 template <int kPairs>
 __device__ __forceinline__ void ll_load_tile(const uint8_t* x, int hidden, int64_t g, int tile, int lane,
                                              vec16 (&in)[kPairs][2]) {
@@ -277,6 +281,20 @@ __global__ __launch_bounds__(kBlockThreads) void ll_move_kernel(const LLDispatch
     ll_store_tile<kPairs, kFp8>(p, g, tile, lane, t, le, slot, in);
 }
 
+// The same for a token that may not be wanted: read through a descriptor of the row, which has no bytes then - the loads bring zeros
+// and touch no memory.
+template <int kPairs>
+__device__ __forceinline__ void ll_load_tile_if(bool wanted, const uint8_t* x, int hidden, int64_t g, int tile, int lane,
+                                                vec16 (&in)[kPairs][2]) {
+    const auto row = buffer_of(x + g * (int64_t(hidden) * 2), wanted ? hidden * 2 : 0);
+#pragma unroll
+    for (int q = 0; q < kPairs; ++q) {
+        const int at = min((tile * kPairs + q) * 1024 + lane * 16, hidden - 16);
+        in[q][0] = buffer_load16_as<false>(row, at * 2);
+        in[q][1] = buffer_load16_as<false>(row, at * 2 + 16);
+    }
+}
+
 // Single-kernel path for decode-sized calls.  Every workgroup first rebuilds the complete routing picture in
 // LDS - one bit per (local expert, token), set from its own pass over all topk_idx rows (tens of KB, L2
 // resident) - so slots are prefix popcounts and no workgroup waits for another: no second launch, no ticket,
@@ -284,10 +302,10 @@ __global__ __launch_bounds__(kBlockThreads) void ll_move_kernel(const LLDispatch
 // workgroups move one (token, column tile) each.
 //
 // The kernel is bound by the chain of dependent phases of one wavefront, not by memory bandwidth: the routing pass alone
-// costs every workgroup a dozen instructions per index entry.  So the index loads are the first thing on the memory
-// pipeline (the pass can start as soon as they are back), the payload loads queue up behind them and land while the pass
-// runs, and the pass itself is kept short: one token id per pair of entries, unpredicated 32-bit LDS atomics, range and
-// duplicate checks left to the wavefront that later moves the token.
+// costs every workgroup a dozen instructions per index entry.  So the token's own selections and the index loads are the
+// first things on the memory pipeline (the pass can start as soon as they are back), the payload is asked for when the
+// selections show a local expert and lands while the pass runs, and the pass itself is kept short: one token id per pair of
+// entries, unpredicated 32-bit LDS atomics, range and duplicate checks left to the wavefront that later moves the token.
 template <int kPairs, bool kFp8, int kFusedThreads>
 __global__ __launch_bounds__(kFusedThreads) void ll_fused_kernel(const LLDispatchParams p, const int tiles) {
     constexpr int kFusedWaves = kFusedThreads / kWaveSize;
@@ -316,22 +334,24 @@ __global__ __launch_bounds__(kFusedThreads) void ll_fused_kernel(const LLDispatc
     // Everything up to the pass is straight-line code without a branch around any load: where control flow merges the
     // compiler can no longer tell how many loads are younger than the one it waits for and waits for all of them - the
     // pass would sit there until the payload had arrived.  So addresses are clamped instead of predicated (the launcher
-    // sends only calls with an aligned table of at least two entries here), and wavefronts without a work item load
-    // the tile of token 0 and drop it.
+    // sends only calls with an aligned table of at least two entries here), and what is not wanted is loaded through a
+    // descriptor without bytes.
     const int total_entries = total_tokens * p.K;
     const int pairs_total = total_entries / 2;
     const vec16* idx2 = reinterpret_cast<const vec16*>(p.topk_idx);
     constexpr int kBatch = 8;
     for (int i = tid; i < p.E_l * words; i += kFusedThreads) bits[i] = 0ull;
     __syncthreads();            // here, where no wavefront is held up by the memory pipeline yet: they arrive together
+    // this token's own selections, in front of everything: the payload waits for them alone
+    const int64_t own_loaded = p.topk_idx[g * p.K + min(lane, p.K - 1)];
     vec16 v[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) v[u] = idx2[min(tid + u * kFusedThreads, pairs_total - 1)];
-    // this token's own selections: behind the routing pass they would be one more trip to the L2 on the critical path
-    const int64_t own_loaded = p.topk_idx[g * p.K + min(lane, p.K - 1)];
-    // the payload tile: queued behind the index loads, in flight while the routing pass runs
+    __builtin_amdgcn_sched_barrier(0);
+    // the payload tile of a token with a local expert: in flight while the routing pass runs
+    const bool stays = lane < p.K && uint64_t(own_loaded) - uint64_t(p.expert_begin) < uint64_t(p.E_l);
     vec16 in[kPairs][2];
-    ll_load_tile<kPairs>(p.x, p.H, g, tile, lane, in);
+    ll_load_tile_if<kPairs>(live && __ballot(stays) != 0ull, p.x, p.H, g, tile, lane, in);
     __builtin_amdgcn_sched_barrier(0);
 
     // An entry sets a bit iff it names a local expert: a negative or oversized id has a non-zero upper half or a lower

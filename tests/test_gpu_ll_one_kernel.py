@@ -45,3 +45,40 @@ def test_single_kernel_lines(R, T, H, E, K, payload):
         assert_equal(got[e, :n], px[e, :n], f"packed_recv_x[{e}]")
         if fp8:
             assert_equal(recv[1][e, :n], oracle.pack_ue8m0(ps[e, :n]) if ue8m0 else ps[e, :n], f"scales[{e}]")
+
+
+@pytest.mark.parametrize("H,payload", [(4112, "bf16"), (4608, "ue8m0")])
+@pytest.mark.parametrize("which", ["none", "last", "every_third", "all"])
+def test_single_kernel_reads_the_tokens_that_stay(which, H, payload):
+    """Payloads of tokens without a local expert are not read: destinations no token, one, some and every token goes to, the others' rows
+    NaN.  The combine goes through the rows the dispatch recorded."""
+    import deep_ep
+    R, T, E, K, M, dst = 3, 37, 12, 3, 40, 1
+    x, idx, w = rc.c5_sources(seed=29, R=R, T=T, H=H, E=E, K=K)
+    E_l = E // R
+    token = torch.arange(R * T).view(R, T, 1)
+    stays = {"none": token < 0, "last": token == R * T - 1, "every_third": token % 3 == 1, "all": token >= 0}[which]
+    others = torch.tensor([0, 1, 2, 3, 8, 9, 10, 11])
+    away = others[torch.rand((R, T, 8), generator=torch.Generator().manual_seed(2)).argsort(dim=2)[..., :K]]
+    here = torch.stack([away[..., 0], dst * E_l + token[..., 0] % E_l, away[..., 2]], dim=2)
+    idx = torch.where(stays, here, away)
+    x = x.masked_fill(~stays, float("nan"))
+    fp8 = payload != "bf16"
+    buf = deep_ep.Buffer(deep_ep.LogicalGroup(dst, R), low_latency_mode=True)
+    recv, count, handle, _, _ = buf.low_latency_dispatch(x.cuda(), idx.cuda(), M, E, use_fp8=fp8, round_scale=fp8, use_ue8m0=fp8)
+    px, ps, cnt, info, rng = oracle.ll_dispatch(list(x), list(idx), M, E, R, dst, fp8, round_scale=fp8)
+    assert int(cnt.sum()) == int(stays.sum())
+    assert_equal(count, cnt, "packed_recv_count")
+    assert_equal(handle[1], rng, "packed_recv_layout_range")
+    got = recv[0] if fp8 else recv
+    y = torch.zeros((E_l, R * M, H), dtype=torch.bfloat16)
+    for e in range(E_l):
+        n = int(cnt[e])
+        assert_equal(handle[0][e, :n], info[e, :n], f"src_info[{e}]")
+        assert_equal(got[e, :n], px[e, :n], f"packed_recv_x[{e}]")
+        if fp8:
+            assert_equal(recv[1][e, :n], oracle.pack_ue8m0(ps[e, :n]), f"scales[{e}]")
+        y[e, :n] = torch.randn((n, H), generator=torch.Generator().manual_seed(e)).to(torch.bfloat16)
+    out, _, _ = buf.low_latency_combine(y.cuda(), idx.cuda(), w.cuda(), handle)
+    for s in range(R):
+        assert_equal(out[s] + 0.0, oracle.ll_combine(y, idx[s], w[s], info, rng, s, E, R, dst) + 0.0, f"combined from source {s}")
