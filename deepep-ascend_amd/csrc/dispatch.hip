@@ -1140,6 +1140,28 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))
     dispatch_cast<kPairs, true, kBlocked>(p);
 }
 
+// Loads the scales of a block (kernels.h) and leaves them in LDS as [row][G + 1].  kBatch loads of a thread are in flight at once, and
+// `meanwhile` runs behind the first of them: a workgroup of the pad kernel has one block, and what it costs is its trips to memory.  With one
+// load at a time in front of its LDS store the pad kernel took 17.1 us at 2048 x 12288 top-4 of 64 experts and 51 at 4096 x 16384 top-8 of
+// 256 (11.2 and 41.4 with scales stored into their columns by the move); it takes 11.9 and 42.
+template <int kBatch, typename Meanwhile>
+__device__ __forceinline__ void load_block(const PadParams& p, uint32_t* scales, int rows, int64_t r0, Meanwhile&& meanwhile) {
+    const int places = rows * p.num_sf_packs;
+    const float rcp_G = 1.0f / float(p.num_sf_packs);
+    for (int first = threadIdx.x; first - int(threadIdx.x) < places; first += kBatch * kThreads) {
+        uint32_t v[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+            v[u] = p.recv_sf[place_in_block(min(first + u * kThreads, places - 1), kScaleBlockRows, rows, r0, p.rsf_hs)];
+        if (first < kThreads) meanwhile();
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            const int i = first + u * kThreads;
+            if (i < places) scales[i + small_div(i, rcp_G)] = v[u];
+        }
+    }
+}
+
 // ---- zero the alignment padding rows of the expanded layout, and put scales that came in blocks into their columns ----
 // Workgroups [0, scale_blocks) turn a block each, those behind them zero rows.
 __global__ __launch_bounds__(kThreads) void zero_padding_kernel(const PadParams p, const int scale_blocks) {
@@ -1152,19 +1174,18 @@ __global__ __launch_bounds__(kThreads) void zero_padding_kernel(const PadParams 
         const int64_t total = int64_t(p.psum_expert[p.E - 1]) - last + (int64_t(last) + p.A - 1) / p.A * p.A;
         if (r0 >= total) return;
         const int rows = int(min(p.expanded_capacity - r0, int64_t(kScaleBlockRows)));
-        const float rcp_G = 1.0f / float(G);
         if (tid == 0) padding = 0ull;
-        for (int i = tid; i < rows * G; i += kThreads) {
-            const int r = small_div(i, rcp_G);
-            scales[r * (G + 1) + (i - r * G)] = p.recv_sf[place_in_block(i, kScaleBlockRows, rows, r0, p.rsf_hs)];
-        }
         __syncthreads();
-        for (int e = tid; e < p.E; e += kThreads) {
-            const int cnt = p.num_unaligned[e];
-            const int64_t from = max(int64_t(p.psum_expert[e]) - r0, int64_t(0));
-            const int64_t to = min(int64_t(p.psum_expert[e]) + ((cnt + p.A - 1) / p.A * p.A - cnt) - r0, int64_t(kScaleBlockRows));
-            if (from < to) atomicOr(&padding, (to == 64 ? ~0ull : (1ull << to) - 1ull) & ~((1ull << from) - 1ull));
-        }
+        const auto note_padding = [&] {
+            for (int e = tid; e < p.E; e += kThreads) {
+                const int cnt = p.num_unaligned[e];
+                const int64_t from = max(int64_t(p.psum_expert[e]) - r0, int64_t(0));
+                const int64_t to = min(int64_t(p.psum_expert[e]) + ((cnt + p.A - 1) / p.A * p.A - cnt) - r0, int64_t(kScaleBlockRows));
+                if (from < to) atomicOr(&padding, (to == 64 ? ~0ull : (1ull << to) - 1ull) & ~((1ull << from) - 1ull));
+            }
+        };
+        if (rows * G <= 4 * kThreads) load_block<4>(p, scales, rows, r0, note_padding);
+        else load_block<8>(p, scales, rows, r0, note_padding);
         __syncthreads();
         const unsigned long long none = padding | (total - r0 < kScaleBlockRows ? ~((1ull << (total - r0)) - 1ull) : 0ull);
         for (int i = tid; i < rows * G; i += kThreads) {
@@ -1598,18 +1619,21 @@ hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream) {
     }
 }
 
-// From 128 K scales on.  Move + pad kernel in us, scales stored into their columns / in blocks, fused cast and pass-through of the
-// same rows, top-8 of 256 experts, alignment 128: 8192 x 7168 134.2 + 19.7 / 117.4 + 22.1 and 106.8 + 19.5 / 100.0 + 21.3; 2048 x
-// 7168 37.1 + 20.0 / 35.5 + 18.4; 512 x 7168 11.9 + 31.9 / 11.4 + 28.4 (a padding row's zeroes are single dwords too); top-6 of 64
-// experts, 8192 x 1024 21.8 + 5.0 / 19.7 + 4.5, 1024 x 2048 in one launch (98 K scales) 15.7 + 4.4 / 15.6 + 4.9; 64 x 2048 6.7 + 6.0 /
-// 7.2 + 6.1.
+// From 128 K scales on, where there are rows enough: padding rows count double, as their zeroes are single dwords too, against the two
+// trips to memory a block costs.  Move + pad kernel in us, scales stored into their columns / in blocks, fused cast, top-8 of 256 experts,
+// alignment 128: 8192 x 7168 134.0 + 20.0 / 115.5 + 23.4; 512 x 7168 19.1 + 32.0 / 18.1 + 28.0; 4096 x 16384 150.4 + 41.4 / 138 + 42;
+// 2048 x 12288 top-4 of 64 40.3 + 11.2 / 37.4 + 11.8 (16.3 K rows so counted); top-6 of 64, 8192 x 1024 30.2 + 5.1 / 29.5 + 5.1.  Below the
+// line of rows, layout, move and pad together, of 32 experts: 1024 x 8192 top-4, alignment 16 (4.6 K rows) 24.3 / 26.6; 2000 x 16384 top-4,
+// alignment 64 (10 K) 56.0 / 59.5; 3000 x 12288 top-4, alignment 16 (12.5 K) 69.0 / 70.6.  Above it: 700 x 7168 top-8 of 128, alignment 128
+// (21.9 K) 36.7 / 34.1; 3000 x 7168 top-6 of 64, alignment 16 (19 K) 50.1 / 49.4.
 bool scales_in_blocks(const MoveParams& m, int alignment) {
-    constexpr int64_t kFromScales = int64_t(1) << 17;
+    constexpr int64_t kFromScales = int64_t(1) << 17, kFromRows = 14000;
+    const int64_t selections = int64_t(m.T) * m.K;
     const bool tile_known = m.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? m.cast_pairs >= 0 && m.cast_pairs <= 2
                                                                       : m.copy_vecs >= 0 && m.copy_vecs <= 4 && m.copy_vecs != 3;
     return m.do_expand && alignment > 1 && m.payload != DEEP_EP_HIP_PAYLOAD_BF16 && m.recv_sf != nullptr && m.rsf_ts == 1 &&
            m.rsf_hs >= m.expanded_capacity && m.num_sf_packs >= 2 && m.num_sf_packs <= kMaxBlockedScales && tile_known &&
-           int64_t(m.T) * m.K * m.num_sf_packs >= kFromScales;
+           selections * m.num_sf_packs >= kFromScales && selections + int64_t(m.E) * (alignment - 1) >= kFromRows;
 }
 
 hipError_t launch_zero_padding(const PadParams& p, hipStream_t stream) {

@@ -1,5 +1,5 @@
 """Column-major scales of zero-padded expanded dispatches (stored in blocks of 64 rows by the move kernel, put into their columns by the
-pad kernel from 131072 scales on) against the oracle: last blocks that are not full, odd and many scales a row, both payloads,
+pad kernel from 131072 scales on, with rows enough) against the oracle: last blocks that are not full, odd and many scales a row, both payloads,
 exact, worst-case and cached outputs."""
 import pytest
 import torch
@@ -18,6 +18,10 @@ pytestmark = pytest.mark.gpu
     (300, 16384, 16, 2, 4, 2),         # as many scales a row as a block may have
     (300, 16512, 16, 2, 4, 2),         # one more: stored into their columns at once
     (2048, 1024, 8, 1, 7, 128),        # short of the line
+    (1300, 2048, 32, 8, 8, 128),       # padding rows fill whole blocks, past the line of rows (14000, padding counted double)
+    (300, 16384, 128, 2, 4, 128),      # as many scales a row as a block may have, past that line: eight trips a thread, blocks of padding alone
+    (2300, 2944, 8, 4, 6, 64),         # 23 scales: the last trip of a block is not full
+    (1755, 2048, 8, 4, 8, 2), (1749, 2048, 8, 4, 8, 2),       # both sides of that line
 ], ids=lambda v: str(v))
 @pytest.mark.parametrize("cast", [True, False])
 def test_blocked_scales_match_the_oracle(T, H, E, R, K, alignment, cast):
