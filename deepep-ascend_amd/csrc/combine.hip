@@ -301,33 +301,28 @@ int workgroups_per_cu(const CombineParams& p) {
     return rows >= 5.8 ? 5 : 6;
 }
 
-// Column tile per wavefront: 1 KB of a BF16 row (512 channels, 41 registers, eight wavefronts per SIMD), or 2 KB.  us with 1 / 2 KB:
-// - many rows a token: 1 KB, at the residency above.  8 ranks top-8, compact: 8192 x 7168 120.7 / 125.3, 2048 x 4096 22.0 / 22.6, 1365 x
-//   2048 11.0 / 11.7, 512 x 1024 7.4 / 8.0; expanded 512 x 7168 16.8 / 18.2, 128 x 2048 8.4 / 9.5.
-// - few rows a token (top-2, or two ranks): 2 KB from one and a half wavefronts per place on (two and a half for rows past 8 KB).
-//   Compact, 2 ranks: 16384 x 7168 107.3 / 98.5, 2048 x 4096 13.2 / 12.5 (8 ranks 13.7 / 13.3), 2048 x 2888 11.6 / 11.1, 2048 x 2048
-//   9.0 / 9.5; 8 ranks 1365 x 7168 15.1 / 15.5.  4 of 4 ranks (2.7 rows) 16384 x 7168 137 / 145.  Expanded rows, whose routing is one trip longer, from half a wavefront per place on: top-2 16384 x 7168
-//   146.5 / 128.5, 1237 x 2048 9.2 / 8.5, 512 x 7168 10.3 / 9.9, 512 x 2048 7.3 / 7.5.
-// - expanded rows of up to 6 KB that fill half of the places to all of them: 2 KB.  Top-4: 1237 x 2048 11.0 / 10.5, 2048 x 2048 13.6 / 12.9,
-//   4096 x 1024 13.5 / 13.0; top-8 the same within 0.2.
-// - compact rows of up to 6 KB and four rows a token and more that fill seven eighths of the places: 2 KB.  1237 x 2888, top-9 of 6 ranks
-//   13.4 / 12.9, top-8 of 8 13.7 / 13.2; 2048 x 2048 13.6 / 13.4 and 13.9 / 13.9; 4 of 4 ranks 1237 x 3072 9.6 / 10.2.
-// - V1 rows of 2 KB that fill half of the places: 2 KB.  2048 x 1024, top-9 of 6 ranks 10.5 / 10.1, top-8 of 8 10.7 / 10.4; 2048 x 2048
-//   14.5 / 15.1 and 14.9 / 15.6.
+// Column tile per wavefront: 1 KB of a BF16 row (512 channels, 41 registers, eight wavefronts per SIMD), or 2 KB, which repeats the routing
+// work half as often and has half the wavefronts to hide its loads with.  2 KB for few rows a token (top-2, or two ranks), where the routing is
+// as much as the rows, from three quarters of the places on; V1 rows, whose routing is shorter, from a full round on.  Change by 2 KB tiles in %
+// at 0.55 / 0.8 / 1.0 / 1.1 / 1.4 / 4 times as many wavefronts of 1 KB as places (730 shapes, rows of 2 to 14 KB):
+//   compact, top-2 of 2 ranks, 8 KB rows    +1.2 / -2.2 / -4.0 / -8.0 / -7.6 / -8.5;   top-2 of 8 ranks +0.6 / +0.5 / -1.5 / -5.8 / -8.2 / -4.4
+//   expanded, top-2                          +0.5 / -3.0 / -6.1 / -7.9 / -1.3 / -2.7
+//   V1, top-2 of 8 ranks, 4 KB rows          +2.4 / +3.2 / +1.0 / -5.8 / -5.1
+//   more rows a token, up to one round: compact top-8 of 8 ranks -3 to +5, expanded top-8 -2 to +9, V1 top-8 -1 to +9
+// A last tile that is half idle costs what the others gain: rows of 3 KB, expanded, top-2, 0.0 / +3.0 / +12.3 / +4.6 / +1.6 / +5.4; compact
+// +0.6 / -0.5 / +2.0 / -7.1 / -8.1 / -2.2.
 bool takes_two_kb_tiles(const CombineParams& p) {
     const int kb = (p.H * 2 + 1023) / 1024;
-    if (kb < 2) return false;
+    if (kb < 2 || rows_per_token(p) >= 2.3) return false;
     const int64_t places = int64_t(compute_units()) * 8 * kWavesPerBlock, waves = int64_t(p.T) * kb;
-    const bool expanded = p.do_expand && !p.rank_mode, fits = kb <= 6 && waves <= places;
-    const double rows = rows_per_token(p);
-    if (rows < 2.3 && 2 * waves >= (expanded ? 1 : kb <= 8 ? 3 : 5) * places) return true;
-    if (p.rank_mode) return kb == 2 && fits && 2 * waves >= places;
-    return fits && (expanded ? 2 * waves > places : rows >= 4.0 && 8 * waves > 7 * places);
+    if (p.rank_mode) return waves > places;
+    const bool half_idle = kb % 2 == 1 && kb < 8;
+    return 4 * waves >= 3 * places && (!half_idle || (!p.do_expand && waves > places));
 }
 
 // The rows a combine adds up have just been written, by the experts or by the dispatch itself: up to 110 MB of them are read with plain
 // loads, which find them in the memory-side cache.  Dispatch and combine of BF16 rows, us, streaming / plain rows (the dispatch stores
-// accordingly, keeps_rows): 4096 x 2048 top-6 of 8 ranks, forward and backward (74 MB) 91.2 / 84.9, 16384 x 2048 of 2 ranks (100 MB) 77.5
+// accordingly, cached_side): 4096 x 2048 top-6 of 8 ranks, forward and backward (74 MB) 91.2 / 84.9, 16384 x 2048 of 2 ranks (100 MB) 77.5
 // / 76.0; combine of rows an expert has just written, with an FP8 dispatch in front, 1024 x 7168 (78 MB) 42.3 / 36.7, 700 x 4096 (30 MB) 27.4 /
 // 26.6; rows that are in HBM while the cache is full of what others have written are the other way round (41.0 / 53.5).  More rows than
 // the cache holds beside other traffic are read past it: 2100 x 7168 (160 MB) 67.5 / 74.0, 4096 x 7168 (311 MB) 134 / 170.

@@ -12,6 +12,10 @@ pytestmark = pytest.mark.gpu
     ("compact", 1195, 3064, 72, 6, 9), ("compact", 1194, 3064, 72, 6, 9),          # many: past seven eighths of 8192
     ("expanded", 512, 4096, 8, 2, 2), ("expanded", 511, 4096, 8, 2, 2),            # 4096
     ("expanded", 1025, 2040, 64, 4, 4), ("expanded", 1024, 2040, 64, 4, 4), ("expanded", 2049, 2048, 64, 4, 4),
+    ("compact", 768, 4096, 8, 2, 2), ("compact", 767, 4096, 8, 2, 2),              # few: three quarters of 8192
+    ("expanded", 768, 4096, 8, 2, 2), ("expanded", 767, 4096, 8, 2, 2),
+    ("compact", 2731, 1536, 8, 2, 2), ("compact", 2730, 1536, 8, 2, 2), ("expanded", 2731, 1536, 8, 2, 2),       # 3 KB rows: a round
+    ("v1", 1025, 4096, 64, 8, 2), ("v1", 1024, 4096, 64, 8, 2),                    # a round
     ("v1", 2048, 1024, 64, 8, 8), ("v1", 2047, 1024, 64, 8, 8), ("v1", 1, 520, 64, 8, 8),
 ])
 def test_the_tile_does_not_show(layout, T, H, E, R, K):
