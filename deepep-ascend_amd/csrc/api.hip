@@ -346,8 +346,10 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
         m.gates_finished = reinterpret_cast<uint32_t*>(ws + w.gates_finished);
         if (plan.fused) fill_fused(m, lay, plan, ws, w);
         m.sf_blocked = a->do_zero_padding && scales_in_blocks(m, a->expert_alignment) ? 1 : 0;
-
-        m.zeroed_rows = a->do_zero_padding ? int(std::min<int64_t>(int64_t(E) * (a->expert_alignment - 1) / 2, INT32_MAX)) : 0;
+        if (a->do_zero_padding) {
+            const int64_t selections = int64_t(T) * K, regions = std::min<int64_t>(E, selections) * a->expert_alignment;
+            m.zeroed_rows = int(std::min<int64_t>(std::max(int64_t(E) * (a->expert_alignment - 1) / 2, regions - selections), INT32_MAX));
+        }
 
         hipError_t err = launch_dispatch_move(m, stream);
         if (err != hipSuccess) return hip_fail(err, "dispatch move launch");

@@ -1477,7 +1477,10 @@ void plan_cache_warming(MoveParams& p) {
 }
 
 // Which side of a copy goes through the memory-side cache (256 MB).
-// - BF16, up to 110 MB of rows: the rows, which whoever is next then finds there; the combine reads as many with plain loads.
+// - BF16, up to 110 MB of rows and 140 MB with the padding rows zeroed behind them: the rows, which whoever is next then finds there.
+//   Dispatch and combine, us, neither / rows, input just written: 277 x 6072 over 8 ranks (18 MB) 24.0 / 22.0, 1024 x 7168 (77 MB) 54.3 / 40.7,
+//   4096 x 2048 top-6 (74 MB) 55.7 / 44.1; with a pass over the rows in between that writes as many 30.9 / 31.6, 66.1 / 65.3, 67.7 / 66.4.  With more
+//   padding the rows leave the cache again before they are read: 300 x 7168 over 256 experts aligned to 128 (470 MB) 104.2 / 113.4.
 // - BF16, more: the input, which the layer in front has just written; so many rows would drive it and each other out.  Dispatch and
 //   combine, us, neither / input: 2600 x 7168 over 8 ranks (198 MB) 103.4 / 96.5, 3400 x 7168 (258 MB) 123.7 / 116.5, 8192 x 7168 (622 MB) 261.7 /
 //   261.5, V1 4096 x 7168 150.2 / 141.8, expanded 4096 x 4096 top-8 143.3 / 134.8; with the input just written behind 400 MB of other writes 103.7 /
@@ -1485,13 +1488,13 @@ void plan_cache_warming(MoveParams& p) {
 //   131.3, 265.4 / 275.7, 153.2 / 159.4, 146.1 / 150.6.
 // - FP8: neither.  Cast, dispatch and combine, neither / input / rows: 1024 x 7168 (39 MB) 43.2 / 44.3 / 43.4, 2100 x 7168 (80 MB) 71.0 / 71.4 /
 //   69.1, 4096 x 7168 (156 MB) 130.1 / 127.4 / 125.4 with three inputs in turn, 126.9 / - / 129.4 with more.
-// - BF16, the input larger than that cache or followed by 150 MB and more of zeroed rows (half an alignment for each expert): neither.
+// - BF16, the input larger than that cache or followed by 150 MB and more of zeroed rows: neither.
 //   Input called over and over, 20000 x 7168 (287 MB) 597.7 / 603.0; expanded over 256 experts aligned to 128 rows 4883 x 6728 (220 MB of zeros)
 //   309.7 / 313.2, 10714 x 6896 (225 MB) 601.2 / 611.5; over 128 (113 MB) it is 567.3 / 565.9 and, input just written, 580.1 / 552.4.
 static int cached_side(const MoveParams& p) {
     if (p.payload != DEEP_EP_HIP_PAYLOAD_BF16) return kNeither;
-    if (row_bytes_out(p) <= 110e6) return kRows;
     const double zeroed = p.zeroed_rows * double(p.row_bytes);
+    if (row_bytes_out(p) <= 110e6 && row_bytes_out(p) + zeroed <= 140e6) return kRows;
     return double(p.T) * p.row_bytes <= 256e6 && zeroed < 150e6 ? kInput : kNeither;
 }
 

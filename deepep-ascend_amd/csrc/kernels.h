@@ -155,7 +155,8 @@ struct MoveParams {
     int row_bytes;       // input row bytes
     int tiles;           // column tiles per token
     int sf_blocked;      // recv_sf is column-major and the pad kernel follows: scales go out in blocks (below)
-    int zeroed_rows;     // rows the pad kernel behind this one zeroes, as expected: half an alignment for each expert
+    int zeroed_rows;     // rows the pad kernel behind this one zeroes, as expected: half an alignment for each expert, or what is
+                         // left of one alignment for each where an expert has fewer rows than that
     int row_by_row;      // a wavefront waits for the stores of a row before it starts the next (set by the launcher)
     unsigned warm_lds_offset;   // single-launch cast: byte offset (in the dynamic LDS) of the 4 KB landing area of the
                                 // cache-warming loads, 0 = none
