@@ -1622,21 +1622,21 @@ hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream) {
     }
 }
 
-// From 128 K scales on, where there are rows enough: padding rows count double, as their zeroes are single dwords too, against the two
-// trips to memory a block costs.  Move + pad kernel in us, scales stored into their columns / in blocks, fused cast, top-8 of 256 experts,
-// alignment 128: 8192 x 7168 134.0 + 20.0 / 115.5 + 23.4; 512 x 7168 19.1 + 32.0 / 18.1 + 28.0; 4096 x 16384 150.4 + 41.4 / 138 + 42;
-// 2048 x 12288 top-4 of 64 40.3 + 11.2 / 37.4 + 11.8 (16.3 K rows so counted); top-6 of 64, 8192 x 1024 30.2 + 5.1 / 29.5 + 5.1.  Below the
-// line of rows, layout, move and pad together, of 32 experts: 1024 x 8192 top-4, alignment 16 (4.6 K rows) 24.3 / 26.6; 2000 x 16384 top-4,
-// alignment 64 (10 K) 56.0 / 59.5; 3000 x 12288 top-4, alignment 16 (12.5 K) 69.0 / 70.6.  Above it: 700 x 7168 top-8 of 128, alignment 128
-// (21.9 K) 36.7 / 34.1; 3000 x 7168 top-6 of 64, alignment 16 (19 K) 50.1 / 49.4.
+// From 850 K scales and 14000 rows on, padding rows, whose zeroes are single dwords too, counted double: what is saved is a partial line for
+// each of them, against the two trips to memory a block costs.  Layout, move and pad kernel in us, scales stored into their columns / in
+// blocks, fused cast, 8 ranks, top-k of experts, alignment: 8192 x 7168 8 of 256, 128 (5.5 M scales) 168.2 / 151.9; 2048 x 12288 4 of 64, 128
+// (1.6 M) 55.1 / 50.7; 512 x 7168 8 of 256, 128 (2.0 M) 67.9 / 61.7; 700 x 7168 8 of 128, 128 (1.2 M) 36.7 / 34.2; 3000 x 7168 6 of 64, 16 (1.1 M)
+// 50.1 / 49.4.  Short of scales: 1640 x 6272 9 of 32, 16 (0.75 M) 40.4 / 42.9; 2568 x 3968 8 of 64, 64 (0.76 M), move and pad 29.9 / 31.2; 4096 x
+// 4096 4 of 64, 64 (0.65 M) 38.0 / 38.2.  Short of rows: 3000 x 12288 4 of 32, 16 (12.5 K) 69.0 / 70.6; 4096 x 16384 2 of 32, 128 (12.3 K) 81.9 /
+// 82.2, and 79.9 / 83.3 with the input just written; 2000 x 16384 4 of 32, 64 (10 K) 56.0 / 59.5.
 bool scales_in_blocks(const MoveParams& m, int alignment) {
-    constexpr int64_t kFromScales = int64_t(1) << 17, kFromRows = 14000;
-    const int64_t selections = int64_t(m.T) * m.K;
+    constexpr int64_t kFromScales = 850000, kFromRows = 14000;
+    const int64_t rows = int64_t(m.T) * m.K + int64_t(m.E) * (alignment - 1);
     const bool tile_known = m.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? m.cast_pairs >= 0 && m.cast_pairs <= 2
                                                                       : m.copy_vecs >= 0 && m.copy_vecs <= 4 && m.copy_vecs != 3;
     return m.do_expand && alignment > 1 && m.payload != DEEP_EP_HIP_PAYLOAD_BF16 && m.recv_sf != nullptr && m.rsf_ts == 1 &&
            m.rsf_hs >= m.expanded_capacity && m.num_sf_packs >= 2 && m.num_sf_packs <= kMaxBlockedScales && tile_known &&
-           selections * m.num_sf_packs >= kFromScales && selections + int64_t(m.E) * (alignment - 1) >= kFromRows;
+           rows * m.num_sf_packs >= kFromScales && rows >= kFromRows;
 }
 
 hipError_t launch_zero_padding(const PadParams& p, hipStream_t stream) {

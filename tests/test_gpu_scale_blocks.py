@@ -1,5 +1,5 @@
 """Column-major scales of zero-padded expanded dispatches (stored in blocks of 64 rows by the move kernel, put into their columns by the
-pad kernel from 131072 scales on, with rows enough) against the oracle: last blocks that are not full, odd and many scales a row, both payloads,
+pad kernel, in large calls) against the oracle: last blocks that are not full, odd and many scales a row, both payloads,
 exact, worst-case and cached outputs."""
 import pytest
 import torch
@@ -12,16 +12,18 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,H,E,R,K,alignment", [
-    (2050, 1024, 8, 2, 8, 2),          # just past the line; two rows a token and expert: few padding rows
+    (2050, 1024, 8, 2, 8, 2),          # two rows a token and expert: few padding rows
     (2048, 1152, 12, 4, 8, 6),         # odd number of scales, regions of 6: blocks start inside padding
     (1100, 2048, 32, 8, 8, 128),       # padding rows fill whole blocks
     (300, 16384, 16, 2, 4, 2),         # as many scales a row as a block may have
     (300, 16512, 16, 2, 4, 2),         # one more: stored into their columns at once
-    (2048, 1024, 8, 1, 7, 128),        # short of the line
-    (1300, 2048, 32, 8, 8, 128),       # padding rows fill whole blocks, past the line of rows (14000, padding counted double)
-    (300, 16384, 128, 2, 4, 128),      # as many scales a row as a block may have, past that line: eight trips a thread, blocks of padding alone
-    (2300, 2944, 8, 4, 6, 64),         # 23 scales: the last trip of a block is not full
-    (1755, 2048, 8, 4, 8, 2), (1749, 2048, 8, 4, 8, 2),       # both sides of that line
+    (2048, 1024, 8, 1, 7, 128),        # narrow rows
+    # in blocks from 850000 scales and 14000 rows on, padding rows counted double:
+    (1300, 2048, 128, 8, 8, 512),      # padding rows fill whole blocks
+    (100, 16384, 128, 2, 4, 128),      # as many scales a row as a block may have, an expert's few rows alone in its region
+    (2300, 2944, 64, 4, 6, 400),       # 23 scales: the last trip of a block is not full
+    (1803, 7168, 8, 4, 8, 128), (1768, 7168, 8, 4, 8, 128),       # 56 scales: both sides of the line of scales
+    (14011, 7808, 8, 4, 1, 2), (13940, 7808, 8, 4, 1, 8),         # 61: both sides of the line of rows, the last block not full
 ], ids=lambda v: str(v))
 @pytest.mark.parametrize("cast", [True, False])
 def test_blocked_scales_match_the_oracle(T, H, E, R, K, alignment, cast):
