@@ -803,9 +803,16 @@ hipError_t launch_ll_combine(const LLCombineParams& p, hipStream_t stream) {
     int vecs = p.vecs;
     if (vecs != 1 && vecs != 2 && vecs != 4 && vecs != 7) {
         // 2 KB is the widest tile whose whole grid is resident at once at decode sizes (1024 tokens x 7168: 1 KB 8.4 us, 2 KB 7.9, 4 KB
-        // 9.2, 7 KB 9.3), and the best one in large batches (8192 tokens x 7168 over 8 ranks 48.0 / 43.7 / 45.4 / 47.7, over 16 ranks
-        // 43.6 / 34.2 / 35.6 / 38.3, 8192 x 2048 17.8 / 16.4 / 16.7 / 21.5).
-        vecs = p.H * 2 <= 1024 ? 1 : 2;
+        // 9.2, 7 KB 9.3), and the best one in large batches whose tokens have half a row here and more (us with 1 / 2 / 4 / 7 KB, 16384 tokens x
+        // 7168 top-8 over 8 ranks 88.8 / 80.8 / 84.3 / 88.4, top-4 80.9 / 63.2 / 65.2 / 69.8; 12800 x 7168 top-8 over 16 64.6 / 50.7 / 52.8 / 56.2).
+        // With fewer rows most wavefronts read the routing and store zeros: 4 KB from an eighth of a row down (16384 x 7168 top-1 over 8 74.0 /
+        // 62.4 / 50.0 / 56.0, 12800 x 5120 top-2 over 16 44.7 / 37.9 / 35.8 / 43.1), at up to a quarter where a row is one tile or
+        // its last one leaves little idle (9600 x 1536 top-2 over 8 14.8 / 15.0 / 14.2 / 18.3, 16384 x 7168 78.1 / 58.6 / 55.5 / 61.9; 5120 channels
+        // 58.2 / 44.1 / 47.2 / 57.3).
+        const int kb = (p.H * 2 + 1023) / 1024, idle = (kb + 3) / 4 * 4 - kb;
+        const int64_t tokens = int64_t(p.S) * p.src_token_stride, local = int64_t(p.K) * p.E_l;        // rows a token: local / E
+        const bool few_rows = 8 * local <= p.E || (4 * local <= p.E && (kb <= 4 || 7 * idle <= kb));
+        vecs = p.H * 2 <= 1024 ? 1 : tokens > 4096 && few_rows ? 4 : 2;
     }
     if (p.use_logfmt) vecs = p.H % 1024 == 0 ? 2 : 1;                                     // one codec chunk per wavefront
     const int tiles = (p.H * 2 + vecs * 1024 - 1) / (vecs * 1024);
