@@ -741,6 +741,18 @@ size_t deep_ep_hip_ll_workspace_bytes(int num_src_ranks, int src_token_stride, i
     return off;
 }
 
+int deep_ep_hip_ll_dispatch_threads(const deep_ep_hip_ll_dispatch_args* a) {
+    REQUIRE(a != nullptr, "args is NULL");
+    REQUIRE(a->num_src_ranks >= 1 && a->src_token_stride >= 1 && a->num_topk >= 1 && a->num_topk <= DEEP_EP_HIP_MAX_TOPK &&
+            a->num_local_experts >= 1 && a->num_local_experts <= DEEP_EP_HIP_MAX_EXPERTS && a->hidden >= 16 && a->hidden % 16 == 0, "bad shape");
+    LLDispatchParams p{};
+    p.S = a->num_src_ranks; p.src_token_stride = a->src_token_stride;
+    p.H = a->hidden; p.K = a->num_topk; p.E_l = a->num_local_experts; p.use_fp8 = a->use_fp8 ? 1 : 0;
+    p.topk_idx = a->topk_idx;
+    p.pairs = a->tuning.ll_pairs; p.threads = a->tuning.ll_threads; p.two_kernels = a->tuning.ll_two_kernels;
+    return ll_single_kernel_threads(p);
+}
+
 int deep_ep_hip_launch_ll_dispatch(const deep_ep_hip_ll_dispatch_args* a, void* stream) {
     REQUIRE(a != nullptr, "args is NULL");
     REQUIRE(a->num_src_ranks >= 1 && a->src_token_stride >= 1, "need at least one source rank and one token slot");

@@ -311,6 +311,8 @@ int compute_units();
 // LDS a workgroup asks for so that a CU holds at most `per_cu` of them (0: no limit).
 size_t lds_for_residency(int per_cu);
 
+// Threads of a workgroup where the dispatch is a single kernel, 0 where it is the counting and the move kernel.
+int ll_single_kernel_threads(const LLDispatchParams& p);
 hipError_t launch_ll_dispatch(const LLDispatchParams& p, hipStream_t stream);
 
 struct LLCombineParams {

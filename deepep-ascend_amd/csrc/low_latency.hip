@@ -221,6 +221,9 @@ __device__ __forceinline__ void ll_store_tile(const LLDispatchParams& p, int64_t
 // the tokens with top-8 over 8 ranks).  The chunk totals in front of the token are asked for ahead of the payload and summed
 // while it is on its way.  4096 tokens of 7168 channels to FP8, bound by memory and by its single-dword scale stores: 17.3 us, 19.4
 // with every payload read and exponents stored byte by byte; counting and moving together 25.0, 32.9 before.
+// The totals in front of a token are a loop of one trip per 64 chunks.  Dispatch of 8192 / 16384 / 32768 / 65536 tokens of 7168 channels to FP8 over 8
+// ranks (32 to 256 chunks) 45 / 66 / 142 / 257 us, 65536 of 2048 channels 73, over 64 ranks 31; with bases from a last workgroup of the counting
+// kernel 55 / 105 / 220 / 365, 156 and 130.
 template <int kPairs, bool kFp8, int kBlockThreads>
 __global__ __launch_bounds__(kBlockThreads) void ll_move_kernel(const LLDispatchParams p, const int tiles) {
     const int lane = threadIdx.x & 63;
@@ -745,42 +748,42 @@ hipError_t launch_fused_by_width(const LLDispatchParams& p, hipStream_t stream, 
     }
 }
 
+static size_t fused_lds_bytes(const LLDispatchParams& p) {      // the routing table, plus one spare 32-bit word per lane
+    return size_t(p.E_l) * ((int64_t(p.S) * p.src_token_stride + 63) / 64) * sizeof(uint64_t) + kWaveSize * sizeof(uint32_t);
+}
+
 // Decode-sized calls: one kernel, every workgroup of which derives the slots itself.  How many threads a workgroup has, or 0 for the
-// two kernels.  Every workgroup passes over all selections, so the more there are the fewer workgroups a CU may have and the more
-// wavefronts share a pass.  Dispatch, us, 256 / 512 / 1024 threads / two kernels, FP8, top-1 over 16 ranks, top-4 over 4, the rest 8:
-//   up to 4096 selections       2048 x 2048 top-1 8.7 / 9.2 / 10.1 / 10.2;   1024 x 4096 top-4 8.6 / 10.1 / 12.1 / 11.7;
-//                               3072 x 7168 top-1 (6144 wavefronts) 13.6 / 13.9 / 15.8 / 13.9;   2048 x 7168 top-2 12.4 / 12.9 / 13.3 / 13.5
-//   up to 8192, 16 a CU         2240 x 2048 top-2 9.6 / 9.2 / 9.9 / 10.8;   1024 x 7168 top-8 12.0 / 11.0 / 14.2 / 13.1;   2048 x 7168 top-4
-//                               (4096 wavefronts) 15.7 / 14.6 / 15.4 / 15.9;   2560 x 7168 top-2 (5120) 15.5 / 14.6 / 17.0 / 14.6
-//   more, 8 wavefronts a CU     2048 x 2048 top-8 12.8 / 10.8 / 10.9 / 11.8;   2048 x 4096 top-8 15.1 / 13.3 / 13.3 / 14.1
-//   up to 16384, 16 a CU, 2048 tokens   1280 x 7168 top-8 15.0 / 15.1 / 13.2 / 14.1;   2048 x 7168 19.8 / 17.6 / 15.9 / 16.4
-//                               (over 16 ranks 18.3 / 15.4 / 14.7 / 14.5: the one point of the line where the two kernels are ahead)
-//   up to 24576, 16 a CU, 2048 channels   2288 x 1024 top-8 13.3 / 12.2 / 11.5 / 11.8;   2560 x 2048 top-6 13.4 / 12.0 / 10.8 / 11.6;   3072 x 2048
-//                               top-8 17.3 / 14.4 / 12.9 / 12.5, where a launch less is worth more than that: dispatch and combine of the
-//                               first 18.8 in three launches, 15.1 in two
-//   beyond                      2240 x 4096 top-8 17.7 / 16.9 / 14.5 / 14.1;   3072 x 7168 top-8 29.0 / 23.9 / 24.0 / 18.6
-static int fused_threads(const LLDispatchParams& p) {
+// two kernels.  Every workgroup passes over all selections, so the more there are the more wavefronts share a pass, as long as the
+// workgroups (one of 1024 threads to a CU) are all resident at once.  500 shapes (64 to 3072 tokens, 1024 to 7168 channels, top-1 to
+// top-32 over 4 to 16 ranks), tokens in the cache and just written, on average behind the fastest of the four, in %, 256 / 512 / 1024 threads /
+// two kernels, by wavefronts a CU and selections:
+//   up to 4096 selections    0 / 5 to 10 / 10 to 32 / 23 to 40
+//   up to 8, 6144 7.3 / 0.0 / 18.2 / 29.0;   24576 14.2 / 1.4 / 8.7 / 16.6;   more, up to 6 wavefronts a CU (half the CUs of 1024 threads would
+//   have no workgroup) 22 / 0.3 / 6 / 26, up to 8 39 / 14 / 0 / 21
+//   up to 12, 6144 7.3 / 0.3 / 9.1 / 15.2;   12288 13.8 / 10.1 / 0.2 / 12.7;   24576 26.0 / 9.4 / 2.1 / 3.5;   more 67 / 28 / 0 / 7.5
+//   up to 16, 8192 7.2 / 1.7 / 12.3 / 18.0;   16384 to FP8 23 / 4.1 / 0.2 / 8, BF16 12 / 5.6 / 10 / 6;   24576 21.2 / 2.3 / 10.2 / 0.0;   more
+//   19 / 17 / 10 / 3.4
+//   more, 6144 11.3 / 0.0 / 27.0 / 9.3;   12288 8.6 / 7.7 / 9.1 / 1.9;   24576 28.2 / 14.5 / 22.8 / 1.1
+int ll_single_kernel_threads(const LLDispatchParams& p) {
     const int64_t tokens = int64_t(p.S) * p.src_token_stride, selections = tokens * p.K;
-    const int64_t waves = tokens * ((p.H + fused_pairs(p) * 1024 - 1) / (fused_pairs(p) * 1024)), per_cu_8 = int64_t(compute_units()) * 8;
+    const bool table_fits = (reinterpret_cast<uintptr_t>(p.topk_idx) & 15) == 0 && selections >= 2 && p.H >= 16 && tokens <= kFusedTokens &&
+                            fused_lds_bytes(p) <= 33 * 1024;
+    if (p.two_kernels || !table_fits) return 0;
     if (p.threads == 256 || p.threads == 512 || p.threads == 1024) return p.threads;
+    const int64_t waves = tokens * ((p.H + fused_pairs(p) * 1024 - 1) / (fused_pairs(p) * 1024)), cus = compute_units();
     if (selections <= 4096) return 256;
-    if (waves <= per_cu_8) return 512;
-    if (waves > 2 * per_cu_8) return 0;
-    if (selections <= 8192) return 512;
-    return selections <= 24576 && (p.H <= 2048 || (selections <= 16384 && tokens <= 2048)) ? 1024 : 0;
+    if (waves <= 8 * cus) return selections <= 24576 || waves <= 6 * cus ? 512 : 1024;
+    if (waves <= 12 * cus) return selections <= 8192 ? 512 : 1024;
+    if (waves <= 16 * cus && selections <= 16384) return selections <= 8192 || !p.use_fp8 ? 512 : 1024;
+    return selections <= 6144 ? 512 : 0;
 }
 
 hipError_t launch_ll_dispatch(const LLDispatchParams& p, hipStream_t stream) {
     if (p.S <= 0 || p.src_token_stride <= 0) return hipSuccess;
-    const int64_t total_tokens = int64_t(p.S) * p.src_token_stride;
-    // the routing table of the single-kernel path, plus one spare 32-bit word per lane
-    const size_t fused_lds = size_t(p.E_l) * ((total_tokens + 63) / 64) * sizeof(uint64_t) + kWaveSize * sizeof(uint32_t);
-    const bool table_fits = (reinterpret_cast<uintptr_t>(p.topk_idx) & 15) == 0 && total_tokens * p.K >= 2 && p.H >= 16;
-    const int threads = fused_threads(p);
-    if (threads != 0 && total_tokens <= kFusedTokens && fused_lds <= 33 * 1024 && table_fits && !p.two_kernels) {
-        if (threads == 256) return launch_fused_by_width<256>(p, stream, fused_lds);
-        if (threads == 1024) return launch_fused_by_width<1024>(p, stream, fused_lds);
-        return launch_fused_by_width<512>(p, stream, fused_lds);
+    switch (ll_single_kernel_threads(p)) {
+        case 256: return launch_fused_by_width<256>(p, stream, fused_lds_bytes(p));
+        case 512: return launch_fused_by_width<512>(p, stream, fused_lds_bytes(p));
+        case 1024: return launch_fused_by_width<1024>(p, stream, fused_lds_bytes(p));
     }
 
     const int chunks_per_src = (p.src_token_stride + kThreads - 1) / kThreads;

@@ -393,6 +393,10 @@ typedef struct {
 /* Bytes of (zero-initialised, reusable) workspace a low-latency dispatch of this shape needs.  A memory of its own: it
  * must not overlap the workspace of deep_ep_hip_launch_dispatch (see deep_ep_hip_workspace_control_bytes). */
 size_t deep_ep_hip_ll_workspace_bytes(int num_src_ranks, int src_token_stride, int num_topk, int num_local_experts);
+/* How deep_ep_hip_launch_ll_dispatch would run for these sizes (num_src_ranks, src_token_stride, hidden, num_topk,
+ * num_local_experts, use_fp8, tuning, the alignment of topk_idx): threads of a workgroup of the single kernel (256, 512, 1024), or 0 for
+ * the counting and the move kernel.  Negative: an error code.  No counterpart in the reference. */
+int deep_ep_hip_ll_dispatch_threads(const deep_ep_hip_ll_dispatch_args* args);
 int deep_ep_hip_launch_ll_dispatch(const deep_ep_hip_ll_dispatch_args* args, void* stream);
 
 typedef struct {

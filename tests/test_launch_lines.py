@@ -1,4 +1,5 @@
-"""Which dispatches take one launch: both sides of the lines drawn by bytes and by rounds of workgroups, and GPU results on both sides of
+"""Which dispatches take one launch: both sides of the lines drawn by bytes and by rounds of workgroups, which low-latency dispatches take the
+single kernel and in workgroups of how many threads, and GPU results on both sides of
 the two lines against the other way of launching (the ways themselves are compared with the oracle elsewhere)."""
 import ctypes
 
@@ -25,6 +26,44 @@ def test_launches(payload, T, H, R, K, E, launches):
     a.payload = {"bf16": _abi.PAYLOAD_BF16, "fp8": _abi.PAYLOAD_FP8, "cast": _abi.PAYLOAD_CAST_FP8}[payload]
     a.num_tokens, a.hidden, a.num_topk, a.num_experts, a.num_ranks, a.expert_alignment = T, H, K, E, R, 1
     assert _abi.lib.deep_ep_hip_dispatch_kernel_launches(ctypes.byref(a)) == launches
+
+
+LL_LINES = [
+    # source ranks, tokens of each, hidden, top-k, local experts, threads (0: two kernels); 256 compute units
+    (8, 512, 512, 1, 32, 0),                                                            # 4096 tokens: past 3072
+    (8, 384, 7168, 1, 32, 256), (4, 512, 1152, 2, 4, 256), (4, 513, 1152, 2, 4, 512),   # 4096 selections
+    (8, 256, 1024, 12, 4, 512), (8, 256, 1024, 13, 4, 1024),                            # eight wavefronts a unit: 24576
+    (8, 192, 1024, 32, 4, 512), (8, 193, 1024, 32, 4, 1024),                            # ... and six
+    (8, 257, 512, 3, 4, 512), (8, 257, 512, 4, 4, 1024),                                # twelve: 8192
+    (8, 384, 512, 2, 4, 512), (8, 384, 512, 3, 4, 1024), (8, 384, 512, 32, 4, 1024),
+    (8, 193, 4112, 3, 4, 512), (8, 193, 4112, 10, 4, 512), (8, 193, 4112, 11, 4, 0),    # 1544 tokens of two wavefronts, sixteen: 16384
+    (8, 256, 7168, 8, 32, 512), (8, 256, 7168, 9, 32, 0), (8, 257, 7168, 7, 32, 0),     # 4096 wavefronts, and more: 6144
+    (8, 384, 7168, 2, 32, 512), (8, 380, 7168, 3, 32, 0),
+    (8, 384, 512, 8, 86, 1024), (8, 384, 512, 8, 88, 0),                                # 33 KB of routing table
+    (1, 1, 7168, 1, 32, 0), (1, 2, 7168, 1, 32, 256),                                   # two selections
+]
+
+
+def _ll_threads(S, stride, H, K, E_l, use_fp8=0, **knobs):
+    a = _abi.LLDispatchArgs()
+    a.num_src_ranks, a.src_token_stride, a.hidden, a.num_topk, a.num_local_experts, a.use_fp8 = S, stride, H, K, E_l, use_fp8
+    for k, v in knobs.items():
+        setattr(a.tuning, k, v)
+    return _abi.lib.deep_ep_hip_ll_dispatch_threads(ctypes.byref(a))
+
+
+@pytest.mark.parametrize("S,stride,H,K,E_l,threads", LL_LINES)
+def test_low_latency_threads(S, stride, H, K, E_l, threads):
+    assert _ll_threads(S, stride, H, K, E_l) == threads
+
+
+def test_low_latency_threads_by_knob_and_errors():
+    assert _ll_threads(8, 128, 7168, 8, 32, ll_two_kernels=1) == 0
+    assert [_ll_threads(8, 128, 7168, 8, 32, ll_threads=n) for n in (256, 512, 1024, 128)] == [256, 512, 1024, 512]
+    assert [_ll_threads(8, 256, 7168, K, 32, use_fp8=1) for K in (4, 5, 8, 9)] == [512, 1024, 1024, 0]       # sixteen: the cast is shared by more
+    assert _ll_threads(8, 512, 7168, 8, 32, ll_threads=1024) == 0                       # 4096 tokens take two kernels whatever is asked for
+    assert _ll_threads(8, 128, 7168, 33, 32) < 0 and _ll_threads(0, 128, 7168, 8, 32) < 0 and _ll_threads(8, 128, 100, 8, 32) < 0
+    assert _abi.lib.deep_ep_hip_ll_dispatch_threads(None) < 0
 
 
 @pytest.mark.gpu
