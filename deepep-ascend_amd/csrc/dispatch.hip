@@ -1507,7 +1507,7 @@ hipError_t launch_copy_cached(const MoveParams& p, unsigned blocks, hipStream_t 
     const bool plain = kPlain == kNoScales && p.recv_sf == nullptr && (rows_per_token(p) < 5.0 || p.row_bytes < 4096);
     auto kernel = p.fused ? (plain ? dispatch_copy_single_launch_kernel<kVecs, kPlain, kCached> : dispatch_copy_single_launch_kernel<kVecs, kScalesInPlace, kCached>)
                           : (plain ? dispatch_copy_kernel<kVecs, kPlain, kCached> : dispatch_copy_kernel<kVecs, kScalesInPlace, kCached>);
-    if constexpr (kVecs <= 4)
+    if constexpr (kVecs <= 4 && kCached == kNeither)            // scales come with FP8 rows
         if (p.sf_blocked) kernel = p.fused ? dispatch_copy_single_launch_kernel<kVecs, kScalesInBlocks, kCached> : dispatch_copy_kernel<kVecs, kScalesInBlocks, kCached>;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), move_lds_bytes(p), stream, p);
     return hipGetLastError();
