@@ -8,8 +8,11 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,H,E,R,K,sync", [
-    (17700, 2056, 32, 2, 2, True), (18100, 2056, 32, 2, 2, True),         # two launches: 109 and 112 MB of rows
+    (17700, 2056, 32, 2, 2, True), (18100, 2056, 32, 2, 2, True),         # two launches: 109 and 112 MB of rows, compact
     (5050, 2056, 256, 8, 8, False), (5200, 2056, 256, 8, 8, False),       # one launch
+    (19500, 2056, 32, 2, 2, True),                                        # 116 MB returned, compact: the combine's side too
+    (13200, 2056, 32, 2, 2, True), (14300, 2056, 32, 2, 2, True),         # expanded, 109 and 118 MB of rows, 103 and 112 returned
+    (3250, 2056, 256, 8, 8, False), (3600, 2056, 256, 8, 8, False),       # 107 and 118, 102 and 113
 ])
 @pytest.mark.parametrize("expand", [False, True])
 def test_rows_and_sums(T, H, E, R, K, sync, expand):
