@@ -322,7 +322,7 @@ bool takes_two_kb_tiles(const CombineParams& p) {
 
 // The rows a combine adds up have just been written, by the experts or by the dispatch itself: up to 110 MB of them are read with plain
 // loads, which find them in the memory-side cache.  Dispatch and combine of BF16 rows, us, streaming / plain rows (the dispatch stores
-// accordingly, cached_side): 4096 x 2048 top-6 of 8 ranks, forward and backward (74 MB) 91.2 / 84.9, 16384 x 2048 of 2 ranks (100 MB) 77.5
+// by the same line, for the rows even routing would give, cached_side): 4096 x 2048 top-6 of 8 ranks, forward and backward (74 MB) 91.2 / 84.9, 16384 x 2048 of 2 ranks (100 MB) 77.5
 // / 76.0; combine of rows an expert has just written, with an FP8 dispatch in front, 1024 x 7168 (78 MB) 42.3 / 36.7, 700 x 4096 (30 MB) 27.4 /
 // 26.6; rows that are in HBM while the cache is full of what others have written are the other way round (41.0 / 53.5).  More rows than
 // the cache holds beside other traffic are read past it: 2100 x 7168 (160 MB) 67.5 / 74.0, 4096 x 7168 (311 MB) 134 / 170.  So are

@@ -73,12 +73,16 @@ typedef struct {
                                   the front of the move kernel) where the shape allows it (num_topk <= 8, num_ranks +
                                   num_experts <= 512, num_ranks * ceil(num_tokens / 256) <= 1024, num_tokens * num_topk
                                   <= 131072; with do_expand also ceil(num_tokens / 256) * num_experts <= 8192 and
-                                  num_tokens * num_topk + num_experts * expert_alignment < 2^18) and it pays (at most
-                                  16384 mover workgroups; with do_expand less than 64 MB of input); 1 = a single launch
-                                  wherever the shape allows it; 2 = always layout kernel + move kernel */
+                                  num_tokens * num_topk + num_experts * expert_alignment < 2^18) and it pays: at most 16384
+                                  mover workgroups; rows copied as they are from less than 64 MB of input, and less than 300 MB
+                                  of them (345 MB of rows of up to 4 KB); no compact cast of four rows a token and more with
+                                  movers + counting workgroups >= 6 and movers <= 7 for each compute unit; with do_expand less
+                                  than 64 MB of input.  1 = a single launch wherever the shape allows it; 2 = always layout
+                                  kernel + move kernel */
     int32_t cast_pairs;        /* fused FP8 cast: 1024-channel segments per wavefront (1, 2, 4, 7, 8; above 2: two launches) */
     int32_t copy_vecs;         /* pass-through payloads: KB of row per wavefront (1, 2, 4, 7, 8) */
-    int32_t plain_loads;       /* 1: payload loads allocate in the caches (for inputs known to be cache resident) */
+    int32_t plain_loads;       /* fused FP8 cast, 1: payload loads allocate in the caches (for inputs known to be cache resident; BF16 copies
+                                  and low-latency dispatches choose by themselves) */
     int32_t xcd_remap;         /* 1: consecutive workgroups of a dispatch share an XCD */
     int32_t combine_vecs;      /* combine: KB of row per wavefront (1, 2, 4) */
     int32_t ll_pairs;          /* low-latency dispatch: 1024-channel segments per wavefront (1, 2, 4) */
