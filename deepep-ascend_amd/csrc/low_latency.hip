@@ -125,7 +125,7 @@ constexpr int kFusedTokens = 3072;      // the single-kernel path: a lane per 64
 // memory-side cache holds unwritten takes longer.  A line that is not there pushes another out, which has to be written to HBM first
 // where the cache is full of what others have written, so nothing is loaded that is not stored.  Dispatch, us, tokens in the cache
 // (called over and over) / just written behind 400 MB of other writes / in HBM / in HBM behind 1 GB of other writes:
-//   plain          1024 x 7168 FP8 9.8 / 11.2 / 10.9 / 12.3;   2048 x 7168 BF16 17.9 / 19.9 / 20.8 / 22.3;   4096 x 7168 (two kernels) 21.4 / 25.3 /
+//   plain          1024 x 7168 FP8 9.8 / 11.2 / 10.9 / 12.3;   2048 x 7168 BF16, 1024 threads 17.9 / 19.9 / 20.8 / 22.3;   4096 x 7168 (two kernels) 21.4 / 25.3 /
 //                  24.6 / 30.1
 //   streaming      10.4 / 12.1 / 11.2 / 11.9;   20.1 / 22.1 / 21.0 / 21.6;   26.1 / 28.3 / 25.7 / 26.3
 //   plain, also the tokens that stay nowhere here   10.6 / 11.9 / 11.4 / 14.4;   20.2 / 22.0 / 23.6 / 27.8
