@@ -326,11 +326,11 @@ bool takes_two_kb_tiles(const CombineParams& p) {
 // / 76.0; combine of rows an expert has just written, with an FP8 dispatch in front, 1024 x 7168 (78 MB) 42.3 / 36.7, 700 x 4096 (30 MB) 27.4 /
 // 26.6; rows that are in HBM while the cache is full of what others have written are the other way round (41.0 / 53.5).  More rows than
 // the cache holds beside other traffic are read past it: 2100 x 7168 (160 MB) 67.5 / 74.0, 4096 x 7168 (311 MB) 134 / 170.  So are
-// expanded rows among padding rows that are zeroed behind them, from 140 MB of both on: 300 x 7168 top-8 over 256 experts aligned to 128 (34 of
-// 470 MB) 14.5 / 22.9; 1500 x 2048 (49 of 134 MB), rows just written by an expert, 19.1 / 17.1.
+// expanded rows among padding rows that are zeroed behind them, from 240 MB of both on: top-8, aligned to 128, input just written, 400 x 7168 of
+// 128 experts (46 of 235 MB) 16.3 / 15.1, of 144 (264 MB) 16.3 / 16.2, of 160 (294 MB) 16.7 / 23.7, 300 x 7168 of 256 (470 MB) 14.9 / 23.8.
 bool reads_past_the_cache(const CombineParams& p) {
     const double row_bytes = p.H * 2.0;
-    const bool between_padding = p.do_expand && !p.rank_mode && p.num_x_rows * row_bytes > 140e6;
+    const bool between_padding = p.do_expand && !p.rank_mode && expanded_rows_in_use(p.num_x_rows, p.num_meta_rows, p.T, p.K, p.E, p.R, p.M) * row_bytes > kExpandedBytesInCache;
     return between_padding || rows_per_token(p) * p.T * row_bytes > 110e6;
 }
 

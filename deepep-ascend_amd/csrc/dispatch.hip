@@ -1477,10 +1477,12 @@ void plan_cache_warming(MoveParams& p) {
 }
 
 // Which side of a copy goes through the memory-side cache (256 MB).
-// - BF16, up to 110 MB of rows and 140 MB with the padding rows zeroed behind them: the rows, which whoever is next then finds there.
+// - BF16, up to 110 MB of rows and 240 MB with the padding rows zeroed behind them: the rows, which whoever is next then finds there.
 //   Dispatch and combine, us, neither / rows, input just written: 277 x 6072 over 8 ranks (18 MB) 24.0 / 22.0, 1024 x 7168 (77 MB) 54.3 / 40.7,
 //   4096 x 2048 top-6 (74 MB) 55.7 / 44.1; with a pass over the rows in between that writes as many 30.9 / 31.6, 66.1 / 65.3, 67.7 / 66.4.  With more
-//   padding the rows leave the cache again before they are read: 300 x 7168 over 256 experts aligned to 128 (470 MB) 104.2 / 113.4.
+//   padding the rows leave the cache again before they are read.  Top-8, aligned to 128, streaming / rows: 646 x 2136 of 384 experts (210 MB)
+//   61.4 / 60.0, 400 x 7168 of 112 (206 MB) 62.8 / 61.6, of 128 (235 MB) 67.2 / 66.5, of 144 (264 MB) 72.2 / 72.2, of 160 (294 MB) 78.0 /
+//   84.4, 300 x 7168 of 256 (470 MB) 104.4 / 115.5.
 // - BF16, more: the input, which the layer in front has just written; so many rows would drive it and each other out.  Dispatch and
 //   combine, us, neither / input: 2600 x 7168 over 8 ranks (198 MB) 103.4 / 96.5, 3400 x 7168 (258 MB) 123.7 / 116.5, 8192 x 7168 (622 MB) 261.7 /
 //   261.5, V1 4096 x 7168 150.2 / 141.8, expanded 4096 x 4096 top-8 143.3 / 134.8; with the input just written behind 400 MB of other writes 103.7 /
@@ -1494,7 +1496,8 @@ void plan_cache_warming(MoveParams& p) {
 static int cached_side(const MoveParams& p) {
     if (p.payload != DEEP_EP_HIP_PAYLOAD_BF16) return kNeither;
     const double zeroed = p.zeroed_rows * double(p.row_bytes);
-    if (row_bytes_out(p) <= 110e6 && row_bytes_out(p) + zeroed <= 140e6) return kRows;
+    const bool among_padding = p.do_expand && expanded_rows_in_use(p.expanded_capacity, p.recv_capacity, p.T, p.K, p.E, p.R, p.M) * p.row_bytes > kExpandedBytesInCache;
+    if (row_bytes_out(p) <= 110e6 && !among_padding) return kRows;
     return double(p.T) * p.row_bytes <= 256e6 && zeroed < 150e6 ? kInput : kNeither;
 }
 

@@ -6,6 +6,9 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <cmath>
+
 namespace deep_ep_hip {
 
 // Single-launch dispatch: number of completion counters ("gates") the movers spread over, and the distance between
@@ -235,6 +238,19 @@ struct FillTailParams {
 };
 
 hipError_t launch_fill_tail(const FillTailParams& p, hipStream_t stream);
+
+// Rows of an expanded output that a call writes or zeroes, for the two sides of the memory-side cache: the dispatch and the combine of
+// its rows have to come to the same answer, and these arguments are the same for both.  An output of exact size: all of it.  One of
+// worst-case size (M tokens of each rank, M * min(K, E) + E * (alignment - 1) rows), with even routing: one alignment for each expert that
+// has a row where next to none (two deviations) needs a second one, otherwise the selections and half an alignment for each.
+inline double expanded_rows_in_use(int64_t rows, int64_t meta_rows, int T, int K, int E, int R, int M) {
+    if (meta_rows < int64_t(M) * R) return double(rows);
+    const double padding = std::max(double(rows) - double(M) * std::min(K, E), 0.0), alignment = padding / E + 1.0;
+    const double selections = double(T) * K, each = selections / E;
+    if (each + 2.0 * std::sqrt(each) <= alignment) return E * (1.0 - std::exp(-each)) * alignment;
+    return selections + 0.5 * padding;
+}
+constexpr double kExpandedBytesInCache = 240e6;
 
 struct CombineParams {
     const uint8_t* x;
