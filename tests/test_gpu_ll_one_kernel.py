@@ -29,6 +29,7 @@ pytestmark = pytest.mark.gpu
     (8, 385, 4112, 16, 2, "bf16"),         # 3080 tokens: two kernels
     (8, 384, 4112, 16, 2, "bf16"),         # 6144 selections, 6144 wavefronts: 512
     (8, 192, 4112, 16, 6, "bf16"),         # 3072 wavefronts: 1024
+    (8, 384, 512, 64, 32, "fp8"),          # 98304 selections: 1024
 ], ids=lambda v: str(v))
 def test_single_kernel_lines(R, T, H, E, K, payload):
     import deep_ep
