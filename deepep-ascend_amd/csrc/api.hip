@@ -53,7 +53,7 @@ struct LaunchPlan {
     bool fused;       // one launch: counting workgroups at the front of the move kernel
 };
 
-LaunchPlan plan_launches(int T, int K, int E, int R, bool do_layout, bool do_move, bool do_expand, int alignment, int payload, int H,
+LaunchPlan plan_launches(int T, int K, int E, int R, bool do_layout, bool do_move, bool do_expand, bool do_zero_padding, int alignment, int payload, int H,
                          int row_bytes, const deep_ep_hip_tuning& tuning, int64_t rows_of_rank_lanes = -1 /* no top-k: rows received */) {
     LaunchPlan q{};
     q.chunks = T > 0 ? (T + kLayoutChunk - 1) / kLayoutChunk : 1;
@@ -75,6 +75,14 @@ LaunchPlan plan_launches(int T, int K, int E, int R, bool do_layout, bool do_mov
     // first microsecond (8192 x 7168: 123-128 us against 130-134 us; from 4096 tokens down the single launch is ahead,
     // 66.5 against 72.8 us).
     if (q.fused && do_expand && tuning.dispatch_launches != 1 && int64_t(T) * row_bytes >= (int64_t(64) << 20)) q.fused = false;
+    // A move on a finished layout zeroes the padding rows beside its own work, a single launch leaves them to one more launch.  One / two
+    // launches, us, padding included: BF16, over 44 shapes of 13 to 64 MB of input two are ahead by 4 % on average and never 2.5 % behind
+    // (6485 x 1280 top-2 of 64 24.1 / 22.6, 4462 x 5120 top-8 of 64 85.2 / 84.9; 1992 x 4224 top-4 of 256, alignment 4, 23.6 / 24.2); FP8 rows 300 x
+    // 7168 top-8 of 256 47.5 / 41.1, 72 x 3968 top-10 of 16 19.1 / 14.1, 2613 x 6144 fp8 49.6 / 49.1; but many of them from a large input, whose
+    // first loads hide the layout: cast, 3000 x 7168 top-6 of 64 49.8 / 52.9, 5346 x 3712 top-4 of 16 36.2 / 40.5, fp8 5342 x 6272 top-6 61.3 / 72.8,
+    // 8417 x 5120 top-4 of 128 63.8 / 65.0; with many narrow rows two again (cast, 13820 x 1280 top-6 54.0 / 48.5, 12640 x 2432 77.7 / 72.0).
+    if (q.fused && do_zero_padding && alignment > 1 && tuning.dispatch_launches != 1)
+        q.fused = payload != DEEP_EP_HIP_PAYLOAD_BF16 && int64_t(T) * row_bytes >= 26000000 && int64_t(T) * K * H >= 80000000 && T <= 10000;
     if (q.fused && tuning.dispatch_launches != 1) {
         MoveParams probe{};
         probe.T = T; probe.H = H; probe.row_bytes = row_bytes; probe.payload = payload; probe.do_expand = do_expand ? 1 : 0;
@@ -288,7 +296,7 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
     // chunk), the first row of that chunk's share of the bucket; the move kernel adds the two.  Layout and move in
     // one call: the counting workgroups ride at the front of the move kernel (one launch); shapes that does not
     // cover run the layout kernel first.
-    const LaunchPlan plan = plan_launches(T, K, E, R, do_layout, do_move, a->do_expand != 0, a->expert_alignment, a->payload, H,
+    const LaunchPlan plan = plan_launches(T, K, E, R, do_layout, do_move, a->do_expand != 0, a->do_zero_padding != 0, a->expert_alignment, a->payload, H,
                                           H * elem_in, a->tuning);
     LayoutParams lay{};
     lay.topk_idx = a->topk_idx;
@@ -351,11 +359,9 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
             m.zeroed_rows = int(std::min<int64_t>(std::max(int64_t(E) * (a->expert_alignment - 1) / 2, regions - selections), INT32_MAX));
         }
 
-        hipError_t err = launch_dispatch_move(m, stream);
-        if (err != hipSuccess) return hip_fail(err, "dispatch move launch");
-
-        if (a->do_zero_padding && a->expert_alignment > 1) {
-            PadParams z{};
+        const bool pads = a->do_zero_padding && a->expert_alignment > 1;
+        PadParams z{};
+        if (pads) {
             z.recv_x = static_cast<uint8_t*>(a->recv_x);
             z.recv_sf = (a->payload != DEEP_EP_HIP_PAYLOAD_BF16) ? static_cast<uint32_t*>(a->recv_sf) : nullptr;
             z.rsf_ts = a->recv_sf_token_stride; z.rsf_hs = a->recv_sf_hidden_stride;
@@ -367,7 +373,18 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
             z.E = E; z.A = a->expert_alignment;
             z.out_row_bytes = H * elem_out;
             z.sf_blocked = m.sf_blocked;
-            err = launch_zero_padding(z, stream);
+            z.slices = pad_slices(E, a->expert_alignment, z.out_row_bytes);
+            if (!plan.fused) {
+                m.pad = z;
+                m.pad_blocks = unsigned(E) * unsigned(z.slices);
+            }
+        }
+
+        hipError_t err = launch_dispatch_move(m, stream);
+        if (err != hipSuccess) return hip_fail(err, "dispatch move launch");
+
+        if (pads) {
+            err = launch_zero_padding(z, plan.fused, stream);
             if (err != hipSuccess) return hip_fail(err, "zero padding launch");
         }
     }
@@ -461,7 +478,7 @@ int deep_ep_hip_dispatch_kernel_launches(const deep_ep_hip_dispatch_args* a) {
     if (a->num_tokens == 0) return do_layout ? 1 : 0;      // an empty move launches nothing
     const int elem_in = a->payload == DEEP_EP_HIP_PAYLOAD_FP8 ? 1 : 2;
     const LaunchPlan plan = plan_launches(a->num_tokens, a->num_topk, a->num_experts, a->num_ranks, do_layout, do_move,
-                                          a->do_expand != 0, a->expert_alignment, a->payload, a->hidden, a->hidden * elem_in,
+                                          a->do_expand != 0, a->do_zero_padding != 0, a->expert_alignment, a->payload, a->hidden, a->hidden * elem_in,
                                           a->tuning);
     return plan.fused ? 1 : int(do_layout) + int(do_move);
 }
@@ -612,7 +629,7 @@ int deep_ep_hip_launch_intranode_dispatch(const deep_ep_hip_intranode_dispatch_a
     pub.expert_start = reinterpret_cast<int32_t*>(ws + w.expert_start);
     pub.totals_out = reinterpret_cast<int32_t*>(ws + w.totals);
 
-    const LaunchPlan plan = plan_launches(T, K, E, R, do_layout, do_move, false, 1, a->payload, H, H * elem_in, a->tuning,
+    const LaunchPlan plan = plan_launches(T, K, E, R, do_layout, do_move, false, false, 1, a->payload, H, H * elem_in, a->tuning,
                                           with_topk ? -1 : a->recv_capacity);
     LayoutParams lay{};
     lay.topk_idx = a->topk_idx;

@@ -678,6 +678,36 @@ __device__ __forceinline__ bool warm_next_rounds_of_rows(const MoveParams& p, un
     return true;
 }
 
+// ---- alignment padding of the expanded layout ----
+//
+// The padding rows of an expert lie side by side, so its payload, its weights and, in every column (row), its scales are runs of zeros:
+// p.slices workgroups share an expert's evenly.  Workgroup `block` of E * slices; needs the finished layout.
+__device__ __forceinline__ void zero_padding_rows(const PadParams& p, const unsigned block) {
+    const int e = int(block / unsigned(p.slices)), slice = int(block) - e * p.slices;
+    const int cnt = p.num_unaligned[e];
+    const int64_t first = p.psum_expert[e];                  // start + actual count
+    const int n = int(min(int64_t((cnt + p.A - 1) / p.A * p.A - cnt), p.expanded_capacity - first));
+    if (n <= 0) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int64_t vecs = int64_t(n) * (p.out_row_bytes / 16);
+    const int64_t share = (vecs + int64_t(p.slices) * kThreads - 1) / (int64_t(p.slices) * kThreads) * kThreads;
+    const int64_t end = min((slice + 1) * share, vecs);
+    uint8_t* rows = p.recv_x + first * p.out_row_bytes;
+    const vec16 zero{0, 0, 0, 0};
+    for (int64_t i = slice * share + tid; i < end; i += kThreads) store16(rows + i * 16, zero);
+    if (p.recv_sf != nullptr && !p.sf_blocked) {
+        // a wavefront to a column, or to a row, whichever is contiguous
+        const bool columns = p.rsf_ts == 1;
+        const int outer = columns ? p.num_sf_packs : n, inner = columns ? n : p.num_sf_packs;
+        const int64_t os = columns ? p.rsf_hs : p.rsf_ts, is = columns ? p.rsf_ts : p.rsf_hs;
+        uint32_t* scales = p.recv_sf + first * p.rsf_ts;
+        for (int o = slice * kWavesPerBlock + (tid >> 6); o < outer; o += p.slices * kWavesPerBlock)
+            for (int i = lane; i < inner; i += kWaveSize) scales[o * os + i * is] = 0u;
+    }
+    if (p.recv_topk_weights != nullptr && slice == 0)
+        for (int i = tid; i < n; i += kThreads) p.recv_topk_weights[first + i] = 0.f;
+}
+
 // ---- pass-through payload (BF16, or FP8 with caller-provided scale packs) ----
 // kScales: rows may come with scale packs (p.recv_sf).
 enum : int { kNoScales = 0, kScalesInPlace = 1, kScalesInBlocks = 2 };
@@ -691,6 +721,12 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
         if (blockIdx.x <= unsigned(p.count_blocks)) {
             if (blockIdx.x < unsigned(p.count_blocks)) fused_count_block(p);
             else fused_publish_block(p);
+            return;
+        }
+    }
+    if constexpr (!kFused) {
+        if (blockIdx.x >= p.num_movers) {                   // behind the movers of a call that zeroes its padding
+            zero_padding_rows(p.pad, blockIdx.x - p.num_movers);
             return;
         }
     }
@@ -789,6 +825,12 @@ __device__ __forceinline__ void dispatch_cast(const MoveParams& p) {
         if (blockIdx.x <= unsigned(p.count_blocks)) {
             if (blockIdx.x < unsigned(p.count_blocks)) fused_count_block(p);
             else fused_publish_block(p);
+            return;
+        }
+    }
+    if constexpr (!kFused) {
+        if (blockIdx.x >= p.num_movers) {                   // behind the movers of a call that zeroes its padding
+            zero_padding_rows(p.pad, blockIdx.x - p.num_movers);
             return;
         }
     }
@@ -1162,7 +1204,7 @@ __device__ __forceinline__ void load_block(const PadParams& p, uint32_t* scales,
     }
 }
 
-// ---- zero the alignment padding rows of the expanded layout, and put scales that came in blocks into their columns ----
+// ---- put scales that came in blocks into their columns, and zero the padding rows behind a single launch ----
 // Workgroups [0, scale_blocks) turn a block each, those behind them zero rows.
 __global__ __launch_bounds__(kThreads) void zero_padding_kernel(const PadParams p, const int scale_blocks) {
     extern __shared__ uint32_t scales[];              // [kScaleBlockRows][G + 1]
@@ -1195,23 +1237,7 @@ __global__ __launch_bounds__(kThreads) void zero_padding_kernel(const PadParams 
         }
         return;
     }
-    const int lane = threadIdx.x & 63;
-    const int64_t work = int64_t(int(blockIdx.x) - scale_blocks) * kWavesPerBlock + (threadIdx.x >> 6);
-    const int pad_slots = p.A - 1;
-    if (work >= int64_t(p.E) * pad_slots) return;
-    const int e = int(work / pad_slots);
-    const int i = int(work - int64_t(e) * pad_slots);
-    const int cnt = p.num_unaligned[e];
-    const int aligned = (cnt + p.A - 1) / p.A * p.A;
-    if (i >= aligned - cnt) return;
-    const int64_t row = int64_t(p.psum_expert[e]) + i;      // start + actual count + i
-    if (row >= p.expanded_capacity) return;
-    uint8_t* dst = p.recv_x + row * p.out_row_bytes;
-    const vec16 zero{0, 0, 0, 0};
-    for (int off = lane * 16; off < p.out_row_bytes; off += kWaveSize * 16) store16(dst + off, zero);
-    if (p.recv_sf != nullptr && !p.sf_blocked)
-        for (int g = lane; g < p.num_sf_packs; g += kWaveSize) p.recv_sf[row * p.rsf_ts + int64_t(g) * p.rsf_hs] = 0u;
-    if (p.recv_topk_weights != nullptr && lane == 0) p.recv_topk_weights[row] = 0.f;
+    zero_padding_rows(p, blockIdx.x - unsigned(scale_blocks));
 }
 
 // ---- stand-alone per-token cast (identity routing) ----
@@ -1452,10 +1478,10 @@ size_t move_lds_bytes(const MoveParams& p) {
     return p.warm_lds_offset != 0 ? size_t(p.warm_lds_offset) + size_t(kWavesPerBlock) * 1024 : bytes;
 }
 
-// Grid: the counting workgroups of a single-launch dispatch come first.
+// Grid: the counting workgroups of a single-launch dispatch come first; those that zero padding rows last.
 unsigned move_grid(MoveParams& p, int64_t waves) {
     p.num_movers = unsigned((waves + kWavesPerBlock - 1) / kWavesPerBlock);
-    return p.num_movers + unsigned(p.fused ? p.count_blocks + 1 : 0);
+    return p.num_movers + (p.fused ? unsigned(p.count_blocks) + 1u : p.pad_blocks);
 }
 
 // Single launch: the movers that are resident at launch warm the caches for the round after next (warm_next_rounds).
@@ -1625,30 +1651,40 @@ hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream) {
     }
 }
 
-// From 850 K scales and 14000 rows on, padding rows, whose zeroes are single dwords too, counted double: what is saved is a partial line for
-// each of them, against the two trips to memory a block costs.  Layout, move and pad kernel in us, scales stored into their columns / in
-// blocks, fused cast, 8 ranks, top-k of experts, alignment: 8192 x 7168 8 of 256, 128 (5.5 M scales) 168.2 / 151.9; 2048 x 12288 4 of 64, 128
-// (1.6 M) 55.1 / 50.7; 512 x 7168 8 of 256, 128 (2.0 M) 67.9 / 61.7; 700 x 7168 8 of 128, 128 (1.2 M) 36.7 / 34.2; 3000 x 7168 6 of 64, 16 (1.1 M)
-// 50.1 / 49.4.  Short of scales: 1640 x 6272 9 of 32, 16 (0.75 M) 40.4 / 42.9; 2568 x 3968 8 of 64, 64 (0.76 M), move and pad 29.9 / 31.2; 4096 x
-// 4096 4 of 64, 64 (0.65 M) 38.0 / 38.2.  Short of rows: 3000 x 12288 4 of 32, 16 (12.5 K) 69.0 / 70.6; 4096 x 16384 2 of 32, 128 (12.3 K) 81.9 /
-// 82.2, and 79.9 / 83.3 with the input just written; 2000 x 16384 4 of 32, 64 (10 K) 56.0 / 59.5.
+// Scales stored into their columns are a partial line for every row that is moved; in blocks they cost a launch behind the move, which
+// otherwise zeroes the padding rows itself.  Layout, move and pad kernel in us, columns / blocks, alignment 128:
+//   cast         7564 x 5376 10 of 48 (76 K rows, 3.2 M scales) 131.4 / 122.3; 13983 x 3328 4 of 16 (56 K, 1.5 M) 76.4 / 73.3; 5754 x 5376 8 of 16
+//                (46 K, 1.9 M) 80.5 / 79.3; short of rows 4984 x 5760 8 of 64 (40 K, 1.8 M) 77.7 / 79.6; 2425 x 6144 10 of 32 (24 K, 1.2 M) 53.0 /
+//                58.3; short of scales 11586 x 1664 4 of 64 (46 K, 0.6 M) 40.8 / 42.4; 300 x 7168 8 of 256 (2.4 K) 41.1 / 46.9
+//   FP8 pairs    9468 x 6016 4 of 256 (38 K, 1.8 M) 104.4 / 99.3; 9219 x 6400 8 of 16 (74 K, 3.7 M) 138.6 / 133.0; 9043 x 5504 8 of 32 118.3 / 118.1;
+//                narrower rows, whose scales one wavefront has all of, 12085 x 4096 8 of 32 (97 K, 3.1 M) 109.5 / 113.5
+// Behind a single launch, where the padding rows take that launch too, padding counts: 3000 x 7168 cast 6 of 64, 16 (1.1 M) 50.1 / 49.4; 700 x 7168
+// 8 of 128, 128 (1.2 M) 36.7 / 34.2; short of scales 2568 x 3968 8 of 64, 64 (0.76 M), move and pad 29.9 / 31.2; 4096 x 4096 4 of 64, 64 (0.65 M) 38.0 /
+// 38.2; short of rows 2000 x 16384 4 of 32, 64 (10 K) 56.0 / 59.5.
 bool scales_in_blocks(const MoveParams& m, int alignment) {
-    constexpr int64_t kFromScales = 850000, kFromRows = 14000;
-    const int64_t rows = int64_t(m.T) * m.K + int64_t(m.E) * (alignment - 1);
-    const bool tile_known = m.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? m.cast_pairs >= 0 && m.cast_pairs <= 2
-                                                                      : m.copy_vecs >= 0 && m.copy_vecs <= 4 && m.copy_vecs != 3;
-    return m.do_expand && alignment > 1 && m.payload != DEEP_EP_HIP_PAYLOAD_BF16 && m.recv_sf != nullptr && m.rsf_ts == 1 &&
-           m.rsf_hs >= m.expanded_capacity && m.num_sf_packs >= 2 && m.num_sf_packs <= kMaxBlockedScales && tile_known &&
-           rows * m.num_sf_packs >= kFromScales && rows >= kFromRows;
+    const bool cast = m.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8;
+    const bool tile_known = cast ? m.cast_pairs >= 0 && m.cast_pairs <= 2 : m.copy_vecs >= 0 && m.copy_vecs <= 4 && m.copy_vecs != 3;
+    if (!m.do_expand || alignment <= 1 || m.payload == DEEP_EP_HIP_PAYLOAD_BF16 || m.recv_sf == nullptr || m.rsf_ts != 1 ||
+        m.rsf_hs < m.expanded_capacity || m.num_sf_packs < 2 || m.num_sf_packs > kMaxBlockedScales || !tile_known)
+        return false;
+    const int64_t moved = int64_t(m.T) * m.K, rows = moved + int64_t(m.E) * (alignment - 1);
+    if (m.fused) return rows * m.num_sf_packs >= 850000 && rows >= 14000;
+    if (cast) return moved * m.num_sf_packs >= 1200000 && moved >= 44000;
+    return moved * m.num_sf_packs >= 1700000 && moved >= 36000 && m.num_sf_packs > 40;
 }
 
-hipError_t launch_zero_padding(const PadParams& p, hipStream_t stream) {
-    if (p.A <= 1 || p.E == 0) return hipSuccess;
-    const int64_t waves = int64_t(p.E) * (p.A - 1);
-    const unsigned blocks = unsigned((waves + kWavesPerBlock - 1) / kWavesPerBlock);
+// 32 KB of an expert's largest padding to a workgroup, and no more than about 4096 of them.
+int pad_slices(int experts, int alignment, int out_row_bytes) {
+    const int64_t wanted = (int64_t(alignment - 1) * out_row_bytes + 32767) / 32768;
+    return int(std::max<int64_t>(std::min<int64_t>(wanted, 4096 / experts), 1));
+}
+
+hipError_t launch_zero_padding(const PadParams& p, bool rows, hipStream_t stream) {
+    const unsigned row_blocks = rows ? unsigned(p.E) * unsigned(p.slices) : 0u;
     const int scale_blocks = p.sf_blocked ? int((p.expanded_capacity + kScaleBlockRows - 1) / kScaleBlockRows) : 0;
+    if (row_blocks + unsigned(scale_blocks) == 0) return hipSuccess;
     const size_t lds = p.sf_blocked ? size_t(kScaleBlockRows) * (p.num_sf_packs + 1) * sizeof(uint32_t) : 0;
-    hipLaunchKernelGGL(zero_padding_kernel, dim3(blocks + unsigned(scale_blocks)), dim3(kThreads), lds, stream, p, scale_blocks);
+    hipLaunchKernelGGL(zero_padding_kernel, dim3(row_blocks + unsigned(scale_blocks)), dim3(kThreads), lds, stream, p, scale_blocks);
     return hipGetLastError();
 }
 

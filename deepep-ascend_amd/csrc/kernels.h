@@ -131,6 +131,23 @@ struct IntranodePrefixParams {
 hipError_t launch_layout_kernel(const LayoutParams& p, const IntranodePrefixParams& prefix, hipStream_t stream);
 hipError_t launch_intranode_prefix(const IntranodePrefixParams& p, hipStream_t stream);
 
+// Alignment padding of an expanded layout: the rows behind the actual ones of every expert.
+struct PadParams {
+    uint8_t* recv_x;
+    uint32_t* recv_sf;
+    int64_t rsf_ts, rsf_hs;
+    int num_sf_packs;
+    float* recv_topk_weights;
+    const int32_t* psum_expert;     // start + actual count (expanded convention)
+    const int32_t* num_unaligned;
+    int64_t expanded_capacity;
+    int E, A, out_row_bytes;
+    int sf_blocked;                  // recv_sf is in blocks: turned by zero_padding_kernel
+    int slices;                      // workgroups that share the padding of an expert (pad_slices)
+};
+
+int pad_slices(int experts, int alignment, int out_row_bytes);
+
 struct MoveParams {
     const uint8_t* x;
     const uint32_t* sf;
@@ -158,7 +175,7 @@ struct MoveParams {
     int row_bytes;       // input row bytes
     int tiles;           // column tiles per token
     int sf_blocked;      // recv_sf is column-major and the pad kernel follows: scales go out in blocks (below)
-    int zeroed_rows;     // rows the pad kernel behind this one zeroes, as expected: half an alignment for each expert, or what is
+    int zeroed_rows;     // padding rows this call zeroes, as expected: half an alignment for each expert, or what is
                          // left of one alignment for each where an expert has fewer rows than that
     int row_by_row;      // a wavefront waits for the stores of a row before it starts the next (set by the launcher)
     unsigned warm_lds_offset;   // single-launch cast: byte offset (in the dynamic LDS) of the 4 KB landing area of the
@@ -197,25 +214,15 @@ struct MoveParams {
     int zero_nonlocal_w;     // weights of lanes routed to another rank are delivered as 0
     int32_t* send_head;      // [T, R] out: receive row of token t on rank r, or -1
     int32_t* recv_src_idx;   // [recv_capacity] out: source token of each receive row
+    // A move on a finished layout zeroes the padding too: pad_blocks workgroups behind the movers, 0 = not wanted
+    unsigned pad_blocks;
+    PadParams pad;
 };
 
 hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream);
 // A call for which the layout kernel and a move of its own are faster than one launch (p.T, p.H, p.row_bytes, p.payload, the
 // routing shape and the tile overrides set, p.fused = 1).
 bool move_prefers_finished_layout(const MoveParams& p, int count_blocks);
-
-struct PadParams {
-    uint8_t* recv_x;
-    uint32_t* recv_sf;
-    int64_t rsf_ts, rsf_hs;
-    int num_sf_packs;
-    float* recv_topk_weights;
-    const int32_t* psum_expert;     // start + actual count (expanded convention)
-    const int32_t* num_unaligned;
-    int64_t expanded_capacity;
-    int E, A, out_row_bytes;
-    int sf_blocked;                  // recv_sf is in blocks: turned here
-};
 
 // Column-major scales of an expanded dispatch on their way.  A row's scales belong into as many columns as it has scales, a
 // dword each, 128 bytes of a column being the work of 32 rows that are moved far apart in time and by different XCDs: every
@@ -227,7 +234,8 @@ constexpr int kMaxBlockedScales = 128;     // scales of a row: the pad kernel tu
 
 bool scales_in_blocks(const MoveParams& m, int alignment);
 
-hipError_t launch_zero_padding(const PadParams& p, hipStream_t stream);
+// What the move has left to do: blocked scales, and the padding rows if `rows`.
+hipError_t launch_zero_padding(const PadParams& p, bool rows, hipStream_t stream);
 
 // V1 (intranode) handle bookkeeping computed from is_token_in_rank, and the -1 fill of unused recv_topk_idx rows.
 struct FillTailParams {
