@@ -154,6 +154,24 @@ __device__ __forceinline__ vec16 buffer_load16_as(__amdgpu_buffer_rsrc_t from, i
     return vec16{v.x, v.y, v.z, v.w};
 }
 
+// One or two 32-bit words; stores past the end are dropped.
+template <typename Words>
+__device__ __forceinline__ Words buffer_load_words(__amdgpu_buffer_rsrc_t from, uint32_t offset) {
+    if constexpr (sizeof(Words) == 4) {
+        return __builtin_amdgcn_raw_buffer_load_b32(from, int(offset), 0, 0);
+    } else {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b64(from, int(offset), 0, 0);
+        return Words{v[0], v[1]};
+    }
+}
+__device__ __forceinline__ void buffer_store_words(__amdgpu_buffer_rsrc_t to, uint32_t offset, uint32_t v) {
+    __builtin_amdgcn_raw_buffer_store_b32(v, to, int(offset), 0, 0);
+}
+__device__ __forceinline__ void buffer_store_words(__amdgpu_buffer_rsrc_t to, uint32_t offset, const uint2& v) {
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{v.x, v.y}, to, int(offset), 0, 0);
+}
+
 // Inclusive prefix sum across the wave, as DPP operand modifiers: inside each row of 16 lanes by shifts of 1, 2, 4 and 8,
 // then the last lane of row 0 / 2 into row 1 / 3 and lane 31 into the upper half (bpermutes through LDS, as a shuffle
 // compiles to, took six dependent trips).  All lanes of the wavefront must be active.

@@ -103,6 +103,7 @@ struct LayoutParams {
     const uint8_t* route_mask;       // [T, R] bool: when set, lane r of token t is "rank r, if the mask says so" (K = E = R)
     int T, K, E, R, E_l;
     int vec_idx;          // topk_idx is 16-byte aligned (set by the launcher)
+    int lds_totals;       // layout kernel of one workgroup: where its totals lie in LDS, bytes (set by the launcher)
     uint8_t* is_token_in_rank;       // optional
     int64_t* copied_topk_idx;        // optional
     PublishParams pub;

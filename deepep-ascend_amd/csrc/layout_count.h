@@ -18,6 +18,12 @@
 
 namespace deep_ep_hip {
 
+// With few ranks most lanes of a wavefront would meet on the same few rank words, so the rank bitmaps are taken by
+// ballot instead: one per rank over "this token goes to rank r", no atomics.  Past 16 ranks the ballots cost more than the
+// atomics (layout launch of 4096 tokens, top-8: 24 ranks 8.2 us by ballot and 7.7 by atomics, 32 ranks 8.7 and 7.8, 64 ranks
+// 9.9 and 7.8; 4096 x 2048 fused cast in one launch over 64 ranks 28.5 and 24.2).
+constexpr int kBallotRanks = 16;
+
 static_assert(kLayoutChunk == 4 * kWaveSize, "the packed before-wave word holds three fields");
 
 // LDS the counting step needs: the bitmap words [(R + E)][4] and one packed word per bucket (see below).
@@ -25,15 +31,12 @@ __host__ __device__ inline size_t count_lds_bytes(int R, int E) {
     return size_t(R + E) * (kLayoutChunk / kWaveSize) * sizeof(uint64_t) + size_t(R + E) * sizeof(uint32_t);
 }
 
+// The counting step of a single launch's front workgroups, which share the registers of its movers.
 // bitmap: LDS of count_lds_bytes(R, E) bytes.  Must be called by all 256 threads of the workgroup.
-// kThrough: positions are stored at agent scope (workgroups of the same launch read them) and carry, like the copy of
-// the rank totals in p.tagged_rank, the launch's tag.  Chunk totals always go out at agent scope, to the count tables,
-// unless `lds_totals` is given: then the call's only chunk leaves them there ([R + E]).
-// hand_off() is called by all threads once the totals and the flags are on their way and before the positions are
-// stored: whoever waits for the totals does not wait for those.
-template <int KMAX, bool kThrough, typename HandOff>
-__device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chunk, const int num_chunks, uint64_t* bitmap,
-                                            int* lds_totals, HandOff hand_off) {
+// Positions are stored at agent scope (movers of the same launch read them) and carry, like the copy of the rank totals in
+// p.tagged_rank, the launch's tag; chunk totals go out at agent scope, to the count tables.
+template <int KMAX>
+__device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chunk, const int num_chunks, uint64_t* bitmap) {
     constexpr int kThreads = kLayoutChunk;
     constexpr int kWaves = kThreads / kWaveSize;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -41,8 +44,7 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
     const int n = p.R + p.E;
     const bool active = t < p.T;
     uint32_t tag = 0;
-    if constexpr (kThrough)
-        if (p.generation != nullptr) tag = (*p.generation + 1u) << kTagShift;     // constant while the launch reads it
+    if (p.generation != nullptr) tag = (*p.generation + 1u) << kTagShift;     // constant while the launch reads it
 
     // The index loads go out first (they are the longest wait of the pass), before anything that could alias
     // them is stored; the bitmap is cleared while they are in flight.
@@ -67,18 +69,8 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
             for (int k = 0; k < KMAX; ++k) raw[k] = -1;
         }
     } else {
-        // Clamped columns instead of a branch around each load: all of a token's loads go out together.  Not beside movers,
-        // whose payload the loads of absent lanes would wait with.
 #pragma unroll
-        for (int k = 0; k < KMAX; ++k) raw[k] = kThrough && active && k < p.K ? p.topk_idx[int64_t(t) * p.K + k] : int64_t(-1);
-        if (!kThrough && active) {
-            const int64_t* row = p.topk_idx + int64_t(t) * p.K;
-#pragma unroll
-            for (int k = 0; k < KMAX; ++k) raw[k] = row[min(k, p.K - 1)];
-#pragma unroll
-            for (int k = 0; k < KMAX; ++k)
-                if (k >= p.K) raw[k] = -1;
-        }
+        for (int k = 0; k < KMAX; ++k) raw[k] = active && k < p.K ? p.topk_idx[int64_t(t) * p.K + k] : int64_t(-1);
     }
 
     for (int i = tid; i < n * kWaves; i += kThreads) bitmap[i] = 0ull;
@@ -87,14 +79,8 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
     // Straight-line code from here on, no branch per routing lane: the LDS atomics of all lanes issue back to back, and
     // so do the LDS reads of the position step further down.  A lane without an expert ORs nothing into a word of its
     // own (not one word for all of them: atomics of one wavefront on one address take turns).
-    // With few ranks most lanes of a wavefront would meet on the same few rank words, so the rank bitmaps are taken by
-    // ballot instead: one per rank over "this token goes to rank r", no atomics.  Past 16 ranks the ballots cost more than the
-    // atomics (layout launch of 4096 tokens, top-8: 24 ranks 8.2 us by ballot and 7.7 by atomics, 32 ranks 8.7 and 7.8, 64 ranks
-    // 9.9 and 7.8; 4096 x 2048 fused cast in one launch over 64 ranks 28.5 and 24.2).
-    constexpr int kBallotRanks = 16;
     const bool ranks_by_ballot = p.R <= kBallotRanks;
     int e[KMAX], d[KMAX];
-    unsigned long long seen = 0;
     int flags = 0;
     const float rcp_experts_per_rank = 1.0f / float(p.E_l);
     const uint64_t my_bit = 1ull << lane;
@@ -108,8 +94,7 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
         d[k] = valid ? small_div(e[k], rcp_experts_per_rank) : -1;
         const uint64_t bit = valid ? my_bit : 0ull;
         unsigned long long* word = reinterpret_cast<unsigned long long*>(&bitmap[valid ? (p.R + e[k]) * kWaves + wave : idle_word]);
-        if constexpr (kThrough) atomicOr(word, bit);          // see the pairwise comparison below
-        else seen |= atomicOr(word, bit) & bit;              // a bit that is set already: the token names the expert twice
+        atomicOr(word, bit);
         if (valid) my_ranks |= 1ull << (d[k] & 63);            // used when num_ranks <= kBallotRanks
     }
     if (ranks_by_ballot) {
@@ -125,15 +110,11 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
             atomicOr(reinterpret_cast<unsigned long long*>(&bitmap[d[k] >= 0 ? d[k] * kWaves + wave : idle_word]),
                      d[k] >= 0 ? my_bit : 0ull);
     }
-    // The caller's copy of the indices: behind the hand-off, unless the registers they would occupy until then are scarce
-    // (the counting workgroups of a single launch are held to those of its movers).
-    auto copy_indices = [&] {
-        if (p.copied_topk_idx == nullptr || !active) return;
+    if (p.copied_topk_idx != nullptr && active) {             // now: the registers are scarce
 #pragma unroll
         for (int k = 0; k < KMAX; ++k)
             if (k < p.K) p.copied_topk_idx[int64_t(t) * p.K + k] = raw[k];
-    };
-    if constexpr (kThrough) copy_indices();
+    }
     __syncthreads();
 
     // Per bucket: the chunk total goes out and the bits set by the wavefronts before each wavefront are packed into one LDS word (three 10-bit fields),
@@ -143,28 +124,21 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
         const int c0 = __popcll(bitmap[j * kWaves]), c1 = __popcll(bitmap[j * kWaves + 1]);
         const int c2 = __popcll(bitmap[j * kWaves + 2]), c3 = __popcll(bitmap[j * kWaves + 3]);
         before_wave[j] = uint32_t(c0) | (uint32_t(c0 + c1) << 10) | (uint32_t(c0 + c1 + c2) << 20);
-        if (!kThrough && lds_totals != nullptr) {
-            lds_totals[j] = c0 + c1 + c2 + c3;
-            continue;
-        }
         int32_t* at = j < p.R ? p.tab.rank_counts + int64_t(j) * p.tab.chunks_padded + chunk
                               : p.tab.expert_counts + int64_t(chunk) * p.tab.experts_padded + (j - p.R);
         store_agent(at, c0 + c1 + c2 + c3);
-        if constexpr (kThrough) {
-            if (j < p.R && p.tagged_rank != nullptr)
-                store_agent(reinterpret_cast<int*>(p.tagged_rank) + j * p.tab.chunks_padded + chunk, int(uint32_t(c0 + c1 + c2 + c3) | tag));
-            if (j >= p.R && p.tagged_expert_counts != nullptr)
-                store_agent(reinterpret_cast<int*>(p.tagged_expert_counts) + chunk * p.tab.experts_padded + (j - p.R),
-                            int(uint32_t(c0 + c1 + c2 + c3) | tag));
-        }
+        if (j < p.R && p.tagged_rank != nullptr)
+            store_agent(reinterpret_cast<int*>(p.tagged_rank) + j * p.tab.chunks_padded + chunk, int(uint32_t(c0 + c1 + c2 + c3) | tag));
+        if (j >= p.R && p.tagged_expert_counts != nullptr)
+            store_agent(reinterpret_cast<int*>(p.tagged_expert_counts) + chunk * p.tab.experts_padded + (j - p.R),
+                        int(uint32_t(c0 + c1 + c2 + c3) | tag));
     }
     const int pad = p.tab.chunks_padded - num_chunks;  // the padding columns of the rank table are cleared by the first workgroup
-    if (chunk == 0 && lds_totals == nullptr) {
+    if (chunk == 0) {
         for (int i = tid; i < p.R * pad; i += kThreads) {
             const int at = (i / pad) * p.tab.chunks_padded + num_chunks + i % pad;
             store_agent(p.tab.rank_counts + at, 0);
-            if constexpr (kThrough)
-                if (p.tagged_rank != nullptr) store_agent(reinterpret_cast<int*>(p.tagged_rank) + at, int(tag));
+            if (p.tagged_rank != nullptr) store_agent(reinterpret_cast<int*>(p.tagged_rank) + at, int(tag));
         }
     }
     __syncthreads();
@@ -211,11 +185,10 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
         }
 #pragma unroll
         for (int k = 0; k < KMAX; ++k) {
-            if constexpr (kThrough) {      // a mover's register budget does not hold eight answers of the LDS: compared pairwise
+            // a mover's register budget does not hold eight answers of the LDS: compared pairwise
 #pragma unroll
-                for (int j = k + 1; j < KMAX; ++j)
-                    if (e[k] >= 0 && e[j] == e[k]) flags |= DEEP_EP_HIP_STATUS_DUPLICATE_EXPERT;
-            }
+            for (int j = k + 1; j < KMAX; ++j)
+                if (e[k] >= 0 && e[j] == e[k]) flags |= DEEP_EP_HIP_STATUS_DUPLICATE_EXPERT;
             packed[k] = (master[k] ? position(word_r[k], before_r[k]) : kNoPosition) | tag;
         }
         if (p.expert_bases) {                         // only the expanded layout places rows by expert
@@ -233,35 +206,20 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
             for (int k = 0; k < KMAX; ++k) packed[k] |= kNoPosition << kExpertPositionShift;
         }
     }
-    if (p.pos != nullptr && seen != 0) flags |= DEEP_EP_HIP_STATUS_DUPLICATE_EXPERT;
 
-    auto store_positions = [&] {
-        if (!active || p.pos == nullptr) return;
+    if (active && p.pos != nullptr) {                        // movers of this launch are waiting for them
         if (KMAX == 8 && p.K == 8) {
             vec16* dst = reinterpret_cast<vec16*>(p.pos + int64_t(t) * 8);
-            const vec16 lo{packed[0], packed[1], packed[2], packed[3]}, hi{packed[4], packed[5], packed[6], packed[7]};
-            if constexpr (kThrough) {
-                store16_agent(dst, lo);
-                store16_agent(dst + 1, hi);
-            } else {
-                dst[0] = lo;
-                dst[1] = hi;
-            }
+            store16_agent(dst, vec16{packed[0], packed[1], packed[2], packed[3]});
+            store16_agent(dst + 1, vec16{packed[4], packed[5], packed[6], packed[7]});
         } else {
 #pragma unroll
             for (int k = 0; k < KMAX; ++k)
-                if (k < p.K) store_word<kThrough>(reinterpret_cast<int*>(p.pos) + int64_t(t) * p.K + k, int(packed[k]));
+                if (k < p.K) store_agent(reinterpret_cast<int*>(p.pos) + int64_t(t) * p.K + k, int(packed[k]));
         }
-    };
-    if constexpr (kThrough) store_positions();           // movers of this launch are waiting for them
+    }
     if (flags != 0) atomicOr(p.status, flags);
 
-    hand_off();
-
-    if constexpr (!kThrough) {
-        store_positions();
-        copy_indices();
-    }
     if (active && p.is_token_in_rank != nullptr) {
         for (int r = 0; r < p.R; ++r)
             p.is_token_in_rank[int64_t(t) * p.R + r] = uint8_t((bitmap[r * kWaves + wave] >> lane) & 1ull);

@@ -4,6 +4,8 @@
 // deep_ep/include/deep_ep/impls/dispatch.cuh:200-257 publish.
 #pragma once
 
+#include <type_traits>
+
 #include "device_utils.h"
 #include "kernels.h"
 
@@ -286,8 +288,8 @@ __device__ bool write_expert_bases_from_registers(const LayoutTables& t, const u
 // own on the critical path of every call: what it costs is the chain of barriers, LDS trips and instruction fetches, so
 // there is one trip to memory (every thread first loads all it needs: up to 16 consecutive entries of the flattened rank
 // table and its experts' columns of chunk totals, of which 32 stay in registers), one pair of prefix sums, taken
-// together, and two barriers; outputs go out from registers.  kOneChunk: `totals` ([R + E], LDS) holds the only
-// chunk's totals and nothing is loaded.  scratch: LDS of publish_scratch_ints.
+// together, and two barriers; outputs go out from registers.  kHeldChunks > 0: `totals` ([R + E][kHeldChunks], LDS) holds all
+// chunks' totals and nothing is loaded.  scratch: LDS of publish_scratch_ints.
 // From the ticket to the end it took 3.4 us at 16 chunks, 9 us at 64 chunks over 32 ranks, with LDS scans of five
 // barriers and 32 chunks at most; the whole launch went from 10.0 to 8.3 and from 14.8 to 11.5 us.
 // Chunks past the 32 in registers are read again for the expert bases, sixteen a trip: one at a time, each load behind the store
@@ -301,62 +303,79 @@ inline bool fits_one_trip(int per_thread, int R, int E, int chunks_padded, int t
 
 inline __host__ __device__ int publish_scratch_ints(int R, int threads) { return R + 2 * (threads / kWaveSize); }
 
-template <int kThreads, bool kOneChunk, int kPerThread>
+template <int kThreads, int kHeldChunks, int kPerThread>
 __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutTables& t, int num_chunks, bool expert_bases,
                                            int* totals, int* scratch) {
     constexpr int kWavesHere = kThreads / kWaveSize;
-    constexpr int kMaxVecs = kOneChunk ? 1 : 4, kColumn = kOneChunk ? 1 : 32 / kPerThread;
+    static_assert(kHeldChunks <= 4 && (kPerThread == 1 || kHeldChunks <= 1), "rows of four chunks; for_host lies over the totals");
+    constexpr bool kHeld = kHeldChunks > 0;
+    constexpr int kMaxVecs = kHeld ? 1 : 4, kColumn = kHeld ? kHeldChunks : 32 / kPerThread;
     int* rank_end = scratch;                             // [R] inclusive prefix sum over the ranks
     int* wave_sums = scratch + q.R;                      // [2][kWavesHere]
     // kPerThread > 1: [E] what the mailbox gets, of which a thread writes the entries it has read the totals from
-    int* for_host = kOneChunk ? totals + q.R : scratch + publish_scratch_ints(q.R, kThreads);
+    int* for_host = kHeld ? totals + q.R : scratch + publish_scratch_ints(q.R, kThreads);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int first_expert = tid * kPerThread;
     const bool has_expert = first_expert < q.E;
     const int status = status_for_host(q);
     const int flat = q.R * t.chunks_padded;              // a multiple of 4: four entries share a row
-    const int vecs = kOneChunk ? 1 : (flat + 4 * kThreads - 1) / (4 * kThreads);
+    const int vecs = kHeld ? 1 : (flat + 4 * kThreads - 1) / (4 * kThreads);
     // The thread's experts of a chunk: columns the table pads with (experts_padded is a multiple of 32) come along and count nothing.
-    struct alignas(4 * kPerThread) Columns { int of[kPerThread]; };
+    // Tables are read and written through descriptors that end with them: chunks there are none of count zero and are not stored, with no
+    // test and no address for each (a wavefront here has its SIMD to itself: every instruction counts).
+    using Columns = std::conditional_t<kPerThread == 1, uint32_t, uint2>;
+    const auto of = [](auto& columns, int j) -> uint32_t& { return reinterpret_cast<uint32_t*>(&columns)[j]; };
+    const uint32_t row_bytes = uint32_t(t.experts_padded) * 4u, my_columns = uint32_t(has_expert ? first_expert : 0) * 4u;
+    const auto expert_counts = buffer_of(reinterpret_cast<const uint8_t*>(t.expert_counts), kHeld ? 0 : num_chunks * int(row_bytes));
     vec16 rv[kMaxVecs];
     Columns v[kColumn];
     int rows = 0, count[kPerThread] = {};
-    const int column = has_expert ? first_expert : 0;
-    auto load_sixteen = [&](int first, Columns* to) {
+    auto load_rows = [&](int first, auto& to, int from, int n) {
+        uint32_t at = uint32_t(first) * row_bytes + my_columns;
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            // a row start common to the workgroup plus the thread's column: one address register serves all loads
-            const int row_start = __builtin_amdgcn_readfirstlane(min(first + u, num_chunks - 1) * t.experts_padded);
-            to[u] = *reinterpret_cast<const Columns*>(t.expert_counts + row_start + column);
-        }
+        for (int u = 0; u < 16; ++u, at += row_bytes)
+            if (u < n) to[from + u] = buffer_load_words<Columns>(expert_counts, at);
     };
-    if constexpr (kOneChunk) {
-        rv[0] = vec16{tid < q.R ? uint32_t(totals[tid]) : 0u, 0, 0, 0};          // rows of four, three of them padding
+    if constexpr (kHeld) {
+        const auto total = [&](int bucket, int chunk, bool there) { return there && chunk < kHeldChunks ? totals[bucket * kHeldChunks + min(chunk, kHeldChunks - 1)] : 0; };
+        const bool has_rank = tid < q.R;                 // rows of four, some of them padding
+        rv[0] = vec16{uint32_t(total(tid, 0, has_rank)), uint32_t(total(tid, 1, has_rank)), uint32_t(total(tid, 2, has_rank)), uint32_t(total(tid, 3, has_rank))};
 #pragma unroll
-        for (int j = 0; j < kPerThread; ++j) v[0].of[j] = count[j] = first_expert + j < q.E ? totals[q.R + first_expert + j] : 0;
-        rows = int(rv[0].x);
+        for (int c = 0; c < kHeldChunks; ++c)
+#pragma unroll
+            for (int j = 0; j < kPerThread; ++j) {
+                of(v[c], j) = uint32_t(total(q.R + first_expert + j, c, first_expert + j < q.E));
+                count[j] += int(of(v[c], j));
+            }
+        rows = int(rv[0].x) + int(rv[0].y) + int(rv[0].z) + int(rv[0].w);
     } else {
+        const auto rank_counts = buffer_of(reinterpret_cast<const uint8_t*>(t.rank_counts), flat * 4);
 #pragma unroll
         for (int i = 0; i < kMaxVecs; ++i) {
             rv[i] = vec16{0, 0, 0, 0};
-            const int begin = (tid * vecs + i) * 4;
-            if (i < vecs && begin < flat) rv[i] = load16(t.rank_counts + begin);
+            if (i < vecs) rv[i] = buffer_load16_as<false>(rank_counts, (tid * vecs + i) * 16);
         }
-        auto sum_sixteen = [&](int first, const Columns* of) {
+        auto sum_rows = [&](auto& of_chunks, int n) {
 #pragma unroll
-            for (int u = 0; u < 16; ++u)
+            for (int u = 0; u < n; ++u)
 #pragma unroll
-                for (int j = 0; j < kPerThread; ++j) count[j] += first + u < num_chunks ? of[u].of[j] : 0;
+                for (int j = 0; j < kPerThread; ++j) count[j] += int(of(of_chunks[u], j));
         };
-        load_sixteen(0, v);
-        if (kColumn > 16 && num_chunks > 16) load_sixteen(16, v + (kColumn - 16));
+#pragma unroll
+        for (int c0 = 0; c0 < kColumn; c0 += 8) {
+            if (c0 < num_chunks) {
+                load_rows(c0, v, c0, 8);
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[c0 + u] = Columns{};
+            }
+        }
         for (int c0 = kColumn; c0 < num_chunks; c0 += 16) {
             Columns w[16];
-            load_sixteen(c0, w);
-            sum_sixteen(c0, w);
+            load_rows(c0, w, 0, 16);
+            sum_rows(w, 16);
         }
-        sum_sixteen(0, v);
-        if (kColumn > 16 && num_chunks > 16) sum_sixteen(16, v + (kColumn - 16));
+        sum_rows(v, kColumn);
 #pragma unroll
         for (int i = 0; i < kMaxVecs; ++i) rows += int(rv[i].x) + int(rv[i].y) + int(rv[i].z) + int(rv[i].w);
     }
@@ -382,7 +401,7 @@ __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutT
     }
     Columns base;                                        // the region of an expert starts at the aligned rows of those before it
 #pragma unroll
-    for (int j = 0, at = start; j < kPerThread; at += aligned[j], ++j) base.of[j] = at;
+    for (int j = 0, at = start; j < kPerThread; at += aligned[j], ++j) of(base, j) = uint32_t(at);
 
 #pragma unroll
     for (int j = 0; j < kPerThread; ++j) {
@@ -393,9 +412,9 @@ __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutT
         if (q.num_tokens_per_expert != nullptr) q.num_tokens_per_expert[e] = count[j];
         if (q.num_unaligned != nullptr) q.num_unaligned[e] = count[j];
         if (q.cumulative_stats != nullptr) q.cumulative_stats[e] += count[j];
-        if (q.expert_start != nullptr) q.expert_start[e] = base.of[j];
-        if (q.psum_expert != nullptr) q.psum_expert[e] = q.do_expand ? base.of[j] + count[j] : base.of[j] + aligned[j];
-        if (e == q.E - 1 && q.totals_out != nullptr) q.totals_out[1] = base.of[j] + aligned[j];
+        if (q.expert_start != nullptr) q.expert_start[e] = int(of(base, j));
+        if (q.psum_expert != nullptr) q.psum_expert[e] = q.do_expand ? int(of(base, j)) + count[j] : int(of(base, j)) + aligned[j];
+        if (e == q.E - 1 && q.totals_out != nullptr) q.totals_out[1] = int(of(base, j)) + aligned[j];
     }
     // ranks: the exclusive prefix over the flattened table is the first compact row of every (rank, chunk)
     const float rcp_row = 1.0f / float(t.chunks_padded);
@@ -425,21 +444,29 @@ __device__ void publish_layout_in_one_trip(const PublishParams& q, const LayoutT
     if (tid == 0 && q.host_counts != nullptr) store_system(q.host_counts + q.R + q.E, -status - 1);
 
     if (t.expert_bases != nullptr && expert_bases && has_expert) {
-        auto store_base = [&](int chunk, const Columns& counts) {
-            *reinterpret_cast<Columns*>(t.expert_bases + __builtin_amdgcn_readfirstlane(chunk * t.experts_padded) + first_expert) = base;
+        const auto table = buffer_of(reinterpret_cast<const uint8_t*>(t.expert_bases), num_chunks * int(row_bytes));
+        uint32_t at = my_columns;
+        auto store_base = [&](Columns& counts) {
+            buffer_store_words(table, at, base);
+            at += row_bytes;
 #pragma unroll
-            for (int j = 0; j < kPerThread; ++j) base.of[j] += counts.of[j];
+            for (int j = 0; j < kPerThread; ++j) of(base, j) += of(counts, j);
         };
+        if constexpr (kHeld) {
 #pragma unroll
-        for (int u = 0; u < kColumn; ++u)
-            if (u < num_chunks) store_base(u, v[u]);
-        if constexpr (!kOneChunk) {
+            for (int u = 0; u < kColumn; ++u) store_base(v[u]);
+        } else {
+#pragma unroll
+            for (int c0 = 0; c0 < kColumn; c0 += 8) {
+                if (c0 >= num_chunks) break;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) store_base(v[c0 + u]);
+            }
             for (int c0 = kColumn; c0 < num_chunks; c0 += 16) {
                 Columns w[16];
-                load_sixteen(c0, w);
+                load_rows(c0, w, 0, 16);
 #pragma unroll
-                for (int u = 0; u < 16; ++u)
-                    if (c0 + u < num_chunks) store_base(c0 + u, w[u]);
+                for (int u = 0; u < 16; ++u) store_base(w[u]);
             }
         }
     }
