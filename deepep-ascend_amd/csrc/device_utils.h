@@ -154,6 +154,12 @@ __device__ __forceinline__ vec16 buffer_load16_as(__amdgpu_buffer_rsrc_t from, i
     return vec16{v.x, v.y, v.z, v.w};
 }
 
+template <bool kStream>
+__device__ __forceinline__ void buffer_store16_as(__amdgpu_buffer_rsrc_t to, int offset, const vec16& v) {
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(u32x4{v.x, v.y, v.z, v.w}, to, offset, 0, kStream ? 2 /* nt */ : 0);
+}
+
 // One or two 32-bit words; stores past the end are dropped.
 template <typename Words>
 __device__ __forceinline__ Words buffer_load_words(__amdgpu_buffer_rsrc_t from, uint32_t offset) {

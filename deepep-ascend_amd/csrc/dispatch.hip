@@ -157,11 +157,13 @@ __device__ __forceinline__ Route resolve_route(const MoveParams& p, const RouteI
         if (lane < p.R) p.send_head[int64_t(t) * p.R + lane] = row_on_rank;
     }
 
-    // Every valid lane learns the compact row of its destination rank from that rank's master lane.
-    for (int j = 0; j < p.K; ++j) {
-        const int dj = read_lane(r.d, j);
-        const int rj = read_lane(r.row_c, j);
-        if (r.d >= 0 && dj == r.d && rj >= 0) r.my_row = rj;
+    // Expanded rows of a cached handle are named by the rank's compact row: every valid lane learns it from the master lane.
+    if (p.do_expand && p.cached) {
+        for (int j = 0; j < p.K; ++j) {
+            const int dj = read_lane(r.d, j);
+            const int rj = read_lane(r.row_c, j);
+            if (r.d >= 0 && dj == r.d && rj >= 0) r.my_row = rj;
+        }
     }
     if (p.do_expand && r.e >= 0) {
         if (p.cached) {
@@ -178,49 +180,58 @@ __device__ __forceinline__ Route resolve_route(const MoveParams& p, const RouteI
 
 // Token-level metadata, written once per token (by the wave that owns column tile 0).
 //
-// Compact layout with K <= 15: a destination row's recv_topk_idx (2 dwords per lane), recv_topk_weights and
-// recv_src_metadata entries go out in ONE dword store instruction: wave lanes take the roles
-//   [0, 2K) index dwords | [2K, 3K) weights | [3K, 4K + 2) metadata columns,
-// each role reading the routing lane it needs through a shuffle done once per token.
+// What a destination row gets besides its payload goes out in ONE dword store instruction.  Wave lanes take the roles
+//   [0, 2K) index dwords | [2K, 3K) weights | [3K, 4K + 2) metadata columns        compact, K <= 15
+//   [0, K + 2) metadata columns                                                    expanded
+// and a lane's place (a base and a stride by rows) and its word where the row's rank is that of its routing lane, and where not, are
+// worked out once: a row then costs an address and a select.  This wavefront's chain is the longest of its token's, and with a branch per
+// role and row it was 250 instructions longer at top-8 over 8 ranks.
 __device__ __forceinline__ void write_token_metadata(const MoveParams& p, const Route& r, int t, int lane) {
-    uint64_t masters = __ballot(r.row_c >= 0);
     const int K = p.K;
-    if (!p.do_expand && 4 * K + 2 <= kWaveSize) {
-        int src;           // routing lane this wave lane reports on
-        if (lane < 2 * K) src = lane >> 1;
-        else if (lane < 3 * K) src = lane - 2 * K;
-        else src = lane - 3 * K - 2;                       // metadata columns 2.. (negative for columns 0 and 1)
-        const int src_c = src < 0 ? 0 : (src >= K ? 0 : src);
-        const int e_src = __shfl(r.e, src_c, kWaveSize);
-        const int d_src = __shfl(r.d, src_c, kWaveSize);
-        const uint32_t w_src = __float_as_uint(__shfl(r.w, src_c, kWaveSize));
-        while (masters) {
-            const int j = __builtin_ctzll(masters);
-            masters &= masters - 1;
-            const int row = read_lane(r.row_c, j);
-            const int dj = read_lane(r.d, j);
-            if (row >= p.recv_capacity) {
-                if (lane == 0) atomicOr(p.status, DEEP_EP_HIP_STATUS_ROW_OVERFLOW);
-                continue;
+    uint64_t masters = __ballot(r.row_c >= 0 && r.row_c < p.recv_capacity);
+    if (__ballot(r.row_c >= p.recv_capacity) != 0ull && lane == 0) atomicOr(p.status, DEEP_EP_HIP_STATUS_ROW_OVERFLOW);
+    if (p.do_expand && p.recv_topk_weights != nullptr && r.erow >= 0 && r.erow < p.expanded_capacity)
+        p.recv_topk_weights[r.erow] = r.w;
+    if (p.do_expand || 4 * K + 2 <= kWaveSize) {
+        const int col = p.do_expand ? lane : lane - 3 * K;                        // metadata column (negative: none)
+        int src = col - 2;                                                        // routing lane this wave lane reports on
+        if (!p.do_expand && lane < 2 * K) src = lane >> 1;
+        else if (!p.do_expand && lane < 3 * K) src = lane - 2 * K;
+        src = src < 0 || src >= K ? 0 : src;
+        const int e_src = __shfl(r.e, src, kWaveSize), d_src = __shfl(r.d, src, kWaveSize);
+        const uint32_t w_src = __float_as_uint(__shfl(r.w, src, kWaveSize));
+        const int erow_src = p.do_expand ? __shfl(r.erow, src, kWaveSize) : -1;
+        uint8_t* base = nullptr;
+        uint32_t stride = uint32_t(K) * 4u, match = ~0u, other = ~0u;
+        if (!p.do_expand && lane < 2 * K) {
+            if (p.recv_topk_idx != nullptr) base = reinterpret_cast<uint8_t*>(p.recv_topk_idx) + lane * 4;
+            stride *= 2u;
+            match = (lane & 1) ? 0u : uint32_t(e_src - d_src * p.E_l);
+        } else if (!p.do_expand && lane < 3 * K) {
+            if (p.recv_topk_weights != nullptr) base = reinterpret_cast<uint8_t*>(p.recv_topk_weights) + (lane - 2 * K) * 4;
+            match = w_src;
+            other = p.zero_nonlocal_w ? 0u : w_src;
+        } else if (col < K + 2) {
+            stride += 8u;
+            if (!p.cached && p.recv_src_metadata != nullptr) base = reinterpret_cast<uint8_t*>(p.recv_src_metadata) + col * 4;
+            match = uint32_t(erow_src);
+            if (col == 0) {
+                match = other = uint32_t(p.rank_idx * p.M + t);
+                if (p.recv_src_idx != nullptr) {             // V1: in place of the columns
+                    base = reinterpret_cast<uint8_t*>(p.recv_src_idx);
+                    stride = 4u;
+                    match = other = uint32_t(t);
+                }
             }
-            uint32_t* dst = nullptr;
-            uint32_t v = 0;
-            if (lane < 2 * K) {
-                const int local = (d_src == dj) ? e_src - dj * p.E_l : -1;
-                v = (lane & 1) ? (local < 0 ? 0xffffffffu : 0u) : uint32_t(local);
-                if (p.recv_topk_idx != nullptr) dst = reinterpret_cast<uint32_t*>(p.recv_topk_idx + int64_t(row) * K) + lane;
-            } else if (lane < 3 * K) {
-                v = (p.zero_nonlocal_w && d_src != dj) ? 0u : w_src;
-                if (p.recv_topk_weights != nullptr)
-                    dst = reinterpret_cast<uint32_t*>(p.recv_topk_weights + int64_t(row) * K) + (lane - 2 * K);
-            } else if (lane < 4 * K + 2) {
-                const int col = lane - 3 * K;
-                v = col == 0 ? uint32_t(p.rank_idx * p.M + t) : col == 1 ? uint32_t(p.rank_idx * K + j) : 0xffffffffu;
-                if (!p.cached && p.recv_src_metadata != nullptr)
-                    dst = reinterpret_cast<uint32_t*>(p.recv_src_metadata + int64_t(row) * (K + 2)) + col;
-                if (col == 0 && p.recv_src_idx != nullptr) p.recv_src_idx[row] = t;
+        }
+        if (base != nullptr) {
+            while (masters) {
+                const int j = __builtin_ctzll(masters);
+                masters &= masters - 1;
+                const uint32_t v = d_src == read_lane(r.d, j) ? match : other;
+                *reinterpret_cast<uint32_t*>(base + uint64_t(uint32_t(read_lane(r.row_c, j))) * stride) =
+                    col == 1 ? uint32_t(p.rank_idx * K + j) : v;
             }
-            if (dst != nullptr) *dst = v;
         }
         return;
     }
@@ -229,28 +240,19 @@ __device__ __forceinline__ void write_token_metadata(const MoveParams& p, const 
         masters &= masters - 1;
         const int row = read_lane(r.row_c, j);
         const int dj = read_lane(r.d, j);
-        if (row >= p.recv_capacity) {
-            if (lane == 0) atomicOr(p.status, DEEP_EP_HIP_STATUS_ROW_OVERFLOW);
-            continue;
-        }
-        if (!p.do_expand && lane < p.K) {
+        if (lane < K) {
             if (p.recv_topk_idx != nullptr)
-                p.recv_topk_idx[int64_t(row) * p.K + lane] = (r.d == dj) ? int64_t(r.e - dj * p.E_l) : int64_t(-1);
+                p.recv_topk_idx[int64_t(row) * K + lane] = (r.d == dj) ? int64_t(r.e - dj * p.E_l) : int64_t(-1);
             if (p.recv_topk_weights != nullptr)
-                p.recv_topk_weights[int64_t(row) * p.K + lane] = (p.zero_nonlocal_w && r.d != dj) ? 0.f : r.w;
+                p.recv_topk_weights[int64_t(row) * K + lane] = (p.zero_nonlocal_w && r.d != dj) ? 0.f : r.w;
         }
         if (lane == 0 && p.recv_src_idx != nullptr) p.recv_src_idx[row] = t;
-        if (!p.cached && p.recv_src_metadata != nullptr && lane < p.K + 2) {
-            int v;
-            if (lane < p.K) v = (p.do_expand && r.d == dj) ? r.erow : -1;
-            else if (lane == p.K) v = p.rank_idx * p.M + t;
-            else v = p.rank_idx * p.K + j;
-            const int col = lane < p.K ? 2 + lane : lane - p.K;
-            p.recv_src_metadata[int64_t(row) * (p.K + 2) + col] = v;
+        if (!p.cached && p.recv_src_metadata != nullptr && lane < K + 2) {
+            const int v = lane < K ? -1 : lane == K ? p.rank_idx * p.M + t : p.rank_idx * K + j;
+            const int col = lane < K ? 2 + lane : lane - K;
+            p.recv_src_metadata[int64_t(row) * (K + 2) + col] = v;
         }
     }
-    if (p.do_expand && p.recv_topk_weights != nullptr && r.erow >= 0 && r.erow < p.expanded_capacity)
-        p.recv_topk_weights[r.erow] = r.w;
 }
 
 // Bit mask of lanes that name a destination row, and the row each of them names.
@@ -749,14 +751,12 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
     bool warmed = false;
     if constexpr (kFused) warmed = warm_next_rounds_of_rows<kVecs>(p, work, lane);
 
+    // Rows are read and written through a descriptor each, which ends with the row: no address and no branch for each vector.
     vec16 v[kVecs];
-    const uint8_t* src = p.x + int64_t(t) * p.row_bytes;
+    const auto src = buffer_of(p.x + int64_t(t) * p.row_bytes, has_work ? p.row_bytes : 0);
+    const int at = tile * (kVecs * 1024) + lane * 16;
 #pragma unroll
-    for (int i = 0; i < kVecs; ++i) {
-        const int off = (tile * kVecs + i) * 1024 + lane * 16;
-        v[i] = vec16{0, 0, 0, 0};
-        if (has_work && off < p.row_bytes) v[i] = load16_as<kCached != kInput>(src + off);
-    }
+    for (int i = 0; i < kVecs; ++i) v[i] = buffer_load16_as<kCached != kInput>(src, at + i * 1024);
 
     // The caller's scale packs ride with tile 0: requested with the payload, once, not per destination row.
     const bool packs = kScales != kNoScales && has_work && tile == 0 && p.recv_sf != nullptr;
@@ -794,18 +794,16 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
         const int j = __builtin_ctzll(dests);
         dests &= dests - 1;
         const int row = read_lane(row_of_lane, j);
-        uint8_t* dst = p.recv_x + int64_t(row) * p.row_bytes;
+        const auto dst = buffer_of(p.recv_x + int64_t(row) * p.row_bytes, p.row_bytes);
 #pragma unroll
-        for (int i = 0; i < kVecs; ++i) {
-            const int off = (tile * kVecs + i) * 1024 + lane * 16;
-            if (off < p.row_bytes) store16_as<kCached != kRows>(dst + off, v[i]);
-        }
+        for (int i = 0; i < kVecs; ++i)                       // vectors wholly past the row's end are not issued
+            if (i == 0 || (tile * kVecs + i) * 1024 < p.row_bytes) buffer_store16_as<kCached != kRows>(dst, at + i * 1024, v[i]);
         if (packs) {
             if (lane < p.num_sf_packs) *scale_place<kScales == kScalesInBlocks>(p, row, lane) = pack;
             for (int g = lane + kWaveSize; g < p.num_sf_packs; g += kWaveSize)        // rows beyond 8192 channels
                 *scale_place<kScales == kScalesInBlocks>(p, row, g) = p.sf[int64_t(t) * p.sf_ts + int64_t(g) * p.sf_hs];
-            if (!kFused && p.row_by_row) wait_for_own_stores();
         }
+        if (!kFused && p.row_by_row) wait_for_own_stores();
     }
 }
 
@@ -857,20 +855,19 @@ __device__ __forceinline__ void dispatch_cast(const MoveParams& p) {
     if constexpr (kFused) warmed = warm_next_rounds<kPairs>(p, work, lane);
 
     vec16 in[kPairs][2];
-    const uint8_t* src = p.x + int64_t(t) * p.row_bytes;
+    const auto src = buffer_of(p.x + int64_t(t) * p.row_bytes, has_work ? p.row_bytes : 0);
+    const int at = tile * (kPairs * 1024) + lane * 16;      // channel, and byte of an output row
+    if (p.plain_loads) {
 #pragma unroll
-    for (int q = 0; q < kPairs; ++q) {
-        const int elem = (tile * kPairs + q) * 1024 + lane * 16;
-        in[q][0] = vec16{0, 0, 0, 0};
-        in[q][1] = vec16{0, 0, 0, 0};
-        if (has_work && elem < p.H) {
-            if (p.plain_loads) {
-                in[q][0] = load16(src + int64_t(elem) * 2);
-                in[q][1] = load16(src + int64_t(elem) * 2 + 16);
-            } else {
-                in[q][0] = load16_stream(src + int64_t(elem) * 2);
-                in[q][1] = load16_stream(src + int64_t(elem) * 2 + 16);
-            }
+        for (int q = 0; q < kPairs; ++q) {
+            in[q][0] = buffer_load16_as<false>(src, at * 2 + q * 2048);
+            in[q][1] = buffer_load16_as<false>(src, at * 2 + q * 2048 + 16);
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < kPairs; ++q) {
+            in[q][0] = buffer_load16_as<true>(src, at * 2 + q * 2048);
+            in[q][1] = buffer_load16_as<true>(src, at * 2 + q * 2048 + 16);
         }
     }
 
@@ -931,12 +928,10 @@ __device__ __forceinline__ void dispatch_cast(const MoveParams& p) {
         const int j = __builtin_ctzll(dests);
         dests &= dests - 1;
         const int row = read_lane(row_of_lane, j);
-        uint8_t* dst = p.recv_x + int64_t(row) * p.H;
+        const auto dst = buffer_of(p.recv_x + int64_t(row) * p.H, p.H);
 #pragma unroll
-        for (int q = 0; q < kPairs; ++q) {
-            const int elem = (tile * kPairs + q) * 1024 + lane * 16;
-            if (elem < p.H) store16_stream(dst + elem, out[q]);
-        }
+        for (int q = 0; q < kPairs; ++q)
+            if (q == 0 || (tile * kPairs + q) * 1024 < p.H) buffer_store16_as<true>(dst, at + q * 1024, out[q]);
         if (owns_scale) *scale_place<kBlocked>(p, row, group) = __float_as_uint(my_scale);
     }
 #ifdef DEEP_EP_HIP_WAVE_STAMPS
@@ -1355,11 +1350,110 @@ static double row_bytes_out(const MoveParams& p) {
 
 static bool is_large_input(const MoveParams& p) { return int64_t(p.T) * p.row_bytes >= (int64_t(64) << 20); }
 
+// Which side of a copy goes through the memory-side cache (256 MB).
+// - BF16, up to 110 MB of rows and 240 MB with the padding rows zeroed behind them: the rows, which whoever is next then finds there.
+//   Dispatch and combine, us, neither / rows, input just written: 277 x 6072 over 8 ranks (18 MB) 24.0 / 22.0, 1024 x 7168 (77 MB) 54.3 / 40.7,
+//   4096 x 2048 top-6 (74 MB) 55.7 / 44.1; with a pass over the rows in between that writes as many 30.9 / 31.6, 66.1 / 65.3, 67.7 / 66.4.  With more
+//   padding the rows leave the cache again before they are read.  Top-8, aligned to 128, streaming / rows: 646 x 2136 of 384 experts (210 MB)
+//   61.4 / 60.0, 400 x 7168 of 112 (206 MB) 62.8 / 61.6, of 128 (235 MB) 67.2 / 66.5, of 144 (264 MB) 72.2 / 72.2, of 160 (294 MB) 78.0 /
+//   84.4, 300 x 7168 of 256 (470 MB) 104.4 / 115.5.
+// - BF16, more: the input, which the layer in front has just written; so many rows would drive it and each other out.  Dispatch and
+//   combine, us, neither / input: 2600 x 7168 over 8 ranks (198 MB) 103.4 / 96.5, 3400 x 7168 (258 MB) 123.7 / 116.5, 8192 x 7168 (622 MB) 261.7 /
+//   261.5, V1 4096 x 7168 150.2 / 141.8, expanded 4096 x 4096 top-8 143.3 / 134.8; with the input just written behind 400 MB of other writes 103.7 /
+//   99.4, 125.8 / 118.2, 274.8 / 247.4, 151.5 / 141.5, 143.9 / 137.5; with an input that has left the cache by then 103.3 / 110.1, 125.7 /
+//   131.3, 265.4 / 275.7, 153.2 / 159.4, 146.1 / 150.6.
+// - FP8: neither.  Cast, dispatch and combine, neither / input / rows: 1024 x 7168 (39 MB) 43.2 / 44.3 / 43.4, 2100 x 7168 (80 MB) 71.0 / 71.4 /
+//   69.1, 4096 x 7168 (156 MB) 130.1 / 127.4 / 125.4 with three inputs in turn, 126.9 / - / 129.4 with more.
+// - BF16, the input larger than that cache or followed by 150 MB and more of zeroed rows: neither.
+//   Input called over and over, 20000 x 7168 (287 MB) 597.7 / 603.0; expanded over 256 experts aligned to 128 rows 4883 x 6728 (220 MB of zeros)
+//   309.7 / 313.2, 10714 x 6896 (225 MB) 601.2 / 611.5; over 128 (113 MB) it is 567.3 / 565.9 and, input just written, 580.1 / 552.4.
+static int cached_side(const MoveParams& p) {
+    if (p.payload != DEEP_EP_HIP_PAYLOAD_BF16) return kNeither;
+    const double zeroed = p.zeroed_rows * double(p.row_bytes);
+    const bool among_padding = p.do_expand && expanded_rows_in_use(p.expanded_capacity, p.recv_capacity, p.T, p.K, p.E, p.R, p.M) * p.row_bytes > kExpandedBytesInCache;
+    if (row_bytes_out(p) <= 110e6 && !among_padding) return kRows;
+    return double(p.T) * p.row_bytes <= 256e6 && zeroed < 150e6 ? kInput : kNeither;
+}
+
 // A launch of so many workgroups of this tile that they fill `rounds` rounds of eight per CU.
 static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
     const int bytes = p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? p.H : p.row_bytes;
     const int64_t wavefronts = int64_t(p.T) * ((bytes + tile * 1024 - 1) / (tile * 1024));
     return wavefronts >= int64_t(compute_units()) * rounds * 8 * kWavesPerBlock;
+}
+
+// Large moves on a finished layout: tile, and workgroups a CU holds at a time (0: as many as fit).  Scattered stores stream fastest when not too
+// many rows are being written at once: a wavefront writes its tile to every row of its token, so what counts is tile x workgroups x rows a token,
+// about 20 KB in a fourth of a CU.  Move and combine together, us, best of 1 KB / 2 KB / 4 KB tiles with the workgroups in brackets, and what
+// these calls took before, mostly with five or six workgroups of 1 KB or eight of 4 KB:
+//   BF16 past the memory-side cache (cached_side):
+//     10967 x 5848 of 8 ranks (5.6 rows) 333.1 (4) / 331.9 (2) / 356.6 (8), before 361.5;   8371 x 5048 204.5 (3) / 204.4 (2) / 208.2 (2), 217.8;
+//     6221 x 4488 of 64 ranks (9.3) 255.7 / 249.7 / 249.3 (2 each), 263.6;   from 90 MB of input, up to 5.2 rows, 17335 x 3712 (4.4) 250.2 with
+//     three of 2 KB, 261.5 with two, 265.1;   15819 x 6096 (2.7) 247 (8) / 243.3 (3) / 249 (2), 245.1;   16746 x 8072 (2.0) 283.5 (8) / 278.1 (8),
+//     280.9 with five, 281.6 with four;   rows of 3 and 4 KB 21387 x 1048 (6.5) 174.0 / 171.9 / 165.2 (2 each), 174.1;
+//   - many expanded rows over fewer than 32 ranks in 1 KB tiles (6706 x 4000 top-8 of 64 181.9 (2) / 173.7 (2)): 17091 x 2552 top-8 304.8 (2) / 313.3 / 315 (2), 329.3;   6490 x 5408 211.1 (2) / 219.3 (2), 221.2;   10922 x
+//     5096 top-9 430.7 / 446.7, 461.5;   up to 300 MB of them they are level (2270 x 5192 88.7 / 90.2, 1646 x 5032 78.2 / 75.2);
+//   - rows of whole KB, whose wavefronts run more alike, up to 430 MB in four or five workgroups of 1 KB: 6608 x 2048 of 8 ranks (5.9) 67.4 (5) / 68.3
+//     (4), 72.4;   2805 x 3072 of 32 (8.0) 57.5 (4) / 57.5 (2), 61.2;   and beyond with each row's stores awaited before the next row's are issued, so that
+//     a wavefront has one row under way however long that takes; without / with the wait: 20000 x 4096 of 8 (5.3), move alone, 177.4 (2 of 2 KB) / 170.5
+//     (6), before 188.5;   whole passes with a layer's other kernels around them, five without / six with the wait: 32000 x 2048 of 32 ranks (7.2) 403.6 /
+//     404.4, before 407.3;   8192 x 7168 of 32 348.4 / 345.3, 346.1;   9800 x 7168 of 16 (7.0) 407.5 / 406.6, 410.6;   16384 x 5120 of 64 (7.6) 532.2 / 530.0,
+//     534.9;   13211 x 4096 of 16 353.0 / 348.2, 360.1;   16384 x 7168 of 16 (6.5) 607.0 / 609.9, 611.2;   of 32 685.1 / 686.4, 685.5, with five and
+//     the wait 710;   on a handle, moves alone, five / six with the wait: 16384 x 7168 of 32 337.6 / 354.5, 350;   32768 x 2048 195.3 / 203.7, 197;   of 16
+//     302 / 302, 298;
+//     rows of 8 and 16 KB, top-6, in three of 2 KB: 24000 x 4096 of 8 ranks (4.4) 361.4 / 369.9 (6), 373.8;   14000 x 8192 418.2 / 430.7 (6), 450.2;
+//     where a token goes to fewer than four rows: 14174 x 8192 (3.3) 348 (8 of 1 KB) / 336.8 (4 of 2 KB), 337.5;   16380 x 7168 (3.6) 353.9 (3 of 2 KB),
+//     360.9;   17516 x 3584 (3.7) 204.7 (3 of 2 KB) / 197.8 (8 of 1 KB with the wait), 199.5;   without top-k tensors, moves alone, 8192 x 7168 of 4 ranks
+//     (2.7) 73.8 (8 of 1 KB) / 75.2 with the wait, 76.1 (4 of 2 KB);   16384 x 4096 top-4 of 8 (3.3) 102.5 / 99.0 with it, 103.3;
+//     expanded 25983 x 2560 top-2 156.2 (8 of 2 KB), 173.4;
+//   fused cast, expanded, 8192 x 7168 top-8 315.4 (4) / 312.4 (3), 320.6;   16316 x 4608 403.9 (4) / 393.9 (3), 418.5;   compact, 25585 x 3072 of 32
+//     ranks 352.5 (4) / 351.8 (4), 364.5;   8192 x 7168 of 8 200.2 (6) / 199.3 (4), 200.4;   12006 x 5120 top-6 (4.4) 204.4 (8) / 202.9 (5), 205.1;   with
+//     blocked scales, whose rows have no single-dword stores, 8192 x 7168 318.1 (5) / 324.0 (3): left alone;
+//   FP8 pairs, expanded, 24963 x 3584 top-9 505.7 (5) / 495.9 (3) / 496.9 (2), 521.1;   compact, 28277 x 4864 (5.9) 485.8 (8) / 473.2 (3) / 474.1 (2),
+//     487.5;   35472 x 3968 (4.4) 438.3 (8) / 427.7 (4) / 437.9 (6), 438.3;   rows of whole KB like those of BF16, move alone, without / with the wait: 16384 x 7168 of 32
+//     ranks 174.8 (5) / 175.0 (6), 181.6 (8);   32768 x 2048 103.7 (5) / 102.0 (8), 109.0 (8);   8192 x 7168 of 8 66.9 / 64.9 (8);   20000 x 4096 95.0 / 91.3 (8);
+//     12000 x 3072 of 16, top-6 45.3 / 44.2 (8);   4096 x 7168 36.0 / 35.4 (8);   12000 x 5120 of 32 101.9 (4) / 105.1 (6), 105.2.
+struct MoveShape {
+    int tile, per_cu;
+    bool in_turn;        // the stores of a row are awaited before the next row's
+};
+
+static bool large_move_shape(const MoveParams& p, MoveShape& q) {
+    const int bytes = p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? p.H : p.row_bytes, kb = (bytes + 1023) / 1024;
+    const double rows = rows_per_token(p), out = row_bytes_out(p);
+    if (p.fused || p.cast_pairs != 0 || p.copy_vecs != 0 || kb < 2 || p.sf_blocked) return false;
+    if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) {
+        if (out < 220e6 || rows < 3.5) return false;
+        q = {2, rows < 5.0 ? 5 : p.do_expand ? 3 : 4, false};
+        return true;
+    }
+    const bool whole = bytes % 1024 == 0;
+    if (p.payload == DEEP_EP_HIP_PAYLOAD_FP8) {
+        if (rows < 3.2 || out < (whole && !p.do_expand ? 100e6 : 280e6)) return false;
+        if (whole && !p.do_expand) q = {1, rows < 6.0 ? 0 : 6, true};
+        else q = {2, rows < 5.0 ? 4 : 3, false};
+        return true;
+    }
+    if (cached_side(p) == kRows || (whole && kb == 2)) return false;
+    if (rows < 2.4) {
+        q = {2, rows < 1.7 || p.do_expand ? 0 : p.R >= 64 ? 4 : 5, false};
+        return whole || kb < 3 || kb > 4;
+    }
+    if (whole) {
+        if (p.rank_lanes && rows < 3.9) q = {1, 0, rows >= 3.0};
+        else if (rows < 3.9 && (rows < 3.5 || kb >= 8 || out < 430e6)) q = {2, rows < 3.5 || kb < 8 ? 4 : 3, false};
+        else if (out < 430e6) q = {1, rows < 6.4 ? 5 : 4, false};
+        else if ((kb & (kb - 1)) == 0 && kb >= 8 && rows < 5.0) q = {2, 3, false};
+        else q = {1, rows < 4.2 ? 0 : p.cached && rows >= 6.0 ? 5 : 6, true};
+        return true;
+    }
+    if (kb == 3 || kb == 4) {
+        q = {4, 2, false};
+        return rows >= 3.2;
+    }
+    if (p.do_expand && rows >= 8.0 && out >= 300e6 && kb >= 5 && p.R < 32) q = {1, 2, false};
+    else q = {2, rows < 4.3 || (rows < 5.2 && double(p.T) * p.row_bytes >= 90e6) ? 3 : 2, false};
+    return true;
 }
 
 // Column tile of a move launch: 1024-channel segments per wavefront for the fused cast, KB of row per wavefront for
@@ -1372,7 +1466,13 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 // 2 KB), 512 x 7168 23.0 / 20.6 / 19.7 (3584): left alone; fused cast, 1 / 2 segments, 300 x 7168 18.0 / 18.3, 512 x 2048 16.8 / 17.4,
 // 512 x 7168 (3584) 19.2 / 18.9.  Not in a single launch, where neighbours of the counting workgroups wait: 512 x 2048 BF16 16.7 / 16.5
 // / 15.6, though 300 x 7168 takes 16.7 / 16.3 / 17.5.
+// BF16 rows that stay in the memory-side cache, up to 60 wavefronts of 1 KB per CU, take 1 KB as well: move and combine of 2001 x 2048 over 8
+// ranks 23.8 us, 26.7 with 2 KB, 30.3 with 4.  Beyond, tokens of three rows and more of 4, 8 or 12 KB take 2 KB, 1 / 2 / 4 KB: 4096 x 2048 top-6
+// 38.0 / 38.5 / 43.0;  6000 x 2048 top-4 42.0 / 40.9 / 45.3;  2200 x 6144 top-4 44.1 / 42.2 / 45.7;  3000 x 4096 expanded top-4 47.6 / 46.2 /
+// 50.6; others the widest: 1400 x 7168 47.1 / 47.5 / 44.9, 3500 x 2560 43.7 / 45.7 / 43.7, 9000 x 1400 top-4 45.5 / 45.5 / 43.2.
 static int move_tile(const MoveParams& p) {
+    MoveShape large{};
+    if (large_move_shape(p, large)) return large.tile;
     const double rows = rows_per_token(p);
     const auto wavefronts_per_cu_at_most = [&](int tile, int most) {
         const int bytes = p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? p.H : p.row_bytes;
@@ -1394,16 +1494,18 @@ static int move_tile(const MoveParams& p) {
     if (p.copy_vecs != 0) return p.copy_vecs;
     const int kb = (p.row_bytes + 1023) / 1024;
     if (wavefronts_per_cu_at_most(1, 8)) return 1;
+    if (p.payload == DEEP_EP_HIP_PAYLOAD_BF16 && !p.fused && cached_side(p) == kRows) {
+        if (int64_t(p.T) * kb <= int64_t(compute_units()) * 60) return 1;
+        if (kb % 4 == 0 && rows >= 3.0) return 2;
+    }
     if (kb > 2 && wavefronts_per_cu_at_most(2, 10)) return 2;
     const int widest = kb <= 1 ? 1 : kb <= 2 ? 2 : 4;
     // Small, latency-bound calls: up to 4 KB per wavefront, so that fewer wavefronts repeat the routing work (4096 rows
     // of 4 KB: 19.5 us against 21.1 us with 1 KB tiles).  Calls that write 200 MB and more are bound by their stores.
     // Rows of up to 3 KB then take 2 KB (32768 x 1536 top-8: 8 ranks 97 against 104 us, 64 ranks 133 against 146), wider
     // (whole KB in the expanded layout and in V1 calls without top-k tensors, which write little or nothing beside the rows, 1 KB:
-// 32768 x 1024 top-8 over 8 ranks 119 against 127 us, cached V1 77 against 84) ones 1 KB where a token goes to 3.5 rows and more (BF16, 8 ranks: 4096 x 7168 66.5 against 73.4 us, 8192 x 7168 126
-    // against 145; 16384 x 7168 top-4 of 16 ranks, 3.6 rows, 194 against 206), 2 KB where it goes to fewer (8192 x 7168, 4 of
-    // 4 ranks: 75.6 us with four workgroups per CU against 79.4 with 1 KB and 84.9 with 4 KB) and, below five, over 64 ranks
-    // (32768 x 2048 top-4: 126 us against 147).  At 183 MB (16384 x 2048, 4 of 4 ranks) 2 and 4 KB measured the same.
+    // 32768 x 1024 top-8 over 8 ranks 119 against 127 us, cached V1 77 against 84) ones 1 KB where a token goes to 3.5 rows and more,
+    // 2 KB where it goes to fewer and, below five, over 64 ranks.  At 183 MB (16384 x 2048, 4 of 4 ranks) 2 and 4 KB measured the same.
     if (p.fused || row_bytes_out(p) < 200e6) return widest;
     const bool whole = p.row_bytes * 8 > kb * 7 * 1024;           // no wavefront of 1 KB would be half idle
     if (kb <= 3) return kb == 1 || (p.rank_lanes && rows >= 5.0) || ((p.rank_lanes || p.do_expand) && whole) ? 1 : 2;
@@ -1416,31 +1518,28 @@ static int move_tile(const MoveParams& p) {
 // for 141, 64 ranks 134 for 164; 16384 tokens over 8 ranks 30.5 for 30.9.  Wider rows gain by it over 64 ranks and lose over 8
 // (32768 x 4096: 231 us for 246, 162 for 157).
 static bool stores_row_by_row(const MoveParams& p) {
+    MoveShape large{};
+    if (large_move_shape(p, large)) return large.in_turn;
     return !p.fused && p.payload != DEEP_EP_HIP_PAYLOAD_CAST_FP8 && p.recv_sf != nullptr && p.row_bytes <= 1024 &&
            rows_per_token(p) >= 3.5 && fills_rounds(p, 1, 2);
 }
 
 // How many workgroups of a move kernel launched on a finished layout a CU should hold at a time (0: as many as fit).
 // Scattered stores stream fastest when not too many are under way: the more rows a token has, the more ranks they are spread
-// over and the wider they are, the fewer.  Move phase in us, inputs read from memory, with 8 / 6 / 5 / 4 workgroups per CU:
+// over and the wider they are, the fewer.  What large_move_shape leaves, move phase in us, inputs read from memory, with 8 / 6 / 5 / 4 per CU:
 //   fused cast, 8192 x 7168, 8 ranks           81.4 / 80.8 / 80.6 / 82.2;   16384 x 7168, 64 ranks 1 KB 272 / 241 / 228
 //   fused cast, expanded, 16384 x 4096 top-8   134 / 139 / 141: left alone;           8192 x 7168 top-8 1 KB 122 / 123 / 121,
 //                                              and 2 % of the whole pass with inputs that change
-//   BF16, 16384 x 7168, 32 ranks, 1 KB         363 / 362 / 354 / 346;       16 ranks 312 / 312 / 304 / 314
-//   BF16, 16384 x 7168, 8 ranks, 1 KB          255 / 249 / 254 / 271;       16384 x 2048 80.8 / 82.2 / 86.8: left alone
-//   BF16, 16384 x 2048, 64 ranks top-6, 1 KB   116 /  95 /  97 / 105;       16 ranks top-8 99.7 / 99.7 / 101 / 109
-//   BF16, 65536 x 768, 2 KB, top-8: 8 ranks    122 / 117 / 116 / 122;       64 ranks top-6 203 / 168 / 143 / 140
-//   BF16, 65536 x 768, 2 KB, top-2 of 2 ranks 50.9 / 52.1 / 55.0 / 62.0: left alone
 //   BF16, 65536 x 512, 64 ranks top-6, 1 KB    140 / 122 / 118 / 123;       65536 x 256 77 / 83 / 88 / 98 (8 ranks): left alone
-//   BF16, 8192 x 7168, 4 of 4 ranks, 2 KB       82 /  80 /  77 /  76;       32768 x 2048, 2 of 2 ranks 60.4 / 62.5 / 63 / 64.3
-//   BF16, 16384 x 7168 top-2 of 8 ranks, 2 KB 123 / 121 / 119 / 118;       the same in FP8 63.5 / 67.1 / 66 / 68.4: left alone
-//   BF16, cached V1, 32768 x 2048, 32 ranks    201 / 211, 65536 x 768, 16 ranks 137 / 137 / 153: left alone
+//   FP8, 16384 x 7168 top-2 of 8 ranks, 2 KB   63.5 / 67.1 / 66 / 68.4: left alone
 // Launches that would not fill two rounds of eight per CU, and copies of less than 200 MB (but for rows of 2 KB over 64 ranks:
 // 32768 x 768 top-4, 198 MB, 70 us without, 58 with four), are left alone.
 static int move_workgroups_per_cu(const MoveParams& p) {
     if (p.fused) return 0;
     if (p.move_workgroups_per_cu != 0)       // two is the least an LDS share within a workgroup's 64 KB can enforce
         return p.move_workgroups_per_cu >= 8 ? 0 : (p.move_workgroups_per_cu < 2 ? 2 : p.move_workgroups_per_cu);
+    MoveShape large{};
+    if (large_move_shape(p, large)) return large.per_cu;
     const int tile = move_tile(p);
     if (!fills_rounds(p, tile, 2)) return 0;
     const double rows = rows_per_token(p);
@@ -1502,38 +1601,13 @@ void plan_cache_warming(MoveParams& p) {
     p.warm_ahead = rounds * first_round * unsigned(kWavesPerBlock);
 }
 
-// Which side of a copy goes through the memory-side cache (256 MB).
-// - BF16, up to 110 MB of rows and 240 MB with the padding rows zeroed behind them: the rows, which whoever is next then finds there.
-//   Dispatch and combine, us, neither / rows, input just written: 277 x 6072 over 8 ranks (18 MB) 24.0 / 22.0, 1024 x 7168 (77 MB) 54.3 / 40.7,
-//   4096 x 2048 top-6 (74 MB) 55.7 / 44.1; with a pass over the rows in between that writes as many 30.9 / 31.6, 66.1 / 65.3, 67.7 / 66.4.  With more
-//   padding the rows leave the cache again before they are read.  Top-8, aligned to 128, streaming / rows: 646 x 2136 of 384 experts (210 MB)
-//   61.4 / 60.0, 400 x 7168 of 112 (206 MB) 62.8 / 61.6, of 128 (235 MB) 67.2 / 66.5, of 144 (264 MB) 72.2 / 72.2, of 160 (294 MB) 78.0 /
-//   84.4, 300 x 7168 of 256 (470 MB) 104.4 / 115.5.
-// - BF16, more: the input, which the layer in front has just written; so many rows would drive it and each other out.  Dispatch and
-//   combine, us, neither / input: 2600 x 7168 over 8 ranks (198 MB) 103.4 / 96.5, 3400 x 7168 (258 MB) 123.7 / 116.5, 8192 x 7168 (622 MB) 261.7 /
-//   261.5, V1 4096 x 7168 150.2 / 141.8, expanded 4096 x 4096 top-8 143.3 / 134.8; with the input just written behind 400 MB of other writes 103.7 /
-//   99.4, 125.8 / 118.2, 274.8 / 247.4, 151.5 / 141.5, 143.9 / 137.5; with an input that has left the cache by then 103.3 / 110.1, 125.7 /
-//   131.3, 265.4 / 275.7, 153.2 / 159.4, 146.1 / 150.6.
-// - FP8: neither.  Cast, dispatch and combine, neither / input / rows: 1024 x 7168 (39 MB) 43.2 / 44.3 / 43.4, 2100 x 7168 (80 MB) 71.0 / 71.4 /
-//   69.1, 4096 x 7168 (156 MB) 130.1 / 127.4 / 125.4 with three inputs in turn, 126.9 / - / 129.4 with more.
-// - BF16, the input larger than that cache or followed by 150 MB and more of zeroed rows: neither.
-//   Input called over and over, 20000 x 7168 (287 MB) 597.7 / 603.0; expanded over 256 experts aligned to 128 rows 4883 x 6728 (220 MB of zeros)
-//   309.7 / 313.2, 10714 x 6896 (225 MB) 601.2 / 611.5; over 128 (113 MB) it is 567.3 / 565.9 and, input just written, 580.1 / 552.4.
-static int cached_side(const MoveParams& p) {
-    if (p.payload != DEEP_EP_HIP_PAYLOAD_BF16) return kNeither;
-    const double zeroed = p.zeroed_rows * double(p.row_bytes);
-    const bool among_padding = p.do_expand && expanded_rows_in_use(p.expanded_capacity, p.recv_capacity, p.T, p.K, p.E, p.R, p.M) * p.row_bytes > kExpandedBytesInCache;
-    if (row_bytes_out(p) <= 110e6 && !among_padding) return kRows;
-    return double(p.T) * p.row_bytes <= 256e6 && zeroed < 150e6 ? kInput : kNeither;
-}
-
 template <int kVecs, int kCached>
 hipError_t launch_copy_cached(const MoveParams& p, unsigned blocks, hipStream_t stream) {
-    // Rows without scale packs, in tiles of one and two KB: a kernel without the branch on the packs, with which they took 3 to 8 %
-    // longer (16384 x 7168 top-2, 1 KB tiles: 126 against 119 us; 65536 x 256 top-8 84.4 against 77.1).  Tiles of four KB and many wide
-    // rows to a token are the other way round (8192 x 2048 top-2 21.9 us without the branch, 20.5 with it; 16384 x 7168 top-8 254, 249).
+    // Rows without scale packs, in tiles of one and two KB: a kernel without the branch on the packs (6490 x 5408 top-8, expanded 101.2 us with the
+    // branch, 97.0 without; 16384 x 7168 of 32 ranks 341.1 / 340.3, 10113 x 6392 226.3 / 226.9).  Tiles of four KB have the one with it (8192 x 2048 top-2 21.9 us
+    // without the branch, 20.5 with it).
     constexpr int kPlain = kVecs <= 2 ? kNoScales : kScalesInPlace;
-    const bool plain = kPlain == kNoScales && p.recv_sf == nullptr && (rows_per_token(p) < 5.0 || p.row_bytes < 4096);
+    const bool plain = kPlain == kNoScales && p.recv_sf == nullptr;
     auto kernel = p.fused ? (plain ? dispatch_copy_single_launch_kernel<kVecs, kPlain, kCached> : dispatch_copy_single_launch_kernel<kVecs, kScalesInPlace, kCached>)
                           : (plain ? dispatch_copy_kernel<kVecs, kPlain, kCached> : dispatch_copy_kernel<kVecs, kScalesInPlace, kCached>);
     if constexpr (kVecs <= 4 && kCached == kNeither)            // scales come with FP8 rows
