@@ -288,6 +288,11 @@ double rows_per_token(const CombineParams& p) {
 //   2048 channels (32768 tokens) 8 ranks 142 / 139 / 139;                64 ranks 205 / 199 / 195
 //   8192 channels (16384 tokens) top-6 of 8 ranks 238 / 247 / 252;   4096 channels (8192) of 64 ranks 79.5 / 83.2 / 83.2: rows a
 //   power of two apart are left alone
+//   a GB of rows and seven a token, of whole KB, a dispatch in front, 6 / 5 / 4: 16384 x 7168 of 32 ranks 669.8 / 659.2 / 653.6, of 64 713 / 705.6 /
+//   697.4;   16000 x 6144 565 / 558.3 / 554.3;   20000 x 5120 587 / 578.2 / 576.8;   behind a fused cast, 16384 x 7168 of 32 541.7 / 538.2 / 527.9;   other
+//   rows 12000 x 6000 of 32 455.2 / 454.0 / 456.4;   14000 x 7000 of 64 681.9 / 676.2 / 676.4
+//   whole passes with 5 / 4: 6000 x 7168 of 32 (619 MB) 252.8 / 254.8; V1 12000 x 5120 of 32 372.4 / 383.9; 30000 x 3072 of 32 547.1 / 549.9; 16384 x 7168 of 64, cast, 615.6 / 604.3
+//   from 500 MB on: 8000 x 5120 of 16 (532 MB) 188.2 without, 184.2 with five; 10000 x 5000 of 8 (530 MB) 241.6, 239.4 with six; 8307 x 4736 of 32 ranks behind a cast (567 MB) 181.7 without a limit, 178.6 with five
 // Smaller calls lose by any limit (4096 x 2048 top-6: 17.3 / 18.3), and so do narrower rows (65536 x 768 over 16 ranks 125 / 137 /
 // 146).
 // The limit is kept with LDS, which a product on another stream then lacks: beside products of 4096^3 BF16 that share the GPU,
@@ -297,7 +302,8 @@ double rows_per_token(const CombineParams& p) {
 int workgroups_per_cu(const CombineParams& p) {
     const double rows = rows_per_token(p), bytes = rows * p.T * p.H * 2;
     if ((p.do_expand && !p.rank_mode) || p.H < 2048 || p.H % 4096 == 0) return 0;
-    if (p.H < 6144 ? rows < 5.0 || bytes < 600e6 : rows >= 5.0 ? bytes < 300e6 : rows < 3.5 || bytes < 450e6) return 0;
+    if (p.H < 6144 ? rows < 5.0 || bytes < 500e6 : rows >= 5.0 ? bytes < 300e6 : rows < 3.5 || bytes < 450e6) return 0;
+    if (rows >= 7.0 && bytes >= 1e9 && p.H >= 5120 && p.H % 512 == 0 && !p.rank_mode) return 4;
     return rows >= 5.8 ? 5 : 6;
 }
 
