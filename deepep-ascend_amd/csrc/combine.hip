@@ -307,25 +307,6 @@ int workgroups_per_cu(const CombineParams& p) {
     return rows >= 5.8 ? 5 : 6;
 }
 
-// Column tile per wavefront: 1 KB of a BF16 row (512 channels, 41 registers, eight wavefronts per SIMD), or 2 KB, which repeats the routing
-// work half as often and has half the wavefronts to hide its loads with.  2 KB for few rows a token (top-2, or two ranks), where the routing is
-// as much as the rows, from three quarters of the places on; V1 rows, whose routing is shorter, from a full round on.  Change by 2 KB tiles in %
-// at 0.55 / 0.8 / 1.0 / 1.1 / 1.4 / 4 times as many wavefronts of 1 KB as places (730 shapes, rows of 2 to 14 KB):
-//   compact, top-2 of 2 ranks, 8 KB rows    +1.2 / -2.2 / -4.0 / -8.0 / -7.6 / -8.5;   top-2 of 8 ranks +0.6 / +0.5 / -1.5 / -5.8 / -8.2 / -4.4
-//   expanded, top-2                          +0.5 / -3.0 / -6.1 / -7.9 / -1.3 / -2.7
-//   V1, top-2 of 8 ranks, 4 KB rows          +2.4 / +3.2 / +1.0 / -5.8 / -5.1
-//   more rows a token, up to one round: compact top-8 of 8 ranks -3 to +5, expanded top-8 -2 to +9, V1 top-8 -1 to +9
-// A last tile that is half idle costs what the others gain: rows of 3 KB, expanded, top-2, 0.0 / +3.0 / +12.3 / +4.6 / +1.6 / +5.4; compact
-// +0.6 / -0.5 / +2.0 / -7.1 / -8.1 / -2.2.
-bool takes_two_kb_tiles(const CombineParams& p) {
-    const int kb = (p.H * 2 + 1023) / 1024;
-    if (kb < 2 || rows_per_token(p) >= 2.3) return false;
-    const int64_t places = int64_t(compute_units()) * 8 * kWavesPerBlock, waves = int64_t(p.T) * kb;
-    if (p.rank_mode) return waves > places;
-    const bool half_idle = kb % 2 == 1 && kb < 8;
-    return 4 * waves >= 3 * places && (!half_idle || (!p.do_expand && waves > places));
-}
-
 // The rows a combine adds up have just been written, by the experts or by the dispatch itself: up to 110 MB of them are read with plain
 // loads, which find them in the memory-side cache.  Dispatch and combine of BF16 rows, us, streaming / plain rows (the dispatch stores
 // by the same line, for the rows even routing would give, cached_side): 4096 x 2048 top-6 of 8 ranks, forward and backward (74 MB) 91.2 / 84.9, 16384 x 2048 of 2 ranks (100 MB) 77.5
@@ -338,6 +319,29 @@ bool reads_past_the_cache(const CombineParams& p) {
     const double row_bytes = p.H * 2.0;
     const bool between_padding = p.do_expand && !p.rank_mode && expanded_rows_in_use(p.num_x_rows, p.num_meta_rows, p.T, p.K, p.E, p.R, p.M) * row_bytes > kExpandedBytesInCache;
     return between_padding || rows_per_token(p) * p.T * row_bytes > 110e6;
+}
+
+// Column tile per wavefront: 1 KB of a BF16 row (512 channels, 41 registers, eight wavefronts per SIMD), or 2 KB, which repeats the routing
+// work half as often and has half the wavefronts to hide its loads with.  2 KB for few rows a token (top-2, or two ranks), where the routing is
+// as much as the rows, from three quarters of the places on, beyond what kb_of_wavefront settles; V1 rows, whose routing is shorter, from a full round on.  Change by 2 KB tiles in %
+// at 0.55 / 0.8 / 1.0 / 1.1 / 1.4 / 4 times as many wavefronts of 1 KB as places (730 shapes, rows of 2 to 14 KB):
+//   compact, top-2 of 2 ranks, 8 KB rows    +1.2 / -2.2 / -4.0 / -8.0 / -7.6 / -8.5;   top-2 of 8 ranks +0.6 / +0.5 / -1.5 / -5.8 / -8.2 / -4.4
+//   expanded, top-2                          +0.5 / -3.0 / -6.1 / -7.9 / -1.3 / -2.7
+//   V1, top-2 of 8 ranks, 4 KB rows          +2.4 / +3.2 / +1.0 / -5.8 / -5.1
+//   more rows a token, up to one round: compact top-8 of 8 ranks -3 to +5, expanded top-8 -2 to +9, V1 top-8 -1 to +9
+// A last tile that is half idle costs what the others gain: rows of 3 KB, expanded, top-2, 0.0 / +3.0 / +12.3 / +4.6 / +1.6 / +5.4; compact
+// +0.6 / -0.5 / +2.0 / -7.1 / -8.1 / -2.2.
+bool takes_two_kb_tiles(const CombineParams& p) {
+    const int kb = (p.H * 2 + 1023) / 1024;
+    if (!reads_past_the_cache(p)) {
+        const int same = kb_of_wavefront(p.T, p.H * 2, rows_per_token(p), false);
+        if (same != 0) return same == 2;
+    }
+    if (kb < 2 || rows_per_token(p) >= 2.3) return false;
+    const int64_t places = int64_t(compute_units()) * 8 * kWavesPerBlock, waves = int64_t(p.T) * kb;
+    if (p.rank_mode) return waves > places;
+    const bool half_idle = kb % 2 == 1 && kb < 8;
+    return 4 * waves >= 3 * places && (!half_idle || (!p.do_expand && waves > places));
 }
 
 template <int kVecs, int kLayout>

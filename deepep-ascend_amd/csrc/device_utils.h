@@ -217,6 +217,13 @@ __device__ __forceinline__ unsigned xcd_contiguous_block(unsigned block, unsigne
     return (block % kXcds) * per + block / kXcds;
 }
 
+// Logical workgroup of the `block`-th workgroup behind `front` others, such that logical workgroup i runs on XCD i % 8 as in a launch
+// without them.
+__device__ __forceinline__ unsigned xcd_aligned_block(unsigned block, unsigned front, unsigned num_blocks) {
+    const unsigned eight = block & ~7u;
+    return eight + 8u <= num_blocks ? eight + ((block + front) & 7u) : block;
+}
+
 // Index of this wavefront's work item, as a wave-uniform 32-bit value (kept in scalar registers, so the
 // divisions that split it into (token, tile) are short 32-bit sequences instead of per-lane 64-bit ones).
 __device__ __forceinline__ unsigned wave_work_index(unsigned block, unsigned waves_per_block) {

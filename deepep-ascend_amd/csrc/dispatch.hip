@@ -734,7 +734,10 @@ __device__ __forceinline__ void dispatch_copy(const MoveParams& p) {
     }
     const int lane = threadIdx.x & 63;
     const unsigned mover = blockIdx.x - (kFused ? unsigned(p.count_blocks) + 1u : 0u);
-    const unsigned block = p.xcd_remap ? xcd_contiguous_block(mover, p.num_movers) : mover;
+    unsigned block = p.xcd_remap ? xcd_contiguous_block(mover, p.num_movers) : mover;
+    // the workgroup of the combine that has this one's number runs on the same XCD (kb_of_wavefront)
+    if constexpr (kFused && kCached == kRows)
+        if (!p.xcd_remap) block = xcd_aligned_block(mover, unsigned(p.count_blocks) + 1u, p.num_movers);
     const unsigned work = wave_work_index(block, kWavesPerBlock);
     const bool has_work = work < unsigned(p.T) * unsigned(p.tiles);
     if (!has_work && !kFused) return;
@@ -1466,10 +1469,10 @@ static bool large_move_shape(const MoveParams& p, MoveShape& q) {
 // 2 KB), 512 x 7168 23.0 / 20.6 / 19.7 (3584): left alone; fused cast, 1 / 2 segments, 300 x 7168 18.0 / 18.3, 512 x 2048 16.8 / 17.4,
 // 512 x 7168 (3584) 19.2 / 18.9.  Not in a single launch, where neighbours of the counting workgroups wait: 512 x 2048 BF16 16.7 / 16.5
 // / 15.6, though 300 x 7168 takes 16.7 / 16.3 / 17.5.
-// BF16 rows that stay in the memory-side cache, up to 60 wavefronts of 1 KB per CU, take 1 KB as well: move and combine of 2001 x 2048 over 8
-// ranks 23.8 us, 26.7 with 2 KB, 30.3 with 4.  Beyond, tokens of three rows and more of 4, 8 or 12 KB take 2 KB, 1 / 2 / 4 KB: 4096 x 2048 top-6
-// 38.0 / 38.5 / 43.0;  6000 x 2048 top-4 42.0 / 40.9 / 45.3;  2200 x 6144 top-4 44.1 / 42.2 / 45.7;  3000 x 4096 expanded top-4 47.6 / 46.2 /
-// 50.6; others the widest: 1400 x 7168 47.1 / 47.5 / 44.9, 3500 x 2560 43.7 / 45.7 / 43.7, 9000 x 1400 top-4 45.5 / 45.5 / 43.2.
+// BF16 rows that stay in the memory-side cache take the tile of the combine (kb_of_wavefront); beyond its lines tokens of three rows and more of 4, 8
+// or 12 KB take 2 KB, move and combine with 1 / 2 / 4 KB: 4096 x 2048 top-6 38.0 / 38.5 / 43.0;  6000 x 2048 top-4 42.0 / 40.9 / 45.3;  2200 x 6144
+// top-4 44.1 / 42.2 / 45.7;  3000 x 4096 expanded top-4 47.6 / 46.2 / 50.6; others the widest: 1400 x 7168 47.1 / 47.5 / 44.9, 3500 x 2560 43.7 /
+// 45.7 / 43.7, 9000 x 1400 top-4 45.5 / 45.5 / 43.2.
 static int move_tile(const MoveParams& p) {
     MoveShape large{};
     if (large_move_shape(p, large)) return large.tile;
@@ -1493,11 +1496,13 @@ static int move_tile(const MoveParams& p) {
     }
     if (p.copy_vecs != 0) return p.copy_vecs;
     const int kb = (p.row_bytes + 1023) / 1024;
-    if (wavefronts_per_cu_at_most(1, 8)) return 1;
-    if (p.payload == DEEP_EP_HIP_PAYLOAD_BF16 && !p.fused && cached_side(p) == kRows) {
-        if (int64_t(p.T) * kb <= int64_t(compute_units()) * 60) return 1;
-        if (kb % 4 == 0 && rows >= 3.0) return 2;
+    const bool rows_cached = p.payload == DEEP_EP_HIP_PAYLOAD_BF16 && cached_side(p) == kRows;
+    if (rows_cached) {
+        const int same = kb_of_wavefront(p.T, p.row_bytes, rows, p.fused != 0);
+        if (same != 0) return same;
     }
+    if (wavefronts_per_cu_at_most(1, 8)) return 1;
+    if (rows_cached && !p.fused && kb % 4 == 0 && rows >= 3.0) return 2;
     if (kb > 2 && wavefronts_per_cu_at_most(2, 10)) return 2;
     const int widest = kb <= 1 ? 1 : kb <= 2 ? 2 : 4;
     // Small, latency-bound calls: up to 4 KB per wavefront, so that fewer wavefronts repeat the routing work (4096 rows

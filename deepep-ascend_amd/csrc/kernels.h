@@ -333,6 +333,23 @@ struct LLDispatchParams {
 // Compute units of the current device (asked once per device).
 int compute_units();
 
+// BF16 rows few enough to be read from the caches (T tokens that go to `rows` rows each): the KB of a row that a wavefront of the dispatch writes and
+// a wavefront of the combine reads, the same for both, so that what an XCD has written it finds in its own L2 (0: each takes its own).  Dispatch and
+// combine, us, rows combined as the dispatch has left them / with a pass in between that writes as many others:
+//   a single launch, 4 KB and 1 KB, 2 KB both   206 x 7960 over 8 ranks 24.6 / 29.6, 17.7 / 27.4;   1009 x 3568 28.1 / 37.1, 23.7 / 36.9;   635 x 6808 of 4 27.3
+//                                               / 34.9, 20.6 / 33.2;   past 22 wavefronts of 2 KB a CU 3382 x 1512 top-6 33.4 / 46.3, 34.0 / 48.9: left alone
+//   a move, 4 KB and 1 KB, 1 KB both, 2 KB both 1237 x 2888 top-9 24.5 / 31.9, 19.3 / 32.0, 18.6 / 31.2;   2970 x 1568 31.6 / 39.6, 26.8 / 41.7, 23.2 / 37.7;
+//                                               1982 x 3256 of 32 ranks (7.2 rows) 41.2 / 65.6, 41.4 / 67.9, 38.3 / 65.3;   past 30 a CU 1324 x 5672 expanded 46.7 /
+//                                               66.6, 43.1 / 69.6, 39.7 / 66.2;  2270 x 4000 33.6 / 45.6, 32.4 / 49.0, 30.4 / 47.4: left alone
+// From six and a half rows a token on small calls have 1 KB both (144 x 7072 expanded 25.0 / 30.6, 20.3 / 29.6, on two launches 532 x 5792 of 32 ranks 26.3 / 44.7,
+// with 2 KB 27.3 / 45.4), and so have moves of rows that leave a fourth of their 2 KB tiles empty (2362 x 1064 23.9 / 38.4, with 2 KB 24.7 / 39.2).
+inline int kb_of_wavefront(int64_t T, int row_bytes, double rows, bool single_launch) {
+    const int kb = (row_bytes + 1023) / 1024, tiles = (kb + 1) / 2;
+    const int64_t cus = compute_units();
+    if (rows < 6.5 && row_bytes >= tiles * 1536) return T * tiles <= cus * (single_launch ? 22 : 30) ? 2 : 0;
+    return T * kb <= cus * (single_launch ? 12 : 30) && (rows >= 6.5 || !single_launch) ? 1 : 0;
+}
+
 // LDS a workgroup asks for so that a CU holds at most `per_cu` of them (0: no limit).
 size_t lds_for_residency(int per_cu);
 

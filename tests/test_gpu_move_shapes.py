@@ -59,3 +59,24 @@ def test_every_word_is_its_tokens(name):
     for got, want in zip((recv,) if payload == "bf16" else recv, pair):
         assert torch.equal(got[at].view(torch.uint8), want[tokens].view(torch.uint8))
     buf.check_device_status()
+
+
+@pytest.mark.parametrize("T,H,E,R,K", [
+    (211, 7960, 64, 8, 8), (1, 4096, 8, 4, 2), (7, 2040, 64, 8, 8), (352, 7168, 64, 8, 8), (353, 7168, 64, 8, 8),   # 2 KB; 22 wavefronts of 7168 per CU
+    (437, 7168, 256, 32, 8), (439, 7168, 256, 32, 8), (1409, 4096, 64, 8, 4), (1407, 4088, 64, 8, 4),              # 1 KB: 12
+])
+def test_rows_of_a_single_launch_and_their_sum(T, H, E, R, K):
+    import deep_ep
+    small = rc.small("single", T, 16, E, R, K, seed=62, masked_ratio=0.05)
+    ref = oracle.dispatch(small.x, small.topk_idx, small.topk_weights, E, R, 0, T)
+    x = torch.randn((T, H), generator=torch.Generator(device="cuda").manual_seed(63), device="cuda", dtype=torch.bfloat16)
+    buf = deep_ep.ElasticBuffer(deep_ep.LogicalGroup(0, R), num_max_tokens_per_rank=T, hidden=H, num_topk=K)
+    recv, _, w, handle, _ = buf.dispatch(x, small.topk_idx.cuda(), small.topk_weights.cuda(), num_experts=E, do_cpu_sync=False)
+    n = ref.recv_src_metadata.shape[0]
+    assert torch.equal(handle.recv_src_metadata[:n].cpu(), ref.recv_src_metadata)
+    tokens = handle.recv_src_metadata[:n, 0].long()
+    assert torch.equal(recv[:n].view(torch.int16), x[tokens].view(torch.int16))
+    out, _, _ = buf.combine(recv, handle, topk_weights=w)
+    count = torch.zeros(T, device="cuda").index_add_(0, tokens, torch.ones(n, device="cuda"))
+    assert torch.equal(out, (x.float() * count[:, None]).to(torch.bfloat16))         # equal terms: exact but for the last rounding
+    buf.check_device_status()
