@@ -77,7 +77,9 @@ typedef struct {
                                   mover workgroups; rows copied as they are from less than 64 MB of input, and less than 300 MB
                                   of them (345 MB of rows of up to 4 KB); no compact cast of four rows a token and more with
                                   movers + counting workgroups >= 6 and movers <= 7 for each compute unit; with do_expand less
-                                  than 64 MB of input.  1 = a single launch wherever the shape allows it; 2 = always layout
+                                  than 64 MB of input; with do_zero_padding and an alignment only FP8 rows and casts of 26 to
+                                  64 MB of input, up to 10000 tokens, that make 80 M channels of rows
+                                  and more.  1 = a single launch wherever the shape allows it; 2 = always layout
                                   kernel + move kernel */
     int32_t cast_pairs;        /* fused FP8 cast: 1024-channel segments per wavefront (1, 2, 4, 7, 8; above 2: two launches) */
     int32_t copy_vecs;         /* pass-through payloads: KB of row per wavefront (1, 2, 4, 7, 8) */
@@ -220,9 +222,10 @@ typedef struct {
 int deep_ep_hip_launch_dispatch(const deep_ep_hip_dispatch_args* args, void* stream);
 
 /* How many kernels deep_ep_hip_launch_dispatch would launch for the layout and move phases of these arguments (shape,
- * phases, payload, do_expand, expert_alignment and tuning are read; no pointer is dereferenced, nothing is launched): 1
- * where layout and move share a launch, else one per requested phase; 0 for a move of no tokens.  The zero-padding
- * kernel of an expanded dispatch is not counted.  Negative: an error code.  No counterpart in the reference; for callers
+ * phases, payload, do_expand, do_zero_padding, expert_alignment and tuning are read; no pointer is dereferenced, nothing is
+ * launched): 1 where layout and move share a launch, else one per requested phase; 0 for a move of no tokens.  Padding rows are
+ * zeroed by the move launch; the kernel that does it behind a shared launch, or turns scales stored in blocks into their columns,
+ * is not counted.  Negative: an error code.  No counterpart in the reference; for callers
  * that size graphs or want to know which path a shape takes. */
 int deep_ep_hip_dispatch_kernel_launches(const deep_ep_hip_dispatch_args* args);
 
