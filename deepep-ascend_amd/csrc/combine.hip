@@ -133,17 +133,16 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const CombineParams p
             if (slot < p.num_x_rows) row_c = slot;
             else atomicOr(p.status, DEEP_EP_HIP_STATUS_ROW_OVERFLOW);
         }
-        const uint64_t rows_of_token = __ballot(row_c >= 0);      // taken with every lane active
-        if (tile == 0 && p.out_w != nullptr && lane < p.Kw) {
+        uint64_t rows = __ballot(row_c >= 0);
+        if (tile == 0 && p.out_w != nullptr) {
             float w = 0.f;
-            uint64_t rows = rows_of_token;
-            while (rows) {
+            while (rows) {                                        // by all lanes: any of them is read from
                 const int j = __builtin_ctzll(rows);
                 rows &= rows - 1;
                 const int row = read_lane(row_c, j);
-                if (p.topk_weights != nullptr) w += p.topk_weights[int64_t(row) * p.Kw + lane];
+                if (p.topk_weights != nullptr && lane < p.Kw) w += p.topk_weights[int64_t(row) * p.Kw + lane];
             }
-            p.out_w[int64_t(t) * p.Kw + lane] = w;
+            if (lane < p.Kw) p.out_w[int64_t(t) * p.Kw + lane] = w;
         }
     } else {
         if (lane < p.K && raw >= 0 && raw < p.E) {

@@ -23,6 +23,7 @@ __device__ __forceinline__ uint64_t lanes_below(int lane) {
 }
 
 // Broadcast the value held by `src_lane` (wave-uniform index) to every lane.
+// Lane src_lane must be active: what the compiler moves or reloads inside a branch it fills in for the lanes that took it.
 __device__ __forceinline__ int read_lane(int v, int src_lane) {
     return __builtin_amdgcn_readlane(v, src_lane);
 }

@@ -224,14 +224,14 @@ __device__ __forceinline__ void write_token_metadata(const MoveParams& p, const 
                 }
             }
         }
-        if (base != nullptr) {
-            while (masters) {
-                const int j = __builtin_ctzll(masters);
-                masters &= masters - 1;
-                const uint32_t v = d_src == read_lane(r.d, j) ? match : other;
-                *reinterpret_cast<uint32_t*>(base + uint64_t(uint32_t(read_lane(r.row_c, j))) * stride) =
-                    col == 1 ? uint32_t(p.rank_idx * K + j) : v;
-            }
+        // All lanes walk the rows, also those that store nothing: a lane that is off may not be read from (read_lane).
+        if (__ballot(base != nullptr) == 0ull) return;
+        while (masters) {
+            const int j = __builtin_ctzll(masters);
+            masters &= masters - 1;
+            const uint64_t at = uint64_t(uint32_t(read_lane(r.row_c, j))) * stride;
+            const uint32_t v = d_src == read_lane(r.d, j) ? match : other;
+            if (base != nullptr) *reinterpret_cast<uint32_t*>(base + at) = col == 1 ? uint32_t(p.rank_idx * K + j) : v;
         }
         return;
     }

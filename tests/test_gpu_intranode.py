@@ -214,3 +214,29 @@ def test_per_source_calls_compose_into_the_world():
         assert_equal(torch.cat([p[2] for p in parts[j]]), world[j].recv_topk_weights, f"recv_topk_weights of rank {j}")
         assert_equal(torch.cat([p[3] for p in parts[j]]), world[j].recv_src_idx, f"recv_src_idx of rank {j}")
     assert_equal(prefix_sum, world[0].rank_prefix_matrix, "rank_prefix_matrix summed over the calls")
+
+
+@pytest.mark.parametrize("T,E,R,K", [(37, 64, 64, 1), (261, 32, 32, 1), (130, 62, 31, 2)])
+def test_more_ranks_than_selections(T, E, R, K):
+    """Lanes that store nothing - of ranks past the selections' weights, of rows without top-k tensors - are the ones rows are read from."""
+    import deep_ep
+    c = rc.small("ranks", T, 64, E, R, K, seed=T, masked_ratio=0.05)
+    idx, w = c.topk_idx.cuda(), c.topk_weights.cuda()
+    buf = deep_ep.Buffer(deep_ep.LogicalGroup(0, R))
+    per_rank, _, per_expert, mask_d, _ = buf.get_dispatch_layout(idx, E)
+    mask = oracle.layout(c.topk_idx, E, R)[2]
+    for with_topk in ([True, False] if R <= 32 else [True]):
+        ref = oracle.intranode_dispatch(c.x, mask, c.topk_idx if with_topk else None, c.topk_weights if with_topk else None, E, R, 0, 1, 10)
+        kw = dict(topk_idx=idx, topk_weights=w) if with_topk else {}
+        recv, ri, rw, _, handle, _ = buf.dispatch(c.x.cuda(), num_tokens_per_rank=per_rank, is_token_in_rank=mask_d, num_tokens_per_expert=per_expert, **kw)
+        assert_equal(recv.view(torch.int16), ref.recv_x.view(torch.int16), "recv_x")
+        assert_equal(handle[3], ref.recv_src_idx, "recv_src_idx")
+        assert_equal(handle[5], ref.send_head, "send_head")
+        out, out_w, _ = buf.combine(recv, handle, topk_weights=rw)
+        ref_out, ref_w = oracle.intranode_combine(ref.recv_x, ref.send_head, ref.recv_topk_weights if with_topk else None, None)
+        assert_equal(out + 0.0, ref_out + 0.0, "combined_x")
+        if with_topk:
+            assert_equal(ri, ref.recv_topk_idx, "recv_topk_idx")
+            assert_equal(rw, ref.recv_topk_weights, "recv_topk_weights")
+            assert_equal(out_w, ref_w, "combined_topk_weights")
+    buf.runtime.check_device_status("intranode")
