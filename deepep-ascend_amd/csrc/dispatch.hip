@@ -193,7 +193,7 @@ __device__ __forceinline__ void write_token_metadata(const MoveParams& p, const 
     if (p.do_expand && p.recv_topk_weights != nullptr && r.erow >= 0 && r.erow < p.expanded_capacity)
         p.recv_topk_weights[r.erow] = r.w;
     if (p.do_expand || 4 * K + 2 <= kWaveSize) {
-        const int col = p.do_expand ? lane : lane - 3 * K;                        // metadata column (negative: none)
+        int col = p.do_expand ? lane : lane - 3 * K;                              // metadata column (negative: none)
         int src = col - 2;                                                        // routing lane this wave lane reports on
         if (!p.do_expand && lane < 2 * K) src = lane >> 1;
         else if (!p.do_expand && lane < 3 * K) src = lane - 2 * K;
@@ -224,14 +224,33 @@ __device__ __forceinline__ void write_token_metadata(const MoveParams& p, const 
                 }
             }
         }
-        // All lanes walk the rows, also those that store nothing: a lane that is off may not be read from (read_lane).
-        if (__ballot(base != nullptr) == 0ull) return;
-        while (masters) {
-            const int j = __builtin_ctzll(masters);
-            masters &= masters - 1;
-            const uint64_t at = uint64_t(uint32_t(read_lane(r.row_c, j))) * stride;
-            const uint32_t v = d_src == read_lane(r.d, j) ? match : other;
-            if (base != nullptr) *reinterpret_cast<uint32_t*>(base + at) = col == 1 ? uint32_t(p.rank_idx * K + j) : v;
+        // The routing lanes walk the rows with those that store, as they are read from (read_lane): one that has nothing to store itself (V1 without
+        // top-k tensors) repeats what the first lane that has stores, the same word to the same place.
+        const uint64_t storing = __ballot(base != nullptr);
+        if (storing == 0ull) return;
+        int rank = d_src;
+        if (__ballot(lane < K && base == nullptr) != 0ull) {
+            const int like = __builtin_ctzll(storing);
+            const uint32_t lo = uint32_t(read_lane(int(uint64_t(base)), like)), hi = uint32_t(read_lane(int(uint64_t(base) >> 32), like));
+            const uint32_t its_match = uint32_t(read_lane(int(match), like)), its_other = uint32_t(read_lane(int(other), like));
+            const int its_rank = read_lane(d_src, like), its_col = read_lane(col, like), its_stride = read_lane(int(stride), like);
+            if (lane < K && base == nullptr) {
+                base = reinterpret_cast<uint8_t*>(uint64_t(hi) << 32 | lo);
+                stride = uint32_t(its_stride);
+                match = its_match;
+                other = its_other;
+                rank = its_rank;
+                col = its_col;
+            }
+        }
+        if (base != nullptr) {
+            while (masters) {
+                const int j = __builtin_ctzll(masters);
+                masters &= masters - 1;
+                const uint32_t v = rank == read_lane(r.d, j) ? match : other;
+                *reinterpret_cast<uint32_t*>(base + uint64_t(uint32_t(read_lane(r.row_c, j))) * stride) =
+                    col == 1 ? uint32_t(p.rank_idx * K + j) : v;
+            }
         }
         return;
     }
