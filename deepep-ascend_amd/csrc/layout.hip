@@ -74,6 +74,11 @@ __global__ __launch_bounds__(kThreads) void intranode_prefix_kernel(const Intran
     channel_prefix_block<kWaves>(p, int(blockIdx.x), reinterpret_cast<int*>(bitmap));
 }
 
+// Up to so many selections a token there is a kernel for each number of them, of 30 KB; beyond, one for up to 12, 16, 20 and 32.  Layout and a move of
+// 16 channels, us, with a kernel for up to 8 (and two chunks in a workgroup each) / its own: 450 tokens top-3 of 64 10.0 / 8.6, top-5 10.4 / 9.2, top-7 10.7 / 9.7;
+// 4096 top-3 of 256 12.0 / 11.4, top-7 12.9 / 12.7; 12000 of 32 ranks top-3 17.6 / 16.9, top-5 19.5 / 19.1.
+constexpr int kOwnKernels = 10;
+
 // LDS of a counting workgroup: bitmap words [R + E][waves], spare 32-bit words, and the packed words of the buckets' chunks [R + E][chunks].
 constexpr int kSpareWords = kWaveSize;
 
@@ -296,12 +301,12 @@ __global__ __launch_bounds__(kThreads * (kHeldChunks > 1 ? kHeldChunks : 1)) voi
 template <int KMAX, bool kExact>
 void launch_layout(const LayoutParams& q, const IntranodePrefixParams& prefix, dim3 grid, size_t lds, int held_chunks, hipStream_t stream) {
     const bool by_one = fits_one_trip(1, q.R, q.E, q.tab.chunks_padded, kThreads), by_two = fits_one_trip(2, q.R, q.E, q.tab.chunks_padded, kThreads);
-    constexpr int kMostHeld = kExact ? 2 : 1;
-    auto kernel = held_chunks == 2   ? layout_kernel<KMAX, kExact, kMostHeld, 1>
-                  : held_chunks == 1 ? (by_one ? layout_kernel<KMAX, kExact, 1, 1> : layout_kernel<KMAX, kExact, 1, 2>)
-                  : by_one           ? layout_kernel<KMAX, kExact, 0, 1>
-                  : by_two           ? layout_kernel<KMAX, kExact, 0, 2>
-                                     : layout_kernel<KMAX, kExact, 0, 0>;
+    auto kernel = held_chunks == 1 ? (by_one ? layout_kernel<KMAX, kExact, 1, 1> : layout_kernel<KMAX, kExact, 1, 2>)
+                  : by_one         ? layout_kernel<KMAX, kExact, 0, 1>
+                  : by_two         ? layout_kernel<KMAX, kExact, 0, 2>
+                                   : layout_kernel<KMAX, kExact, 0, 0>;
+    if constexpr (kExact)
+        if (held_chunks == 2) kernel = layout_kernel<KMAX, kExact, 2, 1>;
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads * std::max(held_chunks, 1)), lds, stream, q, prefix);
 }
 
@@ -321,10 +326,9 @@ hipError_t launch_layout_kernel(const LayoutParams& p, const IntranodePrefixPara
     // totals and the publishing step's scratch behind it.
     // Two chunks in one workgroup / in one each, us, 450 tokens: top-8 of 256 over 8 ranks 6.4 / 6.8, top-3 of 64 5.2 / 6.7; of more buckets than threads,
     // or with a kernel for up to so many selections, the one workgroup is behind: top-12 of 256 over 64 ranks 12.6 / 10.5, top-16 of 512 17.0 / 13.7.
-    const bool one_kernel_each = p.K <= 10 && p.K != 3 && p.K != 5 && p.K != 7;
-    const int held_chunks = num_chunks == 1 && p.R <= kThreads && p.E <= 2 * kThreads                                  ? 1
-                            : num_chunks == 2 && one_kernel_each && p.R + p.E <= 320 && p.R <= kThreads                ? 2
-                                                                                                                       : 0;
+    const int held_chunks = num_chunks == 1 && p.R <= kThreads && p.E <= 2 * kThreads                      ? 1
+                            : num_chunks == 2 && p.K <= kOwnKernels && p.R + p.E <= 320 && p.R <= kThreads ? 2
+                                                                                                           : 0;
     const int chunks = std::max(held_chunks, 1);
     LayoutParams q = p;
     q.vec_idx = (reinterpret_cast<uintptr_t>(p.topk_idx) % 16 == 0) ? 1 : 0;
@@ -334,18 +338,21 @@ hipError_t launch_layout_kernel(const LayoutParams& p, const IntranodePrefixPara
     if (held_chunks == 0) lds = std::max(lds, publish_lds_bytes(p.R, p.E, kThreads));
     if (prefix.R != 0) lds = std::max(lds, size_t(prefix.C) * sizeof(int));
     const dim3 grid((held_chunks > 0 ? 1 : num_chunks) + prefix.R);
-    const auto launch = [&](auto kernels) { kernels(q, prefix, grid, lds, held_chunks, stream); };      // one_kernel_each: the numbers of selections in use
+    const auto launch = [&](auto kernels) { kernels(q, prefix, grid, lds, held_chunks, stream); };
+    static_assert(kOwnKernels == 10, "one case for each");
     switch (p.K) {
         case 1: launch(launch_layout<1, true>); break;
         case 2: launch(launch_layout<2, true>); break;
+        case 3: launch(launch_layout<3, true>); break;
         case 4: launch(launch_layout<4, true>); break;
+        case 5: launch(launch_layout<5, true>); break;
         case 6: launch(launch_layout<6, true>); break;
+        case 7: launch(launch_layout<7, true>); break;
         case 8: launch(launch_layout<8, true>); break;
         case 9: launch(launch_layout<9, true>); break;
         case 10: launch(launch_layout<10, true>); break;
         default:
-            if (p.K <= 8) launch(launch_layout<8, false>);
-            else if (p.K <= 12) launch(launch_layout<12, false>);
+            if (p.K <= 12) launch(launch_layout<12, false>);
             else if (p.K <= 16) launch(launch_layout<16, false>);
             else if (p.K <= 20) launch(launch_layout<20, false>);
             else launch(launch_layout<32, false>);
