@@ -53,8 +53,9 @@ struct LaunchPlan {
     bool fused;       // one launch: counting workgroups at the front of the move kernel
 };
 
-LaunchPlan plan_launches(int T, int K, int E, int R, bool do_layout, bool do_move, bool do_expand, bool do_zero_padding, int alignment, int payload, int H,
-                         int row_bytes, const deep_ep_hip_tuning& tuning, int64_t rows_of_rank_lanes = -1 /* no top-k: rows received */) {
+LaunchPlan plan_launches(const MoveParams& m, bool do_layout, bool do_move, bool do_zero_padding, int alignment, const deep_ep_hip_tuning& tuning) {
+    const int T = m.T, K = m.K, E = m.E, R = m.R, H = m.H, row_bytes = m.row_bytes, payload = m.payload;
+    const bool do_expand = m.do_expand != 0;
     LaunchPlan q{};
     q.chunks = T > 0 ? (T + kLayoutChunk - 1) / kLayoutChunk : 1;
     q.chunks_padded = (q.chunks + 3) / 4 * 4;
@@ -84,14 +85,87 @@ LaunchPlan plan_launches(int T, int K, int E, int R, bool do_layout, bool do_mov
     if (q.fused && do_zero_padding && alignment > 1 && tuning.dispatch_launches != 1)
         q.fused = payload != DEEP_EP_HIP_PAYLOAD_BF16 && int64_t(T) * row_bytes >= 26000000 && int64_t(T) * K * H >= 80000000 && T <= 10000;
     if (q.fused && tuning.dispatch_launches != 1) {
-        MoveParams probe{};
-        probe.T = T; probe.H = H; probe.row_bytes = row_bytes; probe.payload = payload; probe.do_expand = do_expand ? 1 : 0;
-        probe.cast_pairs = tuning.cast_pairs; probe.copy_vecs = tuning.copy_vecs;
-        probe.K = K; probe.R = R; probe.fused = 1;
-        probe.rank_lanes = rows_of_rank_lanes >= 0 ? 1 : 0; probe.recv_capacity = rows_of_rank_lanes;
-        q.fused = !move_prefers_finished_layout(probe, q.chunks);
+        MoveParams single = m;
+        single.fused = 1;
+        q.fused = !move_prefers_finished_layout(single, q.chunks);
     }
     return q;
+}
+
+int bytes_per_element(int payload) { return payload == DEEP_EP_HIP_PAYLOAD_FP8 ? 1 : 2; }
+
+bool known_payload(int payload) {
+    return payload == DEEP_EP_HIP_PAYLOAD_BF16 || payload == DEEP_EP_HIP_PAYLOAD_FP8 || payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8;
+}
+
+void set_knobs(MoveParams& m, const deep_ep_hip_tuning& tuning) {
+    m.cast_pairs = tuning.cast_pairs; m.copy_vecs = tuning.copy_vecs;
+    m.mover_spin_limit = tuning.mover_spin_limit > 0 ? unsigned(tuning.mover_spin_limit) : (1u << 22);   // seconds
+    m.move_workgroups_per_cu = tuning.move_workgroups_per_cu;
+    m.warm_rounds = tuning.warm_rounds;
+    m.persistent_movers = tuning.persistent_movers;
+    m.plain_loads = tuning.plain_loads; m.xcd_remap = tuning.xcd_remap;
+}
+
+// What a move is chosen by - the launches, its tile, what a CU holds, what goes through the caches - as far as the arguments say it.
+MoveParams shape_of_move(const deep_ep_hip_dispatch_args* a) {
+    MoveParams m{};
+    m.T = a->num_tokens; m.H = a->hidden; m.K = a->num_topk; m.E = a->num_experts; m.R = a->num_ranks; m.E_l = m.E / m.R;
+    m.rank_idx = a->rank_idx; m.M = a->num_max_tokens_per_rank;
+    m.cached = a->cached ? 1 : 0;
+    m.do_expand = a->do_expand ? 1 : 0;
+    m.payload = a->payload;
+    m.row_bytes = m.H * bytes_per_element(a->payload);
+    m.recv_capacity = a->recv_capacity;
+    m.expanded_capacity = a->expanded_capacity;
+    m.num_sf_packs = a->num_sf_packs;
+    m.recv_sf = static_cast<uint32_t*>(a->recv_sf);
+    m.rsf_ts = a->recv_sf_token_stride; m.rsf_hs = a->recv_sf_hidden_stride;
+    if (a->do_zero_padding) {
+        const int64_t selections = int64_t(m.T) * m.K, regions = std::min<int64_t>(m.E, selections) * a->expert_alignment;
+        m.zeroed_rows = int(std::min<int64_t>(std::max(int64_t(m.E) * (a->expert_alignment - 1) / 2, regions - selections), INT32_MAX));
+    }
+    set_knobs(m, a->tuning);
+    return m;
+}
+
+MoveParams shape_of_move(const deep_ep_hip_intranode_dispatch_args* a, bool with_topk) {
+    MoveParams m{};
+    m.T = a->num_tokens; m.H = a->hidden; m.R = a->num_ranks;
+    m.K = with_topk ? a->num_topk : m.R; m.E = with_topk ? a->num_experts : m.R; m.E_l = m.E / m.R;
+    m.rank_idx = a->rank_idx; m.M = m.T > 0 ? m.T : 1;
+    m.cached = a->cached ? 1 : 0;
+    m.payload = a->payload;
+    m.row_bytes = m.H * bytes_per_element(a->payload);
+    m.recv_capacity = a->recv_capacity;
+    m.num_sf_packs = a->num_scales;
+    m.recv_sf = static_cast<uint32_t*>(a->recv_x_scales);
+    m.rsf_ts = a->recv_scale_token_stride; m.rsf_hs = a->recv_scale_hidden_stride;
+    m.rank_lanes = with_topk ? 0 : 1;
+    set_knobs(m, a->tuning);
+    return m;
+}
+
+CombineParams shape_of_combine(const deep_ep_hip_combine_args* a) {
+    CombineParams p{};
+    p.T = a->num_tokens; p.H = a->hidden; p.K = a->num_topk; p.E = a->num_experts; p.R = a->num_ranks; p.E_l = p.E / p.R;
+    p.rank_idx = a->rank_idx; p.M = a->num_max_tokens_per_rank;
+    p.num_x_rows = a->num_x_rows;
+    p.num_meta_rows = a->num_recv_rows;
+    p.do_expand = a->do_expand ? 1 : 0;
+    p.multi_red = a->allow_multiple_reduction ? 1 : 0;
+    p.vecs = a->tuning.combine_vecs;
+    return p;
+}
+
+CombineParams shape_of_combine(const deep_ep_hip_intranode_combine_args* a) {
+    CombineParams p{};
+    p.T = a->num_tokens; p.H = a->hidden; p.K = a->num_ranks; p.E = a->num_ranks; p.R = a->num_ranks; p.E_l = 1;
+    p.num_x_rows = a->num_x_rows;
+    p.rank_mode = 1;
+    p.Kw = a->num_topk;
+    p.vecs = a->tuning.combine_vecs;
+    return p;
 }
 
 LayoutTables carve_tables(uint8_t* ws, const WorkspaceLayout& w, int num_tokens, int num_experts) {
@@ -296,8 +370,8 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
     // chunk), the first row of that chunk's share of the bucket; the move kernel adds the two.  Layout and move in
     // one call: the counting workgroups ride at the front of the move kernel (one launch); shapes that does not
     // cover run the layout kernel first.
-    const LaunchPlan plan = plan_launches(T, K, E, R, do_layout, do_move, a->do_expand != 0, a->do_zero_padding != 0, a->expert_alignment, a->payload, H,
-                                          H * elem_in, a->tuning);
+    MoveParams m = shape_of_move(a);
+    const LaunchPlan plan = plan_launches(m, do_layout, do_move, a->do_zero_padding != 0, a->expert_alignment, a->tuning);
     LayoutParams lay{};
     lay.topk_idx = a->topk_idx;
     lay.T = T; lay.K = K; lay.E = E; lay.R = R; lay.E_l = E / R;
@@ -315,11 +389,9 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
     }
 
     if (do_move) {
-        MoveParams m{};
         m.x = static_cast<const uint8_t*>(a->x);
         m.sf = static_cast<const uint32_t*>(a->sf);
         m.sf_ts = a->sf_token_stride; m.sf_hs = a->sf_hidden_stride;
-        m.num_sf_packs = a->num_sf_packs;
         m.topk_idx = a->topk_idx;
         m.topk_weights = a->topk_weights;
         m.pos = reinterpret_cast<const uint32_t*>(ws + w.pos);
@@ -329,35 +401,15 @@ int dispatch_with_workspace(const deep_ep_hip_dispatch_args* a, void* workspace,
         m.psum_rank = a->psum_num_recv_tokens_per_rank;
         m.recv_src_metadata = a->recv_src_metadata;
         m.recv_x = static_cast<uint8_t*>(a->recv_x);
-        m.recv_sf = static_cast<uint32_t*>(a->recv_sf);
-        m.rsf_ts = a->recv_sf_token_stride; m.rsf_hs = a->recv_sf_hidden_stride;
         m.recv_topk_idx = a->recv_topk_idx;
         m.recv_topk_weights = a->topk_weights != nullptr ? a->recv_topk_weights : nullptr;
-        m.recv_capacity = a->recv_capacity;
-        m.expanded_capacity = a->expanded_capacity;
-        m.T = T; m.H = H; m.K = K; m.E = E; m.R = R; m.E_l = E / R;
-        m.rank_idx = a->rank_idx; m.M = a->num_max_tokens_per_rank;
-        m.cached = a->cached ? 1 : 0;
-        m.do_expand = a->do_expand ? 1 : 0;
-        m.payload = a->payload;
-        m.row_bytes = H * elem_in;
         m.tab = lay.tab;
         m.pub = pub;
         m.status = status;
-        m.cast_pairs = a->tuning.cast_pairs; m.copy_vecs = a->tuning.copy_vecs;
-        m.mover_spin_limit = a->tuning.mover_spin_limit > 0 ? unsigned(a->tuning.mover_spin_limit) : (1u << 22);   // seconds
-        m.move_workgroups_per_cu = a->tuning.move_workgroups_per_cu;
-        m.warm_rounds = a->tuning.warm_rounds;
-        m.persistent_movers = a->tuning.persistent_movers;
-        m.plain_loads = a->tuning.plain_loads; m.xcd_remap = a->tuning.xcd_remap;
         m.gates = reinterpret_cast<uint32_t*>(ws + w.gates);               // a persistent move kernel keeps its item counter there
         m.gates_finished = reinterpret_cast<uint32_t*>(ws + w.gates_finished);
         if (plan.fused) fill_fused(m, lay, plan, ws, w);
         m.sf_blocked = a->do_zero_padding && scales_in_blocks(m, a->expert_alignment) ? 1 : 0;
-        if (a->do_zero_padding) {
-            const int64_t selections = int64_t(T) * K, regions = std::min<int64_t>(E, selections) * a->expert_alignment;
-            m.zeroed_rows = int(std::min<int64_t>(std::max(int64_t(E) * (a->expert_alignment - 1) / 2, regions - selections), INT32_MAX));
-        }
 
         const bool pads = a->do_zero_padding && a->expert_alignment > 1;
         PadParams z{};
@@ -473,14 +525,60 @@ int deep_ep_hip_dispatch_kernel_launches(const deep_ep_hip_dispatch_args* a) {
     const bool do_layout = (a->phases & DEEP_EP_HIP_PHASE_LAYOUT) != 0;
     const bool do_move = (a->phases & DEEP_EP_HIP_PHASE_MOVE) != 0;
     REQUIRE(do_layout || do_move, "phases selects nothing");
-    REQUIRE(a->payload == DEEP_EP_HIP_PAYLOAD_BF16 || a->payload == DEEP_EP_HIP_PAYLOAD_FP8 ||
-            a->payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8, "unknown payload kind %d", a->payload);
+    REQUIRE(known_payload(a->payload), "unknown payload kind %d", a->payload);
     if (a->num_tokens == 0) return do_layout ? 1 : 0;      // an empty move launches nothing
-    const int elem_in = a->payload == DEEP_EP_HIP_PAYLOAD_FP8 ? 1 : 2;
-    const LaunchPlan plan = plan_launches(a->num_tokens, a->num_topk, a->num_experts, a->num_ranks, do_layout, do_move,
-                                          a->do_expand != 0, a->do_zero_padding != 0, a->expert_alignment, a->payload, a->hidden, a->hidden * elem_in,
-                                          a->tuning);
+    const LaunchPlan plan = plan_launches(shape_of_move(a), do_layout, do_move, a->do_zero_padding != 0, a->expert_alignment, a->tuning);
     return plan.fused ? 1 : int(do_layout) + int(do_move);
+}
+
+static int tell_move_shape(MoveParams m, const LaunchPlan& plan, bool blocked, deep_ep_hip_move_shape* out) {
+    *out = deep_ep_hip_move_shape{};
+    if (m.T == 0) return DEEP_EP_HIP_OK;
+    m.fused = plan.fused ? 1 : 0;
+    m.sf_blocked = blocked ? 1 : 0;
+    const MoveChoice c = choose_move(m);
+    out->single_launch = m.fused;
+    out->tile = c.tile;
+    out->workgroups_per_cu = c.per_cu;
+    out->rows_in_turn = c.in_turn;
+    out->cached_side = c.cached_side;
+    out->blocked_scales = m.sf_blocked;
+    return DEEP_EP_HIP_OK;
+}
+
+int deep_ep_hip_dispatch_move_shape(const deep_ep_hip_dispatch_args* a, deep_ep_hip_move_shape* out) {
+    REQUIRE(a != nullptr && out != nullptr, "args is NULL");
+    if (int rc = check_routing_shape(a->num_tokens, a->num_topk, a->num_experts, a->num_ranks)) return rc;
+    REQUIRE(known_payload(a->payload), "unknown payload kind %d", a->payload);
+    REQUIRE(a->hidden >= 1 && int64_t(a->hidden) * 2 < (int64_t(1) << 30) && a->expert_alignment >= 1, "bad shape");
+    MoveParams m = shape_of_move(a);
+    const LaunchPlan plan = plan_launches(m, (a->phases & DEEP_EP_HIP_PHASE_LAYOUT) != 0, true, a->do_zero_padding != 0, a->expert_alignment, a->tuning);
+    m.fused = plan.fused ? 1 : 0;
+    return tell_move_shape(m, plan, a->do_zero_padding && scales_in_blocks(m, a->expert_alignment), out);
+}
+
+int deep_ep_hip_intranode_move_shape(const deep_ep_hip_intranode_dispatch_args* a, deep_ep_hip_move_shape* out) {
+    REQUIRE(a != nullptr && out != nullptr, "args is NULL");
+    const bool with_topk = a->num_topk > 0;
+    REQUIRE(a->num_ranks >= 1, "num_ranks must be positive");
+    if (int rc = check_routing_shape(a->num_tokens, with_topk ? a->num_topk : a->num_ranks, with_topk ? a->num_experts : a->num_ranks, a->num_ranks)) return rc;
+    REQUIRE(known_payload(a->payload), "unknown payload kind %d", a->payload);
+    REQUIRE(a->hidden >= 1 && int64_t(a->hidden) * 2 < (int64_t(1) << 30), "bad shape");
+    const MoveParams m = shape_of_move(a, with_topk);
+    return tell_move_shape(m, plan_launches(m, (a->phases & DEEP_EP_HIP_PHASE_LAYOUT) != 0, true, false, 1, a->tuning), false, out);
+}
+
+int deep_ep_hip_combine_tile(const deep_ep_hip_combine_args* a) {
+    REQUIRE(a != nullptr, "args is NULL");
+    if (int rc = check_routing_shape(a->num_tokens, a->num_topk, a->num_experts, a->num_ranks)) return rc;
+    REQUIRE(a->hidden >= 1 && a->num_x_rows >= 0, "bad shape");
+    return combine_tile(shape_of_combine(a));
+}
+
+int deep_ep_hip_intranode_combine_tile(const deep_ep_hip_intranode_combine_args* a) {
+    REQUIRE(a != nullptr, "args is NULL");
+    REQUIRE(a->num_tokens >= 0 && a->num_ranks >= 1 && a->num_topk >= 0 && a->hidden >= 1 && a->num_x_rows >= 0, "bad shape");
+    return combine_tile(shape_of_combine(a));
 }
 
 int deep_ep_hip_launch_dispatch_static(const deep_ep_hip_dispatch_args* a, void* stream_) {
@@ -530,26 +628,18 @@ int deep_ep_hip_launch_combine(const deep_ep_hip_combine_args* a, void* stream) 
         if (err != hipSuccess) return hip_fail(err, "slot map launch");
         slot = q.slot;
     }
-    CombineParams p{};
+    CombineParams p = shape_of_combine(a);
     p.x = static_cast<const uint8_t*>(a->x);
-    p.num_x_rows = a->num_x_rows;
     p.topk_weights = a->topk_weights;
     p.bias0 = static_cast<const uint8_t*>(a->bias_0);
     p.bias1 = static_cast<const uint8_t*>(a->bias_1);
     p.topk_idx = a->topk_idx;
     p.slot = slot;
     p.meta = a->recv_src_metadata;
-    p.num_meta_rows = a->num_recv_rows;
     p.psum_rank = a->psum_num_recv_tokens_per_rank;
     p.out = static_cast<uint8_t*>(a->combined_x);
     p.out_w = a->combined_topk_weights;
-    p.T = a->num_tokens; p.H = a->hidden; p.K = a->num_topk; p.E = a->num_experts; p.R = a->num_ranks;
-    p.E_l = p.E / p.R;
-    p.rank_idx = a->rank_idx; p.M = a->num_max_tokens_per_rank;
-    p.do_expand = a->do_expand ? 1 : 0;
-    p.multi_red = a->allow_multiple_reduction ? 1 : 0;
     p.status = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(a->workspace));
-    p.vecs = a->tuning.combine_vecs;
     hipError_t err = launch_combine_kernel(p, static_cast<hipStream_t>(stream));
     if (err != hipSuccess) return hip_fail(err, "combine launch");
     return DEEP_EP_HIP_OK;
@@ -629,8 +719,8 @@ int deep_ep_hip_launch_intranode_dispatch(const deep_ep_hip_intranode_dispatch_a
     pub.expert_start = reinterpret_cast<int32_t*>(ws + w.expert_start);
     pub.totals_out = reinterpret_cast<int32_t*>(ws + w.totals);
 
-    const LaunchPlan plan = plan_launches(T, K, E, R, do_layout, do_move, false, false, 1, a->payload, H, H * elem_in, a->tuning,
-                                          with_topk ? -1 : a->recv_capacity);
+    MoveParams m = shape_of_move(a, with_topk);
+    const LaunchPlan plan = plan_launches(m, do_layout, do_move, false, 1, a->tuning);
     LayoutParams lay{};
     lay.topk_idx = a->topk_idx;
     lay.route_mask = with_topk ? nullptr : a->is_token_in_rank;
@@ -657,47 +747,26 @@ int deep_ep_hip_launch_intranode_dispatch(const deep_ep_hip_intranode_dispatch_a
     }
 
     if (do_move) {
-        MoveParams m{};
         m.x = static_cast<const uint8_t*>(a->x);
         m.sf = static_cast<const uint32_t*>(a->x_scales);
         m.sf_ts = a->scale_token_stride; m.sf_hs = a->scale_hidden_stride;
-        m.num_sf_packs = a->num_scales;
         m.topk_idx = a->topk_idx;
         m.route_mask = (with_topk || a->cached) ? nullptr : a->is_token_in_rank;
         m.topk_weights = a->topk_weights;
         m.pos = reinterpret_cast<const uint32_t*>(ws + w.pos);
         m.expert_start = reinterpret_cast<const int32_t*>(ws + w.expert_start);
         m.cached_slot = a->send_head;
-        m.dst_buffer_slot_idx = nullptr;
         m.psum_rank = a->psum_num_recv_tokens_per_rank;
-        m.recv_src_metadata = nullptr;
         m.recv_x = static_cast<uint8_t*>(a->recv_x);
-        m.recv_sf = static_cast<uint32_t*>(a->recv_x_scales);
-        m.rsf_ts = a->recv_scale_token_stride; m.rsf_hs = a->recv_scale_hidden_stride;
         m.recv_topk_idx = with_topk ? a->recv_topk_idx : nullptr;
         m.recv_topk_weights = with_topk ? a->recv_topk_weights : nullptr;
-        m.recv_capacity = a->recv_capacity;
-        m.expanded_capacity = 0;
-        m.T = T; m.H = H; m.K = K; m.E = E; m.R = R; m.E_l = E / R;
-        m.rank_idx = a->rank_idx; m.M = T > 0 ? T : 1;
-        m.cached = a->cached ? 1 : 0;
-        m.do_expand = 0;
-        m.payload = a->payload;
-        m.row_bytes = H * elem_in;
         m.tab = lay.tab;
         m.pub = pub;
         m.status = status;
-        m.cast_pairs = a->tuning.cast_pairs; m.copy_vecs = a->tuning.copy_vecs;
-        m.mover_spin_limit = a->tuning.mover_spin_limit > 0 ? unsigned(a->tuning.mover_spin_limit) : (1u << 22);   // seconds
-        m.move_workgroups_per_cu = a->tuning.move_workgroups_per_cu;
-        m.warm_rounds = a->tuning.warm_rounds;
-        m.persistent_movers = a->tuning.persistent_movers;
-        m.plain_loads = a->tuning.plain_loads; m.xcd_remap = a->tuning.xcd_remap;
         m.gates = reinterpret_cast<uint32_t*>(ws + w.gates);               // a persistent move kernel keeps its item counter there
         m.gates_finished = reinterpret_cast<uint32_t*>(ws + w.gates_finished);
         if (plan.fused) fill_fused(m, lay, plan, ws, w);
 
-        m.rank_lanes = with_topk ? 0 : 1;
         m.slot_is_row = a->cached ? 1 : 0;
         m.zero_nonlocal_w = 1;
         m.send_head = a->cached ? nullptr : a->send_head;
@@ -730,20 +799,15 @@ int deep_ep_hip_launch_intranode_combine(const deep_ep_hip_intranode_combine_arg
     REQUIRE(!any || a->x != nullptr || a->num_x_rows == 0, "x is NULL");
     REQUIRE(a->num_topk == 0 || a->topk_weights == nullptr || a->combined_topk_weights != nullptr, "combined_topk_weights is NULL");
     REQUIRE(a->workspace != nullptr && a->workspace_bytes >= 256, "workspace is NULL or smaller than 256 bytes");
-    CombineParams p{};
+    CombineParams p = shape_of_combine(a);
     p.x = static_cast<const uint8_t*>(a->x);
-    p.num_x_rows = a->num_x_rows;
     p.topk_weights = a->topk_weights;
     p.bias0 = static_cast<const uint8_t*>(a->bias_0);
     p.bias1 = static_cast<const uint8_t*>(a->bias_1);
     p.slot = a->send_head;
     p.out = static_cast<uint8_t*>(a->combined_x);
     p.out_w = a->num_topk > 0 ? a->combined_topk_weights : nullptr;
-    p.T = a->num_tokens; p.H = a->hidden; p.K = a->num_ranks; p.E = a->num_ranks; p.R = a->num_ranks; p.E_l = 1;
-    p.rank_mode = 1;
-    p.Kw = a->num_topk;
     p.status = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(a->workspace));
-    p.vecs = a->tuning.combine_vecs;
     hipError_t err = launch_combine_kernel(p, static_cast<hipStream_t>(stream));
     if (err != hipSuccess) return hip_fail(err, "intranode combine launch");
     return DEEP_EP_HIP_OK;

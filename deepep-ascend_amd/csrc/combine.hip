@@ -404,10 +404,14 @@ hipError_t launch_rebuild_slot_map(const SlotMapParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
+int combine_tile(const CombineParams& p) {
+    if (p.vecs != 0) return p.vecs == 1 || p.vecs == 4 ? p.vecs : 2;
+    return p.T > 0 && takes_two_kb_tiles(p) ? 2 : 1;
+}
+
 hipError_t launch_combine_kernel(CombineParams p, hipStream_t stream) {
     if (p.T == 0) return hipSuccess;
-    const int vecs = p.vecs != 0 ? p.vecs : takes_two_kb_tiles(p) ? 2 : 1;
-    switch (vecs) {
+    switch (combine_tile(p)) {
         case 1: return launch<1>(p, stream);
         case 4: return launch<4>(p, stream);
         default: return launch<2>(p, stream);

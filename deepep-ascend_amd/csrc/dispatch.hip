@@ -1725,6 +1725,10 @@ bool move_prefers_finished_layout(const MoveParams& p, int count_blocks) {
     return is_large_input(p) || row_bytes_out(p) >= (p.row_bytes > 4096 ? 300e6 : 345e6);
 }
 
+MoveChoice choose_move(const MoveParams& p) {
+    return {move_tile(p), move_workgroups_per_cu(p), stores_row_by_row(p) ? 1 : 0, cached_side(p)};
+}
+
 hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream) {
     if (p.T == 0) return hipSuccess;
     p.rcp_E_l = 1.0f / float(p.E_l);

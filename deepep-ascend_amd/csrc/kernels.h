@@ -221,6 +221,14 @@ struct MoveParams {
 };
 
 hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream);
+// What launch_dispatch_move takes for these parameters (p.fused and p.sf_blocked set).
+struct MoveChoice {
+    int tile;            // KB of row (fused cast: 1024 channels) per wavefront
+    int per_cu;          // workgroups a CU holds at a time, 0 = as many as fit
+    int in_turn;         // a row's stores are awaited before the next row's
+    int cached_side;     // what goes through the memory-side cache: 0 nothing, 1 the input, 2 the rows
+};
+MoveChoice choose_move(const MoveParams& p);
 // A call for which the layout kernel and a move of its own are faster than one launch (p.T, p.H, p.row_bytes, p.payload, the
 // routing shape and the tile overrides set, p.fused = 1).
 bool move_prefers_finished_layout(const MoveParams& p, int count_blocks);
@@ -286,6 +294,8 @@ struct CombineParams {
 };
 
 hipError_t launch_combine_kernel(CombineParams p, hipStream_t stream);
+// KB of row a wavefront of it has.
+int combine_tile(const CombineParams& p);
 
 // dst_buffer_slot_idx of a handle rebuilt from its recv_src_metadata and per-rank prefix (see combine.hip).
 struct SlotMapParams {

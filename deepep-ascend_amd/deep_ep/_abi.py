@@ -233,6 +233,13 @@ class CastArgs(Structure):
     ]
 
 
+class MoveShape(Structure):
+    _fields_ = [
+        ("single_launch", c_int32), ("tile", c_int32), ("workgroups_per_cu", c_int32), ("rows_in_turn", c_int32),
+        ("cached_side", c_int32), ("blocked_scales", c_int32), ("reserved", c_int32 * 2),
+    ]
+
+
 # name -> (restype, argtypes): every symbol include/deep_ep_hip.h declares
 EXPORTS = {
     "deep_ep_hip_abi_version": (c_int, []),
@@ -247,6 +254,10 @@ EXPORTS = {
     "deep_ep_hip_launch_dispatch_static": (c_int, [POINTER(DispatchArgs), c_void_p]),
     "deep_ep_hip_ll_dispatch_threads": (c_int, [POINTER(LLDispatchArgs)]),
     "deep_ep_hip_dispatch_kernel_launches": (c_int, [POINTER(DispatchArgs)]),
+    "deep_ep_hip_dispatch_move_shape": (c_int, [POINTER(DispatchArgs), POINTER(MoveShape)]),
+    "deep_ep_hip_intranode_move_shape": (c_int, [POINTER(IntranodeDispatchArgs), POINTER(MoveShape)]),
+    "deep_ep_hip_combine_tile": (c_int, [POINTER(CombineArgs)]),
+    "deep_ep_hip_intranode_combine_tile": (c_int, [POINTER(IntranodeCombineArgs)]),
     "deep_ep_hip_launch_combine": (c_int, [POINTER(CombineArgs), c_void_p]),
     "deep_ep_hip_combine_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "deep_ep_hip_launch_intranode_dispatch": (c_int, [POINTER(IntranodeDispatchArgs), c_void_p]),

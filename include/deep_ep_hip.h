@@ -229,6 +229,21 @@ int deep_ep_hip_launch_dispatch(const deep_ep_hip_dispatch_args* args, void* str
  * that size graphs or want to know which path a shape takes. */
 int deep_ep_hip_dispatch_kernel_launches(const deep_ep_hip_dispatch_args* args);
 
+/* How the rows of a dispatch would be moved by deep_ep_hip_launch_dispatch with these arguments: the library's choice, knobs included.  Read
+ * are the shape, the phases, the capacities, the strides of recv_sf and whether it is NULL; nothing is dereferenced or launched.
+ * A move of no tokens: all zero. */
+typedef struct {
+    int32_t single_launch;     /* 1: layout and move share a launch */
+    int32_t tile;              /* KB of row per wavefront; fused cast: 1024 channels */
+    int32_t workgroups_per_cu; /* a CU holds at a time; 0 = as many as fit */
+    int32_t rows_in_turn;      /* 1: a wavefront awaits a row's stores before the next row's */
+    int32_t cached_side;       /* what goes through the memory-side cache: 0 nothing, 1 the input, 2 the rows */
+    int32_t blocked_scales;    /* 1: column-major scales go out in blocks, which a launch behind the move turns */
+    int32_t reserved[2];
+} deep_ep_hip_move_shape;
+
+int deep_ep_hip_dispatch_move_shape(const deep_ep_hip_dispatch_args* args, deep_ep_hip_move_shape* out);
+
 /* The same dispatch for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  args->workspace and
  * args->workspace_bytes are ignored: the workspace is a device-resident array built into the library,
@@ -271,6 +286,9 @@ typedef struct {
 } deep_ep_hip_combine_args;
 
 int deep_ep_hip_launch_combine(const deep_ep_hip_combine_args* args, void* stream);
+
+/* KB of row a wavefront of that combine would have (1, 2 or 4; negative: an error code).  The shape and the knobs are read. */
+int deep_ep_hip_combine_tile(const deep_ep_hip_combine_args* args);
 /* Workspace a combine needs when it has to rebuild dst_buffer_slot_idx: the dispatch workspace of the same shape
  * (deep_ep_hip_workspace_bytes, left untouched, so that dispatch and combine can share one allocation) followed by the
  * rebuilt map.  A combine that is given dst_buffer_slot_idx needs 256 bytes (the status word). */
@@ -337,6 +355,8 @@ typedef struct {
 } deep_ep_hip_intranode_dispatch_args;
 
 int deep_ep_hip_launch_intranode_dispatch(const deep_ep_hip_intranode_dispatch_args* args, void* stream);
+/* ... and how its rows would be moved (see deep_ep_hip_dispatch_move_shape; num_topk = 0: routed by rank). */
+int deep_ep_hip_intranode_move_shape(const deep_ep_hip_intranode_dispatch_args* args, deep_ep_hip_move_shape* out);
 
 /* combined_x[t] = bf16( bias_0[t] + bias_1[t] + sum over ranks d ascending with send_head[t][d] >= 0 of
  * x[send_head[t][d]] ) in fp32; combined_topk_weights[t] = sum of the same rows of topk_weights. */
@@ -357,6 +377,8 @@ typedef struct {
 } deep_ep_hip_intranode_combine_args;
 
 int deep_ep_hip_launch_intranode_combine(const deep_ep_hip_intranode_combine_args* args, void* stream);
+/* ... and KB of row a wavefront of it would have. */
+int deep_ep_hip_intranode_combine_tile(const deep_ep_hip_intranode_combine_args* args);
 
 /* ------------------------------------------------------------------------------------------
  * Low-latency packed layout (V1 `Buffer.low_latency_dispatch/combine`) for one logical
