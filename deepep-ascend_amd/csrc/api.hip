@@ -107,6 +107,14 @@ void set_knobs(MoveParams& m, const deep_ep_hip_tuning& tuning) {
     m.plain_loads = tuning.plain_loads; m.xcd_remap = tuning.xcd_remap;
 }
 
+// Does a BF16 dispatch of this shape with both phases in one call take one launch?
+bool copies_in_one_launch(MoveParams m, const deep_ep_hip_tuning& tuning) {
+    m.payload = DEEP_EP_HIP_PAYLOAD_BF16;
+    m.row_bytes = m.H * 2;
+    m.cached = 0;
+    return plan_launches(m, true, true, false, 1, tuning).fused;
+}
+
 // What a move is chosen by - the launches, its tile, what a CU holds, what goes through the caches - as far as the arguments say it.
 MoveParams shape_of_move(const deep_ep_hip_dispatch_args* a) {
     MoveParams m{};
@@ -126,6 +134,8 @@ MoveParams shape_of_move(const deep_ep_hip_dispatch_args* a) {
         m.zeroed_rows = int(std::min<int64_t>(std::max(int64_t(m.E) * (a->expert_alignment - 1) / 2, regions - selections), INT32_MAX));
     }
     set_knobs(m, a->tuning);
+    const bool pads = a->do_zero_padding && a->expert_alignment > 1;
+    m.like_single = m.cached && a->tuning.rows_copied == 2 && !pads && copies_in_one_launch(m, a->tuning) ? 1 : 0;
     return m;
 }
 
@@ -155,6 +165,15 @@ CombineParams shape_of_combine(const deep_ep_hip_combine_args* a) {
     p.do_expand = a->do_expand ? 1 : 0;
     p.multi_red = a->allow_multiple_reduction ? 1 : 0;
     p.vecs = a->tuning.combine_vecs;
+    p.shares_tile = a->tuning.rows_copied != 0 ? 1 : 0;
+    if (a->tuning.rows_copied == 2) {
+        MoveParams m{};
+        m.T = p.T; m.H = p.H; m.K = p.K; m.E = p.E; m.R = p.R; m.E_l = p.E_l; m.M = p.M;
+        m.do_expand = p.do_expand;
+        m.recv_capacity = p.num_meta_rows;
+        m.expanded_capacity = p.num_x_rows;
+        if (copies_in_one_launch(m, a->tuning)) p.shares_tile = 2;
+    }
     return p;
 }
 
@@ -165,6 +184,15 @@ CombineParams shape_of_combine(const deep_ep_hip_intranode_combine_args* a) {
     p.rank_mode = 1;
     p.Kw = a->num_topk;
     p.vecs = a->tuning.combine_vecs;
+    // A V1 handle does not say what made it: taken for BF16, and for a call of both phases where it has a row for every rank.
+    p.shares_tile = 1;
+    if (p.num_x_rows >= int64_t(p.T) * p.R) {
+        MoveParams m{};
+        m.T = p.T; m.H = p.H; m.K = p.Kw > 0 ? p.Kw : p.R; m.E = p.E; m.R = p.R; m.E_l = 1; m.M = p.T;
+        m.recv_capacity = p.num_x_rows;
+        m.rank_lanes = p.Kw > 0 ? 0 : 1;
+        if (copies_in_one_launch(m, a->tuning)) p.shares_tile = 2;
+    }
     return p;
 }
 

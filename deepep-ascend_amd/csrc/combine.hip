@@ -322,7 +322,7 @@ bool reads_past_the_cache(const CombineParams& p) {
 
 // Column tile per wavefront: 1 KB of a BF16 row (512 channels, 41 registers, eight wavefronts per SIMD), or 2 KB, which repeats the routing
 // work half as often and has half the wavefronts to hide its loads with.  2 KB for few rows a token (top-2, or two ranks), where the routing is
-// as much as the rows, from three quarters of the places on, beyond what kb_of_wavefront settles; V1 rows, whose routing is shorter, from a full round on.  Change by 2 KB tiles in %
+// as much as the rows, from three quarters of the places on, where kb_of_wavefront does not settle it; V1 rows, whose routing is shorter, from a full round on.  Change by 2 KB tiles in %
 // at 0.55 / 0.8 / 1.0 / 1.1 / 1.4 / 4 times as many wavefronts of 1 KB as places (730 shapes, rows of 2 to 14 KB):
 //   compact, top-2 of 2 ranks, 8 KB rows    +1.2 / -2.2 / -4.0 / -8.0 / -7.6 / -8.5;   top-2 of 8 ranks +0.6 / +0.5 / -1.5 / -5.8 / -8.2 / -4.4
 //   expanded, top-2                          +0.5 / -3.0 / -6.1 / -7.9 / -1.3 / -2.7
@@ -333,8 +333,9 @@ bool reads_past_the_cache(const CombineParams& p) {
 bool takes_two_kb_tiles(const CombineParams& p) {
     const int kb = (p.H * 2 + 1023) / 1024;
     if (!reads_past_the_cache(p)) {
-        const int same = kb_of_wavefront(p.T, p.H * 2, rows_per_token(p), false);
-        if (same != 0) return same == 2;
+        const int same = shared_tile(p.T, p.H * 2, rows_per_token(p), p.shares_tile == 2);
+        const bool others = p.shares_tile == 0 && int64_t(p.T) * ((kb + 1) / 2) < int64_t(compute_units()) * 18;
+        if (same != 0 && !others) return same == 2;
     }
     if (kb < 2 || rows_per_token(p) >= 2.3) return false;
     const int64_t places = int64_t(compute_units()) * 8 * kWavesPerBlock, waves = int64_t(p.T) * kb;

@@ -55,13 +55,18 @@ py::class_<ElasticBuffer> register_common_apis(py::module_& m) {
              py::arg("expert_alignment"), py::arg("num_sms"), py::arg("num_qps"), py::arg("previous_event"),
              py::arg("previous_event_before_epilogue"), py::arg("async_with_compute_stream"), py::arg("allocate_on_comm_stream"),
              py::arg("do_handle_copy"), py::arg("do_cpu_sync"), py::arg("do_expand"), py::arg("do_zero_padding"),
-             py::arg("use_tma_aligned_col_major_sf"), py::arg("cast_to_fp8") = false)
-        .def("combine", &ElasticBuffer::combine, py::arg("x"), py::arg("topk_weights"), py::arg("bias_0"), py::arg("bias_1"),
-             py::arg("src_metadata"), py::arg("combined_topk_idx"), py::arg("psum_num_recv_tokens_per_scaleup_rank"),
-             py::arg("token_metadata_at_forward"), py::arg("channel_linked_list"), py::arg("num_experts"),
-             py::arg("num_max_tokens_per_rank"), py::arg("num_sms"), py::arg("num_qps"), py::arg("previous_event"),
-             py::arg("previous_event_before_epilogue"), py::arg("async_with_compute_stream"), py::arg("allocate_on_comm_stream"),
-             py::arg("use_expanded_layout"), py::arg("dst_buffer_slot_idx") = py::none());
+             py::arg("use_tma_aligned_col_major_sf"), py::arg("cast_to_fp8") = false);
+    const auto def_combine = [&](const char* name, auto method) {
+        cls.def(name, method, py::arg("x"), py::arg("topk_weights"), py::arg("bias_0"), py::arg("bias_1"),
+                py::arg("src_metadata"), py::arg("combined_topk_idx"), py::arg("psum_num_recv_tokens_per_scaleup_rank"),
+                py::arg("token_metadata_at_forward"), py::arg("channel_linked_list"), py::arg("num_experts"),
+                py::arg("num_max_tokens_per_rank"), py::arg("num_sms"), py::arg("num_qps"), py::arg("previous_event"),
+                py::arg("previous_event_before_epilogue"), py::arg("async_with_compute_stream"), py::arg("allocate_on_comm_stream"),
+                py::arg("use_expanded_layout"), py::arg("dst_buffer_slot_idx") = py::none());
+    };
+    def_combine("combine", &ElasticBuffer::template combine<0>);
+    def_combine("_combine_copied_rows", &ElasticBuffer::template combine<1>);             // for this package alone: EPHandle.rows_copied
+    def_combine("_combine_rows_copied_at_once", &ElasticBuffer::template combine<2>);
     m.def("calculate_elastic_buffer_size", &ElasticBuffer::calculate_buffer_size);
     return cls;
 }

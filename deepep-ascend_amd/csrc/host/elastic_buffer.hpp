@@ -220,6 +220,8 @@ public:
         args.workspace = workspace.data_ptr();
         args.workspace_bytes = static_cast<uint64_t>(workspace.numel());
         args.tuning = process_tuning();
+        // a handle without the counts was made without waiting for them, by both phases in one call
+        if (cached_mode) args.tuning.rows_copied = cached_num_recv_tokens_per_expert_list->empty() ? 2 : 1;
         void* stream_ptr = run.stream();
 
         // Sizes of the outputs.  With a CPU sync they are exact: known before the move is launched, or, for outputs small enough
@@ -344,6 +346,9 @@ public:
     // it produced together with this `src_metadata`, and for a handle it has not seen (or whose tensors were cloned)
     // the library rebuilds the map from `src_metadata[:, 0:2]` and the per-rank prefix, a scatter of one entry per
     // received row.
+    // kRowsCopied: what is known of the dispatch that made the handle (deep_ep_hip_tuning::rows_copied); a method for each, as the
+    // reference's signature has no place for it.
+    template <int kRowsCopied>
     std::tuple<torch::Tensor, std::optional<torch::Tensor>, std::optional<EventHandle>>
     combine(const torch::Tensor& x, const std::optional<torch::Tensor>& topk_weights, const std::optional<torch::Tensor>& bias_0,
             const std::optional<torch::Tensor>& bias_1, const torch::Tensor& src_metadata, const torch::Tensor& combined_topk_idx,
@@ -419,6 +424,7 @@ public:
         args.workspace = workspace.data_ptr();
         args.workspace_bytes = static_cast<uint64_t>(workspace.numel());
         args.tuning = process_tuning();
+        args.tuning.rows_copied = kRowsCopied;
         check_abi(deep_ep_hip_launch_combine(&args, run.stream()), "combine");
 
         std::optional<EventHandle> event = scope.finish({x, topk_weights, bias_0, bias_1, src_metadata, combined_topk_idx,

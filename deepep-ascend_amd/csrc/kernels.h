@@ -178,6 +178,8 @@ struct MoveParams {
     int sf_blocked;      // recv_sf is column-major and the pad kernel follows: scales go out in blocks (below)
     int zeroed_rows;     // padding rows this call zeroes, as expected: half an alignment for each expert, or what is
                          // left of one alignment for each where an expert has fewer rows than that
+    int like_single;     // a cached handle of a single launch: its tile (kb_of_wavefront)
+    int shared_tile;     // the combine has the same tile: workgroups on the XCD of its (set by the launcher)
     int row_by_row;      // a wavefront waits for the stores of a row before it starts the next (set by the launcher)
     unsigned warm_lds_offset;   // single-launch cast: byte offset (in the dynamic LDS) of the 4 KB landing area of the
                                 // cache-warming loads, 0 = none
@@ -291,6 +293,7 @@ struct CombineParams {
     int rank_mode;
     int Kw;
     int vecs;            // forced column tile, 0 = choose
+    int shares_tile;     // the rows are a BF16 dispatch's, on a finished layout (1) or in a single launch (2): kb_of_wavefront; 0: not, or not known
 };
 
 hipError_t launch_combine_kernel(CombineParams p, hipStream_t stream);
@@ -344,20 +347,46 @@ struct LLDispatchParams {
 int compute_units();
 
 // BF16 rows few enough to be read from the caches (T tokens that go to `rows` rows each): the KB of a row that a wavefront of the dispatch writes and
-// a wavefront of the combine reads, the same for both, so that what an XCD has written it finds in its own L2 (0: each takes its own).  Dispatch and
-// combine, us, rows combined as the dispatch has left them / with a pass in between that writes as many others:
-//   a single launch, 4 KB and 1 KB, 2 KB both   206 x 7960 over 8 ranks 24.6 / 29.6, 17.7 / 27.4;   1009 x 3568 28.1 / 37.1, 23.7 / 36.9;   635 x 6808 of 4 27.3
-//                                               / 34.9, 20.6 / 33.2;   past 22 wavefronts of 2 KB a CU 3382 x 1512 top-6 33.4 / 46.3, 34.0 / 48.9: left alone
-//   a move, 4 KB and 1 KB, 1 KB both, 2 KB both 1237 x 2888 top-9 24.5 / 31.9, 19.3 / 32.0, 18.6 / 31.2;   2970 x 1568 31.6 / 39.6, 26.8 / 41.7, 23.2 / 37.7;
-//                                               1982 x 3256 of 32 ranks (7.2 rows) 41.2 / 65.6, 41.4 / 67.9, 38.3 / 65.3;   past 30 a CU 1324 x 5672 expanded 46.7 /
-//                                               66.6, 43.1 / 69.6, 39.7 / 66.2;  2270 x 4000 33.6 / 45.6, 32.4 / 49.0, 30.4 / 47.4: left alone
-// From six and a half rows a token on small calls have 1 KB both (144 x 7072 expanded 25.0 / 30.6, 20.3 / 29.6, on two launches 532 x 5792 of 32 ranks 26.3 / 44.7,
-// with 2 KB 27.3 / 45.4), and so have moves of rows that leave a fourth of their 2 KB tiles empty (2362 x 1064 23.9 / 38.4, with 2 KB 24.7 / 39.2).
+// a wavefront of the combine reads, the same for both, so that what an XCD has written it finds in its own L2 (0: each takes its own).
+// Lines by wavefronts of 2 KB a CU.  Dispatch and combine, us, top-8 of 8 ranks unless said, rows combined as the dispatch has left them / with a pass
+// in between that reads them and writes as many others, which are combined:
+//   two launches                    1 KB both     2 KB both      4 and 1 KB (2 and 1 KB)
+//     128 x 1024 top-2 of 2   1     10.5 / 12.7   10.9 / 13.0    10.9 / 12.9      up to 4: 1 KB, which has twice the wavefronts
+//     256 x 1024              1     12.9 / 16.8   13.5 / 17.4    14.5 / 17.3
+//     146 x 7168              4     14.5 / 26.9   14.5 / 26.8    18.4 / 26.9
+//     292 x 7168              8     18.4 / 29.9   18.1 / 30.1    25.5 / 30.4      up to 30: 2 KB
+//     1706 x 2888             20    35.8 / 53.0   32.4 / 50.3    35.5 / 49.5
+//     950 x 7168              26    40.6 / 63.0   39.1 / 60.7    41.6 / 60.4
+//     1243 x 7168             34    49.8 / 78.2   47.9 / 76.9    49.0 / 74.8      left alone (2901 x 2888 50.6 / 76.8, 48.7 / 74.8, 48.0 / 71.9)
+//     512 x 7168 expanded     14    34.2 / 52.0   34.6 / 53.0    37.4 / 51.2      tokens of seven and a half rows and more: 1 KB up to 15
+//     320 x 8192              5     15.6 / 23.9   16.1 / 27.8    22.5 / 26.2      rows of whole 8 KB (256 x 4096 top-4 12.3 / 18.9, 12.5 / 20.5): 1 KB up to 6
+//   a single launch
+//     73 x 7168               2     15.2 / 21.6   14.1 / 20.6    15.9 / 20.5      up to 22: 2 KB
+//     292 x 7168 of 32        8     20.5 / 33.4   19.6 / 32.4    26.9 / 34.0
+//     731 x 7168              20    32.1 / 49.5   29.4 / 46.9    32.2 / 46.6
+//     950 x 7168              26    40.6 / 62.2   44.4 / 67.5    37.6 / 56.9      left alone
+//     320 x 4096              5     17.4 / 26.6   18.5 / 28.9    21.1 / 27.3      rows of whole 8 KB: 1 KB from 4 to 6 (155 x 4096, one row, 2.4 a CU 17.7, 17.1)
+//     146 x 7168 expanded     4     20.8 / 32.1   21.4 / 33.2    25.8 / 32.5      tokens of seven and a half rows and more: 1 KB up to 4
+// Rows that leave a fourth of their 2 KB tiles empty take 1 KB (2362 x 1064 23.9 / 38.4, with 2 KB 24.7 / 39.2), in a single launch only tokens of many.
+// Past the lines of a single launch its combine has the tile of two launches, which a cached dispatch on the same handle has (shared_tile); behind the single
+// launch that is level with its own (950 x 7168 37.7 / 56.8 with 2 KB, 37.6 / 56.9 with 1 KB).  A combine whose rows are not those of a BF16 dispatch keeps to its own rule
+// below 18 a CU: fused cast, 1 / 2 KB, 1194 x 2944 21.4 / 22.0, 3584 x 1024 22.4 / 22.9, 192 x 4096 19.9 / 21.1; 1706 x 2944 top-4 22.2 / 21.3, 731 x 7168 25.6 / 25.8.
+// V1 handles do not say what made them; level from 8 on (FP8, 682 x 2944 34.2 / 34.3, 512 x 4096 33.2 / 33.9).
 inline int kb_of_wavefront(int64_t T, int row_bytes, double rows, bool single_launch) {
     const int kb = (row_bytes + 1023) / 1024, tiles = (kb + 1) / 2;
-    const int64_t cus = compute_units();
-    if (rows < 6.5 && row_bytes >= tiles * 1536) return T * tiles <= cus * (single_launch ? 22 : 30) ? 2 : 0;
-    return T * kb <= cus * (single_launch ? 12 : 30) && (rows >= 6.5 || !single_launch) ? 1 : 0;
+    const int64_t cus = compute_units(), wavefronts = T * tiles;
+    if (row_bytes < tiles * 1536) return T * kb <= cus * (single_launch ? 12 : 30) && (rows >= 6.5 || !single_launch) ? 1 : 0;
+    if (wavefronts > cus * (single_launch ? 22 : 30)) return 0;
+    const bool many = rows >= 7.5, whole_8kb = row_bytes % 8192 == 0;
+    if (single_launch && whole_8kb && !many) return wavefronts > cus * 4 && wavefronts <= cus * 6 ? 1 : 2;
+    const int one_kb_to = single_launch ? (whole_8kb ? 6 : many ? 4 : 0) : many ? 15 : whole_8kb ? 6 : 4;
+    return wavefronts <= cus * one_kb_to ? 1 : 2;
+}
+
+// The tile of the combine, and of a dispatch on the handle, where the handle is a single launch's or not.
+inline int shared_tile(int64_t T, int row_bytes, double rows, bool single_launch) {
+    const int kb = single_launch ? kb_of_wavefront(T, row_bytes, rows, true) : 0;
+    return kb != 0 ? kb : kb_of_wavefront(T, row_bytes, rows, false);
 }
 
 // LDS a workgroup asks for so that a CU holds at most `per_cu` of them (0: no limit).

@@ -35,14 +35,14 @@ class Tuning(Structure):
         ("dispatch_launches", c_int32), ("cast_pairs", c_int32), ("copy_vecs", c_int32), ("plain_loads", c_int32),
         ("xcd_remap", c_int32), ("combine_vecs", c_int32), ("ll_pairs", c_int32), ("ll_threads", c_int32),
         ("ll_two_kernels", c_int32), ("ll_combine_vecs", c_int32), ("mover_spin_limit", c_int32),
-        ("move_workgroups_per_cu", c_int32), ("warm_rounds", c_int32), ("persistent_movers", c_int32), ("reserved", c_int32 * 2),
+        ("move_workgroups_per_cu", c_int32), ("warm_rounds", c_int32), ("persistent_movers", c_int32), ("rows_copied", c_int32), ("reserved", c_int32 * 1),
     ]
 
     @classmethod
     def from_env(cls) -> "Tuning":
         t = cls()
         for name, _ in cls._fields_:
-            if name != "reserved":
+            if name not in ("rows_copied", "reserved"):          # a fact of each call, and nothing yet
                 setattr(t, name, int(os.environ.get("DEEP_EP_HIP_" + name.upper(), "0")))
         return t
 

@@ -109,7 +109,11 @@ typedef struct {
                                   request the next item's loads before the current item's stores; implies layout kernel +
                                   move kernel.  Calls it does not cover (expanded layout, cached handle, mask routing) run
                                   as if it were 0.  A measured alternative (slower on MI355X), not a default */
-    int32_t reserved[2];
+    int32_t rows_copied;       /* no knob but a fact, of a combine and of a dispatch on a cached handle: the dispatch that made the handle moved
+                                  its rows as 0 = not known, or FP8, 1 = BF16, on a finished layout (phases one by one, or padding
+                                  rows zeroed), 2 = BF16, with both phases in one call.  Rows few enough to lie in the caches are then
+                                  moved and combined in the same column tiles */
+    int32_t reserved[1];
 } deep_ep_hip_tuning;
 
 /* Bytes of workspace needed for dispatches of up to num_max_tokens tokens.  The workspace must

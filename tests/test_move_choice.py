@@ -40,6 +40,22 @@ def v1_move(payload, T, H, R, rows, cached=False):
     return s
 
 
+def combine(T, H, E, R, K, copied, rows=None, expanded=False, meta_rows=None):
+    a = _abi.CombineArgs()
+    a.num_tokens, a.hidden, a.num_topk, a.num_experts, a.num_ranks, a.num_max_tokens_per_rank, a.do_expand = T, H, K, E, R, T, expanded
+    at_once = copied == 2
+    a.num_recv_rows = T * R if at_once else int(T * R * (1 - (1 - 1 / R) ** K))
+    a.num_x_rows = T * K if expanded else a.num_recv_rows
+    a.tuning.rows_copied = copied
+    return _abi.lib.deep_ep_hip_combine_tile(ctypes.byref(a))
+
+
+def v1_combine(T, H, R, K, rows):
+    a = _abi.IntranodeCombineArgs()
+    a.num_tokens, a.hidden, a.num_ranks, a.num_topk, a.num_x_rows = T, H, R, K, rows
+    return _abi.lib.deep_ep_hip_intranode_combine_tile(ctypes.byref(a))
+
+
 def shape(s):
     return s.tile, s.workgroups_per_cu, s.rows_in_turn
 
@@ -77,3 +93,63 @@ def test_what_the_cache_holds_among_padding(E, side):
     """400 x 7168 top-8 aligned to 128, in outputs of worst-case size: 46 MB of rows in 235 and 250 MB that are in use."""
     s = move("bf16", 400, 7168, E, 8, 8, expanded=True, alignment=128, single=True)
     assert s.single_launch == 1 and s.cached_side == side
+
+
+# Rows that lie in the caches: the KB a wavefront of the dispatch writes and one of the combine reads.  2 KB wavefronts per CU are T * 7 / 256 for 7168
+# channels, T * 4 / 256 for 4096 and T * 3 / 256 for 2888.
+SHARED = [
+    # T, hidden, experts, ranks, selections, expanded, both phases in one call, KB of both (0: each its own)
+    (128, 1024, 8, 2, 2, False, False, 1), (1024, 1024, 64, 8, 4, False, False, 1), (1025, 1024, 64, 8, 4, False, False, 2),      # 4
+    (146, 7168, 64, 8, 8, False, False, 1), (147, 7168, 64, 8, 8, False, False, 2),
+    (341, 2888, 64, 8, 8, False, False, 1), (342, 2888, 64, 8, 8, False, False, 2),
+    (384, 4096, 64, 8, 8, False, False, 1), (385, 4096, 64, 8, 8, False, False, 2),                                               # whole 8 KB: 6
+    (548, 7168, 64, 8, 8, True, False, 1), (549, 7168, 64, 8, 8, True, False, 2),                                                 # eight rows: 15
+    (1097, 7168, 64, 8, 4, False, False, 2), (1098, 7168, 64, 8, 4, False, False, 0),                                             # 30
+    (1, 7168, 64, 8, 8, False, True, 2), (804, 7168, 64, 8, 8, False, True, 2),                                                   # 22
+    (292, 7168, 256, 32, 8, False, True, 2), (256, 4096, 64, 8, 8, False, True, 2), (257, 4096, 64, 8, 8, False, True, 1),
+    (384, 4096, 64, 8, 8, False, True, 1), (385, 4096, 64, 8, 8, False, True, 2),                                                 # 4 and 6
+    (146, 7168, 64, 8, 8, True, True, 1), (147, 7168, 64, 8, 8, True, True, 2),
+    (2362, 1064, 64, 8, 8, False, False, 1), (2562, 1064, 64, 8, 4, False, False, 0),                                             # 2128 of 4096 bytes
+]
+
+
+@pytest.mark.parametrize("T,H,E,R,K,expanded,at_once,kb", SHARED)
+def test_dispatch_and_combine_share_a_tile(T, H, E, R, K, expanded, at_once, kb):
+    s = move("bf16", T, H, E, R, K, expanded=expanded, single=at_once)
+    assert s.cached_side == ROWS and s.single_launch == at_once
+    both = combine(T, H, E, R, K, 2 if at_once else 1, expanded=expanded)
+    own = combine(T, H, E, R, K, 0, expanded=expanded)
+    if kb:
+        assert s.tile == both == kb
+    else:
+        assert both == own
+    if R == 8 and K >= 4 and T * ((H + 1023) // 1024) < 18 * 256:
+        assert own == 1                                   # behind FP8 rows, and for handles that do not say
+
+
+def test_past_the_line_of_a_single_launch():
+    """805 x 7168: 22 a CU.  The move has its own tile; the combine and a dispatch on the handle share that of two launches."""
+    a = (805, 7168, 64, 8, 8)
+    assert move("bf16", *a, single=True).tile == 4 and combine(*a, 2) == move("bf16", *a, cached=True, rows_copied=2).tile == 2
+    b = (2370, 1264, 64, 4, 5)                            # a fourth of the 2 KB tiles empty, 1 KB
+    assert move("bf16", *b, expanded=True, cached=True, rows_copied=2).tile == combine(*b, 2, expanded=True) == 1
+
+
+def test_combine_of_rows_no_bf16_dispatch_wrote():
+    assert combine(1535, 2888, 64, 8, 8, 0) == 1 and combine(1536, 2888, 64, 8, 8, 0) == 2                  # 18 a CU
+    assert combine(2561, 2888, 64, 8, 4, 0) == 1                                                          # 30
+
+
+def test_cached_dispatch_has_the_tile_of_the_handle():
+    a = (128, 7168, 64, 8, 8)
+    assert move("bf16", *a, cached=True).tile == move("bf16", *a, cached=True, rows_copied=1).tile == 1
+    assert move("bf16", *a, cached=True, rows_copied=2).tile == move("bf16", *a, single=True).tile == combine(*a, 2) == 2
+    assert move("bf16", 1000, 2048, 64, 8, 9, cached=True, rows_copied=2).tile == 2             # top-9 has no single launch: 8 a CU
+    assert move("bf16", 100, 7168, 64, 8, 8, expanded=True, alignment=16, pads=True, cached=True, rows_copied=2).tile == 1
+
+
+def test_v1_tiles():
+    for T, rows, kb in ((146, 700, 1), (147, 700, 2), (1097, 5000, 2), (1098, 3000, 1), (100, 800, 2)):      # 4 and 30; a row for every rank
+        assert v1_combine(T, 7168, 8, 4, rows) == kb
+    assert v1_combine(146, 7168, 8, 0, 700) == v1_move("bf16", 146, 7168, 8, 700).tile == 1
+    assert v1_combine(147, 7168, 8, 0, 700) == v1_move("bf16", 147, 7168, 8, 700).tile == 2
