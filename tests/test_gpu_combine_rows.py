@@ -44,3 +44,16 @@ def test_combine_reads_its_rows(name, reduce_in_rank, expand):
     assert torch.equal((out.cpu() + 0.0).view(torch.int16), (ref + 0.0).view(torch.int16))
     assert torch.equal(out_w.cpu(), ref_w)
     buf.check_device_status()
+
+
+def test_a_handle_is_what_has_its_fields():
+    """A combine takes whatever carries the reference's handle fields, also without the one this package adds."""
+    import types
+
+    import deep_ep
+    c = rc.small("fields", 40, 128, 16, 4, 3, seed=3)
+    buf = deep_ep.ElasticBuffer(deep_ep.LogicalGroup(0, c.R), num_max_tokens_per_rank=40, hidden=128, num_topk=3)
+    recv, _, w, handle, _ = buf.dispatch(c.x.cuda(), c.topk_idx.cuda(), c.topk_weights.cuda(), num_experts=c.E)
+    like = types.SimpleNamespace(**{k: v for k, v in vars(handle).items() if k != "rows_copied"})
+    for a, b in zip(buf.combine(recv, handle, topk_weights=w)[:2], buf.combine(recv, like, topk_weights=w)[:2]):
+        assert torch.equal(a, b)
