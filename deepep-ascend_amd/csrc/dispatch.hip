@@ -1413,8 +1413,10 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 //     6221 x 4488 of 64 ranks (9.3) 255.7 / 249.7 / 249.3 (2 each), 263.6;   from 90 MB of input, up to 5.2 rows, 17335 x 3712 (4.4) 250.2 with
 //     three of 2 KB, 261.5 with two, 265.1;   15819 x 6096 (2.7) 247 (8) / 243.3 (3) / 249 (2), 245.1;   16746 x 8072 (2.0) 283.5 (8) / 278.1 (8),
 //     280.9 with five, 281.6 with four;   rows of 3 and 4 KB 21387 x 1048 (6.5) 174.0 / 171.9 / 165.2 (2 each), 174.1;
-//   - many expanded rows over fewer than 32 ranks in 1 KB tiles (6706 x 4000 top-8 of 64 181.9 (2) / 173.7 (2)): 17091 x 2552 top-8 304.8 (2) / 313.3 / 315 (2), 329.3;   6490 x 5408 211.1 (2) / 219.3 (2), 221.2;   10922 x
-//     5096 top-9 430.7 / 446.7, 461.5;   up to 300 MB of them they are level (2270 x 5192 88.7 / 90.2, 1646 x 5032 78.2 / 75.2);
+//   - nine and more expanded rows over fewer than 32 ranks in two of 1 KB from 450 MB on, rows that are no whole 64 bytes, in % of two of 2 KB, straight /
+//     with a pass in between: 500 MB top-10 -4.2 / -1.3, top-9 -2.7 / +0.5, 700 MB top-10 -1.3 / -1.5, top-9 -2.5 / -0.5, 1 GB top-10 -3.6 / -1.0;   of eight rows level
+//     / +2.2, of 350 MB of ten +0.7 / -1.3;   rows of whole 64 bytes, which both halves of a KB then share with nobody, +9 to +20 / +10 to +13 (500 MB, 3424 channels
+//     top-8 +19.3 / +13.3, top-10 +10.4 / +11.1);
 //   - rows of whole KB, whose wavefronts run more alike, up to 430 MB in four or five workgroups of 1 KB: 6608 x 2048 of 8 ranks (5.9) 67.4 (5) / 68.3
 //     (4), 72.4;   2805 x 3072 of 32 (8.0) 57.5 (4) / 57.5 (2), 61.2;   and beyond with each row's stores awaited before the next row's are issued, so that
 //     a wavefront has one row under way however long that takes; without / with the wait: 20000 x 4096 of 8 (5.3), move alone, 177.4 (2 of 2 KB) / 170.5
@@ -1473,7 +1475,7 @@ static bool large_move_shape(const MoveParams& p, MoveShape& q) {
         q = {4, 2, false};
         return rows >= 3.2;
     }
-    if (p.do_expand && rows >= 8.0 && out >= 300e6 && kb >= 5 && p.R < 32) q = {1, 2, false};
+    if (p.do_expand && rows >= 9.0 && out >= 450e6 && kb >= 5 && p.R < 32 && bytes % 64 != 0) q = {1, 2, false};
     else q = {2, rows < 4.3 || (rows < 5.2 && double(p.T) * p.row_bytes >= 90e6) ? 3 : 2, false};
     return true;
 }

@@ -153,3 +153,11 @@ def test_v1_tiles():
         assert v1_combine(T, 7168, 8, 4, rows) == kb
     assert v1_combine(146, 7168, 8, 0, 700) == v1_move("bf16", 146, 7168, 8, 700).tile == 1
     assert v1_combine(147, 7168, 8, 0, 700) == v1_move("bf16", 147, 7168, 8, 700).tile == 2
+
+
+def test_large_expanded_rows_of_no_whole_kb():
+    assert shape(move("bf16", 4927, 5080, 72, 8, 9, expanded=True)) == (1, 2, 0)            # 450.6 MB
+    assert shape(move("bf16", 4900, 5080, 72, 8, 9, expanded=True)) == (2, 2, 0)            # 448.1
+    assert shape(move("bf16", 9854, 5080, 72, 8, 8, expanded=True))[:1] == (2,)             # eight rows, 801 MB
+    assert shape(move("bf16", 4927, 5088, 72, 8, 9, expanded=True)) == (2, 2, 0)            # whole 64 bytes
+    assert shape(move("bf16", 4927, 5080, 288, 32, 9, expanded=True)) == (2, 2, 0)
