@@ -1430,6 +1430,8 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 //     360.9;   17516 x 3584 (3.7) 204.7 (3 of 2 KB) / 197.8 (8 of 1 KB with the wait), 199.5;   without top-k tensors, moves alone, 8192 x 7168 of 4 ranks
 //     (2.7) 73.8 (8 of 1 KB) / 75.2 with the wait, 76.1 (4 of 2 KB);   16384 x 4096 top-4 of 8 (3.3) 102.5 / 99.0 with it, 103.3;
 //     expanded 25983 x 2560 top-2 156.2 (8 of 2 KB), 173.4;
+//   - a few rows among much padding, whose zeroes are most of the call, come here too and are level: 17 shapes of 60 to 1000 tokens x 7168 or 2048 of 256 to 512 experts
+//     aligned to 128, layout, move and padding, with a pass over the rows and a combine behind them or not, -0.2 % with four of 2 KB, -1 to +1 without a limit;
 //   fused cast, expanded, 8192 x 7168 top-8 315.4 (4) / 312.4 (3), 320.6;   16316 x 4608 403.9 (4) / 393.9 (3), 418.5;   compact, 25585 x 3072 of 32
 //     ranks 352.5 (4) / 351.8 (4), 364.5;   8192 x 7168 of 8 200.2 (6) / 199.3 (4), 200.4;   12006 x 5120 top-6 (4.4) 204.4 (8) / 202.9 (5), 205.1;   with
 //     blocked scales, whose rows have no single-dword stores, 8192 x 7168 318.1 (5) / 324.0 (3): left alone;

@@ -16,6 +16,8 @@ pytestmark = pytest.mark.gpu
     ("bf16", 130, 264, 48, 6, 9, 128),           # rows of no whole KB, three slices an expert
     ("bf16", 77, 4104, 5, 1, 2, 700),            # an expert's padding in more than a hundred slices
     ("bf16", 600, 1024, 512, 32, 8, 128),        # slices bounded by the number of experts
+    ("bf16", 67, 7168, 256, 8, 8, 128),          # four workgroups a CU, zeroing ones among them
+    ("bf16", 67, 7160, 256, 8, 8, 128),          # two
     ("cast", 72, 2560, 128, 16, 8, 128), ("pair", 201, 640, 24, 4, 10, 16),
     ("cast", 1801, 7168, 16, 4, 8, 128), ("cast", 1820, 7168, 16, 4, 8, 128),    # 25.8 and 26.1 MB of input: two launches and one, with blocks
     ("cast", 5499, 3584, 16, 2, 8, 5), ("cast", 5503, 3584, 16, 2, 8, 5),        # 43992 and 44024 rows: columns and blocks

@@ -161,3 +161,10 @@ def test_large_expanded_rows_of_no_whole_kb():
     assert shape(move("bf16", 9854, 5080, 72, 8, 8, expanded=True))[:1] == (2,)             # eight rows, 801 MB
     assert shape(move("bf16", 4927, 5088, 72, 8, 9, expanded=True)) == (2, 2, 0)            # whole 64 bytes
     assert shape(move("bf16", 4927, 5080, 288, 32, 9, expanded=True)) == (2, 2, 0)
+
+
+def test_few_rows_among_much_padding():
+    few = dict(expanded=True, alignment=128, pads=True)
+    s = move("bf16", 300, 7168, 256, 8, 8, **few)
+    assert s.cached_side == NOTHING and shape(s) == (1, 4, 0)                    # 34 MB among 500
+    assert shape(move("bf16", 300, 7000, 256, 8, 8, **few)) == (2, 2, 0)
