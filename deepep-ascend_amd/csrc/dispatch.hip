@@ -1433,7 +1433,10 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 //   - a few rows among much padding, whose zeroes are most of the call, come here too and are level: 17 shapes of 60 to 1000 tokens x 7168 or 2048 of 256 to 512 experts
 //     aligned to 128, layout, move and padding, with a pass over the rows and a combine behind them or not, -0.2 % with four of 2 KB, -1 to +1 without a limit;
 //   fused cast, expanded, 8192 x 7168 top-8 315.4 (4) / 312.4 (3), 320.6;   16316 x 4608 403.9 (4) / 393.9 (3), 418.5;   compact, 25585 x 3072 of 32
-//     ranks 352.5 (4) / 351.8 (4), 364.5;   8192 x 7168 of 8 200.2 (6) / 199.3 (4), 200.4;   12006 x 5120 top-6 (4.4) 204.4 (8) / 202.9 (5), 205.1;   with
+//     ranks 352.5 (4) / 351.8 (4), 364.5;   8192 x 7168 of 8 200.2 (6) / 199.3 (4), 200.4;   12006 x 5120 top-6 (4.4) 204.4 (8) / 202.9 (5), 205.1;   seven
+//     rows and more of whole KB, move alone and with the combine, four of 1 KB / four of 2 KB: 16384 x 7168 of 32 204.2, 530.8 / 212.8, 534.9;   of 64 223.1, 555.4 / 230.8,
+//     563.6;   8192 x 7168 of 32 110.6, 268.1 / 115.1, 271.9;   of 64 118.0, 280.8 / 125.5, 293.4;   25585 x 3072 of 32 147.3, 352.6 / 144.4, 358.4;   16384 x 4096 of 32 126.5, 307.6 /
+//     131.9, 301.2;   fewer rows or other rows 16384 x 7168 of 16 192.9, 474.5 / 192.4, 470.1;   14000 x 6272 top-10 of 16 176.4, 423.2 / 170.2, 411.8;   with
 //     blocked scales, whose rows have no single-dword stores, 8192 x 7168 318.1 (5) / 324.0 (3): left alone;
 //   FP8 pairs, expanded, 24963 x 3584 top-9 505.7 (5) / 495.9 (3) / 496.9 (2), 521.1;   compact, 28277 x 4864 (5.9) 485.8 (8) / 473.2 (3) / 474.1 (2),
 //     487.5;   35472 x 3968 (4.4) 438.3 (8) / 427.7 (4) / 437.9 (6), 438.3;   rows of whole KB like those of BF16, move alone, without / with the wait: 16384 x 7168 of 32
@@ -1450,7 +1453,8 @@ static bool large_move_shape(const MoveParams& p, MoveShape& q) {
     if (p.fused || p.cast_pairs != 0 || p.copy_vecs != 0 || kb < 2 || p.sf_blocked) return false;
     if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) {
         if (out < 220e6 || rows < 3.5) return false;
-        q = {2, rows < 5.0 ? 5 : p.do_expand ? 3 : 4, false};
+        if (!p.do_expand && rows >= 7.0 && bytes % 1024 == 0) q = {1, 4, false};
+        else q = {2, rows < 5.0 ? 5 : p.do_expand ? 3 : 4, false};
         return true;
     }
     const bool whole = bytes % 1024 == 0;

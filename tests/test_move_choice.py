@@ -168,3 +168,12 @@ def test_few_rows_among_much_padding():
     s = move("bf16", 300, 7168, 256, 8, 8, **few)
     assert s.cached_side == NOTHING and shape(s) == (1, 4, 0)                    # 34 MB among 500
     assert shape(move("bf16", 300, 7000, 256, 8, 8, **few)) == (2, 2, 0)
+
+
+def test_large_casts():
+    assert shape(move("cast", 16384, 7168, 256, 32, 8)) == (1, 4, 0)              # 7.2 rows of 7 KB
+    assert shape(move("cast", 16384, 7168, 256, 16, 8)) == (2, 4, 0)              # 6.5
+    assert shape(move("cast", 16384, 7296, 256, 32, 8)) == (2, 4, 0)
+    assert shape(move("cast", 8192, 7168, 256, 8, 6)) == (2, 5, 0)                # 4.4
+    assert shape(move("cast", 8192, 7168, 256, 8, 8, expanded=True)) == (2, 3, 0)
+    assert shape(move("cast", 5210, 5888, 256, 32, 8)) == (2, 4, 0) and shape(move("cast", 5200, 5888, 256, 32, 8)) == (2, 0, 0)       # 220 MB
