@@ -1423,8 +1423,9 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 //     (6), before 188.5;   whole passes with a layer's other kernels around them, five without / six with the wait: 32000 x 2048 of 32 ranks (7.2) 403.6 /
 //     404.4, before 407.3;   8192 x 7168 of 32 348.4 / 345.3, 346.1;   9800 x 7168 of 16 (7.0) 407.5 / 406.6, 410.6;   16384 x 5120 of 64 (7.6) 532.2 / 530.0,
 //     534.9;   13211 x 4096 of 16 353.0 / 348.2, 360.1;   16384 x 7168 of 16 (6.5) 607.0 / 609.9, 611.2;   of 32 685.1 / 686.4, 685.5, with five and
-//     the wait 710;   on a handle, moves alone, five / six with the wait: 16384 x 7168 of 32 337.6 / 354.5, 350;   32768 x 2048 195.3 / 203.7, 197;   of 16
-//     302 / 302, 298;
+//     the wait 710;   on a handle with the wait, five / six, moves alone and with the combine: 16384 x 7168 of 32 (7.2) 340.0, 646.5 /
+//     344.1, 671.1;   of 16 (6.5) 316.1, 587.0 / 300.7, 572.7;   9800 x 7168 of 16 185.7, 353.2 / 178.0, 346.6;   13211 x 4096 of 16 149.8, 280.9 / 141.7, 274.8;   16384 x 5120 of 64
+//     260.2, 500.2 / 269.1, 505.5;   30000 x 2048 of 32 181.6, 350.9 / 184.5, 348.1;
 //     rows of 8 and 16 KB, top-6, in three of 2 KB: 24000 x 4096 of 8 ranks (4.4) 361.4 / 369.9 (6), 373.8;   14000 x 8192 418.2 / 430.7 (6), 450.2;
 //     where a token goes to fewer than four rows: 14174 x 8192 (3.3) 348 (8 of 1 KB) / 336.8 (4 of 2 KB), 337.5;   16380 x 7168 (3.6) 353.9 (3 of 2 KB),
 //     360.9;   17516 x 3584 (3.7) 204.7 (3 of 2 KB) / 197.8 (8 of 1 KB with the wait), 199.5;   without top-k tensors, moves alone, 8192 x 7168 of 4 ranks
@@ -1474,7 +1475,7 @@ static bool large_move_shape(const MoveParams& p, MoveShape& q) {
         else if (rows < 3.9 && (rows < 3.5 || kb >= 8 || out < 430e6)) q = {2, rows < 3.5 || kb < 8 ? 4 : 3, false};
         else if (out < 430e6) q = {1, rows < 6.4 ? 5 : 4, false};
         else if ((kb & (kb - 1)) == 0 && kb >= 8 && rows < 5.0) q = {2, 3, false};
-        else q = {1, rows < 4.2 ? 0 : p.cached && rows >= 6.0 ? 5 : 6, true};
+        else q = {1, rows < 4.2 ? 0 : p.cached && rows >= 7.0 ? 5 : 6, true};
         return true;
     }
     if (kb == 3 || kb == 4) {

@@ -177,3 +177,23 @@ def test_large_casts():
     assert shape(move("cast", 8192, 7168, 256, 8, 6)) == (2, 5, 0)                # 4.4
     assert shape(move("cast", 8192, 7168, 256, 8, 8, expanded=True)) == (2, 3, 0)
     assert shape(move("cast", 5210, 5888, 256, 32, 8)) == (2, 4, 0) and shape(move("cast", 5200, 5888, 256, 32, 8)) == (2, 0, 0)       # 220 MB
+
+
+def test_large_rows_of_whole_kb():
+    a = (16384, 7168, 256, 32, 8)
+    assert shape(move("bf16", *a)) == (1, 6, 1) and shape(move("bf16", *a, cached=True)) == (1, 5, 1)                     # 7.2 rows
+    assert shape(move("bf16", 16384, 7168, 256, 16, 8, cached=True)) == (1, 6, 1)                                        # 6.5
+    assert shape(move("bf16", 4000, 7168, 256, 32, 8)) == (1, 4, 0) and shape(move("bf16", 4000, 7168, 64, 8, 8)) == (1, 5, 0)      # up to 430 MB
+    assert shape(move("bf16", 24000, 4096, 64, 8, 6)) == (2, 3, 0)                                                       # rows of 8 KB, 4.4
+    assert shape(move("bf16", 16380, 7168, 256, 16, 4)) == (2, 3, 0) and shape(move("bf16", 14174, 8192, 64, 8, 4)) == (2, 4, 0)    # 3.6 and 3.3
+    assert shape(v1_move("bf16", 8192, 7168, 4, 22118)) == (1, 0, 0) and shape(v1_move("bf16", 8192, 7168, 8, 26215)) == (1, 0, 1)  # 2.7 and 3.2, no top-k
+    assert shape(move("fp8", 16384, 7168, 256, 32, 8)) == (1, 6, 1) and shape(move("fp8", 8192, 7168, 64, 8, 8)) == (1, 0, 1)
+    assert shape(move("fp8", 20000, 3968, 64, 8, 6)) == (2, 4, 0) and shape(move("fp8", 17000, 3968, 64, 8, 8, expanded=True)) == (2, 3, 0)
+
+
+def test_large_rows_of_no_whole_kb():
+    assert shape(move("bf16", 16746, 8072, 64, 8, 2)) == (2, 5, 0) and shape(move("bf16", 16746, 8072, 64, 64, 2)) == (2, 4, 0)     # 1.9 and 2.0 rows
+    assert shape(move("bf16", 9000, 8008, 64, 8, 1)) == (2, 0, 0)
+    assert shape(move("bf16", 10000, 1048, 256, 32, 8)) == (4, 2, 0) and shape(move("bf16", 8000, 2040, 64, 8, 8)) == (4, 2, 0)     # 3 and 4 KB
+    assert shape(move("bf16", 2230, 5112, 64, 8, 8)) == (2, 2, 0) and shape(move("bf16", 9000, 5112, 64, 8, 6)) == (2, 3, 0)        # 5.3 rows; 92 MB, 4.4
+    assert shape(move("bf16", 4500, 5112, 64, 4, 4)) == (2, 3, 0)                                                                     # 2.7
