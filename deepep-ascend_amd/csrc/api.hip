@@ -78,12 +78,18 @@ LaunchPlan plan_launches(const MoveParams& m, bool do_layout, bool do_move, bool
     if (q.fused && do_expand && tuning.dispatch_launches != 1 && int64_t(T) * row_bytes >= (int64_t(64) << 20)) q.fused = false;
     // A move on a finished layout zeroes the padding rows beside its own work, a single launch leaves them to one more launch.  One / two
     // launches, us, padding included: BF16, over 44 shapes of 13 to 64 MB of input two are ahead by 4 % on average and never 2.5 % behind
-    // (6485 x 1280 top-2 of 64 24.1 / 22.6, 4462 x 5120 top-8 of 64 85.2 / 84.9; 1992 x 4224 top-4 of 256, alignment 4, 23.6 / 24.2); FP8 rows 300 x
-    // 7168 top-8 of 256 47.5 / 41.1, 72 x 3968 top-10 of 16 19.1 / 14.1, 2613 x 6144 fp8 49.6 / 49.1; but many of them from a large input, whose
-    // first loads hide the layout: cast, 3000 x 7168 top-6 of 64 49.8 / 52.9, 5346 x 3712 top-4 of 16 36.2 / 40.5, fp8 5342 x 6272 top-6 61.3 / 72.8,
-    // 8417 x 5120 top-4 of 128 63.8 / 65.0; with many narrow rows two again (cast, 13820 x 1280 top-6 54.0 / 48.5, 12640 x 2432 77.7 / 72.0).
-    if (q.fused && do_zero_padding && alignment > 1 && tuning.dispatch_launches != 1)
-        q.fused = payload != DEEP_EP_HIP_PAYLOAD_BF16 && int64_t(T) * row_bytes >= 26000000 && int64_t(T) * K * H >= 80000000 && T <= 10000;
+    // (6485 x 1280 top-2 of 64 24.1 / 22.6, 4462 x 5120 top-8 of 64 85.2 / 84.9; 1992 x 4224 top-4 of 256, alignment 4, 23.6 / 24.2), and so are small FP8 calls (300 x
+    // 7168 top-8 of 256 47.5 / 41.1).  Many FP8 rows from a large input, whose first loads hide the layout, are the other way round.  Dispatch and combine in a single launch against
+    // two, in %, 64 experts aligned to 64, input of 28 / 40 / 60 MB:
+    //   fused cast, 4608 to 7168 channels   top-4 -0.9 (60 MB), top-6 -1.1 / -3.0 / -2.3, top-8 +0.6 / -3.2 / -0.5
+    //               2048 to 3584            top-4 +2.2 (60 MB), top-6 +1.9 / -0.4 / +1.9, top-8 +3.2 / -1.0 / +1.1
+    //   FP8 pairs, top-4, 6 and 8, by the rows they make   112 MB +3.0, 160 MB +2.4, 168 MB +2.0, 224 MB -1.4, 240 MB -2.2, 320 MB -0.1, 360 MB +1.6, 480 MB -1.1 (three shapes);
+    //     13309 x 3840 top-6 of 16 ranks (307 MB), dispatch alone, 95.9 / 86.4, 14194 x 2560 top-8 (291 MB) 95.6 / 91.4
+    if (q.fused && do_zero_padding && alignment > 1 && tuning.dispatch_launches != 1) {
+        const int64_t channels = int64_t(T) * K * H;
+        q.fused = payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8 ? H >= 4096 && int64_t(T) * row_bytes >= 26000000 && channels >= 80000000
+                                                          : payload == DEEP_EP_HIP_PAYLOAD_FP8 && channels >= 200000000 && channels <= 260000000;
+    }
     if (q.fused && tuning.dispatch_launches != 1) {
         MoveParams single = m;
         single.fused = 1;

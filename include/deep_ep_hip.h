@@ -77,9 +77,9 @@ typedef struct {
                                   mover workgroups; rows copied as they are from less than 64 MB of input, and less than 300 MB
                                   of them (345 MB of rows of up to 4 KB); no compact cast of four rows a token and more with
                                   movers + counting workgroups >= 6 and movers <= 7 for each compute unit; with do_expand less
-                                  than 64 MB of input; with do_zero_padding and an alignment only FP8 rows and casts of 26 to
-                                  64 MB of input, up to 10000 tokens, that make 80 M channels of rows
-                                  and more.  1 = a single launch wherever the shape allows it; 2 = always layout
+                                  than 64 MB of input; with do_zero_padding and an alignment only casts of 4096 channels and
+                                  more from 26 MB of input on that make 80 M channels of rows and more, and
+                                  200 to 260 MB of FP8 rows.  1 = a single launch wherever the shape allows it; 2 = always layout
                                   kernel + move kernel */
     int32_t cast_pairs;        /* fused FP8 cast: 1024-channel segments per wavefront (1, 2, 4, 7, 8; above 2: two launches) */
     int32_t copy_vecs;         /* pass-through payloads: KB of row per wavefront (1, 2, 4, 7, 8) */

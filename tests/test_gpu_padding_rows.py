@@ -21,7 +21,8 @@ pytestmark = pytest.mark.gpu
     ("cast", 72, 2560, 128, 16, 8, 128), ("pair", 201, 640, 24, 4, 10, 16),
     ("cast", 1801, 7168, 16, 4, 8, 128), ("cast", 1820, 7168, 16, 4, 8, 128),    # 25.8 and 26.1 MB of input: two launches and one, with blocks
     ("cast", 5499, 3584, 16, 2, 8, 5), ("cast", 5503, 3584, 16, 2, 8, 5),        # 43992 and 44024 rows: columns and blocks
-    ("pair", 5182, 5248, 16, 2, 8, 3), ("pair", 5188, 5248, 16, 2, 8, 3),        # 1.6997 and 1.7017 M scales
+    ("pair", 5182, 5248, 16, 2, 8, 3), ("pair", 5188, 5248, 16, 2, 8, 3),        # a single launch, with blocks
+    ("pair", 4146, 5248, 16, 2, 10, 3), ("pair", 4147, 5248, 16, 2, 10, 3),      # 1.6999 and 1.7003 M scales: columns and blocks
 ], ids=lambda v: str(v))
 @pytest.mark.parametrize("columns", [True, False], ids=["columns", "rows"])
 def test_padding_rows_read_zero(payload, T, H, E, R, K, alignment, columns):

@@ -28,6 +28,31 @@ def test_launches(payload, T, H, R, K, E, launches):
     assert _abi.lib.deep_ep_hip_dispatch_kernel_launches(ctypes.byref(a)) == launches
 
 
+PADDED_LINES = [
+    # payload, T, hidden, top-k, launches: expanded, padding rows of 64 experts over 8 ranks, aligned to 128, to be zeroed
+    ("bf16", 600, 2048, 4, 2), ("bf16", 4000, 4096, 8, 2),
+    ("cast", 3173, 4096, 8, 2), ("cast", 3174, 4096, 8, 1),                          # 26 MB of input
+    ("cast", 7999, 5000 // 128 * 128, 2, 2), ("cast", 4882, 4096, 4, 2), ("cast", 4883, 4096, 4, 1),      # 80 M channels of rows
+    ("cast", 5000, 3968, 8, 2), ("cast", 5000, 4096, 8, 1), ("cast", 8191, 4096, 8, 1), ("cast", 8192, 4096, 8, 2),      # 4096 channels; 64 MB of input
+    ("fp8", 6103, 4096, 8, 2), ("fp8", 6104, 4096, 8, 1), ("fp8", 7934, 4096, 8, 1), ("fp8", 7935, 4096, 8, 2),         # 200 and 260 MB of rows
+    ("fp8", 15000, 4096, 4, 1), ("fp8", 4000, 4096, 8, 2),
+]
+
+
+@pytest.mark.parametrize("payload,T,H,K,launches", PADDED_LINES)
+def test_launches_with_padding_to_zero(payload, T, H, K, launches):
+    a = _abi.DispatchArgs()
+    a.phases = _abi.PHASE_LAYOUT | _abi.PHASE_MOVE
+    a.payload = {"bf16": _abi.PAYLOAD_BF16, "fp8": _abi.PAYLOAD_FP8, "cast": _abi.PAYLOAD_CAST_FP8}[payload]
+    a.num_tokens, a.hidden, a.num_topk, a.num_experts, a.num_ranks, a.expert_alignment = T, H, K, 64, 8, 128
+    a.do_expand = a.do_zero_padding = 1
+    assert _abi.lib.deep_ep_hip_dispatch_kernel_launches(ctypes.byref(a)) == launches
+    a.tuning.dispatch_launches = 1
+    assert _abi.lib.deep_ep_hip_dispatch_kernel_launches(ctypes.byref(a)) == 1
+    a.tuning.dispatch_launches, a.expert_alignment = 0, 1                            # nothing to zero: single but for 64 MB of input
+    assert _abi.lib.deep_ep_hip_dispatch_kernel_launches(ctypes.byref(a)) == (2 if T * H * (1 if payload == "fp8" else 2) >= 64 << 20 else 1)
+
+
 LL_LINES = [
     # source ranks, tokens of each, hidden, top-k, local experts, threads (0: two kernels); 256 compute units
     (8, 512, 512, 1, 32, 0),                                                            # 4096 tokens: past 3072

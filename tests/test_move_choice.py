@@ -197,3 +197,13 @@ def test_large_rows_of_no_whole_kb():
     assert shape(move("bf16", 10000, 1048, 256, 32, 8)) == (4, 2, 0) and shape(move("bf16", 8000, 2040, 64, 8, 8)) == (4, 2, 0)     # 3 and 4 KB
     assert shape(move("bf16", 2230, 5112, 64, 8, 8)) == (2, 2, 0) and shape(move("bf16", 9000, 5112, 64, 8, 6)) == (2, 3, 0)        # 5.3 rows; 92 MB, 4.4
     assert shape(move("bf16", 4500, 5112, 64, 4, 4)) == (2, 3, 0)                                                                     # 2.7
+
+
+@pytest.mark.parametrize("payload,T,H,K,blocked", [("cast", 5499, 3584, 8, 0), ("cast", 5501, 3584, 8, 1), ("pair", 4146, 5248, 10, 0), ("pair", 4147, 5248, 10, 1),
+                                                   ("pair", 5188, 5120, 10, 0)])
+def test_scales_in_blocks(payload, T, H, K, blocked):
+    """From 44000 moved rows of a cast on, from 1.7 M scales of FP8 pairs of more than 5120 channels on; column-major scales only."""
+    a = dict(expanded=True, alignment=3, pads=True)
+    payload = "fp8" if payload == "pair" else payload
+    assert move(payload, T, H, 16, 2, K, columns=True, **a).blocked_scales == blocked
+    assert move(payload, T, H, 16, 2, K, **a).blocked_scales == 0
