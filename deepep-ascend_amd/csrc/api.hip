@@ -59,7 +59,7 @@ LaunchPlan plan_launches(const MoveParams& m, bool do_layout, bool do_move, bool
     LaunchPlan q{};
     q.chunks = T > 0 ? (T + kLayoutChunk - 1) / kLayoutChunk : 1;
     q.chunks_padded = (q.chunks + 3) / 4 * 4;
-    q.fused = do_layout && do_move && T > 0 && K <= 8 && (R + E) <= 512 && R * q.chunks_padded <= kTaggedRankWords &&
+    q.fused = do_layout && do_move && T > 0 && K <= kSingleLaunchTopk && (R + E) <= 512 && R * q.chunks_padded <= kTaggedRankWords &&
               int64_t(T) * K <= kTaggedPosWords && tuning.dispatch_launches != 2 &&
               !(tuning.persistent_movers > 0 && payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8);      // the persistent move runs on a finished layout
     if (q.fused && do_expand) {

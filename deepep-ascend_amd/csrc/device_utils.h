@@ -51,17 +51,6 @@ __device__ __forceinline__ void store16_stream(void* p, const vec16& v) {
     __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
 }
 
-template <bool kStream>
-__device__ __forceinline__ vec16 load16_as(const void* p) {
-    if constexpr (kStream) return load16_stream(p);
-    else return load16(p);
-}
-template <bool kStream>
-__device__ __forceinline__ void store16_as(void* p, const vec16& v) {
-    if constexpr (kStream) store16_stream(p, v);
-    else store16(p, v);
-}
-
 // bf16 <-> fp32 on raw bits.
 __device__ __forceinline__ float bf16_lo(uint32_t packed) { return __uint_as_float(packed << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t packed) { return __uint_as_float(packed & 0xffff0000u); }
@@ -261,11 +250,6 @@ template <bool kThrough>
 __device__ __forceinline__ void store_word(int* p, int v) {
     if constexpr (kThrough) store_agent(p, v);
     else *p = v;
-}
-template <bool kAgent>
-__device__ __forceinline__ int load_word(const int* p) {
-    if constexpr (kAgent) return load_agent(p);
-    else return *p;
 }
 // 16 bytes stored at agent scope (written through), as two 8-byte atomic stores: the language offers atomics of at most
 // 8 bytes, and a 16-byte store written as an instruction by hand would sit outside the compiler's hazard tracking

@@ -343,7 +343,7 @@ __device__ __forceinline__ unsigned movers_of_gate(const MoveParams& p, unsigned
 __device__ __forceinline__ void fused_count_block(const MoveParams& p) {
     extern __shared__ uint64_t count_lds[];
     const int c = int(blockIdx.x);
-    count_chunk<8>(p.lay, c, p.count_blocks, count_lds);
+    count_chunk(p.lay, c, p.count_blocks, count_lds);
     wait_for_own_stores();
     __syncthreads();
     if (threadIdx.x == 0) store_agent(p.chunk_done + c, 1);      // for the publisher

@@ -18,6 +18,7 @@ namespace deep_ep_hip {
 constexpr int kDispatchGates = 256;
 constexpr int kDispatchGateStride = 32;
 constexpr int kMaxCountBlocks = 1024;
+constexpr int kSingleLaunchTopk = 8;         // selections a token, at most
 
 // Single-launch dispatch: words that counting and publishing workgroups hand to the movers of the same launch carry
 // the launch's tag in their upper bits, so that a reader knows a word of this launch from what an earlier launch left
@@ -104,7 +105,7 @@ struct LayoutParams {
     int T, K, E, R, E_l;
     int vec_idx;          // topk_idx is 16-byte aligned (set by the launcher)
     int lds_totals;       // layout kernel of one workgroup: where its totals lie in LDS, bytes (set by the launcher)
-    uint8_t* is_token_in_rank;       // optional
+    uint8_t* is_token_in_rank;       // optional, layout launch only
     int64_t* copied_topk_idx;        // optional
     PublishParams pub;
     int32_t* status;

@@ -35,9 +35,8 @@ __host__ __device__ inline size_t count_lds_bytes(int R, int E) {
 // bitmap: LDS of count_lds_bytes(R, E) bytes.  Must be called by all 256 threads of the workgroup.
 // Positions are stored at agent scope (movers of the same launch read them) and carry, like the copy of the rank totals in
 // p.tagged_rank, the launch's tag; chunk totals go out at agent scope, to the count tables.
-template <int KMAX>
 __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chunk, const int num_chunks, uint64_t* bitmap) {
-    constexpr int kThreads = kLayoutChunk;
+    constexpr int KMAX = kSingleLaunchTopk, kThreads = kLayoutChunk;
     constexpr int kWaves = kThreads / kWaveSize;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int t = chunk * kThreads + tid;
@@ -53,7 +52,7 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
 #pragma unroll
         for (int k = 0; k < KMAX; ++k)
             raw[k] = (active && k < p.K && p.route_mask[int64_t(t) * p.K + k] != 0) ? int64_t(k) : int64_t(-1);
-    } else if (KMAX == 8 && p.K == 8 && p.vec_idx) {
+    } else if (p.K == 8 && p.vec_idx) {
         if (active) {
             const vec16* src = reinterpret_cast<const vec16*>(p.topk_idx + int64_t(t) * 8);
             vec16 q[4];
@@ -208,7 +207,7 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
     }
 
     if (active && p.pos != nullptr) {                        // movers of this launch are waiting for them
-        if (KMAX == 8 && p.K == 8) {
+        if (p.K == 8) {
             vec16* dst = reinterpret_cast<vec16*>(p.pos + int64_t(t) * 8);
             store16_agent(dst, vec16{packed[0], packed[1], packed[2], packed[3]});
             store16_agent(dst + 1, vec16{packed[4], packed[5], packed[6], packed[7]});
@@ -219,11 +218,6 @@ __device__ __forceinline__ void count_chunk(const LayoutParams& p, const int chu
         }
     }
     if (flags != 0) atomicOr(p.status, flags);
-
-    if (active && p.is_token_in_rank != nullptr) {
-        for (int r = 0; r < p.R; ++r)
-            p.is_token_in_rank[int64_t(t) * p.R + r] = uint8_t((bitmap[r * kWaves + wave] >> lane) & 1ull);
-    }
 }
 
 }  // namespace deep_ep_hip
