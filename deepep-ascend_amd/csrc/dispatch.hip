@@ -1439,7 +1439,8 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 //     563.6;   8192 x 7168 of 32 110.6, 268.1 / 115.1, 271.9;   of 64 118.0, 280.8 / 125.5, 293.4;   25585 x 3072 of 32 147.3, 352.6 / 144.4, 358.4;   16384 x 4096 of 32 126.5, 307.6 /
 //     131.9, 301.2;   fewer rows or other rows 16384 x 7168 of 16 192.9, 474.5 / 192.4, 470.1;   14000 x 6272 top-10 of 16 176.4, 423.2 / 170.2, 411.8;   with
 //     blocked scales, whose rows have no single-dword stores, 8192 x 7168 318.1 (5) / 324.0 (3): left alone;
-//   FP8 pairs, expanded, 24963 x 3584 top-9 505.7 (5) / 495.9 (3) / 496.9 (2), 521.1;   compact, 28277 x 4864 (5.9) 485.8 (8) / 473.2 (3) / 474.1 (2),
+//   FP8 pairs, expanded, of 210 to 270 MB, top-4 / 6 / 8, against what the smaller tiles' rules take: 4 KB -17.5 / -13.7 / -10.2 %, four of 2 KB -14.3 /
+//     -11.9 / -8.7, three -7.6 / -9.7 / -7.7;   of 320 MB 4 KB against three or four of 2 KB -3.9 / -2.5 / -0.6;   24963 x 3584 top-9 505.7 (5) / 495.9 (3) / 496.9 (2), 521.1;   compact, 28277 x 4864 (5.9) 485.8 (8) / 473.2 (3) / 474.1 (2),
 //     487.5;   35472 x 3968 (4.4) 438.3 (8) / 427.7 (4) / 437.9 (6), 438.3;   rows of whole KB like those of BF16, move alone, without / with the wait: 16384 x 7168 of 32
 //     ranks 174.8 (5) / 175.0 (6), 181.6 (8);   32768 x 2048 103.7 (5) / 102.0 (8), 109.0 (8);   8192 x 7168 of 8 66.9 / 64.9 (8);   20000 x 4096 95.0 / 91.3 (8);
 //     12000 x 3072 of 16, top-6 45.3 / 44.2 (8);   4096 x 7168 36.0 / 35.4 (8);   12000 x 5120 of 32 101.9 (4) / 105.1 (6), 105.2.
@@ -1460,6 +1461,10 @@ static bool large_move_shape(const MoveParams& p, MoveShape& q) {
     }
     const bool whole = bytes % 1024 == 0;
     if (p.payload == DEEP_EP_HIP_PAYLOAD_FP8) {
+        if (p.do_expand && kb >= 3 && rows >= 3.2 && out >= 200e6 && out < 300e6) {
+            q = {4, 0, false};
+            return true;
+        }
         if (rows < 3.2 || out < (whole && !p.do_expand ? 100e6 : 280e6)) return false;
         if (whole && !p.do_expand) q = {1, rows < 6.0 ? 0 : 6, true};
         else q = {2, rows < 5.0 ? 4 : 3, false};

@@ -188,6 +188,8 @@ def test_large_rows_of_whole_kb():
     assert shape(move("bf16", 16380, 7168, 256, 16, 4)) == (2, 3, 0) and shape(move("bf16", 14174, 8192, 64, 8, 4)) == (2, 4, 0)    # 3.6 and 3.3
     assert shape(v1_move("bf16", 8192, 7168, 4, 22118)) == (1, 0, 0) and shape(v1_move("bf16", 8192, 7168, 8, 26215)) == (1, 0, 1)  # 2.7 and 3.2, no top-k
     assert shape(move("fp8", 16384, 7168, 256, 32, 8)) == (1, 6, 1) and shape(move("fp8", 8192, 7168, 64, 8, 8)) == (1, 0, 1)
+    assert shape(move("fp8", 6301, 3968, 64, 8, 8, expanded=True)) == (4, 0, 0) and shape(move("fp8", 9450, 3968, 64, 8, 8, expanded=True)) == (4, 0, 0)   # 200 and 300 MB
+    assert shape(move("fp8", 9453, 3968, 64, 8, 8, expanded=True)) == (2, 3, 0)
     assert shape(move("fp8", 20000, 3968, 64, 8, 6)) == (2, 4, 0) and shape(move("fp8", 17000, 3968, 64, 8, 8, expanded=True)) == (2, 3, 0)
 
 
