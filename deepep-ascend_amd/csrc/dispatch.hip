@@ -1411,8 +1411,8 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 //   BF16 past the memory-side cache (cached_side):
 //     10967 x 5848 of 8 ranks (5.6 rows) 333.1 (4) / 331.9 (2) / 356.6 (8), before 361.5;   8371 x 5048 204.5 (3) / 204.4 (2) / 208.2 (2), 217.8;
 //     6221 x 4488 of 64 ranks (9.3) 255.7 / 249.7 / 249.3 (2 each), 263.6;   from 90 MB of input, up to 5.2 rows, 17335 x 3712 (4.4) 250.2 with
-//     three of 2 KB, 261.5 with two, 265.1;   15819 x 6096 (2.7) 247 (8) / 243.3 (3) / 249 (2), 245.1;   16746 x 8072 (2.0) 283.5 (8) / 278.1 (8),
-//     280.9 with five, 281.6 with four;   rows of 3 and 4 KB 21387 x 1048 (6.5) 174.0 / 171.9 / 165.2 (2 each), 174.1;
+//     three of 2 KB, 261.5 with two, 265.1;   15819 x 6096 (2.7) 247 (8) / 243.3 (3) / 249 (2), 245.1;   two rows, 2 KB without a limit / with five, move and with the combine, 16746 x 8072 of 8
+//     166.9, 303.5 / 163.6, 299.7;   of 32 173.8, 314.3 / 166.5, 308.2;   20000 x 3976 of 8 99.8, 178.4 / 94.5, 173.2;   of 64 16746 x 8072 185.6, 333.2 / 174.7, 315.2 (four);   rows of 3 and 4 KB 21387 x 1048 (6.5) 174.0 / 171.9 / 165.2 (2 each), 174.1;
 //   - nine and more expanded rows over fewer than 32 ranks in two of 1 KB from 450 MB on, rows that are no whole 64 bytes, in % of two of 2 KB, straight /
 //     with a pass in between: 500 MB top-10 -4.2 / -1.3, top-9 -2.7 / +0.5, 700 MB top-10 -1.3 / -1.5, top-9 -2.5 / -0.5, 1 GB top-10 -3.6 / -1.0;   of eight rows level
 //     / +2.2, of 350 MB of ten +0.7 / -1.3;   rows of whole 64 bytes, which both halves of a KB then share with nobody, +9 to +20 / +10 to +13 (500 MB, 3424 channels
@@ -1425,7 +1425,8 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 //     534.9;   13211 x 4096 of 16 353.0 / 348.2, 360.1;   16384 x 7168 of 16 (6.5) 607.0 / 609.9, 611.2;   of 32 685.1 / 686.4, 685.5, with five and
 //     the wait 710;   on a handle with the wait, five / six, moves alone and with the combine: 16384 x 7168 of 32 (7.2) 340.0, 646.5 /
 //     344.1, 671.1;   of 16 (6.5) 316.1, 587.0 / 300.7, 572.7;   9800 x 7168 of 16 185.7, 353.2 / 178.0, 346.6;   13211 x 4096 of 16 149.8, 280.9 / 141.7, 274.8;   16384 x 5120 of 64
-//     260.2, 500.2 / 269.1, 505.5;   30000 x 2048 of 32 181.6, 350.9 / 184.5, 348.1;
+//     260.2, 500.2 / 269.1, 505.5;   30000 x 2048 of 32 181.6, 350.9 / 184.5, 348.1;   with the wait, six / as many as fit, moves and with another pass and the combine: of 8 ranks top-6 (4.4)
+//     7118 x 7168 111.8, 345.9 / 105.8, 346.0;   15502 x 5120 160.6, 536.8 / 157.0, 527.1;   on a handle 155.7, 535.6 / 147.8, 521.3;   of 64 top-5 (4.8) on one 10075 x 7168 150.9, 509.7 / 152.6, 491.9;
 //     rows of 8 and 16 KB, top-6, in three of 2 KB: 24000 x 4096 of 8 ranks (4.4) 361.4 / 369.9 (6), 373.8;   14000 x 8192 418.2 / 430.7 (6), 450.2;
 //     where a token goes to fewer than four rows: 14174 x 8192 (3.3) 348 (8 of 1 KB) / 336.8 (4 of 2 KB), 337.5;   16380 x 7168 (3.6) 353.9 (3 of 2 KB),
 //     360.9;   17516 x 3584 (3.7) 204.7 (3 of 2 KB) / 197.8 (8 of 1 KB with the wait), 199.5;   without top-k tensors, moves alone, 8192 x 7168 of 4 ranks
@@ -1480,7 +1481,7 @@ static bool large_move_shape(const MoveParams& p, MoveShape& q) {
         else if (rows < 3.9 && (rows < 3.5 || kb >= 8 || out < 430e6)) q = {2, rows < 3.5 || kb < 8 ? 4 : 3, false};
         else if (out < 430e6) q = {1, rows < 6.4 ? 5 : 4, false};
         else if ((kb & (kb - 1)) == 0 && kb >= 8 && rows < 5.0) q = {2, 3, false};
-        else q = {1, rows < 4.2 ? 0 : p.cached && rows >= 7.0 ? 5 : 6, true};
+        else q = {1, rows < (p.cached ? 5.0 : 4.5) ? 0 : p.cached && rows >= 7.0 ? 5 : 6, true};
         return true;
     }
     if (kb == 3 || kb == 4) {
