@@ -1434,6 +1434,9 @@ static bool fills_rounds(const MoveParams& p, int tile, int rounds) {
 //     expanded 25983 x 2560 top-2 156.2 (8 of 2 KB), 173.4;
 //   - a few rows among much padding, whose zeroes are most of the call, come here too and are level: 17 shapes of 60 to 1000 tokens x 7168 or 2048 of 256 to 512 experts
 //     aligned to 128, layout, move and padding, with a pass over the rows and a combine behind them or not, -0.2 % with four of 2 KB, -1 to +1 without a limit;
+//   - rows of whole KB, BF16 and FP8, over 56 to 64 ranks, top-4, with the wait / three (BF16) or four (FP8) of 2 KB, moves and with the combine: 64 ranks BF16 14282 x 7168 203.2, 361.1 /
+//     185.4, 347.8;   12496 x 5120 126.1, 228.7 / 122.8, 228.0;   FP8 28564 x 7168 227.1, 543.3 / 200.7, 526.9;   24993 x 5120 145.7, 348.5 / 135.7, 339.8;   move alone of 500 MB, four shapes,
+//     40 ranks +1.3 % by 2 KB, 56 -1.9, 60 -2.6, 63 -2.6, 64 -5.0, 65 (whose lanes read the base of their own rank, as on a handle, not of all) +7.3, 96 +6.0;   of 300 MB level, on a handle +5.8;
 //   fused cast, expanded, 8192 x 7168 top-8 315.4 (4) / 312.4 (3), 320.6;   16316 x 4608 403.9 (4) / 393.9 (3), 418.5;   compact, 25585 x 3072 of 32
 //     ranks 352.5 (4) / 351.8 (4), 364.5;   8192 x 7168 of 8 200.2 (6) / 199.3 (4), 200.4;   12006 x 5120 top-6 (4.4) 204.4 (8) / 202.9 (5), 205.1;   seven
 //     rows and more of whole KB, move alone and with the combine, four of 1 KB / four of 2 KB: 16384 x 7168 of 32 204.2, 530.8 / 212.8, 534.9;   of 64 223.1, 555.4 / 230.8,
@@ -1460,14 +1463,15 @@ static bool large_move_shape(const MoveParams& p, MoveShape& q) {
         else q = {2, rows < 5.0 ? 5 : p.do_expand ? 3 : 4, false};
         return true;
     }
-    const bool whole = bytes % 1024 == 0;
+    const bool whole = bytes % 1024 == 0, many_ranks_few_rows = p.R >= 56 && p.R <= 64 && rows < 4.5 && out >= 350e6 && !p.cached && !p.rank_lanes;
     if (p.payload == DEEP_EP_HIP_PAYLOAD_FP8) {
         if (p.do_expand && kb >= 3 && rows >= 3.2 && out >= 200e6 && out < 300e6) {
             q = {4, 0, false};
             return true;
         }
         if (rows < 3.2 || out < (whole && !p.do_expand ? 100e6 : 280e6)) return false;
-        if (whole && !p.do_expand) q = {1, rows < 6.0 ? 0 : 6, true};
+        if (whole && !p.do_expand && many_ranks_few_rows) q = {2, 4, false};
+        else if (whole && !p.do_expand) q = {1, rows < 6.0 ? 0 : 6, true};
         else q = {2, rows < 5.0 ? 4 : 3, false};
         return true;
     }
@@ -1478,6 +1482,7 @@ static bool large_move_shape(const MoveParams& p, MoveShape& q) {
     }
     if (whole) {
         if (p.rank_lanes && rows < 3.9) q = {1, 0, rows >= 3.0};
+        else if (many_ranks_few_rows) q = {2, 3, false};
         else if (rows < 3.9 && (rows < 3.5 || kb >= 8 || out < 430e6)) q = {2, rows < 3.5 || kb < 8 ? 4 : 3, false};
         else if (out < 430e6) q = {1, rows < 6.4 ? 5 : 4, false};
         else if ((kb & (kb - 1)) == 0 && kb >= 8 && rows < 5.0) q = {2, 3, false};

@@ -38,6 +38,8 @@ CASES = {   # tokens, channels, experts, ranks, selections, payload, expanded, a
     "whole_power_of_two": ((10007, 4096, 64, 8, 8, "bf16", False, 1), (1, 6, 1)),                # 430 MB of 8 KB, 5.3 rows
     "whole_power_of_two_four_rows": ((12503, 4096, 64, 8, 6, "bf16", False, 1), (2, 3, 0)),      # 4.4
     "whole_in_turn_no_limit": ((7507, 7168, 64, 8, 6, "bf16", False, 1), (1, 0, 1)),
+    "whole_many_ranks": ((7001, 7168, 256, 64, 4, "bf16", False, 1), (2, 3, 0)),
+    "fp8_whole_many_ranks": ((14003, 7168, 256, 64, 4, "fp8", False, 1), (2, 4, 0)),
     "whole_few_rows": ((9001, 4096, 64, 8, 4, "bf16", False, 1), (2, 4, 0)),
     "fp8_four_workgroups": ((20011, 3968, 64, 8, 6, "fp8", False, 1), (2, 4, 0)),
     "fp8_three_workgroups": ((17011, 3968, 64, 8, 8, "fp8", True, 1), (2, 3, 0)),

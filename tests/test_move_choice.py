@@ -185,6 +185,10 @@ def test_large_rows_of_whole_kb():
     assert shape(move("bf16", 16384, 7168, 256, 16, 8, cached=True)) == (1, 6, 1)                                        # 6.5
     assert shape(move("bf16", 8000, 7168, 64, 8, 6)) == (1, 0, 1) and shape(move("bf16", 8000, 7168, 256, 32, 5)) == (1, 6, 1)             # 4.4 and 4.7
     assert shape(move("bf16", 8000, 7168, 256, 64, 5, cached=True)) == (1, 0, 1) and shape(move("bf16", 8000, 7168, 64, 8, 8, cached=True)) == (1, 6, 1)   # 4.8, 5.3
+    assert shape(move("bf16", 8000, 7168, 256, 64, 4)) == (2, 3, 0) and shape(move("fp8", 16000, 7168, 256, 64, 4)) == (2, 4, 0)
+    assert shape(move("bf16", 8000, 7168, 260, 65, 4)) == (1, 0, 1) and shape(move("fp8", 16000, 7168, 260, 65, 4)) == (1, 0, 1)
+    assert shape(move("bf16", 8000, 7168, 256, 64, 4, cached=True)) == (1, 0, 1) and shape(move("fp8", 16000, 7168, 220, 55, 4)) == (1, 0, 1)
+    assert shape(move("bf16", 6190, 7168, 256, 64, 4)) == (1, 5, 0) and shape(move("bf16", 6290, 7168, 256, 64, 4)) == (2, 3, 0)             # 347 and 353 MB
     assert shape(move("bf16", 4000, 7168, 256, 32, 8)) == (1, 4, 0) and shape(move("bf16", 4000, 7168, 64, 8, 8)) == (1, 5, 0)      # up to 430 MB
     assert shape(move("bf16", 24000, 4096, 64, 8, 6)) == (2, 3, 0)                                                       # rows of 8 KB, 4.4
     assert shape(move("bf16", 16380, 7168, 256, 16, 4)) == (2, 3, 0) and shape(move("bf16", 14174, 8192, 64, 8, 4)) == (2, 4, 0)    # 3.6 and 3.3
