@@ -273,7 +273,7 @@ double rows_per_token(const CombineParams& p) {
     const int selections = p.rank_mode ? p.Kw : p.K;
     if (selections == 0) return returned;
     const int ranks = p.rank_mode ? p.K : p.R;
-    return std::min(returned, p.do_expand && !p.rank_mode ? double(selections) : ranks * (1.0 - std::pow(1.0 - 1.0 / ranks, selections)));
+    return std::min(returned, p.do_expand && !p.rank_mode ? double(selections) : distinct_ranks(ranks, selections));
 }
 
 // How many workgroups a CU should hold at a time (0: the eight its registers allow).  Scattered rows stream fastest when not

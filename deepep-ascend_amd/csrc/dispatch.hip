@@ -1361,7 +1361,7 @@ static int lds_bytes_per_cu() {
 static double rows_per_token(const MoveParams& p) {
     if (p.rank_lanes) return std::min(double(p.R), double(p.recv_capacity) / p.T);
     if (p.do_expand) return p.K;
-    return p.R * (1.0 - std::pow(1.0 - 1.0 / p.R, p.K));
+    return distinct_ranks(p.R, p.K);
 }
 
 // The bytes of those rows.
