@@ -1502,13 +1502,12 @@ static bool large_move_shape(const MoveParams& p, MoveShape& q) {
 // the pass-through payloads.  A tile of one whose last wavefront of a row would be half idle loses to one of two: 65536
 // tokens x 768 BF16 over 16 ranks 152 against 175 us, fused cast of 32768 x 1152 over 32 ranks 82 against 104 us.
 //
-// Calls that leave the chip half empty take the narrowest tile that still gives a CU no more than eight wavefronts (ten with 2 KB
-// tiles): what a wavefront does is a chain, and a shorter one is over sooner.  Layout and move of compact calls with 1 / 2 / 4 KB tiles, us:
-// BF16 top-8 of 8 ranks 128 x 4096 14.0 / 14.2 / 14.9, 512 x 2048 16.7 / 16.9 / 17.5, 1237 x 2048 18.6 / 18.4 / 19.3 (2474 wavefronts of
-// 2 KB), 512 x 7168 23.0 / 20.6 / 19.7 (3584): left alone; fused cast, 1 / 2 segments, 300 x 7168 18.0 / 18.3, 512 x 2048 16.8 / 17.4,
-// 512 x 7168 (3584) 19.2 / 18.9.  Not in a single launch, where neighbours of the counting workgroups wait: 512 x 2048 BF16 16.7 / 16.5
-// / 15.6, though 300 x 7168 takes 16.7 / 16.3 / 17.5.
-// BF16 rows that stay in the memory-side cache take the tile of the combine (kb_of_wavefront); beyond its lines tokens of three rows and more of 4, 8
+// FP8 rows of calls that leave the chip half empty take the narrowest tile that still gives a CU no more than eight wavefronts (ten with 2 KB
+// tiles): what a wavefront does is a chain, and a shorter one is over sooner.  Layout and move of compact calls, top-8 of 8 ranks, with 1 / 2 / 4 KB
+// tiles, us: pairs 128 x 4096 10.5 / 10.7 / 11.0, 128 x 8192 10.8 / 10.9 / 11.2, 512 x 4096 12.9 / 12.8 / 13.2, 1237 x 4096 15.2 / 15.6 / 15.8 (2474
+// wavefronts of 2 KB), 512 x 14336 18.3 / 17.6 / 17.5 (3584): left alone; fused cast, 1 / 2 segments, 300 x 7168 18.0 / 18.3, 512 x 2048 16.8 / 17.4,
+// 512 x 7168 (3584) 19.2 / 18.9.  Not in a single launch, where neighbours of the counting workgroups wait.
+// BF16 rows that stay in the memory-side cache take the tile of the combine (kb_of_wavefront), the smallest calls too; beyond its lines tokens of three rows and more of 4, 8
 // or 12 KB take 2 KB, move and combine with 1 / 2 / 4 KB: 4096 x 2048 top-6 38.0 / 38.5 / 43.0;  6000 x 2048 top-4 42.0 / 40.9 / 45.3;  2200 x 6144
 // top-4 44.1 / 42.2 / 45.7;  3000 x 4096 expanded top-4 47.6 / 46.2 / 50.6; others the widest: 1400 x 7168 47.1 / 47.5 / 44.9, 3500 x 2560 43.7 /
 // 45.7 / 43.7, 9000 x 1400 top-4 45.5 / 45.5 / 43.2.
