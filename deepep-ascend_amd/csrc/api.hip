@@ -158,6 +158,7 @@ MoveParams shape_of_move(const deep_ep_hip_intranode_dispatch_args* a, bool with
     m.recv_sf = static_cast<uint32_t*>(a->recv_x_scales);
     m.rsf_ts = a->recv_scale_token_stride; m.rsf_hs = a->recv_scale_hidden_stride;
     m.rank_lanes = with_topk ? 0 : 1;
+    m.v1 = 1;
     set_knobs(m, a->tuning);
     return m;
 }
@@ -197,6 +198,7 @@ CombineParams shape_of_combine(const deep_ep_hip_intranode_combine_args* a) {
         m.T = p.T; m.H = p.H; m.K = p.Kw > 0 ? p.Kw : p.R; m.E = p.E; m.R = p.R; m.E_l = 1; m.M = p.T;
         m.recv_capacity = p.num_x_rows;
         m.rank_lanes = p.Kw > 0 ? 0 : 1;
+        m.v1 = 1;
         if (copies_in_one_launch(m, a->tuning)) p.shares_tile = 2;
     }
     return p;

@@ -333,7 +333,7 @@ bool reads_past_the_cache(const CombineParams& p) {
 bool takes_two_kb_tiles(const CombineParams& p) {
     const int kb = (p.H * 2 + 1023) / 1024;
     if (!reads_past_the_cache(p)) {
-        const int same = shared_tile(p.T, p.H * 2, rows_per_token(p), p.shares_tile == 2);
+        const int same = shared_tile(p.T, p.H * 2, rows_per_token(p), p.shares_tile == 2, p.rank_mode != 0);
         const bool others = p.shares_tile == 0 && int64_t(p.T) * ((kb + 1) / 2) < int64_t(compute_units()) * 18;
         if (same != 0 && !others) return same == 2;
     }

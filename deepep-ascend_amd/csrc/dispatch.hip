@@ -1536,7 +1536,7 @@ static int move_tile(const MoveParams& p) {
     const int kb = (p.row_bytes + 1023) / 1024;
     const bool rows_cached = p.payload == DEEP_EP_HIP_PAYLOAD_BF16 && cached_side(p) == kRows;
     if (rows_cached) {
-        const int same = p.fused ? kb_of_wavefront(p.T, p.row_bytes, rows, true) : shared_tile(p.T, p.row_bytes, rows, p.like_single != 0);
+        const int same = p.fused ? kb_of_wavefront(p.T, p.row_bytes, rows, true, p.v1 != 0) : shared_tile(p.T, p.row_bytes, rows, p.like_single != 0, p.v1 != 0);
         if (same != 0) return same;
     }
     if (wavefronts_per_cu_at_most(1, 8)) return 1;
@@ -1754,7 +1754,7 @@ hipError_t launch_dispatch_move(MoveParams p, hipStream_t stream) {
     p.num_cus = p.fused ? compute_units() : 0;
     const int tile = move_tile(p);
     p.row_by_row = stores_row_by_row(p) ? 1 : 0;
-    p.shared_tile = p.payload == DEEP_EP_HIP_PAYLOAD_BF16 && p.copy_vecs == 0 && kb_of_wavefront(p.T, p.row_bytes, rows_per_token(p), p.fused != 0) != 0 ? 1 : 0;
+    p.shared_tile = p.payload == DEEP_EP_HIP_PAYLOAD_BF16 && p.copy_vecs == 0 && kb_of_wavefront(p.T, p.row_bytes, rows_per_token(p), p.fused != 0, p.v1 != 0) != 0 ? 1 : 0;
     if (p.payload == DEEP_EP_HIP_PAYLOAD_CAST_FP8) {
         switch (tile) {
             case 1: return launch_cast<1>(p, stream);

@@ -179,6 +179,7 @@ struct MoveParams {
     int sf_blocked;      // recv_sf is column-major and the pad kernel follows: scales go out in blocks (below)
     int zeroed_rows;     // padding rows this call zeroes, as expected: half an alignment for each expert, or what is
                          // left of one alignment for each where an expert has fewer rows than that
+    int v1;              // a V1 call (kb_of_wavefront)
     int like_single;     // a cached handle of a single launch: its tile (kb_of_wavefront)
     int shared_tile;     // the combine has the same tile: workgroups on the XCD of its (set by the launcher)
     int row_by_row;      // a wavefront waits for the stores of a row before it starts the next (set by the launcher)
@@ -381,22 +382,23 @@ inline double distinct_ranks(int ranks, int selections) {
 // Past the lines of a single launch its combine has the tile of two launches, which a cached dispatch on the same handle has (shared_tile); behind the single
 // launch that is level with its own (950 x 7168 37.7 / 56.8 with 2 KB, 37.6 / 56.9 with 1 KB).  A combine whose rows are not those of a BF16 dispatch keeps to its own rule
 // below 18 a CU: fused cast, 1 / 2 KB, 1194 x 2944 21.4 / 22.0, 3584 x 1024 22.4 / 22.9, 192 x 4096 19.9 / 21.1; 1706 x 2944 top-4 22.2 / 21.3, 731 x 7168 25.6 / 25.8.
-// V1 handles do not say what made them; level from 8 on (FP8, 682 x 2944 34.2 / 34.3, 512 x 4096 33.2 / 33.9).
-inline int kb_of_wavefront(int64_t T, int row_bytes, double rows, bool single_launch) {
+// V1 handles do not say what made them, and the combine behind FP8 rows is ahead with 1 KB up to 8 a CU, BF16 level or ahead there: FP8, 1 / 2 KB, 200 x 7168 18.0 / 18.6, 400 x 4096
+// 19.3 / 20.0, 560 x 2048 19.6 / 19.9, 290 x 7168 20.4 / 20.8;  BF16 19.5 / 19.9, 20.3 / 21.0, 20.8 / 20.8, 21.8 / 21.9.  Level from 8 on (FP8, 682 x 2944 34.2 / 34.3, 512 x 4096 33.2 / 33.9).
+inline int kb_of_wavefront(int64_t T, int row_bytes, double rows, bool single_launch, bool v1) {
     const int kb = (row_bytes + 1023) / 1024, tiles = (kb + 1) / 2;
     const int64_t cus = compute_units(), wavefronts = T * tiles;
     if (row_bytes < tiles * 1536) return T * kb <= cus * (single_launch ? 12 : 30) && (rows >= 6.5 || !single_launch) ? 1 : 0;
     if (wavefronts > cus * (single_launch ? 22 : 30)) return 0;
     const bool many = rows >= 7.5, whole_8kb = row_bytes % 8192 == 0;
     if (single_launch && whole_8kb && !many) return wavefronts > cus * 4 && wavefronts <= cus * 6 ? 1 : 2;
-    const int one_kb_to = single_launch ? (whole_8kb ? 6 : many ? 4 : 0) : many ? 15 : whole_8kb ? 6 : 4;
+    const int one_kb_to = single_launch ? (whole_8kb ? 6 : many ? 4 : 0) : many ? 15 : v1 ? 8 : whole_8kb ? 6 : 4;
     return wavefronts <= cus * one_kb_to ? 1 : 2;
 }
 
 // The tile of the combine, and of a dispatch on the handle, where the handle is a single launch's or not.
-inline int shared_tile(int64_t T, int row_bytes, double rows, bool single_launch) {
-    const int kb = single_launch ? kb_of_wavefront(T, row_bytes, rows, true) : 0;
-    return kb != 0 ? kb : kb_of_wavefront(T, row_bytes, rows, false);
+inline int shared_tile(int64_t T, int row_bytes, double rows, bool single_launch, bool v1) {
+    const int kb = single_launch ? kb_of_wavefront(T, row_bytes, rows, true, v1) : 0;
+    return kb != 0 ? kb : kb_of_wavefront(T, row_bytes, rows, false, v1);
 }
 
 // LDS a workgroup asks for so that a CU holds at most `per_cu` of them (0: no limit).

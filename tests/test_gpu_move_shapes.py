@@ -128,7 +128,7 @@ def test_large_rows_on_a_handle():
     buf.check_device_status()
 
 
-@pytest.mark.parametrize("T,H,R,K,chosen", [(5003, 7168, 4, 4, (1, 0, 0)), (5003, 7168, 8, 4, (1, 0, 1)), (9001, 3968, 8, 3, (2, 3, 0)), (311, 7168, 8, 8, (2, 0, 0))])
+@pytest.mark.parametrize("T,H,R,K,chosen", [(5003, 7168, 4, 4, (1, 0, 0)), (5003, 7168, 8, 4, (1, 0, 1)), (9001, 3968, 8, 3, (2, 3, 0)), (292, 7168, 8, 8, (1, 0, 0)), (293, 7168, 8, 8, (2, 0, 0)), (311, 7168, 8, 8, (2, 0, 0))])
 def test_v1_rows_of_a_mask(T, H, R, K, chosen):
     """V1 calls without top-k tensors, whose routing lanes are ranks, and the same on their handle."""
     import deep_ep

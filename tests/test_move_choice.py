@@ -149,10 +149,11 @@ def test_cached_dispatch_has_the_tile_of_the_handle():
 
 
 def test_v1_tiles():
-    for T, rows, kb in ((146, 700, 1), (147, 700, 2), (1097, 5000, 2), (1098, 3000, 1), (100, 800, 2)):      # 4 and 30; a row for every rank
+    for T, rows, kb in ((146, 700, 1), (292, 1400, 1), (293, 1400, 2), (1097, 5000, 2), (1098, 3000, 1), (100, 800, 2)):      # 8 and 30; a row for every rank
         assert v1_combine(T, 7168, 8, 4, rows) == kb
     assert v1_combine(146, 7168, 8, 0, 700) == v1_move("bf16", 146, 7168, 8, 700).tile == 1
-    assert v1_combine(147, 7168, 8, 0, 700) == v1_move("bf16", 147, 7168, 8, 700).tile == 2
+    assert v1_combine(292, 7168, 8, 0, 1400) == v1_move("bf16", 292, 7168, 8, 1400).tile == 1
+    assert v1_combine(293, 7168, 8, 0, 1400) == v1_move("bf16", 293, 7168, 8, 1400).tile == 2
 
 
 def test_large_expanded_rows_of_no_whole_kb():
